@@ -195,7 +195,7 @@ LatArgs coarse_args(dnsg_t *h) {
     L.red = nullptr;
     L.force = h->d_force;
     L.dsum = nullptr;
-    L.paired = h->cs_pair ? (cs_paired(L.nx, h->elem) ? 1 : 0) | (cs_paired(L.nx, h->elem, true) ? 2 : 0) : 0;
+    L.paired = h->cs_pair && cs_paired(L.nx, L.ny, (int)h->elem);
     set_dest_weights(h, 0, &L);
     return L;
 }
@@ -220,14 +220,14 @@ void band_args(dnsg_t *h, LatArgs *L) {
         L[b].red = nullptr;
         L[b].force = h->d_force;
         L[b].dsum = nullptr;
-        L[b].paired = h->cs_pair ? (cs_paired(g.nx, h->elem) ? 1 : 0) | (cs_paired(g.nx, h->elem, true) ? 2 : 0) : 0;
+        L[b].paired = h->cs_pair && cs_paired(g.nx, g.ny, (int)h->elem);
         set_dest_weights(h, 1 + b, &L[b]);
     }
 }
 
 double *red_coarse(dnsg_t *h) { return h->red; }
 double *red_lower(dnsg_t *h) { return h->red + (size_t)h->coarse.ny * h->coarse.nz * cs_chunks(h->coarse.nx) * RED_W; }
-double *red_upper(dnsg_t *h) { return red_lower(h) + (size_t)h->lower.ny * h->lower.nz * band_cpr(h) * RED_W; }
+double *red_upper(dnsg_t *h) { return red_lower(h) + band_parts_max(h->d) * RED_W; }
 
 void rotate_levels(dnsg_t *h) {  // xcomputations.c:548-556
     // the spare (slot 3) becomes the newest level, the oldest the spare
@@ -328,7 +328,7 @@ static int sec_average(dnsg_t *h, const SecTimer &T, double *ms) {
 int do_step_band2(dnsg_t *h, double *rec, SecTimer *T) {
     const bool flux = h->p.force_mode == DNSG_FORCE_FLUX;
     const bool from_writes = flux && h->flux_fused;
-    h->band_cols = B2_TX;
+    h->band_tiled = true;
     if (T) T->start_step(h->stream);
     if (flux && !from_writes) {
         if (T) T->begin(h->stream, SEC_REDUCE);
@@ -354,7 +354,7 @@ int do_step_band2(dnsg_t *h, double *rec, SecTimer *T) {
     B[1].red = red_upper(h);
     if (flux) {
         B[0].dsum = h->dsum + 2 * (size_t)h->d.Yc * h->d.zdc * cs_chunks(h->d.Xc);
-        B[1].dsum = B[0].dsum + 2 * (size_t)h->d.Yf * (h->d.zdf - 1) * band_cpr(h);
+        B[1].dsum = B[0].dsum + band_dsum_doubles(h);
     }
     if (T) T->begin(h->stream, SEC_BAND);
     HIPCHK(h, launch_band2(h->stream, B, h->p.precision, h->halt()));
@@ -388,7 +388,7 @@ int do_step(dnsg_t *h, double *rec, SecTimer *T = nullptr) {
     // or after the state was changed from outside)
     const bool from_writes = flux && h->flux_fused;
     const int GR = h->d.GR;
-    h->band_cols = CS_THREADS;
+    h->band_tiled = false;
     if (T) T->start_step(h->stream);
     if (flux && !from_writes) {
         if (T) T->begin(h->stream, SEC_REDUCE);
@@ -396,7 +396,7 @@ int do_step(dnsg_t *h, double *rec, SecTimer *T = nullptr) {
         if (T) T->end(h->stream, SEC_REDUCE);
     }
     double *dl = h->dsum + 2 * (size_t)h->d.Yc * h->d.zdc * cs_chunks(h->d.Xc);
-    double *du = dl + 2 * (size_t)h->d.Yf * (h->d.zdf - 1) * band_cpr(h);
+    double *du = dl + band_dsum_doubles(h);
     for (int iter = 1; iter <= GR; iter++) {
         LatArgs L[3];
         LatArgs *B = L;  // the band pair of this substep
@@ -867,19 +867,19 @@ int dnsg::create_ctx(const dnsg_params *p, hipStream_t ext, dnsg_t **out) {
     }
     h->elem = p->precision == DNSG_PREC_FP64 ? 8 : (p->precision == DNSG_PREC_FP32 ? 4 : 2);
     {
-        // gratio 2: both band substeps in one pass (k_band2.hip), by default in the FP64
-        // and FP32 constant-force configurations, where it is the faster path (FP16
-        // storage and the flux controller: one launch per substep); DNSG_BAND2=1 /
-        // DNSG_BAND2=0 in the environment selects it / the one-launch-per-substep path
-        // for any configuration (the same state; the reductions' partials differ)
         // FP32 / FP16 rows of a multiple of 2 CS_THREADS nodes: the paired collide-stream
         // form (k_stream.hip), unless DNSG_CS_PAIRED=0 (the scatter form; same state)
         const char *cp = getenv("DNSG_CS_PAIRED");
         h->cs_pair = !(cp && cp[0] == '0');
+        // gratio 2: both band substeps in one pass (k_band2.hip), by default in FP64 and FP32
+        // where the lattice is large enough (band2_pays); FP16 storage keeps one launch per
+        // substep (Re_tau=180 step 0.92 against 0.94 ms).  DNSG_BAND2=1 / DNSG_BAND2=0 in the
+        // environment selects it / the one-launch-per-substep path (the same state; the
+        // reductions' partials differ)
         const char *e = getenv("DNSG_BAND2");
-        const bool pick = (p->precision == DNSG_PREC_FP64 || p->precision == DNSG_PREC_FP32) &&
-                          p->force_mode == DNSG_FORCE_CONST;
-        h->band2 = h->d.GR == 2 && ((e && e[0]) ? e[0] == '1' : pick);
+        const int elem = (int)h->elem;
+        h->band2 = h->d.GR == 2 && buf_fits(h->d.Xf, h->d.Yf, elem) &&
+                   ((e && e[0]) ? e[0] == '1' : elem != 2 && band2_pays(h->d.Xf, h->d.Yf, h->d.zdf - 1, elem));
     }
     const dnsg_dims &d = h->d;
     h->coarse.nx = d.Xc; h->coarse.ny = d.Yc; h->coarse.nz = d.zdc;
@@ -908,7 +908,7 @@ int dnsg::create_ctx(const dnsg_params *p, hipStream_t ext, dnsg_t **out) {
     HIPCHK(h, hipMalloc(&h->part, h->part_cap * 8));
     {
         const size_t nred =
-            ((size_t)d.Yc * d.zdc * cs_chunks(d.Xc) + 2 * (size_t)d.Yf * (d.zdf - 1) * band_cpr_max(h)) * RED_W;
+            ((size_t)d.Yc * d.zdc * cs_chunks(d.Xc) + 2 * band_parts_max(d)) * RED_W;
         HIPCHK(h, hipMalloc(&h->red, nred * 8));
         HIPCHK(h, hipMemsetAsync(h->red, 0, nred * 8, h->stream));
         HIPCHK(h, hipMalloc(&h->seg, enc_seg_doubles(h) * 8));

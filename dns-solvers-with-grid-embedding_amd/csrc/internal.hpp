@@ -50,7 +50,7 @@ struct LatArgs {
     // klo..khi carry kscale (khalf: half of it), all others 0.
     double *dsum;
     int klo, khi, khalf;
-    int paired;  // the paired collide-stream form (cs_paired): bit 0 in a plain launch, bit 1 in a launch with dsum
+    int paired;  // the paired collide-stream form (cs_paired)
     double kscale;
 };
 
@@ -87,23 +87,16 @@ constexpr int CS_THREADS = DNSG_CS_THREADS;
 __host__ __device__ __forceinline__ int cs_chunks(int nx) { return (nx + CS_THREADS - 1) / CS_THREADS; }
 // lattices narrower than a workgroup: each workgroup takes this many whole rows
 __host__ __device__ __forceinline__ int cs_rows_per_wg(int nx) { return nx >= CS_THREADS ? 1 : CS_THREADS / nx; }
-// Paired collide-stream form (mask bit 0 FP64, bit 1 FP32, bit 2 FP16): rows that are
-// a multiple of 2 CS_THREADS nodes are taken two chunks per workgroup, two adjacent
-// nodes per thread, with 2-value loads and stores.  Measured on the Re_tau=180
-// lattices: FP32 coarse launch 0.956 -> 0.852 ms, FP16 0.599 -> 0.586 ms; FP64 with
-// pairs 0.97 ms against 0.94 ms in the aligned one-node form, so FP64 keeps that.
-// Launches that also sum their writes for the flux controller (LatArgs::dsum) use
-// DNSG_CS_PAIRED_DS_MASK: there FP64 pairs measured faster (the Re_tau=180 band
-// launch 1.032 -> 0.937 ms, the coarse one 1.936 -> 1.898 ms).
-#ifndef DNSG_CS_PAIRED_MASK
-#define DNSG_CS_PAIRED_MASK 6
-#endif
-#ifndef DNSG_CS_PAIRED_DS_MASK
-#define DNSG_CS_PAIRED_DS_MASK 7
-#endif
-__host__ __device__ __forceinline__ bool cs_paired(int nx, int elem, bool ds = false) {
-    const int bit = elem == 8 ? 1 : (elem == 4 ? 2 : 4);
-    return ((ds ? DNSG_CS_PAIRED_DS_MASK : DNSG_CS_PAIRED_MASK) & bit) != 0 && nx % (2 * CS_THREADS) == 0;
+// a layer can be addressed with 31-bit byte offsets (the buffer-resource forms)
+__host__ __device__ __forceinline__ bool buf_fits(int nx, int ny, int elem) {
+    return (size_t)nx * ny * 19 * elem < ((size_t)1 << 31);
+}
+// Paired collide-stream form: rows of FP32 / FP16 values that are a multiple of 2
+// CS_THREADS nodes are taken two chunks per workgroup, two adjacent nodes per thread, with
+// 2-value loads and stores.  Measured on the Re_tau=180 lattices against one node per
+// thread: FP32 coarse launch 0.956 -> 0.852 ms, FP16 0.599 -> 0.586 ms.
+__host__ __device__ __forceinline__ bool cs_paired(int nx, int ny, int elem) {
+    return elem != 8 && nx % (2 * CS_THREADS) == 0 && buf_fits(nx, ny, elem);
 }
 // collide-stream workgroups of one lattice with `rows` rows of nx nodes
 __host__ __device__ __forceinline__ int cs_blocks(int nx, int rows, bool paired) {
@@ -123,10 +116,21 @@ struct Grid {
     void swap() { cur ^= 1; }
 };
 
-// Columns per tile of the two-substep band kernel (k_band2.hip).  When a step runs
-// it, the bands' fused-reduction partials (LatArgs::red, ::dsum) are per (layer, row,
-// B2_TX columns) instead of per CS_THREADS columns; dnsg_ctx::band_cols says which.
-constexpr int B2_TX = 64;
+// Tile of the two-substep band kernel (k_band2.hip): rows of a workgroup (ring
+// included), nodes per lane and output columns for elements of `elem` bytes.  When a
+// step runs it (dnsg_ctx::band_tiled), the bands' fused-reduction partials are per
+// (row, b2_cols columns) instead of per (layer, row, CS_THREADS columns), with the layer
+// weights applied: LatArgs::dsum the pair above, LatArgs::red the B2_RED values
+//   [0], [1] sum of rho, rho u_x weighted by encalc2's layer weights
+//   [2]      sum of rho over the layer whose density wshearstr takes
+//   [3..5]   sum of u_x over the three layers next to the wall, nearest first
+constexpr int B2_RED = 6;
+#ifndef DNSG_B2_ROWS
+#define DNSG_B2_ROWS 12
+#endif
+constexpr int B2_ROWS = DNSG_B2_ROWS;
+constexpr int b2_npl(int elem) { return elem == 8 ? 1 : 2; }
+constexpr int b2_cols(int elem) { return 62 * b2_npl(elem); }
 
 // number of doubles in one diag record written by the reduction finalisers
 constexpr int DIAG_WORDS = 9;
@@ -153,10 +157,10 @@ struct dnsg_ctx {
     // the step's wall-stress check has passed
     void *lev_lo[4] = {nullptr, nullptr, nullptr, nullptr};
     void *lev_up[4] = {nullptr, nullptr, nullptr, nullptr};
-    // the steps use the two-substep band kernel (gratio 2); band_cols: columns per
-    // fused-reduction partial in the bands' partials of the last launch that wrote them
+    // the steps use the two-substep band kernel (gratio 2); band_tiled: the bands'
+    // fused-reduction partials of the last launch that wrote them are that kernel's
     bool band2 = false;
-    int band_cols = dnsg::CS_THREADS;
+    bool band_tiled = false;
     bool cs_pair = true;  // FP32 / FP16: the paired collide-stream form where the rows allow it
     int8_t *wall_lo = nullptr, *wall_up = nullptr;     // [Yf][Xf]
 
@@ -210,10 +214,22 @@ struct dnsg_ctx {
 
 namespace dnsg {
 
-// fused-reduction partials per (layer, row) of a band: in the current layout, and
-// the most any layout needs (the buffers are sized for it)
-inline int band_cpr(const dnsg_ctx *h) { return (h->d.Xf + h->band_cols - 1) / h->band_cols; }
-inline int band_cpr_max(const dnsg_ctx *h) { return (h->d.Xf + B2_TX - 1) / B2_TX; }
+// fused-reduction partials per row of a band (and layer, where not band_tiled) in the
+// current layout, and the partials of RED_W values a band's buffer is sized for in
+// either layout
+inline int band_cpr(const dnsg_ctx *h) {
+    const int cols = h->band_tiled ? b2_cols((int)h->elem) : CS_THREADS;
+    return (h->d.Xf + cols - 1) / cols;
+}
+inline size_t band_parts_max(const dnsg_dims &d) {
+    const size_t b2 = (size_t)d.Yf * ((d.Xf + b2_cols(8) - 1) / b2_cols(8)) * (B2_RED / RED_W);
+    const size_t cs = (size_t)d.Yf * (d.zdf - 1) * cs_chunks(d.Xf);
+    return b2 > cs ? b2 : cs;
+}
+// doubles from the lower band's dsum partials to the upper band's
+inline size_t band_dsum_doubles(const dnsg_ctx *h) {
+    return 2 * (size_t)h->d.Yf * (h->band_tiled ? 1 : h->d.zdf - 1) * band_cpr(h);
+}
 
 // handle set-up and the per-step argument builders shared by the single-solve
 // step and the serving queue
@@ -229,10 +245,12 @@ void rotate_levels(dnsg_t *h);
 hipError_t launch_collide_stream(hipStream_t s, const LatArgs *lats, int nlat, int prec, const int *halt = nullptr);
 // both gratio-2 band substeps of one coarse step in one pass (k_band2.hip): bands[0]
 // the lower band, bands[1] the upper band, as band_args builds them; the first fill
-// must already be in their nxt lattices' interface layers; red / dsum in the B2_TX
-// partial layout
+// must already be in their nxt lattices' interface layers; red / dsum in its own
+// partial layout (B2_RED)
 hipError_t launch_band2(hipStream_t s, const LatArgs *bands, int prec, const int *halt = nullptr);
-int band2_tiles(int nx, int ny, int prec);
+int band2_tiles(int nx, int ny, int elem);
+// the one-pass path is the faster one for a handle's two bands of nx x ny x nz nodes
+bool band2_pays(int nx, int ny, int nz, int elem);
 hipError_t launch_init_lattice(hipStream_t s, dnsg_ctx *h, int grid, void *dst);
 // gl = 1: the host array carries one ghost x-plane and y-row (the reference's in-memory
 // layout); downloads write them as periodic images

@@ -9,16 +9,18 @@
 // fill reads only the interface planes.  So the fill runs first, into the output
 // lattice's interface layer, and one workgroup then carries a tile of the band
 // through both substeps, keeping the intermediate state on chip:
-//   * a tile is 64 x-consecutive columns (one wave per row) by 4 rows (FP64) or 8
-//     rows (FP32, FP16), all layers;
+//   * a workgroup has NR waves, one per row of the tile and its ring; a lane holds NPL
+//     adjacent nodes of its row.  The first substep is collided on all 64 NPL columns
+//     and NR rows, the second on all but the outermost lane and row on each side (the
+//     ring), so a tile is 62 NPL columns by NR - 2 rows, all layers;
 //   * the workgroup marches through the layers from the interface towards the wall.
-//     At layer t it loads and collides the first substep's input on the tile and a
-//     one-node ring around it (the rows above and below, one wave each, and the
-//     columns left and right, one extra wave); then it gathers the first substep's
-//     streamed values of layer t-1 -- along a row by wave shuffles, across rows and
-//     from the ring columns through LDS, across layers from what earlier
-//     iterations kept -- collides them again (the second substep) and pushes the
-//     result to its targets in the output lattice with the wall rules;
+//     At layer t it collides the first substep's input and puts the 18 streamed
+//     values of each node into LDS; after a barrier every node of the tile takes the
+//     values that arrive at it from layer t toward the interface, has everything that
+//     streams into layer t-1 (the rest was kept in registers from earlier layers),
+//     collides that again (the second substep) and pushes the result to its targets
+//     in the output lattice with the wall rules; then it takes the values that stay in
+//     layer t or go on toward the wall out of LDS, and a second barrier frees it;
 //   * the interface layer (t = 0) takes the first fill's values from the output
 //     lattice; the layer next to the wall (t = nz-1) takes its values coming from
 //     the wall by the wall rules in pull form: for a direction b leaving the wall,
@@ -31,10 +33,11 @@
 // from 2 x (19 reads + 19 writes) to 19 reads (+ the ring, largely from L2) and 19
 // writes.
 //
-// The same launch sums the first substep's pre-collision moments per (row, tile
-// column) for encalc2 / wshearstr (LatArgs::red) and, in flux mode, the
-// destination-weighted sums of the second substep's writes (LatArgs::dsum), both in
-// the 64-column partial layout (B2_TX).
+// The same launch sums, per row and tile of b2_cols() columns, the first substep's
+// pre-collision moments for encalc2 and wshearstr (LatArgs::red, B2_RED doubles) or, in
+// flux mode, the destination-weighted sums of the second substep's writes
+// (LatArgs::dsum, 2 doubles) beside the wall-stress part.  A lane adds up its layers and
+// a wave reduces once per tile: reduced at every layer, the sums took 4% of the launch.
 #include <algorithm>
 
 #include "internal.hpp"
@@ -45,19 +48,13 @@ namespace dnsg {
 
 namespace {
 
-constexpr int TX = B2_TX;          // columns per tile = lanes per row wave
-constexpr int CW = TX + 2;         // LDS columns: left ring column, the tile's 64, right ring column
-// Output rows per tile.  The workgroup has a row wave per tile row, one for the ring
-// row above and one for the ring row below, and one wave for the ring columns; a CU
-// holds one workgroup (LDS).  FP64 needs 240 VGPRs, two waves per SIMD: 4 rows, 7
-// waves.  FP32 and FP16 need 160, three waves per SIMD: 8 rows, 11 waves (9 rows,
-// 12 waves, measured slower).
+constexpr int NR = B2_ROWS;  // rows of a workgroup, ring included: one wave each
+constexpr int TY = NR - 2;   // output rows of a tile
+constexpr int B2_THREADS = 64 * NR;
 template <class S>
-constexpr int tile_rows() { return sizeof(S) == 8 ? 4 : 8; }
+constexpr int npl() { return b2_npl(sizeof(S)); }  // nodes per lane
 template <class S>
-constexpr int row_waves() { return tile_rows<S>() + 2; }
-template <class S>
-constexpr int wg_threads() { return 64 * (row_waves<S>() + 1); }
+constexpr bool early() { return sizeof(S) == 8; }  // when the next layer is loaded (band2_tile)
 
 // March coordinate t: 0 at the interface layer, nz-1 next to the wall.  A direction
 // moves t by ez for the upper band (interface = stored layer 0) and by -ez for the
@@ -67,306 +64,394 @@ constexpr int ezt(int q) { return SIDE ? EZ[q] : -EZ[q]; }
 // class of a direction: 0 along the layer, 1 toward the wall, 2 toward the interface
 template <int SIDE>
 constexpr int cls(int q) { return ezt<SIDE>(q) == 0 ? 0 : (ezt<SIDE>(q) > 0 ? 1 : 2); }
-// directions with e_y = 0, register slot within their class: 0 e_x = 0, 1 e_x = +1, 2 e_x = -1
-constexpr int xi(int q) { return EX[q] == 0 ? 0 : (EX[q] > 0 ? 1 : 2); }
-// directions with e_y != 0, LDS slot within their class: along the layer q = 3, 4, 7,
-// 8, 9, 10 -> 0..5; out of the layer e_y = +1 -> 0, e_y = -1 -> 1
-constexpr int yi(int q) {
-    return q == 3 ? 0 : q == 4 ? 1 : q == 7 ? 2 : q == 8 ? 3 : q == 9 ? 4 : q == 10 ? 5 : (EY[q] > 0 ? 0 : 1);
+// register slot of a direction within its class: along the layer (EZ = 0) q = 0..4 ->
+// 0..4, 7..10 -> 5..8; out of the layer by in-plane offset
+constexpr int slot(int q) {
+    if (EZ[q] == 0) return q < 5 ? q : q - 2;
+    return EX[q] > 0 ? 1 : EX[q] < 0 ? 2 : EY[q] > 0 ? 3 : EY[q] < 0 ? 4 : 0;
 }
 
-// Post-collision values of the first substep that cross waves.  y*: directions with
-// e_y != 0, by row and column; h*: ring columns, e_y = 0 directions pointing into
-// the tile (left column: e_x = +1, right column: e_x = -1), by row.  Layer slots:
-// along the layer t & 1 (read one iteration later), toward the wall t % 3 (read two
-// iterations later), toward the interface one (read in the same iteration); two
-// barriers per iteration separate the writes of a layer from the reads of older ones.
-template <class T, int NR>
-struct Lds {
-    T yf[2][6][NR][CW];
-    T yu[3][2][NR][CW];
-    T yd[2][NR][CW];
-    T hf[2][NR][2];
-    T hu[3][NR][2];
-    T hd[NR][2];
-    int8_t wcl[NR][CW];  // the tile's wall codes, ring included
-};
+// LDS plane of a direction: 10 out of the layer, then 8 along it, which are kept twice
+// (even and odd layers): those of a layer are read one layer later
+constexpr int plane(int q) { return EZ[q] != 0 ? (q < 7 ? q - 5 : q - 9) : (q < 5 ? q + 9 : q + 7); }
+constexpr int ALONG = 8, NPLANES = 10 + 2 * ALONG;
 
-// wall codes of scatter_push from the tile's LDS copy: the node at row wave r, LDS
-// column col, and its in-plane neighbours
-struct WallCodesTile {
-    const int8_t (*w)[CW];
-    int r, col;
-    __device__ __forceinline__ int operator()(int, int dx, int dy, int, int) const { return w[r + dy][col + dx]; }
-};
-
+// NPL adjacent values of a lane: one value (FP64) or a pair
+__device__ __forceinline__ void load_n(Rsrc R, unsigned v, unsigned s, const double *p, double (&o)[1]) { o[0] = buf_load(R, v, s, p); }
 template <class S>
-__device__ __forceinline__ typename ComputeOf<S>::T rest_value(int q) {
-    // a harmless stand-in for lanes outside the lattice (rho = 1, u = 0)
-    if constexpr (sizeof(S) == 8) return WQ[q];
-    else return 0.f;
-}
+__device__ __forceinline__ void load_n(Rsrc R, unsigned v, unsigned s, const S *p, float (&o)[2]) { buf_load_pair(R, v, s, p, o[0], o[1]); }
 
 template <class S, int SIDE, bool DS>
-__device__ __forceinline__ void band2_tile(const LatArgs &L, int tile,
-                                           Lds<typename ComputeOf<S>::T, row_waves<S>()> &sm) {
+__device__ __forceinline__ void band2_tile(const LatArgs &L, int tile, typename ComputeOf<S>::T *lds, int8_t *wcl) {
     using T = typename ComputeOf<S>::T;
-    constexpr int TY = tile_rows<S>(), NR = row_waves<S>();
+    constexpr int NPL = npl<S>(), CW = 64 * NPL, OX = 62 * NPL;
+    auto each_n = [](auto &&f) __attribute__((always_inline)) { unroll<0, NPL>(f); };
     const int nx = L.nx, ny = L.ny, nz = L.nz;
-    const int tilesx = (nx + TX - 1) / TX;
+    const int tilesx = (nx + OX - 1) / OX;
     const int tx = tile % tilesx, ty = tile / tilesx;
-    const int x0 = tx * TX, y0 = ty * TY;
-    const int w = min(TX, nx - x0), th = min(TY, ny - y0), nrows = th + 2;
-    // the wave index as a scalar, so that the compiler sees branches on it as uniform
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
-    const int cpr = tilesx;  // partials per (layer, row)
+    const int x0 = tx * OX, y0 = ty * TY;
+    const int w = min(OX, nx - x0), th = min(TY, ny - y0);
+    // the wave index as a scalar: row addresses and row conditions are wave-uniform
+    const int r = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
     const S *__restrict__ cur = static_cast<const S *>(L.cur);
     S *__restrict__ nxt = static_cast<S *>(L.nxt);
     const T G = (T)(L.gscale * L.force[0]);
     const T om = (T)L.omega;
     const int8_t *__restrict__ wc = SIDE ? L.whi : L.wlo;
-    // this thread's node: row wave r, column x (ring wave: ring row r, left or right column)
-    const bool ringw = wave == NR;
-    const int r = ringw ? (lane >> 1) : wave;
-    const int sd = lane & 1;
-    const bool rowok = r < nrows && (!ringw || lane < 2 * NR);
-    const int y = ((y0 - 1 + r) % ny + ny) % ny;
-    const int x = ringw ? (sd ? (x0 + w) % nx : (x0 - 1 + nx) % nx) : x0 + lane;
-    const bool act = rowok && (ringw || lane < w);
-    const int col = ringw ? (sd ? w + 1 : 0) : lane + 1;
-    const bool core = !ringw && r >= 1 && r <= th;
-    // in-row values kept across iterations: along the layer (layer t-1, layer t),
-    // toward the wall (t-2, t-1, t), toward the interface (t)
-    T fprv[3] = {0, 0, 0}, fcur[3] = {0, 0, 0};
-    T uprv2[3] = {0, 0, 0}, uprv[3] = {0, 0, 0}, ucur[3] = {0, 0, 0};
-    T dcur[3] = {0, 0, 0};
+    const bool rowok = r < th + 2, core_row = r >= 1 && r <= th;
+    const int ya = y0 - 1 + r, y = ya < 0 ? ya + ny : (ya >= ny ? ya - ny : ya);
+    const int ym = y == 0 ? ny - 1 : y - 1, yp = y == ny - 1 ? 0 : y + 1;
+    // this lane's first column; lanes past the right ring column repeat it
+    const int lc = min(lane, w / NPL + 1);
+    const int xa = x0 - NPL + NPL * lc, x = xa < 0 ? xa + nx : (xa >= nx ? xa - nx : xa);
+    const bool core = core_row && lane >= 1 && lane <= w / NPL;
+    // byte offsets in a row: this lane's nodes (loads), and the targets of e_x = 0, +1, -1
+    constexpr unsigned ES = sizeof(S);
+    const unsigned vx = (unsigned)x * ES;
+    const unsigned vs0 = core ? vx : DROP;
+    unsigned vsp = DROP, vsm = DROP;
+    if (core && (NPL == 1 || x + NPL != nx)) vsp = x + 1 == nx ? 0 : vx + ES;
+    if (core && (NPL == 1 || x != 0)) vsm = x == 0 ? (unsigned)(nx - 1) * ES : vx - ES;
+    // a pair of targets across the periodic edge is stored one value at a time
+    const bool edge = NPL == 2 && (x0 == 0 || x0 + w == nx);
+    const bool ep = core && x + NPL == nx, em = core && x == 0;
+    const unsigned layer_bytes = (unsigned)ny * Q * nx * ES;
+    auto soff = [&](int yy, int q) { return (unsigned)(yy * Q + q) * nx * ES; };  // row and direction within a layer
+    // LDS: plane q-1 of [NR][CW]; this lane's place in it
+    T *const me = lds + r * CW + NPL * lane;
+    constexpr int PL = NR * CW;
 
-    // gather and collide the second substep at layer t into g (core row waves only)
-    auto second = [&](int t, bool wall, T *g) __attribute__((always_inline)) {
+    T fin[NPL][Q];                       // first-substep input of the next layer
+    T q0[NPL];                           // rest direction of layer t-1
+    T wo[NPL][5], wn[NPL][5];            // arrived toward the wall: from layer t-2, t-1
+    double srho = 0., smom = 0.;         // layer-weighted sums of the first substep's input (encalc2)
+    double sdm = 0., sdd = 0.;           // ... and of the second substep's writes (flux controller)
+    each_n([&](auto nc) {
+        constexpr int n = decltype(nc)::value;
+        q0[n] = T(0);
+#pragma unroll
+        for (int k = 0; k < 5; k++) wo[n][k] = wn[n][k] = T(0);
+    });
+
+    auto layer_rsrc = [&](const S *lat, int t) {
+        return buf_rsrc(lat + (size_t)(SIDE ? t : nz - 1 - t) * ny * Q * nx, layer_bytes);
+    };
+    auto load_q = [&](Rsrc R, int q, T (&v)[NPL]) __attribute__((always_inline)) { load_n(R, vx, soff(y, q), cur, v); };
+    auto load_layer = [&](Rsrc R, T (&f)[NPL][Q]) __attribute__((always_inline)) {
+        unroll<0, Q>([&](auto qc) {
+            constexpr int q = decltype(qc)::value;
+            T v[NPL];
+            load_q(R, q, v);
+            each_n([&](auto nc) { constexpr int n = decltype(nc)::value; f[n][q] = v[n]; });
+        });
+    };
+    // value of direction q arriving at node n of this lane, from the layer whose values are
+    // at m (me, for the directions along a layer plus that layer's copy)
+    auto arrive = [&](auto qc, int n, const T *m) {
+        constexpr int q = decltype(qc)::value;
+        return m[plane(q) * PL - EY[q] * CW + n - EX[q]];
+    };
+    auto collide_all = [&](T (&g)[NPL][Q]) __attribute__((always_inline)) {
+        unroll<0, NPL>([&](auto nc) { collide_any(g[decltype(nc)::value], G, om); });
+    };
+
+    // push of the second substep's result at layer t
+    auto push = [&](int t, const T (&g)[NPL][Q]) __attribute__((always_inline)) {
         const int m = SIDE ? t : nz - 1 - t;
-        const size_t row = (size_t)m * ny + y;
-        if (t == 0) {  // the interface layer: the first fill's values
-            // the addresses are formed here, not kept from the kernel's start: they are
-            // loop-invariant, and holding 19 of them through the march spills registers
-            const S *fill = nxt + lat_at(0, row, x, nx);
-            asm volatile("" : "+v"(fill));
-            unroll<0, Q>([&](auto qc) {
-                constexpr int q = decltype(qc)::value;
-                g[q] = act ? (T)load_s(fill + (size_t)q * nx) : rest_value<S>(q);
-            });
-        } else {
-            const int sf = t & 1, su = (t - 1) % 3, sw = t % 3;
-            unroll<0, Q>([&](auto qc) {
-                constexpr int q = decltype(qc)::value;
-                constexpr int c = cls<SIDE>(q);
-                if constexpr (c == 2) {
-                    if (wall) {  // from the wall: the wall rules (below)
-                        g[q] = T(0);
-                        return;
-                    }
-                }
-                if constexpr (EY[q] == 0) {
-                    constexpr int k = xi(q);
-                    const T v = c == 0 ? fprv[k] : (c == 1 ? uprv2[k] : dcur[k]);
-                    if constexpr (EX[q] == 0) {
-                        g[q] = v;
-                    } else if constexpr (EX[q] > 0) {
-                        const T s = __shfl_up(v, 1, 64);
-                        const T hv = c == 0 ? sm.hf[sf][r][0] : (c == 1 ? sm.hu[su][r][0] : sm.hd[r][0]);
-                        g[q] = lane == 0 ? hv : s;
-                    } else {
-                        const T s = __shfl_down(v, 1, 64);
-                        const T hv = c == 0 ? sm.hf[sf][r][1] : (c == 1 ? sm.hu[su][r][1] : sm.hd[r][1]);
-                        g[q] = lane == w - 1 ? hv : s;
-                    }
+        double sd[3] = {0., 0., 0.}, sx[3] = {0., 0., 0.};  // per class: sums of f and of e_x f
+        auto put = [&](Rsrc R, auto qc) {  // R: the target layer
+            constexpr int q = decltype(qc)::value;
+            const unsigned so = soff(EY[q] > 0 ? yp : (EY[q] < 0 ? ym : y), q);
+            const unsigned vo = EX[q] > 0 ? vsp : (EX[q] < 0 ? vsm : vs0);
+            if constexpr (NPL == 1) {
+                buf_store<0>(R, vo, so, nxt, g[0][q]);
+            } else {
+                // e_x = +-1: a dword-aligned 8-byte store in FP32; FP16 has no such store, so two
+                if constexpr (EX[q] == 0 || sizeof(S) == 4) {
+                    buf_store_pair<0>(R, vo, so, nxt, g[0][q], g[1][q]);
                 } else {
-                    constexpr int j = yi(q);
-                    const int rs = r - EY[q], cs = lane + 1 - EX[q];
-                    if constexpr (c == 0) g[q] = sm.yf[sf][j][rs][cs];
-                    else if constexpr (c == 1) g[q] = sm.yu[su][j][rs][cs];
-                    else g[q] = sm.yd[j][rs][cs];
+                    buf_store<0>(R, vo, so, nxt, g[0][q]);
+                    buf_store<0>(R, vo == DROP ? DROP : vo + ES, so, nxt, g[1][q]);
                 }
-            });
-            if (wall) {
-                // directions leaving the wall (toward the interface) at the layer next to
-                // it, from that layer's toward-the-wall values (layer t, slot sw, uprv)
-                const int own = act ? (int)sm.wcl[r][col] : 0;
-                unroll<0, Q>([&](auto qc) {
-                    constexpr int b = decltype(qc)::value;
-                    if constexpr (cls<SIDE>(b) == 2) {
-                        constexpr int ebx = EX[b], eby = EY[b];
-                        const bool bb = act && own == -1 && sm.wcl[r - eby][col - ebx] == -1;
-                        T vbb, vsp;
-                        if constexpr (eby == 0) {
-                            vbb = uprv[xi(OPP[b])];
-                            const T v = uprv[xi(MIR[b])];
-                            if constexpr (ebx == 0) {
-                                vsp = v;
-                            } else if constexpr (ebx > 0) {
-                                const T s = __shfl_up(v, 1, 64);
-                                vsp = lane == 0 ? sm.hu[sw][r][0] : s;
-                            } else {
-                                const T s = __shfl_down(v, 1, 64);
-                                vsp = lane == w - 1 ? sm.hu[sw][r][1] : s;
-                            }
-                        } else {
-                            vbb = sm.yu[sw][yi(OPP[b])][r][lane + 1];
-                            vsp = sm.yu[sw][yi(MIR[b])][r - eby][lane + 1 - ebx];
-                        }
-                        g[b] = bb ? vbb : vsp;
+                if constexpr (EX[q] != 0) {
+                    if (edge) {
+                        const bool e = EX[q] > 0 ? ep : em;
+                        buf_store<0>(R, e ? (unsigned)(nx - 1) * ES : DROP, so, nxt, g[0][q]);
+                        buf_store<0>(R, e ? 0u : DROP, so, nxt, g[1][q]);
                     }
+                }
+            }
+            if constexpr (DS) {
+                each_n([&](auto nc) {
+                    constexpr int n = decltype(nc)::value;
+                    const double v = read_back<S, q>(g[n][q]);
+                    sd[cls<SIDE>(q)] += v;
+                    if constexpr (EX[q] > 0) sx[cls<SIDE>(q)] += v;
+                    if constexpr (EX[q] < 0) sx[cls<SIDE>(q)] -= v;
                 });
             }
+        };
+        if (t >= 1) {  // along the interface layer: rewritten by the next fill
+            const Rsrc R = layer_rsrc(nxt, t);
+            unroll<0, Q>([&](auto qc) {
+                if constexpr (cls<SIDE>(decltype(qc)::value) == 0) put(R, qc);
+            });
         }
-        collide_any(g, G, om);
-    };
-    // push the second substep's result at layer t to its targets
-    auto push = [&](int t, const T *g) __attribute__((always_inline)) {
-        const int m = SIDE ? t : nz - 1 - t;
-        const size_t row = (size_t)m * ny + y;
-        RowSums rs;
-        if (act) scatter_push<S, DS>(L, nxt, (int)row, x, g, rs, WallCodesTile{sm.wcl, r, col});
-        if (DS && L.dsum) {
-            const double dm = wave_sum64(rs.dm), dd = wave_sum64(rs.dd);
-            if (lane == 0) {
-                const size_t e = row * cpr + tx;
-                L.dsum[2 * e] = dm;
-                L.dsum[2 * e + 1] = dd;
+        if (t >= 2) {  // into the interface layer (t = 1) or out of the band (t = 0): not written
+            const Rsrc R = layer_rsrc(nxt, t - 1);
+            unroll<0, Q>([&](auto qc) {
+                if constexpr (cls<SIDE>(decltype(qc)::value) == 2) put(R, qc);
+            });
+        }
+        if (t < nz - 1) {
+            const Rsrc R = layer_rsrc(nxt, t + 1);
+            unroll<0, Q>([&](auto qc) {
+                if constexpr (cls<SIDE>(decltype(qc)::value) == 1) put(R, qc);
+            });
+        } else if (core) {
+            // onto the wall (xfcomputations.c:230-239): halfway bounce-back where both wall
+            // cells are no-slip, else specular reflection
+            unroll<0, Q>([&](auto qc) {
+                constexpr int q = decltype(qc)::value;
+                if constexpr (cls<SIDE>(q) == 1) {
+                    const int yt = EY[q] > 0 ? yp : (EY[q] < 0 ? ym : y);
+                    unroll<0, NPL>([&](auto nc) {
+                        constexpr int n = decltype(nc)::value;
+                        const int c = NPL * lane + n;
+                        const bool bb = wcl[r * CW + c] == -1 && wcl[(r + EY[q]) * CW + c + EX[q]] == -1;
+                        const int xn = x + n, xt = EX[q] > 0 ? (xn + 1 == nx ? 0 : xn + 1)
+                                                             : (EX[q] < 0 ? (xn == 0 ? nx - 1 : xn - 1) : xn);
+                        if (bb) store_s(nxt + lat_at(OPP[q], (size_t)m * ny + y, xn, nx), g[n][q]);
+                        else store_s(nxt + lat_at(MIR[q], (size_t)m * ny + yt, xt, nx), g[n][q]);
+                        if constexpr (DS) {  // lands in this layer
+                            const double v = read_back<S, q>(g[n][q]);
+                            sd[0] += v;
+                            if constexpr (EX[q] > 0) sx[0] += bb ? -v : v;
+                            if constexpr (EX[q] < 0) sx[0] += bb ? v : -v;
+                        }
+                    });
+                }
+            });
+        }
+        if constexpr (DS) {
+            if (core) {
+                constexpr int up = SIDE ? 1 : -1;  // stored-layer step toward the wall
+                const double w0 = dest_w(L, m), w1 = t < nz - 1 ? dest_w(L, m + up) : 0., w2 = t >= 1 ? dest_w(L, m - up) : 0.;
+                sdm += w0 * sx[0] + w1 * sx[1] + w2 * sx[2];
+                sdd += w0 * sd[0] + w1 * sd[1] + w2 * sd[2];
             }
         }
     };
 
-    // the first substep's input of a layer, loaded one layer ahead: the loads of layer
-    // t+1 are issued at the top of iteration t and waited for just before the second
-    // substep's stores (below), so they overlap both collisions.  The loads are
-    // unconditional, so no join between lanes or waves waits for them: lanes without
-    // a node read the tile's first ring node, whose cache lines lane 0 of the first
-    // row wave fetches anyway, and take rest values at use.
-    const int yl = act ? y : ((y0 - 1) % ny + ny) % ny, xl = act ? x : x0;
-    T fin[Q];
-    auto load_layer = [&](int t) __attribute__((always_inline)) {
-        const size_t row = (size_t)(SIDE ? t : nz - 1 - t) * ny + yl;
-        unroll<0, Q>([&](auto qc) {
-            constexpr int q = decltype(qc)::value;
-            fin[q] = (T)load_s(cur + lat_at(q, row, xl, nx));
-        });
-    };
-    // the tile's wall codes, read at the layer next to the wall
-    if (act) sm.wcl[r][col] = wc[(size_t)y * nx + x];
-    load_layer(0);
-    __builtin_amdgcn_s_waitcnt(0x0F70);  // the first layer is waited for on entry
+    if (rowok) {
+        if (NPL * lane < w + 2 * NPL)  // the tile's wall codes, ring included
+            each_n([&](auto nc) { constexpr int n = decltype(nc)::value; wcl[r * CW + NPL * lane + n] = wc[(size_t)y * nx + x + n]; });
+        load_layer(layer_rsrc(cur, 0), fin);
+    }
+    double *const rec = L.red ? L.red + ((size_t)y * tilesx + tx) * B2_RED : nullptr;
     for (int t = 0; t < nz; t++) {
-        // ---- first substep at layer t: load, sum, collide, share
-        const int m = SIDE ? t : nz - 1 - t;
-        const size_t row = (size_t)m * ny + y;
-        T f[Q];
-        unroll<0, Q>([&](auto qc) {
-            constexpr int q = decltype(qc)::value;
-            f[q] = act ? fin[q] : rest_value<S>(q);
-        });
-        if (t + 1 < nz) load_layer(t + 1);
+        T *const me0 = me + (t & 1) * ALONG * PL;               // along-layer copy of layer t
+        const T *const me1 = me + ((t & 1) ^ 1) * ALONG * PL;   // ... of layer t-1
+        // The next layer's loads: issued here, before this layer's collision, in FP64, so
+        // they have the whole iteration to arrive (Re_tau=180 launch 1.250 -> 1.203 ms);
+        // in FP32 and FP16, whose two nodes per lane would spill (0.749 -> 0.812 ms), after
+        // it, into the registers it frees.
+        T f[NPL][Q];
+        T(&F)[NPL][Q] = early<S>() ? f : fin;
+        if constexpr (early<S>()) {
+            unroll<0, Q>([&](auto qc) {
+                constexpr int q = decltype(qc)::value;
+                each_n([&](auto nc) { f[decltype(nc)::value][q] = fin[decltype(nc)::value][q]; });
+            });
+            if (rowok && t + 1 < nz) load_layer(layer_rsrc(cur, t + 1), fin);
+            __builtin_amdgcn_sched_barrier(0);
+        }
         if (rowok) {
-            if (core && L.red) {
-                RowSums rs;
-                if (act) rs.add<S>(f);
-                const double a = wave_sum64(rs.rho), b = wave_sum64(rs.mom), c = wave_sum64(rs.u);
-                if (lane == 0) {
-                    double *p = L.red + (row * cpr + tx) * RED_W;
-                    p[0] = a;
-                    p[1] = b;
-                    p[2] = c;
+            // ---- first substep at layer t: collide, sum, share
+            PreSums<T> ps[NPL];
+            each_n([&](auto nc) { ps[decltype(nc)::value] = collide_any(F[decltype(nc)::value], G, om); });
+            if (L.red) {
+                const double wt = DS ? 0. : dest_w(L, SIDE ? t : nz - 1 - t);  // flux control: encalc2 comes from the writes
+                if (wt != 0. && core)
+                    each_n([&](auto nc) {
+                        srho += wt * pre_rho(ps[decltype(nc)::value]);
+                        smom += wt * (double)ps[decltype(nc)::value].mx;
+                    });
+                if (t >= nz - 3 && core_row) {  // the layers of the wall-stress stencil
+                    double u = 0., d = 0.;
+                    if (core)
+                        each_n([&](auto nc) {
+                            u += pre_u(ps[decltype(nc)::value]);
+                            d += pre_rho(ps[decltype(nc)::value]);
+                        });
+                    u = wave_sum64(u);
+                    if (lane == 0) rec[3 + (nz - 1 - t)] = u;
+                    if (t == (SIDE ? nz - 3 : nz - 1)) {
+                        d = wave_sum64(d);
+                        if (lane == 0) rec[2] = d;
+                    }
                 }
             }
-            collide_any(f, G, om);
-            if constexpr (sizeof(S) == 2) {
+            each_n([&](auto nc) {
+                constexpr int n = decltype(nc)::value;
                 // FP16 storage: one launch per substep stores this result in FP16 and the
                 // second substep reads it back; round it the same way here
-                unroll<0, Q>([&](auto qc) {
+                if constexpr (sizeof(S) == 2)
+                    unroll<0, Q>([&](auto qc) {
+                        constexpr int q = decltype(qc)::value;
+                        F[n][q] = __half2float(__float2half(F[n][q]));
+                    });
+                unroll<1, Q>([&](auto qc) {
                     constexpr int q = decltype(qc)::value;
-                    f[q] = __half2float(__float2half(f[q]));
+                    (EZ[q] == 0 ? me0 : me)[plane(q) * PL + n] = F[n][q];
                 });
-            }
-            const int sf = t & 1, su = t % 3;
-            unroll<0, Q>([&](auto qc) {
-                constexpr int q = decltype(qc)::value;
-                constexpr int c = cls<SIDE>(q);
-                if constexpr (EY[q] != 0) {
-                    // only nodes of the lattice write: a row wave's lanes past a partial
-                    // tile's last column would overwrite the right ring column
-                    constexpr int j = yi(q);
-                    if (act) {
-                        if constexpr (c == 0) sm.yf[sf][j][r][col] = f[q];
-                        else if constexpr (c == 1) sm.yu[su][j][r][col] = f[q];
-                        else sm.yd[j][r][col] = f[q];
-                    }
-                } else {
-                    constexpr int k = xi(q);
-                    if (ringw) {
-                        // a ring column passes the direction pointing into the tile
-                        if constexpr (k != 0) {
-                            if (act && sd == (k == 1 ? 0 : 1)) {
-                                if constexpr (c == 0) sm.hf[sf][r][sd] = f[q];
-                                else if constexpr (c == 1) sm.hu[su][r][sd] = f[q];
-                                else sm.hd[r][sd] = f[q];
-                            }
-                        }
-                    } else {
-                        if constexpr (c == 0) fcur[k] = f[q];
-                        else if constexpr (c == 1) ucur[k] = f[q];
-                        else dcur[k] = f[q];
-                    }
-                }
             });
         }
+        T f0[NPL];
+        each_n([&](auto nc) { f0[decltype(nc)::value] = F[decltype(nc)::value][0]; });
         __syncthreads();
-        // ---- second substep at layer t-1: gather and collide, then (after the barrier
-        // that frees the layer slots for the next iteration) push
-        T g[Q];
-        if (t >= 1 && core) second(t - 1, false, g);
-        // wait here, on every wave, for every vector memory operation in flight -- the
-        // next layer's loads and the previous layer's stores -- so that the pushes below
-        // are the only ones outstanding when the next iteration first uses the loaded
-        // values (the compiler's own wait there would cover them too).  The wait sits
-        // beside the barrier, in code that every path runs.
-        __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0), no wait on expcnt / lgkmcnt
-        __syncthreads();
-        if (t >= 1 && core) push(t - 1, g);
-#pragma unroll
-        for (int k = 0; k < 3; k++) {
-            fprv[k] = fcur[k];
-            uprv2[k] = uprv[k];
-            uprv[k] = ucur[k];
+        if constexpr (!early<S>()) {
+            if (rowok && t + 1 < nz) load_layer(layer_rsrc(cur, t + 1), fin);
         }
+        __builtin_amdgcn_sched_barrier(0);
+        // ---- second substep at layer t-1
+        T g[NPL][Q];
+        if (t >= 1 && core_row) {
+            unroll<0, Q>([&](auto qc) {
+                constexpr int q = decltype(qc)::value;
+                each_n([&](auto nc) {
+                    constexpr int n = decltype(nc)::value;
+                    if constexpr (q == 0) g[n][q] = q0[n];
+                    else if constexpr (cls<SIDE>(q) == 0) g[n][q] = arrive(qc, n, me1);
+                    else if constexpr (cls<SIDE>(q) == 1) g[n][q] = wo[n][slot(q)];
+                    else g[n][q] = arrive(qc, n, me);
+                });
+            });
+            if (t == 1) {  // the interface layer: the first fill's values (those toward the wall are in wo)
+                const Rsrc R = layer_rsrc(nxt, 0);
+                unroll<0, Q>([&](auto qc) {
+                    constexpr int q = decltype(qc)::value;
+                    if constexpr (cls<SIDE>(q) != 1) {
+                        T v[NPL];
+                        load_q(R, q, v);
+                        each_n([&](auto nc) { g[decltype(nc)::value][q] = v[decltype(nc)::value]; });
+                    }
+                });
+            }
+            collide_all(g);
+        }
+        // every wave waits here for the next layer's loads and the previous layer's stores,
+        // so that the pushes below are the only vector memory operations in flight when the
+        // loaded values are first used
+        __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0), no wait on expcnt / lgkmcnt
+        __builtin_amdgcn_sched_barrier(0);
+        if (t >= 1 && core_row) push(t - 1, g);
+        if (core_row) {
+            each_n([&](auto nc) {
+                constexpr int n = decltype(nc)::value;
+#pragma unroll
+                for (int k = 0; k < 5; k++) wo[n][k] = wn[n][k];
+                q0[n] = f0[n];
+                unroll<1, Q>([&](auto qc) {
+                    constexpr int q = decltype(qc)::value;
+                    if constexpr (cls<SIDE>(q) == 1) wn[n][slot(q)] = arrive(qc, n, me);
+                });
+            });
+            if (t == 0) {  // the interface layer: the first fill's values
+                const Rsrc R = layer_rsrc(nxt, 0);
+                unroll<0, Q>([&](auto qc) {
+                    constexpr int q = decltype(qc)::value;
+                    if constexpr (cls<SIDE>(q) == 1) {
+                        T v[NPL];
+                        load_q(R, q, v);
+                        each_n([&](auto nc) { wo[decltype(nc)::value][slot(q)] = v[decltype(nc)::value]; });
+                    }
+                });
+            }
+        }
+        if (t + 1 < nz) __syncthreads();
     }
-    // ---- second substep at the layer next to the wall
-    if (core) {
-        T g[Q];
-        second(nz - 1, true, g);
+    // ---- second substep at the layer next to the wall; the directions leaving the wall
+    // from this layer's toward-the-wall values (wn, and LDS at this node)
+    if (core_row) {
+        T g[NPL][Q];
+        each_n([&](auto nc) {
+            constexpr int n = decltype(nc)::value;
+            const int c = NPL * lane + n;
+            const bool own = wcl[r * CW + c] == -1;
+            unroll<0, Q>([&](auto qc) {
+                constexpr int q = decltype(qc)::value;
+                if constexpr (q == 0) g[n][q] = q0[n];
+                else if constexpr (cls<SIDE>(q) == 0) g[n][q] = arrive(qc, n, me + ((nz - 1) & 1) * ALONG * PL);
+                else if constexpr (cls<SIDE>(q) == 1) g[n][q] = wo[n][slot(q)];
+                else {
+                    const bool bb = own && core && wcl[(r - EY[q]) * CW + c - EX[q]] == -1;
+                    const T vbb = me[plane(OPP[q]) * PL + n];
+                    g[n][q] = bb ? vbb : wn[n][slot(MIR[q])];
+                }
+            });
+        });
+        collide_all(g);
         push(nz - 1, g);
+        if (!DS && rec) {
+            const double a = wave_sum64(srho), b = wave_sum64(smom);
+            if (lane == 0) {
+                rec[0] = a;
+                rec[1] = b;
+            }
+        }
+        if (DS && L.dsum) {
+            const double a = wave_sum64(sdm), b = wave_sum64(sdd);
+            if (lane == 0) {
+                double *o = L.dsum + 2 * ((size_t)y * tilesx + tx);
+                o[0] = a;
+                o[1] = b;
+            }
+        }
     }
 }
 
 template <class S, bool DS>
-__global__ __launch_bounds__(wg_threads<S>()) void k_band2(Batch<LatArgs> P) {
+__global__ __launch_bounds__(B2_THREADS) void k_band2(Batch<LatArgs> P) {
     using T = typename ComputeOf<S>::T;
-    __shared__ Lds<T, row_waves<S>()> sm;
+    constexpr int CW = 64 * npl<S>(), PAD = 2;  // PAD: ring lanes read one value beside the array and ignore it
+    __shared__ T lds[NPLANES * NR * CW + 2 * PAD];
+    __shared__ int8_t wcl[NR * CW + 2 * PAD];  // the tile's wall codes, ring included
     if (halted(P.halt)) return;
     const int bg = xcd_remap(blockIdx.x, gridDim.x);
     const int it = batch_find(P.first, P.n, bg);
     const LatArgs &L = P.it[it];
     const int tile = bg - P.first[it];
-    if (L.lo_kind == BOUND_WALL) band2_tile<S, 0, DS>(L, tile, sm);
-    else band2_tile<S, 1, DS>(L, tile, sm);
+    if (L.lo_kind == BOUND_WALL) band2_tile<S, 0, DS>(L, tile, lds + PAD, wcl + PAD);
+    else band2_tile<S, 1, DS>(L, tile, lds + PAD, wcl + PAD);
 }
 
 }  // namespace
 
-int band2_tiles(int nx, int ny, int prec) {
-    const int ty = prec == DNSG_PREC_FP64 ? tile_rows<double>() : tile_rows<float>();
-    return ((nx + TX - 1) / TX) * ((ny + ty - 1) / ty);
+int band2_tiles(int nx, int ny, int elem) {
+    const int ox = b2_cols(elem);
+    return ((nx + ox - 1) / ox) * ((ny + TY - 1) / TY);
+}
+
+// Which path a gratio-2 handle takes.  A tile holds a CU to itself and marches nz + 1
+// layers, each a chain of two collisions, two barriers and their memory accesses that
+// takes 6.5-8 us with few tiles and 9-10 us with the chip full, so the pass takes whole
+// rounds of tiles over the CUs; the two launches it replaces move twice the bytes at
+// 5.5 TB/s.  Measured, pass against two launches (band time a step): FP64 512 x 256 x 8
+// bands (468 tiles, 2 rounds) 165 / 237 us, 128 x 64 x 8 (42 tiles) 58 / 47 us, 256 x
+// 256 x 8 (260 tiles, a second round for 4 of them) 124 / 112 us; FP32 420 x 252 x 11
+// (208 tiles) 128 / 154 us, 512 x 256 x 16 (260 tiles) 264 / 251 us.
+bool band2_pays(int nx, int ny, int nz, int elem) {
+    int dev = 0, cus = 0;
+    if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus < 1)
+        return false;
+    const int rounds = (2 * band2_tiles(nx, ny, elem) + cus - 1) / cus;
+    const double pass = rounds * (nz + 1) * 9e-6, two = 2. * 2. * nx * (double)ny * nz * 2 * Q * elem / 5.5e12;
+    return pass <= two;
 }
 
 hipError_t launch_band2(hipStream_t s, const LatArgs *bands, int prec, const int *halt) {
+    const int elem = prec == DNSG_PREC_FP64 ? 8 : (prec == DNSG_PREC_FP32 ? 4 : 2);
     Batch<LatArgs> P;
     P.halt = halt;
     P.n = 2;
@@ -374,11 +459,11 @@ hipError_t launch_band2(hipStream_t s, const LatArgs *bands, int prec, const int
     for (int i = 0; i < BATCH_MAX; i++) {
         P.it[i] = bands[i < 2 ? i : 0];
         P.first[i] = blocks;
-        if (i < 2) blocks += band2_tiles(bands[i].nx, bands[i].ny, prec);
+        if (i < 2) blocks += band2_tiles(bands[i].nx, bands[i].ny, elem);
     }
     P.first[BATCH_MAX] = blocks;
     const bool ds = bands[0].dsum != nullptr || bands[1].dsum != nullptr;
-    const dim3 g(blocks), b(prec == DNSG_PREC_FP64 ? wg_threads<double>() : wg_threads<float>());
+    const dim3 g(blocks), b(B2_THREADS);
     if (prec == DNSG_PREC_FP64) {
         if (ds) hipLaunchKernelGGL((k_band2<double, true>), g, b, 0, s, P);
         else hipLaunchKernelGGL((k_band2<double, false>), g, b, 0, s, P);

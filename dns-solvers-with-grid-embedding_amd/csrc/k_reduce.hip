@@ -146,7 +146,8 @@ static RedSet make_set(dnsg_ctx *h, const double *means_c, const double *means_l
 // ---- encalc2 ---------------------------------------------------------------------------
 struct EncArgs {
     const double *pc, *pl, *pu;
-    int st;            // doubles per partial: [0] sum rho, [1] sum rho u_x
+    int st, stb;       // doubles per partial (coarse, bands): [0] sum rho, [1] sum rho u_x
+    int tiled;         // the bands' partials are per (row, tile), layer weights applied (B2_RED)
     int cpr_c, cpr_f;  // partials per row (coarse, bands)
     int Yc, zdc, Yf, zds, GR, zdf, NZs, Xf, force_mode;
     double ub, g_const;
@@ -156,12 +157,17 @@ struct EncArgs {
 // encalc2 partials as one index space: [lower entries | coarse entries | upper entries]
 struct EncSpace {
     int nl, nc, nu0, nu;  // entries in each part; nu0 = first upper entry used
-    __device__ int total() const { return nl + nc + nu; }
+    __host__ __device__ int total() const { return nl + nc + nu; }
 };
-__device__ __forceinline__ EncSpace enc_space(const EncArgs &A) {
+__host__ __device__ __forceinline__ EncSpace enc_space(const EncArgs &A) {
     EncSpace S;
-    S.nl = A.Yf * (A.zdf - A.GR - 1) * A.cpr_f;  // lower band k = 1 .. zdf-GR-1 (stored m = 0 .. zdf-GR-2)
     S.nc = A.Yc * A.zdc * A.cpr_c;                // every coarse layer
+    if (A.tiled) {
+        S.nl = S.nu = A.Yf * A.cpr_f;
+        S.nu0 = 0;
+        return S;
+    }
+    S.nl = A.Yf * (A.zdf - A.GR - 1) * A.cpr_f;  // lower band k = 1 .. zdf-GR-1 (stored m = 0 .. zdf-GR-2)
     S.nu0 = A.Yf * A.GR * A.cpr_f;                // upper band k = GR .. zdf-2 (stored m = GR .. zds-1)
     S.nu = A.Yf * A.zds * A.cpr_f - S.nu0;
     return S;
@@ -170,8 +176,8 @@ __device__ __forceinline__ EncSpace enc_space(const EncArgs &A) {
 // v += weighted (momentum, density, coarse momentum, coarse density) of entry e
 __device__ __forceinline__ void enc_entry(const EncArgs &A, const EncSpace &S, int e, double *v) {
     if (e < S.nl) {
-        v[0] += A.pl[(size_t)e * A.st + 1];
-        v[1] += A.pl[(size_t)e * A.st + 0];
+        v[0] += A.pl[(size_t)e * A.stb + 1];
+        v[1] += A.pl[(size_t)e * A.stb + 0];
     } else if (e < S.nl + S.nc) {
         e -= S.nl;
         const int z = (e / A.cpr_c) / A.Yc;
@@ -180,9 +186,9 @@ __device__ __forceinline__ void enc_entry(const EncArgs &A, const EncSpace &S, i
         v[0] += m; v[1] += d; v[2] += m; v[3] += d;
     } else {
         e = e - S.nl - S.nc + S.nu0;
-        const double c = ((e / A.cpr_f) / A.Yf == A.GR) ? 0.5 : 1.;  // half weight at k = GR
-        v[0] += c * A.pu[(size_t)e * A.st + 1];
-        v[1] += c * A.pu[(size_t)e * A.st + 0];
+        const double c = (!A.tiled && (e / A.cpr_f) / A.Yf == A.GR) ? 0.5 : 1.;  // half weight at k = GR
+        v[0] += c * A.pu[(size_t)e * A.stb + 1];
+        v[1] += c * A.pu[(size_t)e * A.stb + 0];
     }
 }
 
@@ -225,8 +231,7 @@ __global__ __launch_bounds__(RB) void k_fin_encalc2(EncArgs A, const double *seg
 }
 
 static hipError_t enc_two_stage(hipStream_t s, const EncArgs &A, double *seg) {
-    const int total = A.Yf * (A.zdf - A.GR - 1) * A.cpr_f + A.Yc * A.zdc * A.cpr_c + A.Yf * (A.zds - A.GR) * A.cpr_f;
-    const int nseg = (total + ENC_SEG - 1) / ENC_SEG;
+    const int nseg = (enc_space(A).total() + ENC_SEG - 1) / ENC_SEG;
     hipLaunchKernelGGL(k_enc_seg, dim3(nseg), dim3(RB), 0, s, A, seg);
     hipLaunchKernelGGL(k_fin_encalc2, dim3(1), dim3(RB), 0, s, A, (const double *)seg, nseg);
     return hipGetLastError();
@@ -236,8 +241,8 @@ constexpr int WS_SEG = 512;  // wall-stress entries per first-stage workgroup (l
 
 size_t enc_seg_doubles(const dnsg_ctx *h) {
     const size_t total = (size_t)h->d.Yc * h->d.zdc * cs_chunks(h->d.Xc) +
-                         2 * (size_t)h->d.Yf * (h->d.zdf - 1) * band_cpr_max(h) + (size_t)ftcd_blocks(h);
-    const size_t ws = (size_t)h->d.Yf * band_cpr_max(h);
+                         2 * band_parts_max(h->d) + (size_t)ftcd_blocks(h);
+    const size_t ws = band_parts_max(h->d);
     return 4 * (total / ENC_SEG + 2 + ws / WS_SEG + 1);
 }
 
@@ -251,7 +256,7 @@ size_t enc_seg_doubles(const dnsg_ctx *h) {
 
 size_t dsum_doubles(const dnsg_ctx *h) {
     return 2 * ((size_t)h->d.Yc * h->d.zdc * cs_chunks(h->d.Xc) +
-                2 * (size_t)h->d.Yf * (h->d.zdf - 1) * band_cpr_max(h));
+                2 * band_parts_max(h->d));
 }
 
 void set_dest_weights(const dnsg_ctx *h, int grid, LatArgs *L) {
@@ -316,7 +321,7 @@ __global__ __launch_bounds__(RB) void k_flux_fin(FluxNextArgs A, const double *s
 hipError_t launch_flux_next(hipStream_t s, dnsg_ctx *h) {
     FluxNextArgs A;
     A.nc = h->d.Yc * h->d.zdc * cs_chunks(h->d.Xc);
-    A.nl = A.nu = h->d.Yf * (h->d.zdf - 1) * band_cpr(h);
+    A.nl = A.nu = (int)(band_dsum_doubles(h) / 2);
     A.nf = ftcd_blocks(h);
     A.dc = h->dsum;
     A.dl = A.dc + 2 * (size_t)A.nc;
@@ -335,6 +340,8 @@ static EncArgs enc_args(dnsg_ctx *h, const double *pc, const double *pl, const d
                         double *diag_rec) {
     EncArgs A;
     A.pc = pc; A.pl = pl; A.pu = pu; A.st = st;
+    A.tiled = fused && h->band_tiled;
+    A.stb = A.tiled ? B2_RED : st;
     A.cpr_c = fused ? cs_chunks(h->coarse.nx) : 1;
     A.cpr_f = fused ? band_cpr(h) : 1;
     A.Yc = h->d.Yc; A.zdc = h->d.zdc; A.Yf = h->d.Yf; A.zds = h->lower.nz; A.GR = h->d.GR; A.zdf = h->d.zdf;
@@ -371,7 +378,7 @@ hipError_t launch_flux_many(hipStream_t s, dnsg_ctx *const *hs, int n, double *o
             dnsg_ctx *h = hs[i0 + (i < B.n ? i : 0)];
             const double *pc = h->red;
             const double *pl = pc + (size_t)h->coarse.ny * h->coarse.nz * cs_chunks(h->coarse.nx) * RED_W;
-            const double *pu = pl + (size_t)h->lower.ny * h->lower.nz * band_cpr(h) * RED_W;
+            const double *pu = pl + band_parts_max(h->d) * RED_W;
             B.it[i] = enc_args(h, pc, pl, pu, RED_W, true, out + 2 * (size_t)slot[i0 + (i < B.n ? i : 0)]);
             B.first[i] = i < B.n ? i : B.n;
         }
@@ -443,25 +450,37 @@ __global__ __launch_bounds__(RB) void k_fin_wshear(WsArgs A) {
     if (threadIdx.x == 0) wshear_finish(A, v);
 }
 
-// wall stress from the row sums of the first band substep (RED_W per row):
+// wall stress from the sums of the first band substep, one entry per (row, partial):
 // sum_x (-2u1 + 3u2 - u3) = -2 S1 + 3 S2 - S3 with S_m = sum_x u_x of layer m
-// One workgroup of WSB threads, four entries in flight per thread: the Re_tau=180
-// bands in the two-substep layout give 8192 (row, tile column) entries per layer.
+struct WsSegArgs {
+    const double *pl, *pu;  // the bands' fused-reduction partials
+    int Yf, cpr, nz, tiled;
+};
+
+__device__ __forceinline__ void ws_entry(const WsSegArgs &W, int e, double *v) {
+    if (W.tiled) {
+        const double *l = W.pl + (size_t)e * B2_RED, *u = W.pu + (size_t)e * B2_RED;
+        v[0] += (-2. * l[3] + 3. * l[4] - l[5]);
+        v[1] += l[2];
+        v[2] += -(2. * u[3] - 3. * u[4] + u[5]);
+        v[3] += u[2];
+        return;
+    }
+    const int y = e / W.cpr, c = e % W.cpr;
+    auto at = [&](const double *p, int m, int k) { return p[(((size_t)m * W.Yf + y) * W.cpr + c) * RED_W + k]; };
+    v[0] += (-2. * at(W.pl, 0, 2) + 3. * at(W.pl, 1, 2) - at(W.pl, 2, 2));
+    v[1] += at(W.pl, 0, 0);
+    v[2] += -(2. * at(W.pu, W.nz - 1, 2) - 3. * at(W.pu, W.nz - 2, 2) + at(W.pu, W.nz - 3, 2));
+    v[3] += at(W.pu, W.nz - 3, 0);
+}
+
+// one workgroup of WSB threads, four entries in flight per thread
 constexpr int WSB = 1024;
-__global__ __launch_bounds__(WSB) void k_fin_wshear_fused(WsArgs A, const double *pl, const double *pu, int nz,
-                                                          int cpr) {
+__global__ __launch_bounds__(WSB) void k_fin_wshear_fused(WsArgs A, WsSegArgs W) {
     __shared__ double lds[4][WSB / 64];
     double v[4] = {0., 0., 0., 0.};
-    const int Yf = A.Yf;
-    auto at = [&](const double *p, int m, int y, int c, int k) { return p[(((size_t)m * Yf + y) * cpr + c) * RED_W + k]; };
 #pragma unroll 4
-    for (int e = threadIdx.x; e < Yf * cpr; e += WSB) {
-        const int y = e / cpr, c = e % cpr;
-        v[0] += (-2. * at(pl, 0, y, c, 2) + 3. * at(pl, 1, y, c, 2) - at(pl, 2, y, c, 2));
-        v[1] += at(pl, 0, y, c, 0);
-        v[2] += -(2. * at(pu, nz - 1, y, c, 2) - 3. * at(pu, nz - 2, y, c, 2) + at(pu, nz - 3, y, c, 2));
-        v[3] += at(pu, nz - 3, y, c, 0);
-    }
+    for (int e = threadIdx.x; e < W.Yf * W.cpr; e += WSB) ws_entry(W, e, v);
     block_sum<4, WSB>(v, lds);
     if (threadIdx.x == 0) {
         wshear_finish(A, v);
@@ -490,12 +509,12 @@ __device__ void wshear_finish(const WsArgs &A, const double *v) {
 hipError_t launch_wshear_fused(hipStream_t s, dnsg_ctx *h, double *diag_rec, const double *enc_rec) {
     const int cpr = band_cpr(h);
     const double *pl = h->red + (size_t)h->coarse.ny * h->coarse.nz * cs_chunks(h->coarse.nx) * RED_W;
-    const double *pu = pl + (size_t)h->lower.ny * h->lower.nz * cpr * RED_W;
+    const double *pu = pl + band_parts_max(h->d) * RED_W;
     WsArgs A;
     A.part = nullptr; A.Xf = h->d.Xf; A.Yf = h->d.Yf; A.NZs = h->d.NZs; A.GR = h->d.GR; A.omega_f = h->d.omega_f;
     A.force = h->d_force; A.diag = diag_rec; A.out = nullptr; A.enc = enc_rec;
     A.halt = h->halt_armed ? h->halt_flag : nullptr;
-    hipLaunchKernelGGL(k_fin_wshear_fused, dim3(1), dim3(WSB), 0, s, A, pl, pu, h->lower.nz, cpr);
+    hipLaunchKernelGGL(k_fin_wshear_fused, dim3(1), dim3(WSB), 0, s, A, WsSegArgs{pl, pu, h->d.Yf, cpr, h->lower.nz, h->band_tiled});
     return hipGetLastError();
 }
 
@@ -506,20 +525,6 @@ hipError_t launch_wshear_fused(hipStream_t s, dnsg_ctx *h, double *diag_rec, con
 // and, with the force that sets, wshearstr -- two launches where the separate
 // reductions take three, one of them a single workgroup over all the wall-stress
 // entries.
-struct WsSegArgs {
-    const double *pl, *pu;  // the bands' fused-reduction partials
-    int Yf, cpr, nz;
-};
-
-__device__ __forceinline__ void ws_entry(const WsSegArgs &W, int e, double *v) {
-    const int y = e / W.cpr, c = e % W.cpr;
-    auto at = [&](const double *p, int m, int k) { return p[(((size_t)m * W.Yf + y) * W.cpr + c) * RED_W + k]; };
-    v[0] += (-2. * at(W.pl, 0, 2) + 3. * at(W.pl, 1, 2) - at(W.pl, 2, 2));
-    v[1] += at(W.pl, 0, 0);
-    v[2] += -(2. * at(W.pu, W.nz - 1, 2) - 3. * at(W.pu, W.nz - 2, 2) + at(W.pu, W.nz - 3, 2));
-    v[3] += at(W.pu, W.nz - 3, 0);
-}
-
 __global__ __launch_bounds__(RB) void k_red_seg(EncArgs A, WsSegArgs W, double *seg, int nseg) {
     __shared__ double lds[4][RB / 64];
     double v[4] = {0., 0., 0., 0.};
@@ -553,11 +558,10 @@ __global__ __launch_bounds__(RB) void k_fin_enc_ws(EncArgs A, WsArgs Wf, const d
 hipError_t launch_reductions_fused(hipStream_t s, dnsg_ctx *h, double *diag_rec) {
     const int cpr = band_cpr(h);
     const double *pc = h->red, *pl = pc + (size_t)h->coarse.ny * h->coarse.nz * cs_chunks(h->coarse.nx) * RED_W;
-    const double *pu = pl + (size_t)h->lower.ny * h->lower.nz * cpr * RED_W;
+    const double *pu = pl + band_parts_max(h->d) * RED_W;
     const EncArgs A = enc_args(h, pc, pl, pu, RED_W, true, diag_rec);
-    const int total = A.Yf * (A.zdf - A.GR - 1) * A.cpr_f + A.Yc * A.zdc * A.cpr_c + A.Yf * (A.zds - A.GR) * A.cpr_f;
-    const int nseg = (total + ENC_SEG - 1) / ENC_SEG;
-    const WsSegArgs W = {pl, pu, h->d.Yf, cpr, h->lower.nz};
+    const int nseg = (enc_space(A).total() + ENC_SEG - 1) / ENC_SEG;
+    const WsSegArgs W = {pl, pu, h->d.Yf, cpr, h->lower.nz, h->band_tiled};
     const int nws = (W.Yf * W.cpr + WS_SEG - 1) / WS_SEG;
     WsArgs Wf;
     Wf.part = nullptr; Wf.Xf = h->d.Xf; Wf.Yf = h->d.Yf; Wf.NZs = h->d.NZs; Wf.GR = h->d.GR; Wf.omega_f = h->d.omega_f;

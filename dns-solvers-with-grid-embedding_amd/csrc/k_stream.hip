@@ -20,52 +20,88 @@
 
 namespace dnsg {
 
-// Per storage type: use the aligned-store form (bit 0 FP64, 1 FP32, 2 FP16) and,
-// in it, non-temporal stores.  Measured on the Re_tau=180 lattices: the aligned
-// form with non-temporal stores is fastest in FP64; FP32 and FP16 are fastest in
-// the scatter form.
-#ifndef DNSG_CS_ALIGNED_MASK
-#define DNSG_CS_ALIGNED_MASK 1
-#endif
-#ifndef DNSG_CS_NT_MASK
-#define DNSG_CS_NT_MASK 1
-#endif
+// FP64 rows of whole chunks take the aligned-store form, with non-temporal stores; FP32 and
+// FP16 rows that cannot pair are faster in the scatter form (Re_tau=180 lattices).
 template <class S>
-constexpr int prec_bit() { return sizeof(S) == 8 ? 1 : (sizeof(S) == 4 ? 2 : 4); }
-template <class S>
-constexpr bool cs_aligned() { return (DNSG_CS_ALIGNED_MASK & prec_bit<S>()) != 0; }
-template <class S>
-constexpr bool cs_nt() { return (DNSG_CS_NT_MASK & prec_bit<S>()) != 0; }
-template <class S, class V>
-__device__ __forceinline__ void store_cs(S *p, V v) {
-    if constexpr (cs_nt<S>()) store_nt(p, v);
-    else store_s(p, v);
-}
-// Non-temporal loads of the pre-collision lattice (same mask convention) measured
-// 1.7% slower in FP64 and no faster in FP32 on the Re_tau=180 lattices: off.
-#ifndef DNSG_CS_NTLOAD_MASK
-#define DNSG_CS_NTLOAD_MASK 0
-#endif
-template <class S>
-__device__ __forceinline__ auto load_cs(const S *p) {
-    if constexpr ((DNSG_CS_NTLOAD_MASK & prec_bit<S>()) != 0 && sizeof(S) != 2) return __builtin_nontemporal_load(p);
-    else return load_s(p);
-}
+constexpr bool cs_aligned() { return sizeof(S) == 8; }
 
-// Scatter form for the node at x of row (y, z): collide, then write each
-// direction to its target (x + e_x, y + e_y, z + e_z) with the wall rules.
+// Sums of a node's stores by the layer step k = -1, 0, 1 of their destination; the layer
+// weights are applied once at the end (LatArgs::dsum).  Every direction is added at its
+// own step, stored or not: the layers that take no store (beyond an end, or rewritten by
+// an interface transfer) have weight 0.  The sums stay in registers only while no branch
+// chooses between two of them, so the wall rules select values, not members.
+struct DestSums {
+    double dl = 0., dc = 0., dh = 0., xl = 0., xc = 0., xh = 0.;
+    template <int k>
+    __device__ __forceinline__ void mass(double v) {
+        if constexpr (k < 0) dl += v;
+        if constexpr (k == 0) dc += v;
+        if constexpr (k > 0) dh += v;
+    }
+    template <int k, int ex>
+    __device__ __forceinline__ void mom(double v) {
+        const double e = ex > 0 ? v : -v;
+        if constexpr (ex != 0 && k < 0) xl += e;
+        if constexpr (ex != 0 && k == 0) xc += e;
+        if constexpr (ex != 0 && k > 0) xh += e;
+    }
+    __device__ __forceinline__ void into(RowSums &rs, const LatArgs &L, int z) const {
+        const double wl = dest_w(L, z - 1), wc = dest_w(L, z), wh = dest_w(L, z + 1);
+        rs.dd += wl * dl + wc * dc + wh * dh;
+        rs.dm += wl * xl + wc * xc + wh * xh;
+    }
+};
+
+// Scatter form for the node at x of row (y, z): collide, then write each direction to its
+// target (x + e_x, y + e_y, z + e_z) with the boundary rules above.  With DS, the
+// destination-weighted sums of the writes go into rs.
 template <class S, bool DS, class T>
 __device__ __forceinline__ void cs_scatter(const LatArgs &L, const S *__restrict__ cur, S *__restrict__ nxt, int row,
                                            int x, T G, T om, bool red, RowSums &rs) {
-    const int nx = L.nx;
+    const int nx = L.nx, ny = L.ny, nz = L.nz;
     T f[Q];
     unroll<0, Q>([&](auto qc) {
         constexpr int q = decltype(qc)::value;
-        f[q] = load_cs(cur + (size_t)q * nx + x);
+        f[q] = load_s(cur + (size_t)q * nx + x);
     });
-    if (red) rs.add<S>(f);
-    collide_any(f, G, om);
-    scatter_push<S, DS>(L, nxt, row, x, f, rs, WallCodesGlobal{L});
+    const auto pre = collide_any(f, G, om);
+    if (red) rs.add<S>(pre);
+    const int y = row % ny, z = row / ny;
+    const bool lo_edge = (z == 0), hi_edge = (z == nz - 1);
+    const int ym = (y == 0) ? ny - 1 : y - 1, yp = (y == ny - 1) ? 0 : y + 1;
+    const int xm = (x == 0) ? nx - 1 : x - 1, xp = (x == nx - 1) ? 0 : x + 1;
+    DestSums dst;
+    unroll<0, Q>([&](auto qc) {
+        constexpr int q = decltype(qc)::value;
+        if constexpr (DS) {
+            dst.mass<EZ[q]>(read_back<S, q>(f[q]));
+            dst.mom<EZ[q], EX[q]>(read_back<S, q>(f[q]));
+        }
+        const int xt = (EX[q] > 0) ? xp : (EX[q] < 0 ? xm : x);
+        const int yt = (EY[q] > 0) ? yp : (EY[q] < 0 ? ym : y);
+        if constexpr (EZ[q] != 0) {
+            const bool at_end = (EZ[q] < 0) ? lo_edge : hi_edge;
+            if (at_end) {
+                const int kind = (EZ[q] < 0) ? L.lo_kind : L.hi_kind;
+                if (kind == BOUND_WALL) {
+                    const int8_t *wc = (EZ[q] < 0) ? L.wlo : L.whi;
+                    const bool bb = wc[(size_t)yt * nx + xt] == -1 && wc[(size_t)y * nx + x] == -1;
+                    if (bb) store_s(nxt + lat_at(OPP[q], (size_t)row, x, nx), f[q]);
+                    else store_s(nxt + lat_at(MIR[q], (size_t)z * ny + yt, xt, nx), f[q]);
+                    if constexpr (DS) {  // it lands in this layer
+                        const double v = read_back<S, q>(f[q]);
+                        dst.mass<0>(v);
+                        dst.mom<0, EX[q]>(bb ? -v : v);
+                    }
+                }
+                return;
+            }
+        }
+        const int zt = z + EZ[q];
+        if ((zt == 0 && L.skip_lo) || (zt == nz - 1 && L.skip_hi)) return;
+        store_s(nxt + lat_at(q, (size_t)zt * ny + yt, xt, nx), f[q]);
+    });
+    if constexpr (DS) dst.into(rs, L, z);
 }
 
 // Aligned form for chunk x0 .. x0 + CS_THREADS - 1 of row (y, z) (nx a multiple of
@@ -75,6 +111,31 @@ __device__ __forceinline__ void cs_scatter(const LatArgs &L, const S *__restrict
 // positions of the target row: whole cache lines, written once.  Each thread
 // stores, at its own x, the value arriving there from x - e_x; the set of writes
 // is exactly the scatter form's.
+// The three layers a row's values go to, as buffer resources, and the scalar offsets of
+// their rows y - 1, y, y + 1 and of a direction's line: formed once per workgroup, so a
+// store costs one scalar add.
+template <class S>
+struct RowTargets {
+    Rsrc lo, mid, hi;
+    unsigned ym, yc, yp, line;
+    __device__ __forceinline__ RowTargets(const LatArgs &L, const S *nxt, int y, int z) {
+        line = __builtin_amdgcn_readfirstlane(L.nx * (int)sizeof(S));
+        y = __builtin_amdgcn_readfirstlane(y);
+        const unsigned row = Q * line, bytes = row * (unsigned)L.ny;
+        const char *m = reinterpret_cast<const char *>(nxt) + (size_t)z * bytes;
+        lo = buf_rsrc(z > 0 ? m - bytes : m, bytes);  // the layer beyond an end takes no stores
+        mid = buf_rsrc(m, bytes);
+        hi = buf_rsrc(z < L.nz - 1 ? m + bytes : m, bytes);
+        ym = row * (unsigned)(y == 0 ? L.ny - 1 : y - 1);
+        yc = row * (unsigned)y;
+        yp = row * (unsigned)(y == L.ny - 1 ? 0 : y + 1);
+    }
+    template <int ez>
+    __device__ __forceinline__ Rsrc layer() const { return ez < 0 ? lo : (ez > 0 ? hi : mid); }
+    template <int ey>
+    __device__ __forceinline__ unsigned off(int q) const { return (ey < 0 ? ym : (ey > 0 ? yp : yc)) + q * line; }
+};
+
 template <class S, bool DS, class T>
 __device__ __forceinline__ void cs_aligned_chunk(const LatArgs &L, const S *__restrict__ cur, S *__restrict__ nxt,
                                                  int row, int x0, T G, T om, bool red, RowSums &rs) {
@@ -86,6 +147,10 @@ __device__ __forceinline__ void cs_aligned_chunk(const LatArgs &L, const S *__re
     const bool lo_edge = (z == 0), hi_edge = (z == nz - 1);
     const int ym = (y == 0) ? ny - 1 : y - 1, yp = (y == ny - 1) ? 0 : y + 1;
     const int t = threadIdx.x, lane = t & 63, w = t >> 6, x = x0 + t;
+    constexpr unsigned ES = sizeof(S);
+    constexpr int NT = 2;
+    const unsigned vx = (unsigned)x * ES, lb = __builtin_amdgcn_readfirstlane(nx * (int)ES);
+    const Rsrc in = buf_rsrc(cur, Q * lb);
     if (t == 0 || t == CS_THREADS - 1) {
         const int side = t == 0 ? 0 : 1;
         int xh = side == 0 ? x0 - 1 : x0 + CS_THREADS;
@@ -93,7 +158,7 @@ __device__ __forceinline__ void cs_aligned_chunk(const LatArgs &L, const S *__re
         T g[Q];
         unroll<0, Q>([&](auto qc) {
             constexpr int q = decltype(qc)::value;
-            g[q] = load_cs(cur + (size_t)q * nx + xh);
+            g[q] = load_s(cur + (size_t)q * nx + xh);
         });
         collide_any(g, G, om);
         unroll<0, Q>([&](auto qc) {
@@ -104,10 +169,10 @@ __device__ __forceinline__ void cs_aligned_chunk(const LatArgs &L, const S *__re
     T f[Q];
     unroll<0, Q>([&](auto qc) {
         constexpr int q = decltype(qc)::value;
-        f[q] = load_cs(cur + (size_t)q * nx + x);
+        f[q] = buf_load(in, vx, q * lb, cur);
     });
-    if (red) rs.add<S>(f);
-    collide_any(f, G, om);
+    const auto pre = collide_any(f, G, om);
+    if (red) rs.add<S>(pre);
     unroll<0, Q>([&](auto qc) {
         constexpr int q = decltype(qc)::value;
         if constexpr (EX[q] > 0) {
@@ -117,8 +182,8 @@ __device__ __forceinline__ void cs_aligned_chunk(const LatArgs &L, const S *__re
         }
     });
     __syncthreads();
-    const bool ds = DS && L.dsum != nullptr;  // DS: compiled in only where a launch asks for it
-    const double wz[3] = {ds ? dest_w(L, z - 1) : 0., ds ? dest_w(L, z) : 0., ds ? dest_w(L, z + 1) : 0.};
+    DestSums dst;
+    const RowTargets<S> to(L, nxt, y, z);
     const int xm = (x == 0) ? nx - 1 : x - 1, xp = (x == nx - 1) ? 0 : x + 1;
     unroll<0, Q>([&](auto qc) {
         constexpr int q = decltype(qc)::value;
@@ -130,6 +195,10 @@ __device__ __forceinline__ void cs_aligned_chunk(const LatArgs &L, const S *__re
             v = __shfl_down(f[q], 1, 64);
             if (lane == 63) v = (w == NW - 1) ? hb[1][q] : wb[w + 1][1][q];
         }
+        if constexpr (DS) {
+            dst.mass<EZ[q]>(read_back<S, q>(v));
+            dst.mom<EZ[q], EX[q]>(read_back<S, q>(v));
+        }
         const int yt = (EY[q] > 0) ? yp : (EY[q] < 0 ? ym : y);
         if constexpr (EZ[q] != 0) {
             const bool at_end = (EZ[q] < 0) ? lo_edge : hi_edge;
@@ -139,15 +208,16 @@ __device__ __forceinline__ void cs_aligned_chunk(const LatArgs &L, const S *__re
                     const int8_t *wc = (EZ[q] < 0) ? L.wlo : L.whi;
                     // specular reflection of the source x - e_x into (x, yt), unless it bounces back
                     const int xs = (EX[q] > 0) ? xm : (EX[q] < 0 ? xp : x);
-                    if (!(wc[(size_t)yt * nx + x] == -1 && wc[(size_t)y * nx + xs] == -1)) {
-                        store_cs(nxt + lat_at(MIR[q], (size_t)z * ny + yt, x, nx), v);
-                        if (ds) add_write(rs, wz[1], EX[q], read_back<S, q>(v));
-                    }
+                    const bool spec = !(wc[(size_t)yt * nx + x] == -1 && wc[(size_t)y * nx + xs] == -1);
+                    if (spec) store_s(nxt + lat_at(MIR[q], (size_t)z * ny + yt, x, nx), v);
                     // halfway bounce-back of this node's own value
                     const int xt = (EX[q] > 0) ? xp : (EX[q] < 0 ? xm : x);
-                    if (wc[(size_t)yt * nx + xt] == -1 && wc[(size_t)y * nx + x] == -1) {
-                        store_cs(nxt + lat_at(OPP[q], (size_t)row, x, nx), f[q]);
-                        if (ds) add_write(rs, wz[1], -EX[q], read_back<S, q>(f[q]));
+                    const bool bb = wc[(size_t)yt * nx + xt] == -1 && wc[(size_t)y * nx + x] == -1;
+                    if (bb) store_s(nxt + lat_at(OPP[q], (size_t)row, x, nx), f[q]);
+                    if constexpr (DS) {  // both land in this layer
+                        const double a = spec ? read_back<S, q>(v) : 0., b = bb ? read_back<S, q>(f[q]) : 0.;
+                        dst.mass<0>(a + b);
+                        dst.mom<0, EX[q]>(a - b);
                     }
                 }
                 return;
@@ -155,9 +225,9 @@ __device__ __forceinline__ void cs_aligned_chunk(const LatArgs &L, const S *__re
         }
         const int zt = z + EZ[q];
         if ((zt == 0 && L.skip_lo) || (zt == nz - 1 && L.skip_hi)) return;
-        store_cs(nxt + lat_at(q, (size_t)zt * ny + yt, x, nx), v);
-        if (ds) add_write(rs, wz[EZ[q] + 1], EX[q], read_back<S, q>(v));
+        buf_store<NT>(to.template layer<EZ[q]>(), vx, to.template off<EY[q]>(q), nxt, v);
     });
+    if constexpr (DS) dst.into(rs, L, z);
 }
 
 // Paired form (FP32 / FP16 storage, nx a multiple of 2 CS_THREADS): the workgroup
@@ -168,43 +238,13 @@ __device__ __forceinline__ void cs_aligned_chunk(const LatArgs &L, const S *__re
 // the pair (f(x - 1), f(x)), f(x - 1) being the previous thread's second node; for
 // e_x = -1 the pair (f(x + 1), f(x + 2)).  At a wall end the pair's two positions
 // take the wall rules one value at a time.  The writes are exactly the scatter
-// form's.  rs[0] / rs[1] collect the sums of the first / second chunk's nodes.
-__device__ __forceinline__ void load_pair(const float *p, float &a, float &b) {
-    const float2 v = *reinterpret_cast<const float2 *>(p);
-    a = v.x;
-    b = v.y;
-}
-__device__ __forceinline__ void load_pair(const __half *p, float &a, float &b) {
-    const __half2 v = *reinterpret_cast<const __half2 *>(p);
-    a = __low2float(v);
-    b = __high2float(v);
-}
-__device__ __forceinline__ void load_pair(const double *p, double &a, double &b) {
-    const double2 v = *reinterpret_cast<const double2 *>(p);
-    a = v.x;
-    b = v.y;
-}
+// form's.  Threads below / from CS_THREADS / 2 hold the first / second chunk's nodes.
 // Paired stores are non-temporal, like the aligned form's.  Measured on the
-// Re_tau=180 lattices: the FP64 coarse launch of the flux-controlled step 1.904 ->
-// 1.861 ms; FP32 coarse 0.952 -> 0.938 ms and band 0.479 -> 0.472 ms; FP16 within 1%.
-__device__ __forceinline__ void store_pair2(double *p, double a, double b) {
-    typedef double d2v __attribute__((ext_vector_type(2)));
-    const d2v v = {a, b};
-    __builtin_nontemporal_store(v, reinterpret_cast<d2v *>(p));
-}
-__device__ __forceinline__ void store_pair2(float *p, float a, float b) {
-    typedef float f2v __attribute__((ext_vector_type(2)));
-    const f2v v = {a, b};
-    __builtin_nontemporal_store(v, reinterpret_cast<f2v *>(p));
-}
-__device__ __forceinline__ void store_pair2(__half *p, float a, float b) {
-    const __half2 h = __halves2half2(__float2half(a), __float2half(b));
-    __builtin_nontemporal_store(*reinterpret_cast<const unsigned int *>(&h), reinterpret_cast<unsigned int *>(p));
-}
-
+// Re_tau=180 lattices: FP32 coarse 0.952 -> 0.938 ms and band 0.479 -> 0.472 ms; FP16
+// within 1%.
 template <class S, bool DS, class T>
 __device__ __forceinline__ void cs_paired_chunk(const LatArgs &L, const S *__restrict__ cur, S *__restrict__ nxt,
-                                                int row, int x0, T G, T om, bool red, RowSums *rs) {
+                                                int row, int x0, T G, T om, bool red, RowSums &rs) {
     constexpr int NW = CS_THREADS / 64, NP = 2 * CS_THREADS;
     __shared__ T hb[2][Q];      // post-collision nodes x0 - 1, x0 + NP
     __shared__ T wb[NW][2][Q];  // per wave: last lane's second node e_x > 0, first lane's first node e_x < 0
@@ -213,6 +253,9 @@ __device__ __forceinline__ void cs_paired_chunk(const LatArgs &L, const S *__res
     const bool lo_edge = (z == 0), hi_edge = (z == nz - 1);
     const int ym = (y == 0) ? ny - 1 : y - 1, yp = (y == ny - 1) ? 0 : y + 1;
     const int t = threadIdx.x, lane = t & 63, w = t >> 6, x = x0 + 2 * t;
+    constexpr unsigned ES = sizeof(S);
+    const unsigned vx = (unsigned)x * ES, lb = __builtin_amdgcn_readfirstlane(nx * (int)ES);
+    const Rsrc in = buf_rsrc(cur, Q * lb);
     if (t == 0 || t == CS_THREADS - 1) {
         const int side = t == 0 ? 0 : 1;
         int xh = side == 0 ? x0 - 1 : x0 + NP;
@@ -231,15 +274,14 @@ __device__ __forceinline__ void cs_paired_chunk(const LatArgs &L, const S *__res
     T f0[Q], f1[Q];
     unroll<0, Q>([&](auto qc) {
         constexpr int q = decltype(qc)::value;
-        load_pair(cur + (size_t)q * nx + x, f0[q], f1[q]);
+        buf_load_pair(in, vx, q * lb, cur, f0[q], f1[q]);
     });
-    RowSums &rt = rs[t < CS_THREADS / 2 ? 0 : 1];
-    if (red) {
-        rt.add<S>(f0);
-        rt.add<S>(f1);
-    }
-    collide_any(f0, G, om);
-    collide_any(f1, G, om);
+    const auto p0 = collide_any(f0, G, om);
+    if (red) rs.add<S>(p0);
+    // one collision after the other: interleaved by the scheduler they take 102 VGPRs (FP32)
+    __builtin_amdgcn_sched_barrier(0);
+    const auto p1 = collide_any(f1, G, om);
+    if (red) rs.add<S>(p1);
     unroll<0, Q>([&](auto qc) {
         constexpr int q = decltype(qc)::value;
         if constexpr (EX[q] > 0) {
@@ -249,8 +291,8 @@ __device__ __forceinline__ void cs_paired_chunk(const LatArgs &L, const S *__res
         }
     });
     __syncthreads();
-    const bool ds = DS && L.dsum != nullptr;  // DS: compiled in only where a launch asks for it
-    const double wz[3] = {ds ? dest_w(L, z - 1) : 0., ds ? dest_w(L, z) : 0., ds ? dest_w(L, z + 1) : 0.};
+    DestSums dst;
+    const RowTargets<S> to(L, nxt, y, z);
     unroll<0, Q>([&](auto qc) {
         constexpr int q = decltype(qc)::value;
         // the values arriving at x and x + 1, and the sources they leave from
@@ -266,6 +308,11 @@ __device__ __forceinline__ void cs_paired_chunk(const LatArgs &L, const S *__res
             va = f1[q];
             vb = s;
         }
+        if constexpr (DS) {
+            const double a = read_back<S, q>(va) + read_back<S, q>(vb);
+            dst.mass<EZ[q]>(a);
+            dst.mom<EZ[q], EX[q]>(a);
+        }
         const int yt = (EY[q] > 0) ? yp : (EY[q] < 0 ? ym : y);
         if constexpr (EZ[q] != 0) {
             const bool at_end = (EZ[q] < 0) ? lo_edge : hi_edge;
@@ -276,34 +323,32 @@ __device__ __forceinline__ void cs_paired_chunk(const LatArgs &L, const S *__res
                     // positions x + i (i = 0, 1): the arriving value (source x + i - e_x)
                     // is reflected specularly into (x + i, yt) unless it bounces back,
                     // and the node's own value bounces back where its target is no-slip
-#pragma unroll
-                    for (int i = 0; i < 2; i++) {
+                    unroll<0, 2>([&](auto ic) {
+                        constexpr int i = decltype(ic)::value;
                         const int xi = x + i;
                         const int xm = (xi == 0) ? nx - 1 : xi - 1, xp = (xi == nx - 1) ? 0 : xi + 1;
                         const T v = i == 0 ? va : vb, own = i == 0 ? f0[q] : f1[q];
                         const int xs = (EX[q] > 0) ? xm : (EX[q] < 0 ? xp : xi);
-                        if (!(wc[(size_t)yt * nx + xi] == -1 && wc[(size_t)y * nx + xs] == -1)) {
-                            store_s(nxt + lat_at(MIR[q], (size_t)z * ny + yt, xi, nx), v);
-                            if (ds) add_write(rt, wz[1], EX[q], read_back<S, q>(v));
-                        }
+                        const bool spec = !(wc[(size_t)yt * nx + xi] == -1 && wc[(size_t)y * nx + xs] == -1);
+                        if (spec) store_s(nxt + lat_at(MIR[q], (size_t)z * ny + yt, xi, nx), v);
                         const int xt = (EX[q] > 0) ? xp : (EX[q] < 0 ? xm : xi);
-                        if (wc[(size_t)yt * nx + xt] == -1 && wc[(size_t)y * nx + xi] == -1) {
-                            store_s(nxt + lat_at(OPP[q], (size_t)row, xi, nx), own);
-                            if (ds) add_write(rt, wz[1], -EX[q], read_back<S, q>(own));
+                        const bool bb = wc[(size_t)yt * nx + xt] == -1 && wc[(size_t)y * nx + xi] == -1;
+                        if (bb) store_s(nxt + lat_at(OPP[q], (size_t)row, xi, nx), own);
+                        if constexpr (DS) {
+                            const double a = spec ? read_back<S, q>(v) : 0., b = bb ? read_back<S, q>(own) : 0.;
+                            dst.mass<0>(a + b);
+                            dst.mom<0, EX[q]>(a - b);
                         }
-                    }
+                    });
                 }
                 return;
             }
         }
         const int zt = z + EZ[q];
         if ((zt == 0 && L.skip_lo) || (zt == nz - 1 && L.skip_hi)) return;
-        store_pair2(nxt + lat_at(q, (size_t)zt * ny + yt, x, nx), va, vb);
-        if (ds) {
-            add_write(rt, wz[EZ[q] + 1], EX[q], read_back<S, q>(va));
-            add_write(rt, wz[EZ[q] + 1], EX[q], read_back<S, q>(vb));
-        }
+        buf_store_pair<2>(to.template layer<EZ[q]>(), vx, to.template off<EY[q]>(q), nxt, va, vb);
     });
+    if constexpr (DS) dst.into(rs, L, z);
 }
 
 __device__ __forceinline__ void write_sums(double *red, size_t e, const RowSums &s) {
@@ -312,25 +357,34 @@ __device__ __forceinline__ void write_sums(double *red, size_t e, const RowSums 
     red[e + 2] = s.u;
 }
 
-// workgroup sum of one partial (wave shuffles, then LDS over the waves)
-__device__ __forceinline__ RowSums block_sums(RowSums s) {
-    __shared__ double lds[5][CS_THREADS / 64];
+// Workgroup sums of the fused reductions (wave shuffles, then LDS over the waves), written
+// as `parts` consecutive partials from e on, each over CS_THREADS / parts threads.
+template <bool DS>
+__device__ __forceinline__ void write_block_sums(const LatArgs &L, const RowSums &s, size_t e, int parts) {
+    constexpr int NW = CS_THREADS / 64;
+    __shared__ double lds[5][NW];
     const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-    s.rho = wave_sum64(s.rho);
-    s.mom = wave_sum64(s.mom);
-    s.u = wave_sum64(s.u);
-    s.dm = wave_sum64(s.dm);
-    s.dd = wave_sum64(s.dd);
-    if (lane == 0) {
-        lds[0][wid] = s.rho; lds[1][wid] = s.mom; lds[2][wid] = s.u; lds[3][wid] = s.dm; lds[4][wid] = s.dd;
+    const bool red = L.red != nullptr, ds = DS && L.dsum != nullptr;
+    if (red) {
+        const double a = wave_sum64(s.rho), b = wave_sum64(s.mom), c = wave_sum64(s.u);
+        if (lane == 0) { lds[0][wid] = a; lds[1][wid] = b; lds[2][wid] = c; }
+    }
+    if (ds) {
+        const double a = wave_sum64(s.dm), b = wave_sum64(s.dd);
+        if (lane == 0) { lds[3][wid] = a; lds[4][wid] = b; }
     }
     __syncthreads();
-    RowSums t;
-    if (threadIdx.x == 0)
-        for (int w = 0; w < CS_THREADS / 64; w++) {
-            t.rho += lds[0][w]; t.mom += lds[1][w]; t.u += lds[2][w]; t.dm += lds[3][w]; t.dd += lds[4][w];
+    if ((int)threadIdx.x < parts) {
+        RowSums t;
+        const int nw = NW / parts;
+        for (int w = threadIdx.x * nw; w < (int)(threadIdx.x + 1) * nw; w++) {
+            if (red) { t.rho += lds[0][w]; t.mom += lds[1][w]; t.u += lds[2][w]; }
+            if (ds) { t.dm += lds[3][w]; t.dd += lds[4][w]; }
         }
-    return t;
+        e += threadIdx.x;
+        if (red) write_sums(L.red, e * RED_W, t);
+        if (ds) { L.dsum[2 * e] = t.dm; L.dsum[2 * e + 1] = t.dd; }
+    }
 }
 
 template <class S, bool DS>
@@ -349,23 +403,14 @@ __global__ __launch_bounds__(CS_THREADS) void k_collide_stream(Batch<LatArgs> P)
     const bool red = L.red != nullptr;
     const int rpw = cs_rows_per_wg(nx);
     RowSums rs;
-    {
+    if constexpr (sizeof(S) != 8) {  // compiled out in FP64, which never pairs (cs_paired)
         if (L.paired) {
             // two chunks of one row per workgroup, two nodes per thread
             const int cpr = cs_chunks(nx), ppr = cpr / 2;
             const int row = b / ppr, pc = b % ppr;
-            RowSums r2[2];
-            cs_paired_chunk<S, DS, T>(L, base + (size_t)row * Q * nx, nxt, row, pc * 2 * CS_THREADS, G, om, red, r2);
-            if (red || (DS && L.dsum)) {  // uniform per workgroup
-#pragma unroll
-                for (int c = 0; c < 2; c++) {
-                    if (c) __syncthreads();  // block_sums' shared partials are reused
-                    const RowSums t = block_sums(r2[c]);
-                    const size_t e = (size_t)row * cpr + 2 * pc + c;
-                    if (threadIdx.x == 0 && red) write_sums(L.red, e * RED_W, t);
-                    if (DS && threadIdx.x == 0 && L.dsum) { L.dsum[2 * e] = t.dm; L.dsum[2 * e + 1] = t.dd; }
-                }
-            }
+            cs_paired_chunk<S, DS, T>(L, base + (size_t)row * Q * nx, nxt, row, pc * 2 * CS_THREADS, G, om, red, rs);
+            if (red || (DS && L.dsum))  // uniform per workgroup; its halves are the two chunks
+                write_block_sums<DS>(L, rs, (size_t)row * cpr + 2 * pc, 2);
             return;
         }
     }
@@ -374,18 +419,13 @@ __global__ __launch_bounds__(CS_THREADS) void k_collide_stream(Batch<LatArgs> P)
         const int cpr = cs_chunks(nx);
         const int row = b / cpr, chunk = b % cpr;
         const S *__restrict__ cur = base + (size_t)row * Q * nx;
-        if (cs_aligned<S>() && nx % CS_THREADS == 0) {
+        if (cs_aligned<S>() && nx % CS_THREADS == 0 && buf_fits(nx, ny, (int)sizeof(S))) {
             cs_aligned_chunk<S, DS, T>(L, cur, nxt, row, chunk * CS_THREADS, G, om, red, rs);
         } else {
             const int x = chunk * CS_THREADS + threadIdx.x;
             if (x < nx) cs_scatter<S, DS, T>(L, cur, nxt, row, x, G, om, red, rs);  // a partial chunk still sums below
         }
-        if (red || (DS && L.dsum)) {  // uniform per workgroup
-            const RowSums t = block_sums(rs);
-            const size_t e = (size_t)row * cpr + chunk;
-            if (threadIdx.x == 0 && red) write_sums(L.red, e * RED_W, t);
-            if (DS && threadIdx.x == 0 && L.dsum) { L.dsum[2 * e] = t.dm; L.dsum[2 * e + 1] = t.dd; }
-        }
+        if (red || (DS && L.dsum)) write_block_sums<DS>(L, rs, (size_t)row * cpr + chunk, 1);  // uniform per workgroup
     } else {
         // narrow lattice: rpw whole rows per workgroup, one partial per row summed in x order
         const int r = threadIdx.x / nx, x = threadIdx.x - r * nx;
@@ -430,7 +470,6 @@ hipError_t launch_collide_stream(hipStream_t s, const LatArgs *lats, int nlat, i
         int blocks = 0;
         for (int i = 0; i < BATCH_MAX; i++) {
             P.it[i] = lats[i0 + (i < P.n ? i : 0)];
-            P.it[i].paired = (P.it[i].paired >> (ds ? 1 : 0)) & 1;  // the form for this launch
             P.first[i] = blocks;
             if (i < P.n) blocks += cs_blocks(P.it[i].nx, P.it[i].ny * P.it[i].nz, P.it[i].paired);
         }

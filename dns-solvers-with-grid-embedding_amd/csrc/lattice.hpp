@@ -97,21 +97,44 @@ __device__ __forceinline__ Macro64 macro64(const double *f) {
     return m;
 }
 
+// Moments of a node before its collision, returned by the collisions for the fused
+// reductions: sum f (FP64) or sum g (shifted tiers), sum e_x f and u_x.
+template <class T>
+struct PreSums {
+    T zeroth, mx, u0;
+};
+
 // BGK collision with the first-order body force F = 3 w rho e_x G
 // (xcomputations.c:73-85): f <- f + (F - omega (f - feq)).
-__device__ __forceinline__ void collide64(double *f, double G, double omega) {
-    const Macro64 m = macro64(f);
-    unroll<0, Q>([&](auto qc) {
+// Opposite directions share e.u up to its sign, which 3 e.u and (4.5 e.u) e.u carry
+// exactly, so those are formed once per pair: 36 of about 300 operations less, with
+// every result bit for bit that of feq64 on each direction.
+__device__ __forceinline__ PreSums<double> collide64(double *f, double G, double omega) {
+    const double ux = first_moment<0>(f), uy = first_moment<1>(f), uz = first_moment<2>(f);
+    const double dens = zeroth_moment(f);
+    const double u0 = ux / dens, u1 = uy / dens, u2 = uz / dens;
+    const double c = 1.5 * (u0 * u0 + u1 * u1 + u2 * u2);
+    auto relax = [&](auto qc, double feq) __attribute__((always_inline)) {
         constexpr int q = decltype(qc)::value;
-        const double feq = feq64<q>(m.dens, m.u0, m.u1, m.u2, m.v);
         const double t = omega * (f[q] - feq);
         if constexpr (EX[q] == 0) {
             f[q] = f[q] - t;
         } else {
-            const double Fi = BIQ[q] * m.dens * (EX[q] > 0 ? G : -G);
+            const double Fi = BIQ[q] * dens * (EX[q] > 0 ? G : -G);
             f[q] = f[q] + (Fi - t);
         }
+    };
+    unroll<0, Q>([&](auto qc) {
+        constexpr int q = decltype(qc)::value;
+        if constexpr (q == 0) {
+            relax(qc, WQ[0] * dens * (1. - c));
+        } else if constexpr (OPP[q] > q) {
+            const double eu = edot<q>(u0, u1, u2), a = 3. * eu, b = 4.5 * eu * eu;
+            relax(qc, WQ[q] * dens * (1. + a + b - c));
+            relax(std::integral_constant<int, OPP[q]>{}, WQ[q] * dens * (1. - a + b - c));
+        }
     });
+    return {dens, ux, u0};
 }
 
 // ---- precision tier: shifted storage g = f - w*rho0, FP32 collision ---------
@@ -140,18 +163,34 @@ __device__ __forceinline__ float geq32(const Macro32 &m) {
     return float(WQ[q]) * (m.drho + m.dens * (3.f * eu + 4.5f * eu * eu - 1.5f * m.v));
 }
 
-__device__ __forceinline__ void collide32(float *g, float G, float omega) {
-    const Macro32 m = macro32(g);
-    unroll<0, Q>([&](auto qc) {
+// as collide64: 3 e.u and (4.5 e.u) e.u once per pair of opposite directions, the same
+// bits as geq32 on each
+__device__ __forceinline__ PreSums<float> collide32(float *g, float G, float omega) {
+    const float drho = zeroth_moment(g), dens = 1.f + drho, inv = 1.f / dens;
+    const float mx = first_moment<0>(g);
+    const float u0 = mx * inv, u1 = first_moment<1>(g) * inv, u2 = first_moment<2>(g) * inv;
+    const float c = 1.5f * (u0 * u0 + u1 * u1 + u2 * u2);
+    auto relax = [&](auto qc, float geq) __attribute__((always_inline)) {
         constexpr int q = decltype(qc)::value;
-        const float t = omega * (g[q] - geq32<q>(m));
+        const float t = omega * (g[q] - geq);
         if constexpr (EX[q] == 0) {
             g[q] = g[q] - t;
         } else {
-            const float Fi = float(BIQ[q]) * m.dens * (EX[q] > 0 ? G : -G);
+            const float Fi = float(BIQ[q]) * dens * (EX[q] > 0 ? G : -G);
             g[q] = g[q] + (Fi - t);
         }
+    };
+    unroll<0, Q>([&](auto qc) {
+        constexpr int q = decltype(qc)::value;
+        if constexpr (q == 0) {
+            relax(qc, float(WQ[0]) * (drho + dens * (0.f - c)));
+        } else if constexpr (OPP[q] > q) {
+            const float eu = edot<q>(u0, u1, u2), a = 3.f * eu, b = 4.5f * eu * eu;
+            relax(qc, float(WQ[q]) * (drho + dens * (a + b - c)));
+            relax(std::integral_constant<int, OPP[q]>{}, float(WQ[q]) * (drho + dens * (b - a - c)));
+        }
     });
+    return {drho, mx, u0};
 }
 
 // storage conversions for the shifted tiers

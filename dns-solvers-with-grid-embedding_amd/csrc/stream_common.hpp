@@ -1,7 +1,7 @@
 // stream_common.hpp -- device helpers shared by the collide-stream kernels
 // (k_stream.hip) and the two-substep band kernel (k_band2.hip): the compute type
-// of each storage type, the collision dispatch, the fused-reduction sums and the
-// push of one collided node to its 19 targets with the wall rules.
+// of each storage type, the collision dispatch, row-wise access through buffer
+// resources and the fused-reduction sums.
 #pragma once
 #include "internal.hpp"
 #include "lattice.hpp"
@@ -17,8 +17,75 @@ struct ComputeOf<double> {
     using T = double;
 };
 
-__device__ __forceinline__ void collide_any(double *f, double G, double om) { collide64(f, G, om); }
-__device__ __forceinline__ void collide_any(float *f, float G, float om) { collide32(f, G, om); }
+__device__ __forceinline__ PreSums<double> collide_any(double *f, double G, double om) { return collide64(f, G, om); }
+__device__ __forceinline__ PreSums<float> collide_any(float *f, float G, float om) { return collide32(f, G, om); }
+
+// Row-wise access through buffer resources: the base of a layer and the row and
+// direction offset are scalars, so a lane holds one 32-bit offset for all 19 directions
+// (as 64-bit addresses, 19 loads or stores in flight take 38 VGPRs), and a lane that
+// must not store takes the offset DROP, which lies past every resource and is dropped
+// by the resource's bounds check, so that stores need no branches.  Layers must be
+// below 2 GiB (buf_fits).
+constexpr unsigned DROP = 0x80000000u;
+typedef __amdgpu_buffer_rsrc_t Rsrc;
+typedef unsigned u2v __attribute__((ext_vector_type(2)));
+// p and bytes must be the same over the wave (they are made scalars: without that, where
+// the compiler cannot prove it, each access becomes a loop over the wave's values)
+__device__ __forceinline__ Rsrc buf_rsrc(const void *p, unsigned bytes) {
+    const unsigned long long a = reinterpret_cast<unsigned long long>(p);
+    const unsigned lo = __builtin_amdgcn_readfirstlane((int)(unsigned)a), hi = __builtin_amdgcn_readfirstlane((int)(a >> 32));
+    void *u = reinterpret_cast<void *>((unsigned long long)hi << 32 | lo);
+    return __builtin_amdgcn_make_buffer_rsrc(u, 0, __builtin_amdgcn_readfirstlane((int)bytes), 0x00027000);
+}
+// loads: v the lane's byte offset, s the scalar one; the pointer names the storage type
+__device__ __forceinline__ double buf_load(Rsrc R, unsigned v, unsigned s, const double *) {
+    return __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(R, v, s, 0));
+}
+__device__ __forceinline__ float buf_load(Rsrc R, unsigned v, unsigned s, const float *) {
+    return __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(R, v, s, 0));
+}
+__device__ __forceinline__ float buf_load(Rsrc R, unsigned v, unsigned s, const __half *) {
+    const unsigned short a = __builtin_amdgcn_raw_buffer_load_b16(R, v, s, 0);
+    return __half2float(__builtin_bit_cast(__half, a));
+}
+__device__ __forceinline__ void buf_load_pair(Rsrc R, unsigned v, unsigned s, const float *, float &a, float &b) {
+    const u2v d = __builtin_amdgcn_raw_buffer_load_b64(R, v, s, 0);
+    a = __uint_as_float(d.x);
+    b = __uint_as_float(d.y);
+}
+__device__ __forceinline__ void buf_load_pair(Rsrc R, unsigned v, unsigned s, const __half *, float &a, float &b) {
+    const __half2 d = __builtin_bit_cast(__half2, __builtin_amdgcn_raw_buffer_load_b32(R, v, s, 0));
+    a = __low2float(d);
+    b = __high2float(d);
+}
+// stores; AUX 2: non-temporal.  At most 8 bytes a lane: 16-byte buffer stores of FP64
+// pairs wrote sporadically wrong values here (the data registers can be rewritten before
+// a store of more than 8 bytes has read them, which the compiler does not guard where
+// the scalar offset is a register).
+template <int AUX>
+__device__ __forceinline__ void buf_store(Rsrc R, unsigned v, unsigned s, const double *, double a) {
+    __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u2v, a), R, v, s, AUX);
+}
+template <int AUX>
+__device__ __forceinline__ void buf_store(Rsrc R, unsigned v, unsigned s, const float *, float a) {
+    __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(a), R, v, s, AUX);
+}
+template <int AUX>
+__device__ __forceinline__ void buf_store(Rsrc R, unsigned v, unsigned s, const __half *, float a) {
+    __builtin_amdgcn_raw_buffer_store_b16(__builtin_bit_cast(unsigned short, __float2half(a)), R, v, s, AUX);
+}
+template <int AUX>
+__device__ __forceinline__ void buf_store_pair(Rsrc R, unsigned v, unsigned s, const float *, float a, float b) {
+    asm("" : "+v"(a));  // else the compiler reads the pair as 8 bytes of the array holding a, which keeps it in memory
+    u2v d;
+    d.x = __float_as_uint(a);
+    d.y = __float_as_uint(b);
+    __builtin_amdgcn_raw_buffer_store_b64(d, R, v, s, AUX);
+}
+template <int AUX>
+__device__ __forceinline__ void buf_store_pair(Rsrc R, unsigned v, unsigned s, const __half *, float a, float b) {
+    __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, __halves2half2(__float2half(a), __float2half(b))), R, v, s, AUX);
+}
 
 __device__ __forceinline__ double wave_sum64(double v) {
 #pragma unroll
@@ -35,97 +102,27 @@ __device__ __forceinline__ int xcd_remap(int b, int nb) {
     return (b < (per << 3)) ? (b & 7) * per + (b >> 3) : b;
 }
 
+// density and u_x of a node from its collision's moments, in FP64 in every tier
+__device__ __forceinline__ double pre_rho(const PreSums<double> &p) { return p.zeroth; }
+__device__ __forceinline__ double pre_rho(const PreSums<float> &p) { return 1. + (double)p.zeroth; }
+__device__ __forceinline__ double pre_u(const PreSums<double> &p) { return p.u0; }
+__device__ __forceinline__ double pre_u(const PreSums<float> &p) { return (double)p.mx / pre_rho(p); }
+
 // fused-reduction sums of one thread's nodes: pre-collision moments (rho, mom, u)
 // and the destination-weighted sums of what it writes (dm, dd)
 struct RowSums {
     double rho = 0., mom = 0., u = 0., dm = 0., dd = 0.;
     template <class S, class T>
-    __device__ __forceinline__ void add(const T *f) {
-        double d, m;
-        if constexpr (sizeof(S) == 8) {
-            m = first_moment<0>(f);
-            d = zeroth_moment(f);
-        } else {
-            m = (double)first_moment<0>(f);
-            d = 1. + (double)zeroth_moment(f);
-        }
-        rho += d;
-        mom += m;
-        u += m / d;
+    __device__ __forceinline__ void add(const PreSums<T> &p) {
+        rho += pre_rho(p);
+        mom += (double)p.mx;
+        u += pre_u(p);
     }
 };
 
 // encalc2 weight of a destination layer (LatArgs::dsum)
 __device__ __forceinline__ double dest_w(const LatArgs &L, int zt) {
     return (zt < L.klo || zt > L.khi) ? 0. : (zt == L.khalf ? 0.5 * L.kscale : L.kscale);
-}
-
-// add a store of direction d (e_x = ex) and f-value fv into a layer of weight W
-__device__ __forceinline__ void add_write(RowSums &rs, double W, int ex, double fv) {
-    const double a = W * fv;
-    rs.dd += a;
-    if (ex > 0) rs.dm += a;
-    else if (ex < 0) rs.dm -= a;
-}
-
-
-// Push of the collided node at x of row (y, z) = row: each direction to its target
-// (x + e_x, y + e_y, z + e_z) with the boundary rules at the stored z ends
-// (xfcomputations.c:215-442):
-//   BOUND_DROP  populations leaving the lattice are not written, nor are those
-//               entering a skipped layer (rewritten by an interface transfer)
-//   BOUND_WALL  target on the wall with code s(t) in {-1, -2}, s1 the code below
-//               the source: s(t) = -1 and s1 = -1 -> halfway bounce-back
-//               f(x, opp q); otherwise specular reflection f(x + e_xy, mirror q)
-// With DS and L.dsum, the destination-weighted sums of the writes go into rs.
-// The wall codes come from wcode(zs, dx, dy, xt, yt): the code of the wall at the
-// in-plane offset (dx, dy) from the node, (xt, yt) in lattice coordinates, on the lo
-// (zs < 0) or hi wall.
-struct WallCodesGlobal {
-    const LatArgs &L;
-    __device__ __forceinline__ int operator()(int zs, int, int, int xt, int yt) const {
-        const int8_t *wc = zs < 0 ? L.wlo : L.whi;
-        return wc[(size_t)yt * L.nx + xt];
-    }
-};
-
-template <class S, bool DS, class T, class WC>
-__device__ __forceinline__ void scatter_push(const LatArgs &L, S *__restrict__ nxt, int row, int x, const T *f,
-                                             RowSums &rs, const WC &wcode) {
-    const int nx = L.nx, ny = L.ny, nz = L.nz;
-    const int y = row % ny, z = row / ny;
-    const bool lo_edge = (z == 0), hi_edge = (z == nz - 1);
-    const int ym = (y == 0) ? ny - 1 : y - 1, yp = (y == ny - 1) ? 0 : y + 1;
-    const bool ds = DS && L.dsum != nullptr;  // DS: compiled in only where a launch asks for it
-    const double wz[3] = {ds ? dest_w(L, z - 1) : 0., ds ? dest_w(L, z) : 0., ds ? dest_w(L, z + 1) : 0.};
-    const int xm = (x == 0) ? nx - 1 : x - 1, xp = (x == nx - 1) ? 0 : x + 1;
-    unroll<0, Q>([&](auto qc) {
-        constexpr int q = decltype(qc)::value;
-        const int xt = (EX[q] > 0) ? xp : (EX[q] < 0 ? xm : x);
-        const int yt = (EY[q] > 0) ? yp : (EY[q] < 0 ? ym : y);
-        if constexpr (EZ[q] != 0) {
-            const bool at_end = (EZ[q] < 0) ? lo_edge : hi_edge;
-            if (at_end) {
-                const int kind = (EZ[q] < 0) ? L.lo_kind : L.hi_kind;
-                if (kind == BOUND_WALL) {
-                    const int sld = wcode(EZ[q], EX[q], EY[q], xt, yt);
-                    const int sld1 = wcode(EZ[q], 0, 0, x, y);
-                    if (sld == -1 && sld1 == -1) {
-                        store_s(nxt + lat_at(OPP[q], (size_t)row, x, nx), f[q]);
-                        if (ds) add_write(rs, wz[1], -EX[q], read_back<S, q>(f[q]));
-                    } else {
-                        store_s(nxt + lat_at(MIR[q], (size_t)z * ny + yt, xt, nx), f[q]);
-                        if (ds) add_write(rs, wz[1], EX[q], read_back<S, q>(f[q]));
-                    }
-                }
-                return;
-            }
-        }
-        const int zt = z + EZ[q];
-        if ((zt == 0 && L.skip_lo) || (zt == nz - 1 && L.skip_hi)) return;
-        store_s(nxt + lat_at(q, (size_t)zt * ny + yt, xt, nx), f[q]);
-        if (ds) add_write(rs, wz[EZ[q] + 1], EX[q], read_back<S, q>(f[q]));
-    });
 }
 
 }  // namespace dnsg
