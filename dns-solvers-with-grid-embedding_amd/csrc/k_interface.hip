@@ -681,10 +681,15 @@ struct FltrArgs {
     int zdf, Xc, Yc, GR;
     double fac;             // GR tau_c / tau_f
     void *coarse;           // coarse post-stream lattice
-    double *fneq;           // [side][19][5][Yf][Xf]
+    double *fneq;           // [side][19][5][Yf][fltr_col(0 .. Xf-1)]
     double *psum;           // as FtcdItem::psum
     const int *halt;        // as Batch::halt
 };
+
+// place of fine column i in a row of f_neq: columns of equal i mod 4 together, so that the
+// coarse nodes of a wave, every fourth column, read consecutive values (GR = 4; read
+// through strided lines, the filter launch took 181 us at coarse 128 x 64)
+__device__ __forceinline__ int fltr_col(int i, int Xf) { return (i & 3) * (Xf >> 2) + (i >> 2); }
 
 // the 19 values of fine node (i, j, k) of one band in double: f (FP64) or the
 // shifted g = f - w (FP32 / FP16 storage); the band's wall layer is not stored in
@@ -719,7 +724,7 @@ __global__ __launch_bounds__(256) void k_fltr_slab(FltrArgs A) {
     const int side = l / 5, kk = l % 5;
     double f[Q];
     fltr_node<S>(A, side, i, j, A.kf[side] + kk - 2, f);
-    double *o = A.fneq + ((size_t)side * Q * 5 + kk) * plane + (size_t)j * Xf + i;
+    double *o = A.fneq + ((size_t)side * Q * 5 + kk) * plane + (size_t)j * Xf + fltr_col(i, Xf);
     if constexpr (sizeof(S) == 8) {  // :160-200, the moments in ftcdtransfer's order
         const Macro64 m = macro64(f);
         unroll<0, Q>([&](auto qq) {
@@ -738,76 +743,77 @@ __global__ __launch_bounds__(256) void k_fltr_slab(FltrArgs A) {
     }
 }
 
-// workgroups [0, nb) filter the lower band, [nb, 2 nb) the upper band (k_ftcd's layout)
+// One thread per coarse node and direction (blockIdx.y): the 125 terms of a node are a
+// serial chain of adds in the reference's order, so the parallelism is over nodes and
+// directions: one thread per node left the launch at 64 workgroups with 2375 terms a
+// thread (coarse 128 x 64: 794 us; now 80 us, at 311 MB of reads through L2).  Each thread forms the node's moments from its 19 values
+// again.  A term's weight is 0 or a power of two and so is 1 / GR^3 (GR = 4), so w f_neq /
+// GR^3 is exact and its add one fused operation with the reference's rounding.
+// Workgroups [0, nb) of a direction filter the lower band, [nb, 2 nb) the upper band.
 template <class S>
 __global__ __launch_bounds__(256) void k_fltr(FltrArgs A) {
     if (halted(A.halt)) return;
     const int Xc = A.Xc, Yc = A.Yc, GR = A.GR, Xf = GR * Xc, Yf = GR * Yc;
-    const int n = Xc * Yc, nb = (n + 255) / 256;
+    const int n = Xc * Yc, nb = (n + 255) / 256, q = blockIdx.y;
     const int side = (int)blockIdx.x >= nb ? 1 : 0;
     const int id = ((int)blockIdx.x - side * nb) * 256 + threadIdx.x;
     double sm = 0., sd = 0.;
     if (id < n) {
         const int ic = id % Xc, jc = id / Xc, i = GR * ic, j = GR * jc;
         const size_t plane = (size_t)Xf * Yf;
-        const double *src = A.fneq + (size_t)side * Q * 5 * plane;
-        constexpr double wl[5] = {0.5, 1., 1., 1., 0.5};
-        const double den = (double)GR * GR * GR;
-        double acc[Q];
-        unroll<0, Q>([&](auto qq) { acc[decltype(qq)::value] = 0.; });
-        for (int ii = 0; ii < 5; ii++) {
-            const int in = (i + ii - 2 + Xf) % Xf;
-            for (int jj = 0; jj < 5; jj++) {
-                const int jn = (j + jj - 2 + Yf) % Yf;
-                const double *p = src + (size_t)jn * Xf + in;
-#pragma unroll
-                for (int kk = 0; kk < 5; kk++) {
-                    const double wt = wl[ii] * wl[jj] * wl[kk];
-                    unroll<0, Q>([&](auto qq) {
-                        constexpr int q = decltype(qq)::value;
-                        acc[q] += (wt * p[((size_t)q * 5 + kk) * plane]) / den;
-                    });
-                }
-            }
-        }
+        const double *src = A.fneq + ((size_t)side * Q + q) * 5 * plane;
         double f[Q];
         fltr_node<S>(A, side, i, j, A.kf[side], f);
+        int row[5];
+#pragma unroll
+        for (int jj = 0; jj < 5; jj++) row[jj] = ((j + jj - 2 + Yf) % Yf) * Xf;
+        double acc = 0.;
+        unroll<0, 5>([&](auto ic5) {
+            constexpr int ii = decltype(ic5)::value;
+            const double *col = src + fltr_col((i + ii - 2 + Xf) % Xf, Xf);
+            unroll<0, 5>([&](auto jc5) {
+                constexpr int jj = decltype(jc5)::value;
+                unroll<0, 5>([&](auto kc5) {
+                    constexpr int kk = decltype(kc5)::value;
+                    constexpr double wl[5] = {0.5, 1., 1., 1., 0.5};
+                    acc = fma_exact(wl[ii] * wl[jj] * wl[kk] / 64., col[row[jj] + (size_t)kk * plane], acc);
+                });
+            });
+        });
         S *cs = static_cast<S *>(A.coarse);
-        const size_t drow = (size_t)A.kc[side] * Yc + jc;
+        const size_t at = (((size_t)A.kc[side] * Yc + jc) * Q + q) * Xc + ic;  // lat_at
         // rho and the raw first moments of the coincident node (not divided by rho)
         const double dsum = zeroth_moment(f);
         const double m0 = first_moment<0>(f), m1 = first_moment<1>(f), m2 = first_moment<2>(f);
         const double v = m0 * m0 + m1 * m1 + m2 * m2;
-        if constexpr (sizeof(S) == 8) {
-            unroll<0, Q>([&](auto qq) {
-                constexpr int q = decltype(qq)::value;
-                const double out = feq64<q>(dsum, m0, m1, m2, v) + A.fac * acc[q];
-                cs[lat_at(q, drow, ic, Xc)] = out;
-                sd += out;
-                if constexpr (EX[q] > 0) sm += out;
-                if constexpr (EX[q] < 0) sm -= out;
-            });
-        } else {  // shifted: feq - w = w (drho + rho (3 eu + 4.5 eu^2 - 1.5 v))
-            const double drho = dsum, dens = 1. + drho;
-            unroll<0, Q>([&](auto qq) {
-                constexpr int q = decltype(qq)::value;
-                const double eu = edot<q>(m0, m1, m2);
-                const double geq = WQ[q] * (drho + dens * (3. * eu + 4.5 * eu * eu - 1.5 * v));
-                const float out = (float)(geq + A.fac * acc[q]);
-                store_s(cs + lat_at(q, drow, ic, Xc), out);
-                const double fv = read_back<S, q>(out);
-                sd += fv;
-                if constexpr (EX[q] > 0) sm += fv;
-                if constexpr (EX[q] < 0) sm -= fv;
-            });
-        }
+        double out = 0.;
+        int ex = 0;
+        unroll<0, Q>([&](auto qq) {  // q is uniform over the workgroup
+            constexpr int QD = decltype(qq)::value;
+            if (q != QD) return;
+            ex = EX[QD];
+            if constexpr (sizeof(S) == 8) {
+                out = feq64<QD>(dsum, m0, m1, m2, v) + A.fac * acc;
+                store_s(cs + at, out);
+            } else {  // shifted: feq - w = w (drho + rho (3 eu + 4.5 eu^2 - 1.5 v))
+                const double drho = dsum, dens = 1. + drho;
+                const double eu = edot<QD>(m0, m1, m2);
+                const double geq = WQ[QD] * (drho + dens * (3. * eu + 4.5 * eu * eu - 1.5 * v));
+                const float g = (float)(geq + A.fac * acc);
+                store_s(cs + at, g);
+                out = read_back<S, QD>(g);
+            }
+        });
+        sd = out;
+        sm = ex > 0 ? out : (ex < 0 ? -out : 0.);
     }
     if (A.psum) {  // uniform per workgroup
         const double w = 0.5 * GR * GR * GR;
         sm *= w;
         sd *= w;
         wg_sum2(sm, sd);
-        if (threadIdx.x == 0) { A.psum[2 * blockIdx.x] = sm; A.psum[2 * blockIdx.x + 1] = sd; }
+        const size_t e = (size_t)q * gridDim.x + blockIdx.x;
+        if (threadIdx.x == 0) { A.psum[2 * e] = sm; A.psum[2 * e + 1] = sd; }
     }
 }
 
@@ -818,7 +824,7 @@ template <class S>
 static hipError_t fltr_launch(hipStream_t s, const FltrArgs &A, int nb) {
     const size_t nslab = 10 * (size_t)A.GR * A.Xc * A.GR * A.Yc;
     hipLaunchKernelGGL(k_fltr_slab<S>, dim3((unsigned)((nslab + 255) / 256)), dim3(256), 0, s, A);
-    hipLaunchKernelGGL(k_fltr<S>, dim3(nb), dim3(256), 0, s, A);
+    hipLaunchKernelGGL(k_fltr<S>, dim3(nb, Q), dim3(256), 0, s, A);
     return hipGetLastError();
 }
 
@@ -830,13 +836,13 @@ static hipError_t launch_fltr(hipStream_t s, dnsg_ctx *h, double *psum) {
     FltrArgs A = {{h->lower.n(), h->upper.n()}, {h->fwall, h->fwall + nw}, {zdf - 1 - GR, GR}, {0, h->d.zdc - 1},
                   zdf, h->d.Xc, h->d.Yc, GR, GR * (h->d.omega_f / h->d.omega_c), h->coarse.n(), h->fneq, psum,
                   h->halt()};
-    const int nb = ftcd_blocks(h);
+    const int nb = ftcd_blocks(h) / Q;
     if (h->p.precision == DNSG_PREC_FP64) return fltr_launch<double>(s, A, nb);
     if (h->p.precision == DNSG_PREC_FP32) return fltr_launch<float>(s, A, nb);
     return fltr_launch<__half>(s, A, nb);
 }
 
-int ftcd_blocks(const dnsg_ctx *h) { return 2 * ((h->d.Xc * h->d.Yc + 255) / 256); }
+int ftcd_blocks(const dnsg_ctx *h) { return 2 * ((h->d.Xc * h->d.Yc + 255) / 256) * (h->p.fltr ? Q : 1); }
 
 hipError_t launch_ftcd_many(hipStream_t s, dnsg_ctx *const *hs, int n, double *psum) {
     if (n < 1) return hipSuccess;
