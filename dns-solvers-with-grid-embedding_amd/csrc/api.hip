@@ -195,7 +195,7 @@ LatArgs coarse_args(dnsg_t *h) {
     L.red = nullptr;
     L.force = h->d_force;
     L.dsum = nullptr;
-    L.paired = h->cs_pair && cs_paired(L.nx, L.ny, (int)h->elem);
+    L.form = cs_form(L.nx, L.ny, (int)h->elem, h->cs_pair);
     set_dest_weights(h, 0, &L);
     return L;
 }
@@ -220,13 +220,13 @@ void band_args(dnsg_t *h, LatArgs *L) {
         L[b].red = nullptr;
         L[b].force = h->d_force;
         L[b].dsum = nullptr;
-        L[b].paired = h->cs_pair && cs_paired(g.nx, g.ny, (int)h->elem);
+        L[b].form = cs_form(g.nx, g.ny, (int)h->elem, h->cs_pair);
         set_dest_weights(h, 1 + b, &L[b]);
     }
 }
 
 double *red_coarse(dnsg_t *h) { return h->red; }
-double *red_lower(dnsg_t *h) { return h->red + (size_t)h->coarse.ny * h->coarse.nz * cs_chunks(h->coarse.nx) * RED_W; }
+double *red_lower(dnsg_t *h) { return h->red + coarse_parts_max(h->d) * RED_W; }
 double *red_upper(dnsg_t *h) { return red_lower(h) + band_parts_max(h->d) * RED_W; }
 
 void rotate_levels(dnsg_t *h) {  // xcomputations.c:548-556
@@ -353,8 +353,8 @@ int do_step_band2(dnsg_t *h, double *rec, SecTimer *T) {
     B[0].red = red_lower(h);
     B[1].red = red_upper(h);
     if (flux) {
-        B[0].dsum = h->dsum + 2 * (size_t)h->d.Yc * h->d.zdc * cs_chunks(h->d.Xc);
-        B[1].dsum = B[0].dsum + band_dsum_doubles(h);
+        B[0].dsum = dsum_band(h, 0);
+        B[1].dsum = dsum_band(h, 1);
     }
     if (T) T->begin(h->stream, SEC_BAND);
     HIPCHK(h, launch_band2(h->stream, B, h->p.precision, h->halt()));
@@ -395,8 +395,6 @@ int do_step(dnsg_t *h, double *rec, SecTimer *T = nullptr) {
         HIPCHK(h, launch_encalc2(h->stream, h, rec));
         if (T) T->end(h->stream, SEC_REDUCE);
     }
-    double *dl = h->dsum + 2 * (size_t)h->d.Yc * h->d.zdc * cs_chunks(h->d.Xc);
-    double *du = dl + band_dsum_doubles(h);
     for (int iter = 1; iter <= GR; iter++) {
         LatArgs L[3];
         LatArgs *B = L;  // the band pair of this substep
@@ -414,8 +412,8 @@ int do_step(dnsg_t *h, double *rec, SecTimer *T = nullptr) {
             B[1].red = red_upper(h);
         }
         if (flux && iter == GR) {  // the last substep writes the bands' next state
-            B[0].dsum = dl;
-            B[1].dsum = du;
+            B[0].dsum = dsum_band(h, 0);
+            B[1].dsum = dsum_band(h, 1);
         }
         if (T) T->begin(h->stream, iter == 1 ? SEC_COARSE : SEC_BAND);
         HIPCHK(h, launch_collide_stream(h->stream, L, nl, h->p.precision, h->halt()));
@@ -908,7 +906,7 @@ int dnsg::create_ctx(const dnsg_params *p, hipStream_t ext, dnsg_t **out) {
     HIPCHK(h, hipMalloc(&h->part, h->part_cap * 8));
     {
         const size_t nred =
-            ((size_t)d.Yc * d.zdc * cs_chunks(d.Xc) + 2 * band_parts_max(d)) * RED_W;
+            (coarse_parts_max(d) + 2 * band_parts_max(d)) * RED_W;
         HIPCHK(h, hipMalloc(&h->red, nred * 8));
         HIPCHK(h, hipMemsetAsync(h->red, 0, nred * 8, h->stream));
         HIPCHK(h, hipMalloc(&h->seg, enc_seg_doubles(h) * 8));

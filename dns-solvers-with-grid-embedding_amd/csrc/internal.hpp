@@ -43,14 +43,14 @@ struct LatArgs {
     double gscale;         // G = gscale * force (1 for coarse, 1/GR for the bands)
     double omega;          // 1/tau
     int skip_lo, skip_hi;  // do not write into layer 0 / nz-1 (rewritten by the interface)
-    double *red;           // if set: per-row sums of the pre-collision state, RED_W per row
+    double *red;           // if set: sums of the pre-collision state, RED_W per partial (cs_parts)
     const double *force;   // V.force[0] of the solve this lattice belongs to
-    // if set: per-(row, chunk) sums over the values this launch writes, each weighted
-    // by the encalc2 weight of its destination layer: [sum w e_x f, sum w f].  Layers
+    // if set: per-partial sums over the values this launch writes, each weighted by the
+    // encalc2 weight of its destination layer: [sum w e_x f, sum w f].  Layers
     // klo..khi carry kscale (khalf: half of it), all others 0.
     double *dsum;
     int klo, khi, khalf;
-    int paired;  // the paired collide-stream form (cs_paired)
+    int form;    // how the collide-stream takes the lattice (CsForm)
     double kscale;
 };
 
@@ -79,30 +79,33 @@ __device__ __forceinline__ int batch_find(const int *first, int n, int b) {
 // per-(row, chunk) sums written by the collide-stream kernels when LatArgs::red
 // is set: sum rho, sum rho u_x, sum u_x (u_x = rho u_x / rho)
 constexpr int RED_W = 3;
-// threads (= nodes) per collide-stream workgroup and chunks per lattice row
-#ifndef DNSG_CS_THREADS
-#define DNSG_CS_THREADS 256
-#endif
-constexpr int CS_THREADS = DNSG_CS_THREADS;
+// threads per collide-stream workgroup and chunks of them per lattice row
+constexpr int CS_THREADS = 256;
 __host__ __device__ __forceinline__ int cs_chunks(int nx) { return (nx + CS_THREADS - 1) / CS_THREADS; }
-// lattices narrower than a workgroup: each workgroup takes this many whole rows
-__host__ __device__ __forceinline__ int cs_rows_per_wg(int nx) { return nx >= CS_THREADS ? 1 : CS_THREADS / nx; }
 // a layer can be addressed with 31-bit byte offsets (the buffer-resource forms)
 __host__ __device__ __forceinline__ bool buf_fits(int nx, int ny, int elem) {
     return (size_t)nx * ny * 19 * elem < ((size_t)1 << 31);
 }
-// Paired collide-stream form: rows of FP32 / FP16 values that are a multiple of 2
-// CS_THREADS nodes are taken two chunks per workgroup, two adjacent nodes per thread, with
-// 2-value loads and stores.  Measured on the Re_tau=180 lattices against one node per
-// thread: FP32 coarse launch 0.956 -> 0.852 ms, FP16 0.599 -> 0.586 ms.
-__host__ __device__ __forceinline__ bool cs_paired(int nx, int ny, int elem) {
-    return elem != 8 && nx % (2 * CS_THREADS) == 0 && buf_fits(nx, ny, elem);
+// How the collide-stream takes a lattice (k_stream.hip):
+//   CS_ALIGNED  FP64 rows of whole chunks: stores aligned to the workgroup's own positions
+//   CS_PAIRED   FP32 / FP16 rows of two whole chunks: two adjacent nodes per thread.
+//               Measured on the Re_tau=180 lattices against one node per thread: FP32
+//               coarse launch 0.956 -> 0.852 ms, FP16 0.599 -> 0.586 ms
+//   CS_FLAT     any other rows: consecutive nodes of a layer, whatever rows they fall in
+//   CS_WIDE     layers of 2 GiB and more: one row chunk per workgroup, 64-bit addresses
+enum CsForm { CS_ALIGNED, CS_PAIRED, CS_FLAT, CS_WIDE };
+inline int cs_form(int nx, int ny, int elem, bool pair) {
+    if (!buf_fits(nx, ny, elem)) return CS_WIDE;
+    if (elem == 8 && nx % CS_THREADS == 0) return CS_ALIGNED;
+    if (elem != 8 && pair && nx % (2 * CS_THREADS) == 0) return CS_PAIRED;
+    return CS_FLAT;
 }
-// collide-stream workgroups of one lattice with `rows` rows of nx nodes
-__host__ __device__ __forceinline__ int cs_blocks(int nx, int rows, bool paired) {
-    if (paired) return rows * (cs_chunks(nx) / 2);
-    const int rpw = cs_rows_per_wg(nx);
-    return rpw == 1 ? rows * cs_chunks(nx) : (rows + rpw - 1) / rpw;
+// partials of the fused sums per layer, and workgroups of a launch per layer
+__host__ __device__ __forceinline__ int cs_parts(int form, int nx, int ny) {
+    return form == CS_FLAT ? (nx * ny + CS_THREADS - 1) / CS_THREADS : ny * cs_chunks(nx);
+}
+__host__ __device__ __forceinline__ int cs_blocks(int form, int nx, int ny) {
+    return form == CS_PAIRED ? cs_parts(form, nx, ny) / 2 : cs_parts(form, nx, ny);
 }
 
 struct Grid {
@@ -119,8 +122,8 @@ struct Grid {
 // Tile of the two-substep band kernel (k_band2.hip): rows of a workgroup (ring
 // included), nodes per lane and output columns for elements of `elem` bytes.  When a
 // step runs it (dnsg_ctx::band_tiled), the bands' fused-reduction partials are per
-// (row, b2_cols columns) instead of per (layer, row, CS_THREADS columns), with the layer
-// weights applied: LatArgs::dsum the pair above, LatArgs::red the B2_RED values
+// (row, b2_cols columns) instead of per layer and workgroup, with the layer weights
+// applied: LatArgs::dsum the pair above, LatArgs::red the B2_RED values
 //   [0], [1] sum of rho, rho u_x weighted by encalc2's layer weights
 //   [2]      sum of rho over the layer whose density wshearstr takes
 //   [3..5]   sum of u_x over the three layers next to the wall, nearest first
@@ -161,7 +164,7 @@ struct dnsg_ctx {
     // fused-reduction partials of the last launch that wrote them are that kernel's
     bool band2 = false;
     bool band_tiled = false;
-    bool cs_pair = true;  // FP32 / FP16: the paired collide-stream form where the rows allow it
+    bool cs_pair = true;  // FP32 / FP16: CS_PAIRED where the rows allow it
     int8_t *wall_lo = nullptr, *wall_up = nullptr;     // [Yf][Xf]
 
     // reductions
@@ -214,21 +217,23 @@ struct dnsg_ctx {
 
 namespace dnsg {
 
-// fused-reduction partials per row of a band (and layer, where not band_tiled) in the
-// current layout, and the partials of RED_W values a band's buffer is sized for in
-// either layout
-inline int band_cpr(const dnsg_ctx *h) {
-    const int cols = h->band_tiled ? b2_cols((int)h->elem) : CS_THREADS;
-    return (h->d.Xf + cols - 1) / cols;
+// fused-reduction partials of a coarse layer, and of a band: of a layer, or of the whole
+// band where band_tiled
+inline int coarse_parts(const dnsg_ctx *h) {
+    return cs_parts(cs_form(h->coarse.nx, h->coarse.ny, (int)h->elem, h->cs_pair), h->coarse.nx, h->coarse.ny);
 }
+inline int band_parts(const dnsg_ctx *h) {
+    const Grid &g = h->lower;
+    if (h->band_tiled) return g.ny * ((g.nx + b2_cols((int)h->elem) - 1) / b2_cols((int)h->elem));
+    return cs_parts(cs_form(g.nx, g.ny, (int)h->elem, h->cs_pair), g.nx, g.ny);
+}
+// the partials of RED_W values the buffers are sized for: any layout of the coarse grid,
+// and of one band
+inline size_t coarse_parts_max(const dnsg_dims &d) { return (size_t)d.Yc * d.zdc * cs_chunks(d.Xc); }
 inline size_t band_parts_max(const dnsg_dims &d) {
     const size_t b2 = (size_t)d.Yf * ((d.Xf + b2_cols(8) - 1) / b2_cols(8)) * (B2_RED / RED_W);
     const size_t cs = (size_t)d.Yf * (d.zdf - 1) * cs_chunks(d.Xf);
     return b2 > cs ? b2 : cs;
-}
-// doubles from the lower band's dsum partials to the upper band's
-inline size_t band_dsum_doubles(const dnsg_ctx *h) {
-    return 2 * (size_t)h->d.Yf * (h->band_tiled ? 1 : h->d.zdf - 1) * band_cpr(h);
 }
 
 // handle set-up and the per-step argument builders shared by the single-solve
@@ -295,6 +300,7 @@ hipError_t launch_reductions_fused(hipStream_t s, dnsg_ctx *h, double *diag_rec)
 // G of the next step from the destination-weighted sums of this step's writes
 hipError_t launch_flux_next(hipStream_t s, dnsg_ctx *h);
 size_t dsum_doubles(const dnsg_ctx *h);
+double *dsum_band(const dnsg_ctx *h, int band);  // the lower (0) / upper (1) band's part of dsum
 // encalc2 destination weights of one lattice (0 coarse, 1 lower band, 2 upper band)
 void set_dest_weights(const dnsg_ctx *h, int grid, LatArgs *L);
 hipError_t launch_wshear(hipStream_t s, dnsg_ctx *h, double *diag_rec);

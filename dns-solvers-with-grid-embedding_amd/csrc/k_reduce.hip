@@ -148,7 +148,7 @@ struct EncArgs {
     const double *pc, *pl, *pu;
     int st, stb;       // doubles per partial (coarse, bands): [0] sum rho, [1] sum rho u_x
     int tiled;         // the bands' partials are per (row, tile), layer weights applied (B2_RED)
-    int cpr_c, cpr_f;  // partials per row (coarse, bands)
+    int ppl_c, ppl_f;  // partials per layer (coarse, bands; of a whole band where tiled)
     int Yc, zdc, Yf, zds, GR, zdf, NZs, Xf, force_mode;
     double ub, g_const;
     double *force, *diag;
@@ -161,15 +161,15 @@ struct EncSpace {
 };
 __host__ __device__ __forceinline__ EncSpace enc_space(const EncArgs &A) {
     EncSpace S;
-    S.nc = A.Yc * A.zdc * A.cpr_c;                // every coarse layer
+    S.nc = A.zdc * A.ppl_c;                  // every coarse layer
     if (A.tiled) {
-        S.nl = S.nu = A.Yf * A.cpr_f;
+        S.nl = S.nu = A.ppl_f;
         S.nu0 = 0;
         return S;
     }
-    S.nl = A.Yf * (A.zdf - A.GR - 1) * A.cpr_f;  // lower band k = 1 .. zdf-GR-1 (stored m = 0 .. zdf-GR-2)
-    S.nu0 = A.Yf * A.GR * A.cpr_f;                // upper band k = GR .. zdf-2 (stored m = GR .. zds-1)
-    S.nu = A.Yf * A.zds * A.cpr_f - S.nu0;
+    S.nl = (A.zdf - A.GR - 1) * A.ppl_f;     // lower band k = 1 .. zdf-GR-1 (stored m = 0 .. zdf-GR-2)
+    S.nu0 = A.GR * A.ppl_f;                  // upper band k = GR .. zdf-2 (stored m = GR .. zds-1)
+    S.nu = A.zds * A.ppl_f - S.nu0;
     return S;
 }
 
@@ -180,13 +180,13 @@ __device__ __forceinline__ void enc_entry(const EncArgs &A, const EncSpace &S, i
         v[1] += A.pl[(size_t)e * A.stb + 0];
     } else if (e < S.nl + S.nc) {
         e -= S.nl;
-        const int z = (e / A.cpr_c) / A.Yc;
+        const int z = e / A.ppl_c;
         const double c = (z == 0 || z == A.zdc - 1) ? 0.5 * A.GR * A.GR * A.GR : 1. * A.GR * A.GR * A.GR;
         const double m = c * A.pc[(size_t)e * A.st + 1], d = c * A.pc[(size_t)e * A.st + 0];
         v[0] += m; v[1] += d; v[2] += m; v[3] += d;
     } else {
         e = e - S.nl - S.nc + S.nu0;
-        const double c = (!A.tiled && (e / A.cpr_f) / A.Yf == A.GR) ? 0.5 : 1.;  // half weight at k = GR
+        const double c = (!A.tiled && e / A.ppl_f == A.GR) ? 0.5 : 1.;  // half weight at k = GR
         v[0] += c * A.pu[(size_t)e * A.stb + 1];
         v[1] += c * A.pu[(size_t)e * A.stb + 0];
     }
@@ -240,8 +240,7 @@ static hipError_t enc_two_stage(hipStream_t s, const EncArgs &A, double *seg) {
 constexpr int WS_SEG = 512;  // wall-stress entries per first-stage workgroup (launch_reductions_fused)
 
 size_t enc_seg_doubles(const dnsg_ctx *h) {
-    const size_t total = (size_t)h->d.Yc * h->d.zdc * cs_chunks(h->d.Xc) +
-                         2 * band_parts_max(h->d) + (size_t)ftcd_blocks(h);
+    const size_t total = coarse_parts_max(h->d) + 2 * band_parts_max(h->d) + (size_t)ftcd_blocks(h);
     const size_t ws = band_parts_max(h->d);
     return 4 * (total / ENC_SEG + 2 + ws / WS_SEG + 1);
 }
@@ -254,9 +253,9 @@ size_t enc_seg_doubles(const dnsg_ctx *h) {
 // destination layer's encalc2 weight (encalc2.c:37-105), so G = ub - <rho u> of the
 // next step needs no pass over the lattices.
 
-size_t dsum_doubles(const dnsg_ctx *h) {
-    return 2 * ((size_t)h->d.Yc * h->d.zdc * cs_chunks(h->d.Xc) +
-                2 * band_parts_max(h->d));
+size_t dsum_doubles(const dnsg_ctx *h) { return 2 * (coarse_parts_max(h->d) + 2 * band_parts_max(h->d)); }
+double *dsum_band(const dnsg_ctx *h, int band) {
+    return h->dsum + 2 * (coarse_parts_max(h->d) + band * band_parts_max(h->d));
 }
 
 void set_dest_weights(const dnsg_ctx *h, int grid, LatArgs *L) {
@@ -320,12 +319,12 @@ __global__ __launch_bounds__(RB) void k_flux_fin(FluxNextArgs A, const double *s
 
 hipError_t launch_flux_next(hipStream_t s, dnsg_ctx *h) {
     FluxNextArgs A;
-    A.nc = h->d.Yc * h->d.zdc * cs_chunks(h->d.Xc);
-    A.nl = A.nu = (int)(band_dsum_doubles(h) / 2);
+    A.nc = h->d.zdc * coarse_parts(h);
+    A.nl = A.nu = (h->band_tiled ? 1 : h->d.zdf - 1) * band_parts(h);
     A.nf = ftcd_blocks(h);
     A.dc = h->dsum;
-    A.dl = A.dc + 2 * (size_t)A.nc;
-    A.du = A.dl + 2 * (size_t)A.nl;
+    A.dl = dsum_band(h, 0);
+    A.du = dsum_band(h, 1);
     A.fs = h->fsum;
     A.Xf = h->d.Xf; A.Yf = h->d.Yf; A.NZs = h->d.NZs; A.ub = h->p.ub;
     A.force = h->d_force; A.enc = h->enc_next;
@@ -342,8 +341,8 @@ static EncArgs enc_args(dnsg_ctx *h, const double *pc, const double *pl, const d
     A.pc = pc; A.pl = pl; A.pu = pu; A.st = st;
     A.tiled = fused && h->band_tiled;
     A.stb = A.tiled ? B2_RED : st;
-    A.cpr_c = fused ? cs_chunks(h->coarse.nx) : 1;
-    A.cpr_f = fused ? band_cpr(h) : 1;
+    A.ppl_c = fused ? coarse_parts(h) : h->d.Yc;  // the explicit pass sums rows
+    A.ppl_f = fused ? band_parts(h) : h->d.Yf;
     A.Yc = h->d.Yc; A.zdc = h->d.zdc; A.Yf = h->d.Yf; A.zds = h->lower.nz; A.GR = h->d.GR; A.zdf = h->d.zdf;
     A.NZs = h->d.NZs; A.Xf = h->d.Xf; A.force_mode = h->p.force_mode; A.ub = h->p.ub; A.g_const = h->p.g_const;
     A.force = h->d_force; A.diag = diag_rec;
@@ -377,7 +376,7 @@ hipError_t launch_flux_many(hipStream_t s, dnsg_ctx *const *hs, int n, double *o
         for (int i = 0; i < BATCH_MAX; i++) {
             dnsg_ctx *h = hs[i0 + (i < B.n ? i : 0)];
             const double *pc = h->red;
-            const double *pl = pc + (size_t)h->coarse.ny * h->coarse.nz * cs_chunks(h->coarse.nx) * RED_W;
+            const double *pl = pc + coarse_parts_max(h->d) * RED_W;
             const double *pu = pl + band_parts_max(h->d) * RED_W;
             B.it[i] = enc_args(h, pc, pl, pu, RED_W, true, out + 2 * (size_t)slot[i0 + (i < B.n ? i : 0)]);
             B.first[i] = i < B.n ? i : B.n;
@@ -450,11 +449,11 @@ __global__ __launch_bounds__(RB) void k_fin_wshear(WsArgs A) {
     if (threadIdx.x == 0) wshear_finish(A, v);
 }
 
-// wall stress from the sums of the first band substep, one entry per (row, partial):
+// wall stress from the sums of the first band substep, one entry per partial of a layer:
 // sum_x (-2u1 + 3u2 - u3) = -2 S1 + 3 S2 - S3 with S_m = sum_x u_x of layer m
 struct WsSegArgs {
     const double *pl, *pu;  // the bands' fused-reduction partials
-    int Yf, cpr, nz, tiled;
+    int ppl, nz, tiled;     // partials per layer (of the band where tiled)
 };
 
 __device__ __forceinline__ void ws_entry(const WsSegArgs &W, int e, double *v) {
@@ -466,8 +465,7 @@ __device__ __forceinline__ void ws_entry(const WsSegArgs &W, int e, double *v) {
         v[3] += u[2];
         return;
     }
-    const int y = e / W.cpr, c = e % W.cpr;
-    auto at = [&](const double *p, int m, int k) { return p[(((size_t)m * W.Yf + y) * W.cpr + c) * RED_W + k]; };
+    auto at = [&](const double *p, int m, int k) { return p[((size_t)m * W.ppl + e) * RED_W + k]; };
     v[0] += (-2. * at(W.pl, 0, 2) + 3. * at(W.pl, 1, 2) - at(W.pl, 2, 2));
     v[1] += at(W.pl, 0, 0);
     v[2] += -(2. * at(W.pu, W.nz - 1, 2) - 3. * at(W.pu, W.nz - 2, 2) + at(W.pu, W.nz - 3, 2));
@@ -480,7 +478,7 @@ __global__ __launch_bounds__(WSB) void k_fin_wshear_fused(WsArgs A, WsSegArgs W)
     __shared__ double lds[4][WSB / 64];
     double v[4] = {0., 0., 0., 0.};
 #pragma unroll 4
-    for (int e = threadIdx.x; e < W.Yf * W.cpr; e += WSB) ws_entry(W, e, v);
+    for (int e = threadIdx.x; e < W.ppl; e += WSB) ws_entry(W, e, v);
     block_sum<4, WSB>(v, lds);
     if (threadIdx.x == 0) {
         wshear_finish(A, v);
@@ -507,14 +505,13 @@ __device__ void wshear_finish(const WsArgs &A, const double *v) {
 }
 
 hipError_t launch_wshear_fused(hipStream_t s, dnsg_ctx *h, double *diag_rec, const double *enc_rec) {
-    const int cpr = band_cpr(h);
-    const double *pl = h->red + (size_t)h->coarse.ny * h->coarse.nz * cs_chunks(h->coarse.nx) * RED_W;
+    const double *pl = h->red + coarse_parts_max(h->d) * RED_W;
     const double *pu = pl + band_parts_max(h->d) * RED_W;
     WsArgs A;
     A.part = nullptr; A.Xf = h->d.Xf; A.Yf = h->d.Yf; A.NZs = h->d.NZs; A.GR = h->d.GR; A.omega_f = h->d.omega_f;
     A.force = h->d_force; A.diag = diag_rec; A.out = nullptr; A.enc = enc_rec;
     A.halt = h->halt_armed ? h->halt_flag : nullptr;
-    hipLaunchKernelGGL(k_fin_wshear_fused, dim3(1), dim3(WSB), 0, s, A, WsSegArgs{pl, pu, h->d.Yf, cpr, h->lower.nz, h->band_tiled});
+    hipLaunchKernelGGL(k_fin_wshear_fused, dim3(1), dim3(WSB), 0, s, A, WsSegArgs{pl, pu, band_parts(h), h->lower.nz, h->band_tiled});
     return hipGetLastError();
 }
 
@@ -533,7 +530,7 @@ __global__ __launch_bounds__(RB) void k_red_seg(EncArgs A, WsSegArgs W, double *
         const int e0 = blockIdx.x * ENC_SEG, e1 = min(S.total(), e0 + ENC_SEG);
         for (int e = e0 + threadIdx.x; e < e1; e += RB) enc_entry(A, S, e, v);
     } else {
-        const int e0 = (blockIdx.x - nseg) * WS_SEG, e1 = min(W.Yf * W.cpr, e0 + WS_SEG);
+        const int e0 = (blockIdx.x - nseg) * WS_SEG, e1 = min(W.ppl, e0 + WS_SEG);
         for (int e = e0 + threadIdx.x; e < e1; e += RB) ws_entry(W, e, v);
     }
     block_sum<4>(v, lds);
@@ -556,13 +553,12 @@ __global__ __launch_bounds__(RB) void k_fin_enc_ws(EncArgs A, WsArgs Wf, const d
 }
 
 hipError_t launch_reductions_fused(hipStream_t s, dnsg_ctx *h, double *diag_rec) {
-    const int cpr = band_cpr(h);
-    const double *pc = h->red, *pl = pc + (size_t)h->coarse.ny * h->coarse.nz * cs_chunks(h->coarse.nx) * RED_W;
+    const double *pc = h->red, *pl = pc + coarse_parts_max(h->d) * RED_W;
     const double *pu = pl + band_parts_max(h->d) * RED_W;
     const EncArgs A = enc_args(h, pc, pl, pu, RED_W, true, diag_rec);
     const int nseg = (enc_space(A).total() + ENC_SEG - 1) / ENC_SEG;
-    const WsSegArgs W = {pl, pu, h->d.Yf, cpr, h->lower.nz, h->band_tiled};
-    const int nws = (W.Yf * W.cpr + WS_SEG - 1) / WS_SEG;
+    const WsSegArgs W = {pl, pu, band_parts(h), h->lower.nz, h->band_tiled};
+    const int nws = (W.ppl + WS_SEG - 1) / WS_SEG;
     WsArgs Wf;
     Wf.part = nullptr; Wf.Xf = h->d.Xf; Wf.Yf = h->d.Yf; Wf.NZs = h->d.NZs; Wf.GR = h->d.GR; Wf.omega_f = h->d.omega_f;
     Wf.force = h->d_force; Wf.diag = diag_rec; Wf.out = nullptr; Wf.enc = nullptr;

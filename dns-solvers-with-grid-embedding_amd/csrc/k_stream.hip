@@ -136,6 +136,68 @@ struct RowTargets {
     __device__ __forceinline__ unsigned off(int q) const { return (ey < 0 ? ym : (ey > 0 ? yp : yc)) + q * line; }
 };
 
+// Flat form: the workgroup takes CS_THREADS consecutive nodes of layer z, from node n0 on,
+// so every lane has a node whatever the row length (by rows, a 144-node row filled 144 of
+// 256 lanes and a 285-node one 285 of 512).  A lane's row is its own, so its offsets are
+// per lane, 32 bits each; layer and direction stay scalar.  The writes are the scatter
+// form's.
+template <class S, bool DS, class T>
+__device__ __forceinline__ void cs_flat(const LatArgs &L, const S *__restrict__ lat, S *__restrict__ nxt, int z, int n0,
+                                        T G, T om, bool red, RowSums &rs) {
+    const int nx = L.nx, ny = L.ny, nz = L.nz, n = nx * ny;
+    const bool ok = n0 + (int)threadIdx.x < n;
+    const unsigned id = ok ? n0 + threadIdx.x : n0;
+    const int y = (int)(id / (unsigned)nx), x = (int)id - y * nx;
+    constexpr unsigned ES = sizeof(S);
+    const unsigned line = __builtin_amdgcn_readfirstlane(nx * (int)ES), row = Q * line;
+    const RowTargets<S> in(L, lat, 0, z), to(L, nxt, 0, z);
+    T f[Q];
+    unroll<0, Q>([&](auto qc) {
+        constexpr int q = decltype(qc)::value;
+        f[q] = buf_load(in.mid, y * row + x * ES, q * line, lat);
+    });
+    const auto pre = collide_any(f, G, om);
+    if (red && ok) rs.add<S>(pre);
+    const bool lo_edge = (z == 0), hi_edge = (z == nz - 1);
+    const int ym = (y == 0) ? ny - 1 : y - 1, yp = (y == ny - 1) ? 0 : y + 1;
+    const int xm = (x == 0) ? nx - 1 : x - 1, xp = (x == nx - 1) ? 0 : x + 1;
+    // a lane without a node: every offset at or past DROP
+    const unsigned om_ = ok ? ym * row : DROP, oc = ok ? y * row : DROP, op = ok ? yp * row : DROP;
+    DestSums dst;
+    unroll<0, Q>([&](auto qc) {
+        constexpr int q = decltype(qc)::value;
+        if constexpr (DS) {
+            dst.mass<EZ[q]>(read_back<S, q>(f[q]));
+            dst.mom<EZ[q], EX[q]>(read_back<S, q>(f[q]));
+        }
+        const int xt = (EX[q] > 0) ? xp : (EX[q] < 0 ? xm : x);
+        if constexpr (EZ[q] != 0) {
+            const bool at_end = (EZ[q] < 0) ? lo_edge : hi_edge;
+            if (at_end) {  // uniform over the workgroup
+                const int kind = (EZ[q] < 0) ? L.lo_kind : L.hi_kind;
+                if (kind == BOUND_WALL && ok) {
+                    const int yt = (EY[q] > 0) ? yp : (EY[q] < 0 ? ym : y);
+                    const int8_t *wc = (EZ[q] < 0) ? L.wlo : L.whi;
+                    const bool bb = wc[(size_t)yt * nx + xt] == -1 && wc[(size_t)y * nx + x] == -1;
+                    if (bb) store_s(nxt + lat_at(OPP[q], (size_t)z * ny + y, x, nx), f[q]);
+                    else store_s(nxt + lat_at(MIR[q], (size_t)z * ny + yt, xt, nx), f[q]);
+                    if constexpr (DS) {  // it lands in this layer
+                        const double v = read_back<S, q>(f[q]);
+                        dst.mass<0>(v);
+                        dst.mom<0, EX[q]>(bb ? -v : v);
+                    }
+                }
+                return;
+            }
+        }
+        const int zt = z + EZ[q];
+        if ((zt == 0 && L.skip_lo) || (zt == nz - 1 && L.skip_hi)) return;
+        const unsigned o = ((EY[q] > 0) ? op : (EY[q] < 0 ? om_ : oc)) + xt * ES;
+        buf_store<0>(to.template layer<EZ[q]>(), o, q * line, nxt, f[q]);
+    });
+    if (DS && ok) dst.into(rs, L, z);
+}
+
 template <class S, bool DS, class T>
 __device__ __forceinline__ void cs_aligned_chunk(const LatArgs &L, const S *__restrict__ cur, S *__restrict__ nxt,
                                                  int row, int x0, T G, T om, bool red, RowSums &rs) {
@@ -401,79 +463,72 @@ __global__ __launch_bounds__(CS_THREADS) void k_collide_stream(Batch<LatArgs> P)
     const T G = (T)(L.gscale * L.force[0]);
     const T om = (T)L.omega;
     const bool red = L.red != nullptr;
-    const int rpw = cs_rows_per_wg(nx);
     RowSums rs;
-    if constexpr (sizeof(S) != 8) {  // compiled out in FP64, which never pairs (cs_paired)
-        if (L.paired) {
-            // two chunks of one row per workgroup, two nodes per thread
-            const int cpr = cs_chunks(nx), ppr = cpr / 2;
-            const int row = b / ppr, pc = b % ppr;
-            cs_paired_chunk<S, DS, T>(L, base + (size_t)row * Q * nx, nxt, row, pc * 2 * CS_THREADS, G, om, red, rs);
-            if (red || (DS && L.dsum))  // uniform per workgroup; its halves are the two chunks
-                write_block_sums<DS>(L, rs, (size_t)row * cpr + 2 * pc, 2);
-            return;
-        }
-    }
-    if (rpw == 1) {
-        // one (row, chunk) per workgroup: row, y and z are uniform over the workgroup
-        const int cpr = cs_chunks(nx);
-        const int row = b / cpr, chunk = b % cpr;
-        const S *__restrict__ cur = base + (size_t)row * Q * nx;
-        if (cs_aligned<S>() && nx % CS_THREADS == 0 && buf_fits(nx, ny, (int)sizeof(S))) {
-            cs_aligned_chunk<S, DS, T>(L, cur, nxt, row, chunk * CS_THREADS, G, om, red, rs);
-        } else {
-            const int x = chunk * CS_THREADS + threadIdx.x;
-            if (x < nx) cs_scatter<S, DS, T>(L, cur, nxt, row, x, G, om, red, rs);  // a partial chunk still sums below
-        }
-        if (red || (DS && L.dsum)) write_block_sums<DS>(L, rs, (size_t)row * cpr + chunk, 1);  // uniform per workgroup
+    size_t e;       // first partial of this workgroup
+    int parts = 1;  // ... and how many it writes
+    if (L.form == CS_FLAT) {
+        const int ppl = cs_parts(CS_FLAT, nx, ny), z = b / ppl;
+        cs_flat<S, DS, T>(L, base, nxt, z, (b - z * ppl) * CS_THREADS, G, om, red, rs);
+        e = b;
+    } else if constexpr (sizeof(S) == 8) {
+        // CS_ALIGNED, one (row, chunk) per workgroup: row, y and z are uniform over the workgroup
+        const int cpr = cs_chunks(nx), row = b / cpr, chunk = b % cpr;
+        cs_aligned_chunk<S, DS, T>(L, base + (size_t)row * Q * nx, nxt, row, chunk * CS_THREADS, G, om, red, rs);
+        e = b;
     } else {
-        // narrow lattice: rpw whole rows per workgroup, one partial per row summed in x order
-        const int r = threadIdx.x / nx, x = threadIdx.x - r * nx;
-        const int row = b * rpw + r;
-        if (r < rpw && row < ny * L.nz) cs_scatter<S, DS, T>(L, base + (size_t)row * Q * nx, nxt, row, x, G, om, red, rs);
-        if (red || (DS && L.dsum)) {
-            __shared__ double lr[DS ? 5 : 3][CS_THREADS];
-            lr[0][threadIdx.x] = rs.rho;
-            lr[1][threadIdx.x] = rs.mom;
-            lr[2][threadIdx.x] = rs.u;
-            if constexpr (DS) {
-                lr[3][threadIdx.x] = rs.dm;
-                lr[4][threadIdx.x] = rs.dd;
-            }
-            __syncthreads();
-            const int rr = b * rpw + (int)threadIdx.x;
-            if ((int)threadIdx.x < rpw && rr < ny * L.nz) {
-                RowSums t;
-                for (int k = threadIdx.x * nx; k < (int)(threadIdx.x + 1) * nx; k++) {
-                    t.rho += lr[0][k];
-                    t.mom += lr[1][k];
-                    t.u += lr[2][k];
-                    if constexpr (DS) {
-                        t.dm += lr[3][k];
-                        t.dd += lr[4][k];
-                    }
-                }
-                if (red) write_sums(L.red, (size_t)rr * RED_W, t);
-                if (DS && L.dsum) { L.dsum[2 * (size_t)rr] = t.dm; L.dsum[2 * (size_t)rr + 1] = t.dd; }
-            }
-        }
+        // CS_PAIRED, two chunks of one row per workgroup, two nodes per thread; the
+        // workgroup's halves are the two chunks' partials
+        const int cpr = cs_chunks(nx), ppr = cpr / 2, row = b / ppr, pc = b % ppr;
+        cs_paired_chunk<S, DS, T>(L, base + (size_t)row * Q * nx, nxt, row, pc * 2 * CS_THREADS, G, om, red, rs);
+        e = (size_t)row * cpr + 2 * pc;
+        parts = 2;
     }
+    if (red || (DS && L.dsum)) write_block_sums<DS>(L, rs, e, parts);  // uniform per workgroup
+}
+
+// CS_WIDE: one (row, chunk) of one lattice per workgroup in the scatter form
+template <class S, bool DS>
+__global__ __launch_bounds__(CS_THREADS) void k_collide_wide(LatArgs L, const int *halt) {
+    using T = typename ComputeOf<S>::T;
+    if (halted(halt)) return;
+    const int cpr = cs_chunks(L.nx), row = blockIdx.x / cpr, x = (blockIdx.x % cpr) * CS_THREADS + threadIdx.x;
+    RowSums rs;
+    if (x < L.nx)
+        cs_scatter<S, DS, T>(L, static_cast<const S *>(L.cur) + (size_t)row * Q * L.nx, static_cast<S *>(L.nxt), row, x,
+                             (T)(L.gscale * L.force[0]), (T)L.omega, L.red != nullptr, rs);
+    if (L.red || (DS && L.dsum)) write_block_sums<DS>(L, rs, blockIdx.x, 1);
+}
+
+template <class S>
+static void launch_wide(hipStream_t s, const LatArgs &L, const int *halt) {
+    const dim3 g((unsigned)(L.nz * cs_blocks(CS_WIDE, L.nx, L.ny))), b(CS_THREADS);
+    if (L.dsum) hipLaunchKernelGGL((k_collide_wide<S, true>), g, b, 0, s, L, halt);
+    else hipLaunchKernelGGL((k_collide_wide<S, false>), g, b, 0, s, L, halt);
 }
 
 hipError_t launch_collide_stream(hipStream_t s, const LatArgs *lats, int nlat, int prec, const int *halt) {
-    for (int i0 = 0; i0 < nlat; i0 += BATCH_MAX) {
+    for (int i = 0; i < nlat;) {
         Batch<LatArgs> P;
         P.halt = halt;
-        P.n = nlat - i0 < BATCH_MAX ? nlat - i0 : BATCH_MAX;
+        P.n = 0;
         bool ds = false;
-        for (int i = 0; i < P.n; i++) ds = ds || lats[i0 + i].dsum != nullptr;
         int blocks = 0;
-        for (int i = 0; i < BATCH_MAX; i++) {
-            P.it[i] = lats[i0 + (i < P.n ? i : 0)];
-            P.first[i] = blocks;
-            if (i < P.n) blocks += cs_blocks(P.it[i].nx, P.it[i].ny * P.it[i].nz, P.it[i].paired);
+        for (; i < nlat && P.n < BATCH_MAX; i++) {
+            const LatArgs &L = lats[i];
+            if (L.form == CS_WIDE) {
+                if (prec == DNSG_PREC_FP64) launch_wide<double>(s, L, halt);
+                else if (prec == DNSG_PREC_FP32) launch_wide<float>(s, L, halt);
+                else launch_wide<__half>(s, L, halt);
+                const hipError_t e = hipGetLastError();
+                if (e != hipSuccess) return e;
+                continue;
+            }
+            ds = ds || L.dsum != nullptr;
+            P.it[P.n] = L;
+            P.first[P.n++] = blocks;
+            blocks += L.nz * cs_blocks(L.form, L.nx, L.ny);
         }
-        P.first[BATCH_MAX] = blocks;
+        for (int k = P.n; k <= BATCH_MAX; k++) P.first[k] = blocks;
         if (blocks == 0) continue;
         const dim3 g(blocks), b(CS_THREADS);
         if (prec == DNSG_PREC_FP64) {

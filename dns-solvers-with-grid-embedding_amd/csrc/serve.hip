@@ -61,7 +61,7 @@ size_t solve_bytes(const dnsg_params *p, const dnsg_dims &d) {
     b += 2 * gran((size_t)d.Xf * d.Yf);                     // wall codes
     const size_t rows = (size_t)d.Yc * d.zdc + 2 * (size_t)d.Yf * (d.zdf - 1);
     b += rows * 5 * 8 + (size_t)d.Yf * 4 * 8;               // explicit-pass partials
-    b += ((size_t)d.Yc * d.zdc * cs_chunks(d.Xc) + 2 * band_parts_max(d)) * RED_W * 8 * 2;
+    b += (coarse_parts_max(d) + 2 * band_parts_max(d)) * RED_W * 8 * 2;
     b += (4 * ((size_t)d.zdc + 2 * (d.zdf - 1)) + 2 * 9 * (size_t)d.NZ + 64) * 8 + 14 * (size_t)d.NZ * 8;
     b += 64 * 9 * 8 + 4 * 8;
     return b + GRAN;  // the small buffers' pool
