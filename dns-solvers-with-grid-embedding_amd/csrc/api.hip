@@ -1415,7 +1415,7 @@ int dnsg_velocity_snapshot(dnsg_t *h, int grid, double *vel, double *den) {
     const size_t nn = (size_t)X * Y * Z;
     double *dv = nullptr;
     HIPCHK(h, hipMalloc(&dv, nn * 4 * 8));
-    hipError_t e = launch_snapshot(h, grid, 0, dv, dv + 3 * nn);
+    hipError_t e = launch_snapshot(h, grid, dv, dv + 3 * nn);
     if (e == hipSuccess && vel) e = hipMemcpyAsync(vel, dv, nn * 3 * 8, hipMemcpyDeviceToHost, h->stream);
     if (e == hipSuccess && den) e = hipMemcpyAsync(den, dv + 3 * nn, nn * 8, hipMemcpyDeviceToHost, h->stream);
     if (e == hipSuccess) e = hipStreamSynchronize(h->stream);

@@ -4,17 +4,18 @@
 // The reference computes them offline, one snapshot at a time, with its TKE-budget
 // tool (TKE-budget/computations/budget2D.c:13-1736, reading.c, uv_fluc.c) from the
 // vel-* and den-* files.  Here the same pass runs on the current state:
-//   1. k_bud_fill    velocity and density of every node of the three grids in the
-//                    tool's array layout, [X+4][Y][Z] with two periodic ghost planes
-//                    on each side in x (reading.c:33-57), formed as vel_print does;
-//   2. k_bud_layer   per-layer sums of u, v, w, rho/3 (budget2D.c:177-244), reduced
-//                    in two stages in a fixed order;
-//   3. k_bud_sub     the layer means subtracted in place, ghost planes included
-//                    (:265-309), so every read below sees what the tool's arrays hold,
-//                    also where a one-sided z stencil reaches into the next row;
-//   4. k_bud_nodes   the 44 per-node products and derivative terms of :449-987,
-//                    summed per layer in two stages;
-//   5. the O(NZ) tail on the host: dU/dz, normalisation, production, transport,
+//   1. k_bud_fill    velocity and density of every node of the three grids, formed as
+//                    vel_print does, in planes [u v w rho][layer][y][x] (x fastest, as in
+//                    the lattices, so every pass reads and writes whole lines: in the
+//                    tool's [x][y][z] order the fill alone took 10.7 ms at the Re_tau=180
+//                    size, now 1.0), and the per-layer sums of u, v, w, rho/3
+//                    (budget2D.c:177-244);
+//   2. k_bud_nodes   the 44 per-node products and derivative terms of :449-987 of the
+//                    fluctuations, formed at each read (value - layer mean, :265-309), and
+//                    summed per layer; the tool's periodic x ghost planes are index wraps,
+//                    and where its one-sided z stencil reaches past a layer stack into the
+//                    next row of its array, the same element is read here (bud_at);
+//   3. the O(NZ) tail on the host: dU/dz, normalisation, production, transport,
 //      dissipation (:311-444, :1003-1547).
 // Each node's terms are formed exactly as the tool forms them; the sums over a
 // layer are taken in another order, so the profiles agree with the tool's to
@@ -22,6 +23,7 @@
 #include <algorithm>
 #include <cmath>
 #include <cstring>
+#include <type_traits>
 #include <vector>
 
 #include "internal.hpp"
@@ -40,11 +42,12 @@ enum {
 };
 constexpr int BT = 256;  // threads per workgroup
 
-// one grid of the snapshot in the tool's layout
+// one grid of the snapshot: planes [4][Z][Y][X] of u, v, w, rho
 struct BudGrid {
-    double *vel, *den;  // [X+4][Y][Z][3], [X+4][Y][Z]
+    double *v;
     int X, Y, Z;
     int k0, k1;         // layers taking part in the statistics
+    int m0, m1;         // layers whose mean is taken (and subtracted)
     int base;           // profile index of layer 0
 };
 
@@ -56,51 +59,41 @@ struct BudArgs {
     int NZ;
 };
 
-__device__ __forceinline__ long bidx(const BudGrid &G, int i, int j, int k) {
-    return ((long)i + 2) * G.Y * G.Z + (long)j * G.Z + k;  // the tool's Fb with its +2 plane offset
+// velocity and density of one node as vel_print.c:86-117 forms them
+struct Vel {
+    double u, v, w, rho;
+};
+__device__ __forceinline__ Vel node_vel(const double *f) {
+    Vel r = {0., 0., 0., 0.};
+    unroll<0, Q>([&](auto qq) {
+        constexpr int q = decltype(qq)::value;
+        r.u += (double)EX[q] * f[q];
+        r.v += (double)EY[q] * f[q];
+        r.w += (double)EZ[q] * f[q];
+        r.rho += f[q];
+    });
+    if (r.rho > 0.) { r.u /= r.rho; r.v /= r.rho; r.w /= r.rho; }
+    else r = {0., 0., 0., 0.};
+    return r;
 }
-__device__ __forceinline__ double vat(const BudGrid &G, int i, int j, int k, int c) {
-    return G.vel[bidx(G, i, j, k) * 3 + c];
-}
-
-// 1. velocity and density as vel_print.c:86-117 writes them, [X+2 pad][Y][Z] with
-//    pad periodic ghost planes on each side in x (pad 0: the vel-* / den-* file
-//    layout); the band wall layers come from the wall-layer copies [X][Y][19]
+// node (x, y, k) of a grid whose stored layers start at file layer zlo and whose wall
+// layer kwall (-1: none) comes from the wall-layer copy [X][Y][19]
 template <class S>
-__global__ __launch_bounds__(BT) void k_bud_fill(const S *__restrict__ lat, const double *__restrict__ wall, int X,
-                                                 int Y, int Z, int zlo, int kwall, int pad, double *__restrict__ vel,
-                                                 double *__restrict__ den) {
-    const long n = (long)(X + 2 * pad) * Y * Z;
-    const long id = (long)blockIdx.x * BT + threadIdx.x;
-    if (id >= n) return;
-    const int k = (int)(id % Z), j = (int)((id / Z) % Y), p = (int)(id / ((long)Y * Z));
-    const int x = (p - pad + X) % X;
+__device__ __forceinline__ Vel file_vel(const S *__restrict__ lat, const double *__restrict__ wall, int X, int Y, int zlo,
+                                        int kwall, int x, int y, int k) {
     double f[Q];
     if (k == kwall) {
-        const double *w = wall + ((size_t)x * Y + j) * Q;
+        const double *w = wall + ((size_t)x * Y + y) * Q;
         unroll<0, Q>([&](auto qq) { f[decltype(qq)::value] = w[decltype(qq)::value]; });
     } else {
-        const size_t row = (size_t)(k - zlo) * Y + j;
+        const size_t row = (size_t)(k - zlo) * Y + y;
         unroll<0, Q>([&](auto qq) {
             constexpr int q = decltype(qq)::value;
             f[q] = (double)load_s(lat + lat_at(q, row, x, X));
             if constexpr (sizeof(S) != 8) f[q] += WQ[q];
         });
     }
-    double ux = 0., uy = 0., uz = 0., dens = 0.;
-    unroll<0, Q>([&](auto qq) {
-        constexpr int q = decltype(qq)::value;
-        ux += (double)EX[q] * f[q];
-        uy += (double)EY[q] * f[q];
-        uz += (double)EZ[q] * f[q];
-        dens += f[q];
-    });
-    if (dens > 0.) { ux /= dens; uy /= dens; uz /= dens; }
-    else { ux = 0.; uy = 0.; uz = 0.; dens = 0.; }
-    vel[id * 3] = ux;
-    vel[id * 3 + 1] = uy;
-    vel[id * 3 + 2] = uz;
-    den[id] = dens;
+    return node_vel(f);
 }
 
 // sum of W values over a workgroup into out[0..W) (fixed order: lanes, then waves)
@@ -124,49 +117,62 @@ __device__ __forceinline__ void wg_sum(double *v, double *out) {
     }
 }
 
-// chunks of one layer: a workgroup takes BT consecutive nodes n = i*Y + j
-__host__ __device__ inline int bud_chunks(const BudGrid &G) { return (G.X * G.Y + BT - 1) / BT; }
+// A workgroup takes BT consecutive columns x of BR rows of one layer: its partials are
+// summed over BR nodes per thread before the workgroup reduction (44 values: reduced at
+// every node, the reduction cost more than the terms).
+constexpr int BR = 8;
+__host__ __device__ inline int bud_xc(int X) { return (X + BT - 1) / BT; }
+__host__ __device__ inline int bud_chunks(int X, int Y) { return bud_xc(X) * ((Y + BR - 1) / BR); }
 
-// 2. per-(layer, chunk) sums of u, v, w, rho/3 -> part[(k - k0) * chunks + chunk][4]
-__global__ __launch_bounds__(BT) void k_bud_layer(BudGrid G, double *__restrict__ part) {
-    const int nch = bud_chunks(G);
-    const int k = G.k0 + (int)blockIdx.x / nch, ch = (int)blockIdx.x % nch;
-    const int n = ch * BT + threadIdx.x;
+// 1. planes of one grid, and per-(layer, chunk) sums of u, v, w, rho/3
+template <class S>
+__global__ __launch_bounds__(BT) void k_bud_fill(const S *__restrict__ lat, const double *__restrict__ wall, BudGrid G,
+                                                 int zlo, int kwall, double *__restrict__ part) {
+    const int nch = bud_chunks(G.X, G.Y), nxc = bud_xc(G.X);
+    const int k = (int)blockIdx.x / nch, ch = (int)blockIdx.x % nch;
+    const int x = (ch % nxc) * BT + threadIdx.x, y0 = ch / nxc * BR;
     double v[4] = {0., 0., 0., 0.};
-    if (n < G.X * G.Y) {
-        const int i = n / G.Y, j = n % G.Y;
-        const long e = bidx(G, i, j, k);
-        v[0] = G.vel[e * 3];
-        v[1] = G.vel[e * 3 + 1];
-        v[2] = G.vel[e * 3 + 2];
-        v[3] = (1. / 3.) * G.den[e];
-    }
+    if (x < G.X)
+        for (int y = y0; y < min(y0 + BR, G.Y); y++) {
+            const Vel r = file_vel(lat, wall, G.X, G.Y, zlo, kwall, x, y, k);
+            const size_t plane = (size_t)G.Z * G.Y * G.X, e = ((size_t)k * G.Y + y) * G.X + x;
+            G.v[e] = r.u;
+            G.v[plane + e] = r.v;
+            G.v[2 * plane + e] = r.w;
+            G.v[3 * plane + e] = r.rho;
+            v[0] += r.u;
+            v[1] += r.v;
+            v[2] += r.w;
+            v[3] += (1. / 3.) * r.rho;
+        }
     wg_sum<4>(v, part + (size_t)blockIdx.x * 4);
 }
 
-// sums of nch consecutive partial records of w values, one thread per (segment, value)
+// sums of nch consecutive partial records of w values, one wave per (segment, value)
 __global__ __launch_bounds__(BT) void k_bud_segsum(const double *__restrict__ part, int nseg, int nch, int w,
                                                    double *__restrict__ out) {
-    const int t = blockIdx.x * BT + threadIdx.x;
-    if (t >= nseg * w) return;
+    const int t = (int)(blockIdx.x * (BT / 64) + (threadIdx.x >> 6)), lane = threadIdx.x & 63;
+    if (t >= nseg * w) return;  // uniform over the wave
     const int s = t / w, c = t % w;
     double a = 0.;
-    for (int i = 0; i < nch; i++) a += part[((size_t)s * nch + i) * w + c];
-    out[t] = a;
+    for (int i = lane; i < nch; i += 64) a += part[((size_t)s * nch + i) * w + c];
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) a += __shfl_down(a, o, 64);
+    if (lane == 0) out[t] = a;
 }
 
-// 3. fluctuations in place, ghost planes included
-__global__ __launch_bounds__(BT) void k_bud_sub(BudGrid G, const double *__restrict__ mean, int NZ) {
-    const long n = (long)(G.X + 4) * G.Y * (G.k1 - G.k0);
-    const long id = (long)blockIdx.x * BT + threadIdx.x;
-    if (id >= n) return;
-    const int nk = G.k1 - G.k0;
-    const int k = G.k0 + (int)(id % nk);
-    const long pj = id / nk;  // (p, j)
-    double *v = G.vel + (pj * G.Z + k) * 3;
-    v[0] -= mean[G.base + k];
-    v[1] -= mean[NZ + G.base + k];
-    v[2] -= mean[2 * NZ + G.base + k];
+// Fluctuation of velocity component c at element (i, j, k) of the tool's array of grid g,
+// [x][y][k] behind two ghost planes in x: k outside the layers is the element that lies
+// there, in the next or previous row (j) or plane (i); i is periodic
+__device__ __forceinline__ double bud_at(const BudArgs &A, int g, int i, int j, int k, int c) {
+    const BudGrid &G = A.g[g];
+    while (k >= G.Z) { k -= G.Z; j++; }
+    while (k < 0) { k += G.Z; j--; }
+    if (j >= G.Y) { j -= G.Y; i++; }
+    if (j < 0) { j += G.Y; i--; }
+    i = i < 0 ? i + G.X : (i >= G.X ? i - G.X : i);
+    const double u = G.v[(((size_t)c * G.Z + k) * G.Y + j) * G.X + i];
+    return (k >= G.m0 && k < G.m1) ? u - A.mean[c * A.NZ + G.base + k] : u;
 }
 
 // z derivative of component c at (i, j, k) of grid g (budget2D.c:539-593 lower band,
@@ -175,26 +181,26 @@ __device__ __forceinline__ double bud_ddz(const BudArgs &A, int g, int i, int j,
     const BudGrid &G = A.g[g];
     const int GR = A.GR;
     const double coef = A.coef;
-    auto V = [&](int kk) { return vat(G, i, j, kk, c); };
+    auto V = [&](int kk) { return bud_at(A, g, i, j, kk, c); };
     if (g == 1) {
         if (k == 1) {
             const double tmp = (2. / 3.) * (V(k + 3) - V(k + 1)) - (1. / 12.) * (V(k + 4) - V(k));
             return -(7. / 3.) * V(k) + 6. * V(k + 1) - 3. * V(k + 2) - (2. / 3.) * V(k + 3) + 3. * tmp;
         }
         if (k == G.Z - 1) {
-            const double cc = vat(A.g[0], i / GR, j / GR, 2, c);
+            const double cc = bud_at(A, 0, i / GR, j / GR, 2, c);
             return (coef * (cc - V(k)) + GR * (V(k) - V(k - 1))) * 1. / (1. + GR);
         }
         return 0.5 * (V(k + 1) - V(k - 1));
     }
     if (g == 0) {
-        if (k == 2) return 0.5 * coef * (V(k + 1) - vat(A.g[1], i * GR, j * GR, A.g[1].Z - 1, c));
+        if (k == 2) return 0.5 * coef * (V(k + 1) - bud_at(A, 1, i * GR, j * GR, A.g[1].Z - 1, c));
         if (k == 3 || k == G.Z - 4) return 0.5 * coef * (V(k + 1) - V(k - 1));
-        if (k == G.Z - 3) return 0.5 * coef * (vat(A.g[2], i * GR, j * GR, 0, c) - V(k - 1));
+        if (k == G.Z - 3) return 0.5 * coef * (bud_at(A, 2, i * GR, j * GR, 0, c) - V(k - 1));
         return 0.5 * coef * (V(k + 1) - V(k - 1));
     }
     if (k == 0) {
-        const double cc = vat(A.g[0], i / GR, j / GR, A.g[0].Z - 3, c);
+        const double cc = bud_at(A, 0, i / GR, j / GR, A.g[0].Z - 3, c);
         return (GR * (V(k + 1) - V(k)) + coef * (V(k) - cc)) * 1. / (1. + GR);
     }
     if (k == G.Z - 2) {
@@ -204,71 +210,74 @@ __device__ __forceinline__ double bud_ddz(const BudArgs &A, int g, int i, int j,
     return 0.5 * (V(k + 1) - V(k - 1));
 }
 
-// 4. the per-node terms of grid g (budget2D.c:449-617, :636-797, :800-987), summed
+// 2. the per-node terms of grid g (budget2D.c:449-617, :636-797, :800-987), summed
 //    per (layer, chunk) -> part[(k - k0) * chunks + chunk][NACC]
 __global__ __launch_bounds__(BT) void k_bud_nodes(BudArgs A, int g, double *__restrict__ part) {
     const BudGrid &G = A.g[g];
-    const int nch = bud_chunks(G);
+    const int X = G.X, Y = G.Y, nch = bud_chunks(X, Y), nxc = bud_xc(X);
     const int k = G.k0 + (int)blockIdx.x / nch, ch = (int)blockIdx.x % nch;
-    const int n = ch * BT + threadIdx.x;
+    const int i = (ch % nxc) * BT + threadIdx.x, y0 = ch / nxc * BR;
     double a[NACC];
 #pragma unroll
     for (int c = 0; c < NACC; c++) a[c] = 0.;
-    if (n < G.X * G.Y) {
-        const int Y = G.Y, i = n / Y, j = n % Y;
-        const long e = bidx(G, i, j, k);
-        const double u = G.vel[e * 3], vv = G.vel[e * 3 + 1], w = G.vel[e * 3 + 2];
-        const double dfl = (1. / 3.) * G.den[e] - A.mean[3 * A.NZ + G.base + k];
-        const int jp = j == 0 ? Y - 1 : j - 1, jpp = j == 0 ? Y - 2 : (j == 1 ? Y - 1 : j - 2);
-        const int jn = j == Y - 1 ? 0 : j + 1, jnn = j == Y - 1 ? 1 : (j == Y - 2 ? 0 : j + 2);
-        double d[3][3];
+    const int im = i == 0 ? X - 1 : i - 1, imm = im == 0 ? X - 1 : im - 1;
+    const int ip = i == X - 1 ? 0 : i + 1, ipp = ip == X - 1 ? 0 : ip + 1;
+    const size_t plane = (size_t)Y * X;
+    if (i < X)
+        for (int j = y0; j < min(y0 + BR, Y); j++) {
+            const int jp = j == 0 ? Y - 1 : j - 1, jpp = jp == 0 ? Y - 1 : jp - 1;
+            const int jn = j == Y - 1 ? 0 : j + 1, jnn = jn == Y - 1 ? 0 : jn + 1;
+            double w0[3], d[3][3];
 #pragma unroll
-        for (int c = 0; c < 3; c++) {
-            const double gx = (2. / 3.) * (vat(G, i + 1, j, k, c) - vat(G, i - 1, j, k, c)) -
-                              (1. / 12.) * (vat(G, i + 2, j, k, c) - vat(G, i - 2, j, k, c));
-            const double gy = (2. / 3.) * (vat(G, i, jn, k, c) - vat(G, i, jp, k, c)) -
-                              (1. / 12.) * (vat(G, i, jnn, k, c) - vat(G, i, jpp, k, c));
-            d[c][0] = g == 0 ? A.coef * gx : gx;
-            d[c][1] = g == 0 ? A.coef * gy : gy;
-            d[c][2] = bud_ddz(A, g, i, j, k, c);
+            for (int c = 0; c < 3; c++) {
+                const double *p = G.v + ((size_t)c * G.Z + k) * plane;
+                const double m = (k >= G.m0 && k < G.m1) ? A.mean[c * A.NZ + G.base + k] : 0.;
+                auto at = [&](int ii, int jj) { return p[(size_t)jj * X + ii] - m; };
+                const double gx = (2. / 3.) * (at(ip, j) - at(im, j)) - (1. / 12.) * (at(ipp, j) - at(imm, j));
+                const double gy = (2. / 3.) * (at(i, jn) - at(i, jp)) - (1. / 12.) * (at(i, jnn) - at(i, jpp));
+                w0[c] = at(i, j);
+                d[c][0] = g == 0 ? A.coef * gx : gx;
+                d[c][1] = g == 0 ? A.coef * gy : gy;
+                d[c][2] = bud_ddz(A, g, i, j, k, c);
+            }
+            const double u = w0[0], vv = w0[1], w = w0[2];
+            const double dfl = (1. / 3.) * G.v[((size_t)3 * G.Z + k) * plane + (size_t)j * X + i] - A.mean[3 * A.NZ + G.base + k];
+            const double dudx = d[0][0], dudy = d[0][1], dudz = d[0][2];
+            const double dvdx = d[1][0], dvdy = d[1][1], dvdz = d[1][2];
+            const double dwdx = d[2][0], dwdy = d[2][1], dwdz = d[2][2];
+            const double ox = (dwdy - dvdz), oy = (dudz - dwdx), oz = (dvdx - dudy);
+            a[A_UU] += u * u; a[A_UV] += u * vv; a[A_UW] += u * w; a[A_VV] += vv * vv; a[A_VW] += vv * w; a[A_WW] += w * w;
+            a[A_SKU] += u * u * u; a[A_SKV] += vv * vv * vv; a[A_SKW] += w * w * w; a[A_SKP] += dfl * dfl * dfl;
+            a[A_SKUW] += u * u * u * w * w * w; a[A_SKUV] += u * u * u * vv * vv * vv; a[A_SKVW] += vv * vv * vv * w * w * w;
+            a[A_KUU] += u * u * u * u; a[A_KUV] += vv * vv * vv * vv; a[A_KUW] += w * w * w * w;
+            a[A_KUP] += dfl * dfl * dfl * dfl;
+            a[A_KUUW] += u * u * u * u * w * w * w * w; a[A_KUVW] += vv * vv * vv * vv * w * w * w * w;
+            a[A_KUUV] += u * u * u * u * vv * vv * vv * vv;
+            a[A_DD] += dfl * dfl;
+            a[A_UUW] += u * u * w; a[A_VVW] += vv * vv * w; a[A_WWW] += w * w * w; a[A_UWW] += u * w * w;
+            a[A_PU] += u * dfl; a[A_PV] += vv * dfl; a[A_PW] += w * dfl;
+            a[A_WX] += ox * ox; a[A_WY] += oy * oy; a[A_WZ] += oz * oz;
+            a[A_PAIUU] += dfl * dudx; a[A_PAIVV] += dfl * dvdy; a[A_PAIWW] += dfl * dwdz; a[A_PAIUW] += dfl * (dudz + dwdx);
+            a[A_USUW] += 0.5 * u * (dudz + dwdx); a[A_VSVW] += 0.5 * vv * (dvdz + dwdy);
+            a[A_WSWW] += 0.5 * w * (dwdz + dwdz); a[A_WSUW] += 0.5 * w * (dudz + dwdx); a[A_USWW] += 0.5 * u * (dwdz + dwdz);
+            a[A_EPUU] += dudx * (dudx + dudx) + dudy * (dudy + dvdx) + dudz * (dudz + dwdx);
+            a[A_EPVV] += dvdx * (dvdx + dudy) + dvdy * (dvdy + dvdy) + dvdz * (dvdz + dwdy);
+            a[A_EPWW] += dwdx * (dwdx + dudz) + dwdy * (dwdy + dvdz) + dwdz * (dwdz + dwdz);
+            a[A_EPUW] += dudx * (dwdx + dudz) + dudy * (dwdy + dvdz) + dudz * (dwdz + dwdz) + dwdx * (dudx + dudx) +
+                         dwdy * (dudy + dvdx) + dwdz * (dudz + dwdx);
         }
-        const double dudx = d[0][0], dudy = d[0][1], dudz = d[0][2];
-        const double dvdx = d[1][0], dvdy = d[1][1], dvdz = d[1][2];
-        const double dwdx = d[2][0], dwdy = d[2][1], dwdz = d[2][2];
-        const double ox = (dwdy - dvdz), oy = (dudz - dwdx), oz = (dvdx - dudy);
-        a[A_UU] = u * u; a[A_UV] = u * vv; a[A_UW] = u * w; a[A_VV] = vv * vv; a[A_VW] = vv * w; a[A_WW] = w * w;
-        a[A_SKU] = u * u * u; a[A_SKV] = vv * vv * vv; a[A_SKW] = w * w * w; a[A_SKP] = dfl * dfl * dfl;
-        a[A_SKUW] = u * u * u * w * w * w; a[A_SKUV] = u * u * u * vv * vv * vv; a[A_SKVW] = vv * vv * vv * w * w * w;
-        a[A_KUU] = u * u * u * u; a[A_KUV] = vv * vv * vv * vv; a[A_KUW] = w * w * w * w;
-        a[A_KUP] = dfl * dfl * dfl * dfl;
-        a[A_KUUW] = u * u * u * u * w * w * w * w; a[A_KUVW] = vv * vv * vv * vv * w * w * w * w;
-        a[A_KUUV] = u * u * u * u * vv * vv * vv * vv;
-        a[A_DD] = dfl * dfl;
-        a[A_UUW] = u * u * w; a[A_VVW] = vv * vv * w; a[A_WWW] = w * w * w; a[A_UWW] = u * w * w;
-        a[A_PU] = u * dfl; a[A_PV] = vv * dfl; a[A_PW] = w * dfl;
-        a[A_WX] = ox * ox; a[A_WY] = oy * oy; a[A_WZ] = oz * oz;
-        a[A_PAIUU] = dfl * dudx; a[A_PAIVV] = dfl * dvdy; a[A_PAIWW] = dfl * dwdz; a[A_PAIUW] = dfl * (dudz + dwdx);
-        a[A_USUW] = 0.5 * u * (dudz + dwdx); a[A_VSVW] = 0.5 * vv * (dvdz + dwdy);
-        a[A_WSWW] = 0.5 * w * (dwdz + dwdz); a[A_WSUW] = 0.5 * w * (dudz + dwdx); a[A_USWW] = 0.5 * u * (dwdz + dwdz);
-        a[A_EPUU] = dudx * (dudx + dudx) + dudy * (dudy + dvdx) + dudz * (dudz + dwdx);
-        a[A_EPVV] = dvdx * (dvdx + dudy) + dvdy * (dvdy + dvdy) + dvdz * (dvdz + dwdy);
-        a[A_EPWW] = dwdx * (dwdx + dudz) + dwdy * (dwdy + dvdz) + dwdz * (dwdz + dwdz);
-        a[A_EPUW] = dudx * (dwdx + dudz) + dudy * (dwdy + dvdz) + dudz * (dwdz + dwdz) + dwdx * (dudx + dudx) +
-                    dwdy * (dudy + dvdx) + dwdz * (dudz + dwdx);
-    }
     wg_sum<NACC>(a, part + (size_t)blockIdx.x * NACC);
 }
 
 // the lower band's u', v' at k = 4 (uv_fluc.c:25-33), [Xf][Yf]
-__global__ __launch_bounds__(BT) void k_bud_plane(BudGrid G, int k, double *__restrict__ uo, double *__restrict__ vo) {
+__global__ __launch_bounds__(BT) void k_bud_plane(BudArgs A, int k, double *__restrict__ uo, double *__restrict__ vo) {
     const int n = blockIdx.x * BT + threadIdx.x;
-    if (n >= G.X * G.Y) return;
-    const long e = bidx(G, n / G.Y, n % G.Y, k);
-    uo[n] = G.vel[e * 3];
-    vo[n] = G.vel[e * 3 + 1];
+    if (n >= A.g[1].X * A.g[1].Y) return;
+    uo[n] = bud_at(A, 1, n / A.g[1].Y, n % A.g[1].Y, k, 0);
+    vo[n] = bud_at(A, 1, n / A.g[1].Y, n % A.g[1].Y, k, 1);
 }
 
-// 5. dU/dz of the mean profile (budget2D.c:311-444)
+// 3. dU/dz of the mean profile (budget2D.c:311-444)
 void bud_dudz(const double *U, int zdf, int zdc, int GR, double *dUdz) {
     const double coef = (1. / ((double)GR));
     const int zd = zdf;
@@ -306,7 +315,7 @@ void bud_dudz(const double *U, int zdf, int zdc, int GR, double *dUdz) {
     }
 }
 
-// 5. normalisation and the derived profiles (budget2D.c:1003-1547)
+// 3. normalisation and the derived profiles (budget2D.c:1003-1547)
 void bud_finish(const dnsg_params &p, const double *Um, const double *dUdz, std::vector<double> &a, double *turb,
                 double *vort, double *ke) {
     const int GR = p.gratio, zdf = p.zds + 1, zdc = p.zdv;
@@ -432,25 +441,65 @@ void bud_finish(const dnsg_params &p, const double *Um, const double *dUdz, std:
 
 }  // namespace
 
-// velocity and density of grid g (0 coarse, 1 lower, 2 upper) from the current
-// state into [X + 2 pad][Y][Z][3] and [X + 2 pad][Y][Z]; needs fwall
-hipError_t launch_snapshot(dnsg_ctx *h, int g, int pad, double *vel, double *den) {
+// A snapshot's tile: SX columns x by SZ layers of one row y.  The lattice is read along x
+// and the file order [x][y][k][3] written along k, through LDS (written node by node
+// from threads along k, each of the 19 reads of a node was a line of its own: 0.25 ms for
+// a 420 x 252 x 12 band against 0.05).
+constexpr int SX = 32, SZ = 8;
+template <class S>
+__global__ __launch_bounds__(SX *SZ) void k_snapshot(const S *__restrict__ lat, const double *__restrict__ wall, int X,
+                                                      int Y, int Z, int zlo, int kwall, double *__restrict__ vel,
+                                                      double *__restrict__ den) {
+    __shared__ double sv[SX][3 * SZ + 1], sd[SX][SZ + 1];
+    const int nxc = (X + SX - 1) / SX, nzc = (Z + SZ - 1) / SZ;
+    const int bx = blockIdx.x % nxc, bz = blockIdx.x / nxc % nzc, y = blockIdx.x / (nxc * nzc);
+    const int x0 = bx * SX, z0 = bz * SZ, tx = threadIdx.x % SX, tz = threadIdx.x / SX;
+    if (x0 + tx < X && z0 + tz < Z) {
+        const Vel r = file_vel(lat, wall, X, Y, zlo, kwall, x0 + tx, y, z0 + tz);
+        sv[tx][3 * tz] = r.u;
+        sv[tx][3 * tz + 1] = r.v;
+        sv[tx][3 * tz + 2] = r.w;
+        sd[tx][tz] = r.rho;
+    }
+    __syncthreads();
+    const int nz = min(SZ, Z - z0), nx = min(SX, X - x0);
+    for (int t = threadIdx.x; t < nx * 3 * nz; t += SX * SZ) {
+        const int xx = t / (3 * nz), e = t % (3 * nz);
+        vel[(((size_t)(x0 + xx) * Y + y) * Z + z0) * 3 + e] = sv[xx][e];
+    }
+    for (int t = threadIdx.x; t < nx * nz; t += SX * SZ) {
+        const int xx = t / nz, e = t % nz;
+        den[((size_t)(x0 + xx) * Y + y) * Z + z0 + e] = sd[xx][e];
+    }
+}
+
+// a grid as vel_print sees it: its lattice, extents, first stored file layer, wall layer
+struct FileGrid {
+    const Grid *lat;
+    int X, Y, Z, zlo, kwall;
+    const double *wall;
+};
+FileGrid file_grid(const dnsg_ctx *h, int g) {
     const dnsg_dims &d = h->d;
-    const Grid *lat = g == 0 ? &h->coarse : (g == 1 ? &h->lower : &h->upper);
-    const int X = g == 0 ? d.Xc : d.Xf, Y = g == 0 ? d.Yc : d.Yf, Z = g == 0 ? d.zdc : d.zdf;
-    const int zlo = g == 1 ? 1 : 0, kwall = g == 0 ? -1 : (g == 1 ? 0 : d.zdf - 1);
-    const double *wall = h->fwall + (g == 2 ? (size_t)d.Xf * d.Yf * 19 : 0);
-    const long n = (long)(X + 2 * pad) * Y * Z;
-    const dim3 grd((unsigned)((n + BT - 1) / BT)), blk(BT);
-    if (h->p.precision == DNSG_PREC_FP64)
-        hipLaunchKernelGGL(k_bud_fill<double>, grd, blk, 0, h->stream, (const double *)lat->c(), wall, X, Y, Z, zlo,
-                           kwall, pad, vel, den);
-    else if (h->p.precision == DNSG_PREC_FP32)
-        hipLaunchKernelGGL(k_bud_fill<float>, grd, blk, 0, h->stream, (const float *)lat->c(), wall, X, Y, Z, zlo,
-                           kwall, pad, vel, den);
-    else
-        hipLaunchKernelGGL(k_bud_fill<__half>, grd, blk, 0, h->stream, (const __half *)lat->c(), wall, X, Y, Z, zlo,
-                           kwall, pad, vel, den);
+    if (g == 0) return {&h->coarse, d.Xc, d.Yc, d.zdc, 0, -1, h->fwall};
+    if (g == 1) return {&h->lower, d.Xf, d.Yf, d.zdf, 1, 0, h->fwall};
+    return {&h->upper, d.Xf, d.Yf, d.zdf, 0, d.zdf - 1, h->fwall + (size_t)d.Xf * d.Yf * 19};
+}
+
+template <class F>
+auto by_storage(const dnsg_ctx *h, const void *lat, F f) {
+    if (h->p.precision == DNSG_PREC_FP64) return f((const double *)lat);
+    if (h->p.precision == DNSG_PREC_FP32) return f((const float *)lat);
+    return f((const __half *)lat);
+}
+
+hipError_t launch_snapshot(dnsg_ctx *h, int g, double *vel, double *den) {
+    const FileGrid F = file_grid(h, g);
+    const dim3 grd((unsigned)(((F.X + SX - 1) / SX) * ((F.Z + SZ - 1) / SZ)) * (unsigned)F.Y), blk(SX * SZ);
+    by_storage(h, F.lat->c(), [&](auto *lat) {
+        using S = std::remove_const_t<std::remove_pointer_t<decltype(lat)>>;
+        hipLaunchKernelGGL(k_snapshot<S>, grd, blk, 0, h->stream, lat, F.wall, F.X, F.Y, F.Z, F.zlo, F.kwall, vel, den);
+    });
     return hipGetLastError();
 }
 
@@ -486,92 +535,82 @@ extern "C" int dnsg_budget2d(dnsg_t *h, double *turb, double *vort, double *ke, 
     A.GR = GR;
     A.coef = (1. / ((double)GR));
     A.NZ = NZ;
-    const int X[3] = {d.Xc, d.Xf, d.Xf}, Y[3] = {d.Yc, d.Yf, d.Yf}, Z[3] = {zdc, zdf, zdf};
     const int k0[3] = {2, 1, 0}, k1[3] = {zdc - 2, zdf, zdf - 1};    // node passes
     const int m0[3] = {2, 0, 0}, m1[3] = {zdc - 2, zdf, zdf};        // means and subtraction
     const int base[3] = {zdf - 2, 0, zdf + zdc - 4};
-    size_t npart = 0;
+    size_t npart = 0, nsum = 0, nv = 0;
     std::vector<double> mean(4 * (size_t)NZ, 0.), acc((size_t)NACC * NZ, 0.), dUdz(NZ, 0.), lay;
-    double *dmean = nullptr, *dpart = nullptr, *dsum = nullptr, *dpl = nullptr;
+    double *dmean = nullptr, *dpart = nullptr, *dsum = nullptr, *dpl = nullptr, *dv = nullptr;
     for (int g = 0; g < 3; g++) {
-        A.g[g] = BudGrid{nullptr, nullptr, X[g], Y[g], Z[g], m0[g], m1[g], base[g]};
-        npart = std::max(npart, (size_t)bud_chunks(A.g[g]) * Z[g] * NACC);
+        const FileGrid F = file_grid(h, g);
+        A.g[g] = BudGrid{nullptr, F.X, F.Y, F.Z, k0[g], k1[g], m0[g], m1[g], base[g]};
+        npart = std::max(npart, (size_t)bud_chunks(F.X, F.Y) * F.Z * NACC);
+        nsum = std::max(nsum, (size_t)F.Z * NACC);
+        nv += 4 * (size_t)F.X * F.Y * F.Z;
     }
-    for (int g = 0; g < 3; g++) {
-        const size_t nn = (size_t)(X[g] + 4) * Y[g] * Z[g];
-        BCHK(h, hipMalloc(&A.g[g].vel, nn * 3 * 8));
-        BCHK(h, hipMalloc(&A.g[g].den, nn * 8));
-    }
+    BCHK(h, hipMalloc(&dv, nv * 8));
     BCHK(h, hipMalloc(&dmean, 4 * (size_t)NZ * 8));
     BCHK(h, hipMalloc(&dpart, npart * 8));
-    BCHK(h, hipMalloc(&dsum, (size_t)NACC * NZ * 8));
-    // 1. snapshot arrays
+    BCHK(h, hipMalloc(&dsum, 3 * nsum * 8));
+    A.g[0].v = dv;
+    for (int g = 1; g < 3; g++) A.g[g].v = A.g[g - 1].v + 4 * (size_t)A.g[g - 1].X * A.g[g - 1].Y * A.g[g - 1].Z;
+    lay.resize(3 * nsum);
+    // 1. snapshot planes and layer means
     for (int g = 0; g < 3; g++) {
-        BCHK(h, launch_snapshot(h, g, 2, A.g[g].vel, A.g[g].den));
+        const FileGrid F = file_grid(h, g);
+        const BudGrid &G = A.g[g];
+        const int nch = bud_chunks(G.X, G.Y);
+        by_storage(h, F.lat->c(), [&](auto *lat) {
+            using S = std::remove_const_t<std::remove_pointer_t<decltype(lat)>>;
+            hipLaunchKernelGGL(k_bud_fill<S>, dim3((unsigned)(G.Z * nch)), dim3(BT), 0, h->stream, lat, F.wall, G, F.zlo,
+                               F.kwall, dpart);
+        });
+        hipLaunchKernelGGL(k_bud_segsum, dim3((unsigned)((G.Z * 4 + 3) / 4)), dim3(BT), 0, h->stream,
+                           (const double *)dpart, G.Z, nch, 4, dsum + g * nsum);
+        BCHK(h, hipGetLastError());
     }
-    // 2. layer means
+    BCHK(h, hipMemcpyAsync(lay.data(), dsum, lay.size() * 8, hipMemcpyDeviceToHost, h->stream));
+    BCHK(h, hipStreamSynchronize(h->stream));
     for (int g = 0; g < 3; g++) {
         const BudGrid &G = A.g[g];
-        const int nch = bud_chunks(G), nk = G.k1 - G.k0;
-        hipLaunchKernelGGL(k_bud_layer, dim3((unsigned)(nk * nch)), dim3(BT), 0, h->stream, G, dpart);
-        hipLaunchKernelGGL(k_bud_segsum, dim3((unsigned)((nk * 4 + BT - 1) / BT)), dim3(BT), 0, h->stream,
-                           (const double *)dpart, nk, nch, 4, dsum);
-        BCHK(h, hipGetLastError());
-        lay.resize((size_t)nk * 4);
-        BCHK(h, hipMemcpyAsync(lay.data(), dsum, lay.size() * 8, hipMemcpyDeviceToHost, h->stream));
-        BCHK(h, hipStreamSynchronize(h->stream));
-        for (int k = G.k0; k < G.k1; k++)
+        for (int k = G.m0; k < G.m1; k++)
             for (int c = 0; c < 4; c++)
-                mean[(size_t)c * NZ + G.base + k] = lay[(size_t)(k - G.k0) * 4 + c] / (double)(G.X * G.Y);
+                mean[(size_t)c * NZ + G.base + k] = lay[g * nsum + (size_t)k * 4 + c] / (double)(G.X * G.Y);
     }
     BCHK(h, hipMemcpyAsync(dmean, mean.data(), mean.size() * 8, hipMemcpyHostToDevice, h->stream));
-    // 3. fluctuations
-    for (int g = 0; g < 3; g++) {
-        const BudGrid &G = A.g[g];
-        const long n = (long)(G.X + 4) * G.Y * (G.k1 - G.k0);
-        hipLaunchKernelGGL(k_bud_sub, dim3((unsigned)((n + BT - 1) / BT)), dim3(BT), 0, h->stream, G,
-                           (const double *)dmean, NZ);
-        BCHK(h, hipGetLastError());
-    }
-    // 4. per-node terms over the layers of the node passes
+    // 2. per-node terms over the layers of the node passes
     A.mean = dmean;
     for (int g = 0; g < 3; g++) {
-        A.g[g].k0 = k0[g];
-        A.g[g].k1 = k1[g];
+        const BudGrid &G = A.g[g];
+        const int nch = bud_chunks(G.X, G.Y), nk = G.k1 - G.k0;
+        hipLaunchKernelGGL(k_bud_nodes, dim3((unsigned)(nk * nch)), dim3(BT), 0, h->stream, A, g, dpart);
+        hipLaunchKernelGGL(k_bud_segsum, dim3((unsigned)((nk * NACC + 3) / 4)), dim3(BT), 0, h->stream,
+                           (const double *)dpart, nk, nch, (int)NACC, dsum + g * nsum);
+        BCHK(h, hipGetLastError());
     }
+    BCHK(h, hipMemcpyAsync(lay.data(), dsum, lay.size() * 8, hipMemcpyDeviceToHost, h->stream));
+    BCHK(h, hipStreamSynchronize(h->stream));
     for (int g = 0; g < 3; g++) {
         const BudGrid &G = A.g[g];
-        const int nch = bud_chunks(G), nk = G.k1 - G.k0;
-        hipLaunchKernelGGL(k_bud_nodes, dim3((unsigned)(nk * nch)), dim3(BT), 0, h->stream, A, g, dpart);
-        hipLaunchKernelGGL(k_bud_segsum, dim3((unsigned)((nk * NACC + BT - 1) / BT)), dim3(BT), 0, h->stream,
-                           (const double *)dpart, nk, nch, (int)NACC, dsum);
-        BCHK(h, hipGetLastError());
-        lay.resize((size_t)nk * NACC);
-        BCHK(h, hipMemcpyAsync(lay.data(), dsum, lay.size() * 8, hipMemcpyDeviceToHost, h->stream));
-        BCHK(h, hipStreamSynchronize(h->stream));
         for (int k = G.k0; k < G.k1; k++)
-            for (int c = 0; c < NACC; c++) acc[(size_t)c * NZ + G.base + k] = lay[(size_t)(k - G.k0) * NACC + c];
+            for (int c = 0; c < NACC; c++)
+                acc[(size_t)c * NZ + G.base + k] = lay[g * nsum + (size_t)(k - G.k0) * NACC + c];
     }
     if (ufl) {
-        const BudGrid &G = A.g[1];
-        const size_t np = (size_t)G.X * G.Y;
+        const size_t np = (size_t)A.g[1].X * A.g[1].Y;
         BCHK(h, hipMalloc(&dpl, 2 * np * 8));
-        hipLaunchKernelGGL(k_bud_plane, dim3((unsigned)((np + BT - 1) / BT)), dim3(BT), 0, h->stream, G, 4, dpl,
-                           dpl + np);
+        hipLaunchKernelGGL(k_bud_plane, dim3((unsigned)((np + BT - 1) / BT)), dim3(BT), 0, h->stream, A, 4, dpl, dpl + np);
         BCHK(h, hipGetLastError());
         BCHK(h, hipMemcpyAsync(ufl, dpl, np * 8, hipMemcpyDeviceToHost, h->stream));
         BCHK(h, hipMemcpyAsync(vfl, dpl + np, np * 8, hipMemcpyDeviceToHost, h->stream));
         BCHK(h, hipStreamSynchronize(h->stream));
     }
-    // 5. the profile tail
+    // 3. the profile tail
     bud_dudz(mean.data(), zdf, zdc, GR, dUdz.data());
     bud_finish(h->p, mean.data(), dUdz.data(), acc, turb, vort, ke);
 done:
     if (rc) (void)hipStreamSynchronize(h->stream);
-    for (int g = 0; g < 3; g++) {
-        if (A.g[g].vel) (void)hipFree(A.g[g].vel);
-        if (A.g[g].den) (void)hipFree(A.g[g].den);
-    }
+    if (dv) (void)hipFree(dv);
     if (dmean) (void)hipFree(dmean);
     if (dpart) (void)hipFree(dpart);
     if (dsum) (void)hipFree(dsum);

@@ -8,11 +8,9 @@
 //   E_y(j) = sum_i fac_j 1/2 |c(i, j)|^2   (spanwise index j = 0 .. N1/2)
 // with fac_j = 1 for j = 0 and 2 otherwise (the folded half of the spectrum).
 // Here the velocity planes are formed on the device from the lattice (the
-// vel_print.c formula), transformed with hipFFT in one batched plan, and folded
-// by one thread per output value in the reference's summation order.
+// vel_print.c formula), transformed with hipFFT in one batched plan, and folded by a wave
+// per E_x value and a workgroup per 64 E_y values.
 #include <hipfft/hipfft.h>
-
-#include <vector>
 
 #include "internal.hpp"
 #include "lattice.hpp"
@@ -21,87 +19,91 @@ namespace dnsg {
 
 namespace {
 
-// velocity of every node of nz_st stored layers, into planes k0.. of
-// vel[3][nzg][nx][ny] (y fastest: the DFT's last, halved dimension)
+// Velocity planes vel[3][nzg][nx][ny] (y fastest: the DFT's last, halved dimension) of every
+// layer of a grid's velocity file, its wall layer kwall (-1: none) from the wall-layer copy
+// [nx][ny][19].  A workgroup takes a tile of TS x TS columns of one layer: the lattice is
+// read along x and the planes written along y, through LDS (written along x, the stores
+// were a line each: 0.45 ms for the Re_tau=180 FP32 grids, now 0.1; the wall layer used to
+// be formed on the host).
+constexpr int TS = 32, TB = 256;
 template <class S>
-__global__ __launch_bounds__(256) void k_vel_planes(const S *__restrict__ lat, int nx, int ny, int nz_st, int k0,
-                                                    int nzg, double *__restrict__ vel) {
-    const size_t n = (size_t)nx * ny * nz_st;
-    const size_t id = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (id >= n) return;
-    const int x = (int)(id % nx), y = (int)((id / nx) % ny), m = (int)(id / ((size_t)nx * ny));
-    double ux = 0., uy = 0., uz = 0., dens = 0.;
-    unroll<0, Q>([&](auto qc) {  // vel_print.c:86-104, in its order
-        constexpr int q = decltype(qc)::value;
-        double f = (double)load_s(lat + lat_at(q, (size_t)m * ny + y, x, nx));
-        if constexpr (sizeof(S) != 8) f += WQ[q];
-        ux += (double)EX[q] * f;
-        uy += (double)EY[q] * f;
-        uz += (double)EZ[q] * f;
-        dens += f;
-    });
-    if (dens > 0.) { ux /= dens; uy /= dens; uz /= dens; }
-    else { ux = 0.; uy = 0.; uz = 0.; }
-    const size_t plane = (size_t)nx * ny, at = (size_t)x * ny + y, k = (size_t)(m + k0);
-    vel[(0 * (size_t)nzg + k) * plane + at] = ux;
-    vel[(1 * (size_t)nzg + k) * plane + at] = uy;
-    vel[(2 * (size_t)nzg + k) * plane + at] = uz;
-}
-
-// one output value per thread: E_x(c, i, k) for t < 3 nzg N0, then E_y(c, j, k)
-__global__ __launch_bounds__(256) void k_fold(const double2 *__restrict__ cf, int N0, int N1, int nzg,
-                                              double *__restrict__ ex, double *__restrict__ ey) {
-    const int N1h = N1 / 2 + 1;
-    const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    const long nxo = 3L * nzg * N0, nyo = 3L * nzg * N1h;
-    if (t >= nxo + nyo) return;
-    const double s = 2. * (1. / ((double)(2. * N0 * N1)));  // 1d-spectra-mgrd.c:183
-    auto term = [&](const double2 *p, int i, int j) {
-        if (i == 0 && j == 0) return 0.;  // the mean removed (:195-200)
-        const double2 c = p[(size_t)i * N1h + j];
-        const double re = c.x * s, im = c.y * s;
-        const double fac = j == 0 ? 1. : 2.;
-        return fac * 0.5 * (re * re + im * im);
-    };
-    if (t < nxo) {
-        const int i = (int)(t % N0), k = (int)((t / N0) % nzg), c = (int)(t / ((long)N0 * nzg));
-        const double2 *p = cf + ((size_t)c * nzg + k) * (size_t)N0 * N1h;
-        double e = 0.;
-        for (int j = 0; j < N1h; j++) e += term(p, i, j);
-        ex[((size_t)c * N0 + i) * nzg + k] = e;
-    } else {
-        const long u = t - nxo;
-        const int j = (int)(u % N1h), k = (int)((u / N1h) % nzg), c = (int)(u / ((long)N1h * nzg));
-        const double2 *p = cf + ((size_t)c * nzg + k) * (size_t)N0 * N1h;
-        double e = 0.;
-        for (int i = 0; i < N0; i++) e += term(p, i, j);
-        ey[((size_t)c * N1h + j) * nzg + k] = e;
+__global__ __launch_bounds__(TB) void k_vel_planes(const S *__restrict__ lat, const double *__restrict__ wall, int nx,
+                                                   int ny, int zlo, int kwall, int nzg, double *__restrict__ vel) {
+    __shared__ double t[3][TS][TS + 1];  // [component][y][x]
+    const int nxc = (nx + TS - 1) / TS, nyc = (ny + TS - 1) / TS;
+    const int x0 = (int)(blockIdx.x % nxc) * TS, y0 = (int)(blockIdx.x / nxc % nyc) * TS, k = (int)(blockIdx.x / (nxc * nyc));
+    const int c = threadIdx.x % TS, r0 = threadIdx.x / TS;
+    for (int r = r0; r < TS; r += TB / TS) {
+        const int x = x0 + c, y = y0 + r;
+        if (x >= nx || y >= ny) continue;
+        double ux = 0., uy = 0., uz = 0., dens = 0.;
+        unroll<0, Q>([&](auto qc) {  // vel_print.c:86-104, in its order
+            constexpr int q = decltype(qc)::value;
+            double f;
+            if (k == kwall) {
+                f = wall[((size_t)x * ny + y) * Q + q];
+            } else {
+                f = (double)load_s(lat + lat_at(q, (size_t)(k - zlo) * ny + y, x, nx));
+                if constexpr (sizeof(S) != 8) f += WQ[q];
+            }
+            ux += (double)EX[q] * f;
+            uy += (double)EY[q] * f;
+            uz += (double)EZ[q] * f;
+            dens += f;
+        });
+        if (dens > 0.) { ux /= dens; uy /= dens; uz /= dens; }
+        else { ux = 0.; uy = 0.; uz = 0.; }
+        t[0][r][c] = ux;
+        t[1][r][c] = uy;
+        t[2][r][c] = uz;
+    }
+    __syncthreads();
+    for (int r = r0; r < TS; r += TB / TS) {  // row r: x = x0 + r, lanes along y
+        const int x = x0 + r, y = y0 + c;
+        if (x >= nx || y >= ny) continue;
+#pragma unroll
+        for (int m = 0; m < 3; m++) vel[(((size_t)m * nzg + k) * nx + x) * ny + y] = t[m][c][r];
     }
 }
 
-// vel_print's velocity of one host-kept wall layer [X][Y][19] -> 3 planes [x][y]
-void wall_velocity(const double *w, int nx, int ny, std::vector<double> &out) {
-    static const int ex[19] = {0, 1, -1, 0, 0, 0, 0, 1, -1, -1, 1, 1, 1, -1, -1, 0, 0, 0, 0};
-    static const int ey[19] = {0, 0, 0, 1, -1, 0, 0, 1, 1, -1, -1, 0, 0, 0, 0, 1, 1, -1, -1};
-    static const int ez[19] = {0, 0, 0, 0, 0, 1, -1, 0, 0, 0, 0, 1, -1, -1, 1, 1, -1, -1, 1};
-    const size_t plane = (size_t)nx * ny;
-    out.assign(3 * plane, 0.);
-    for (int i = 0; i < nx; i++)
-        for (int j = 0; j < ny; j++) {
-            const double *f = w + ((size_t)i * ny + j) * 19;
-            double ux = 0., uy = 0., uz = 0., dens = 0.;
-            for (int a = 0; a < 19; a++) {
-                ux += ex[a] * f[a];
-                uy += ey[a] * f[a];
-                uz += ez[a] * f[a];
-                dens += f[a];
-            }
-            if (dens > 0.) { ux /= dens; uy /= dens; uz /= dens; }
-            else { ux = 0.; uy = 0.; uz = 0.; }
-            out[0 * plane + (size_t)i * ny + j] = ux;
-            out[1 * plane + (size_t)i * ny + j] = uy;
-            out[2 * plane + (size_t)i * ny + j] = uz;
-        }
+// E_x(c, i, k) of the DFT coefficients cf[3 nzg][N0][N1h]: one wave per (c, k, i), its lanes
+// along j; then E_y(c, j, k): one thread per value, lanes along j, over i in order
+__device__ __forceinline__ double fold_term(const double2 c, double s, int i, int j) {
+    if (i == 0 && j == 0) return 0.;  // the mean removed (1d-spectra-mgrd.c:195-200)
+    const double re = c.x * s, im = c.y * s;
+    const double fac = j == 0 ? 1. : 2.;
+    return fac * 0.5 * (re * re + im * im);
+}
+__global__ __launch_bounds__(TB) void k_fold_x(const double2 *__restrict__ cf, int N0, int N1, int nzg, double *__restrict__ ex) {
+    const int N1h = N1 / 2 + 1, lane = threadIdx.x & 63;
+    const long t = (long)blockIdx.x * (TB / 64) + (threadIdx.x >> 6);  // (c k, i)
+    if (t >= 3L * nzg * N0) return;
+    const int i = (int)(t % N0), k = (int)((t / N0) % nzg), c = (int)(t / ((long)N0 * nzg));
+    const double s = 2. * (1. / ((double)(2. * N0 * N1)));  // 1d-spectra-mgrd.c:183
+    const double2 *p = cf + (size_t)t * N1h;
+    double e = 0.;
+    for (int j = lane; j < N1h; j += 64) e += fold_term(p[j], s, i, j);
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) e += __shfl_down(e, o, 64);
+    if (lane == 0) ex[((size_t)c * N0 + i) * nzg + k] = e;
+}
+// a workgroup: 64 wavenumbers j of one (c, k), its waves sharing the N0 rows
+__global__ __launch_bounds__(TB) void k_fold_y(const double2 *__restrict__ cf, int N0, int N1, int nzg, double *__restrict__ ey) {
+    __shared__ double l[TB / 64][64];
+    const int N1h = N1 / 2 + 1, njc = (N1h + 63) / 64, lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const int j = (int)(blockIdx.x % njc) * 64 + lane, ck = (int)(blockIdx.x / njc), k = ck % nzg, c = ck / nzg;
+    const double s = 2. * (1. / ((double)(2. * N0 * N1)));
+    const double2 *p = cf + (size_t)ck * N0 * N1h;
+    double e = 0.;
+    if (j < N1h)
+        for (int i = w; i < N0; i += TB / 64) e += fold_term(p[(size_t)i * N1h + j], s, i, j);
+    l[w][lane] = e;
+    __syncthreads();
+    if (w == 0 && j < N1h) {
+        double a = l[0][lane];
+        for (int v = 1; v < TB / 64; v++) a += l[v][lane];
+        ey[((size_t)c * N1h + j) * nzg + k] = a;
+    }
 }
 
 }  // namespace
@@ -131,7 +133,8 @@ extern "C" int dnsg_spectra(dnsg_t *h, int grid, double *ex, double *ey) {
     const int nzg = grid == 0 ? h->d.zdc : h->d.zdf;  // planes in the velocity file
     const int k0 = grid == 1 ? 1 : 0;                 // lower band: the wall is plane 0
     const size_t plane = (size_t)N0 * N1;
-    int rc = DNSG_OK;
+    int rc = ensure_fwall(h);
+    if (rc) return rc;
     double *vel = nullptr, *dex = nullptr, *dey = nullptr;
     double2 *cf = nullptr;
     hipfftHandle plan = 0;
@@ -141,24 +144,16 @@ extern "C" int dnsg_spectra(dnsg_t *h, int grid, double *ex, double *ey) {
     SPCHK(h, hipMalloc(&dex, 3 * (size_t)N0 * nzg * sizeof(double)));
     SPCHK(h, hipMalloc(&dey, 3 * (size_t)N1h * nzg * sizeof(double)));
     {
-        const size_t n = plane * g.nz;
-        const dim3 grd((unsigned)((n + 255) / 256)), blk(256);
+        const int kwall = grid == 0 ? -1 : (grid == 1 ? 0 : nzg - 1);
+        const double *wall = grid == 2 ? h->fwall + plane * Q : h->fwall;
+        const dim3 grd((unsigned)(((N0 + TS - 1) / TS) * ((N1 + TS - 1) / TS) * nzg)), blk(TB);
         if (h->p.precision == DNSG_PREC_FP64)
-            hipLaunchKernelGGL(k_vel_planes<double>, grd, blk, 0, h->stream, (const double *)g.c(), N0, N1, g.nz, k0, nzg, vel);
+            hipLaunchKernelGGL(k_vel_planes<double>, grd, blk, 0, h->stream, (const double *)g.c(), wall, N0, N1, k0, kwall, nzg, vel);
         else if (h->p.precision == DNSG_PREC_FP32)
-            hipLaunchKernelGGL(k_vel_planes<float>, grd, blk, 0, h->stream, (const float *)g.c(), N0, N1, g.nz, k0, nzg, vel);
+            hipLaunchKernelGGL(k_vel_planes<float>, grd, blk, 0, h->stream, (const float *)g.c(), wall, N0, N1, k0, kwall, nzg, vel);
         else
-            hipLaunchKernelGGL(k_vel_planes<__half>, grd, blk, 0, h->stream, (const __half *)g.c(), N0, N1, g.nz, k0, nzg, vel);
+            hipLaunchKernelGGL(k_vel_planes<__half>, grd, blk, 0, h->stream, (const __half *)g.c(), wall, N0, N1, k0, kwall, nzg, vel);
         SPCHK(h, hipGetLastError());
-    }
-    if (grid != 0) {  // the band's wall layer is kept on the host
-        std::vector<double> wv;
-        wall_velocity(grid == 1 ? h->host_wall_lo : h->host_wall_up, N0, N1, wv);
-        const int kw = grid == 1 ? 0 : nzg - 1;
-        for (int c = 0; c < 3; c++)
-            SPCHK(h, hipMemcpyAsync(vel + ((size_t)c * nzg + kw) * plane, wv.data() + c * plane, plane * sizeof(double),
-                                    hipMemcpyHostToDevice, h->stream));
-        SPCHK(h, hipStreamSynchronize(h->stream));  // wv goes out of scope
     }
     {
         int dims[2] = {N0, N1};
@@ -176,9 +171,10 @@ extern "C" int dnsg_spectra(dnsg_t *h, int grid, double *ex, double *ey) {
         }
     }
     {
-        const long nout = 3L * nzg * (N0 + N1h);
-        hipLaunchKernelGGL(k_fold, dim3((unsigned)((nout + 255) / 256)), dim3(256), 0, h->stream, (const double2 *)cf, N0,
-                           N1, nzg, dex, dey);
+        hipLaunchKernelGGL(k_fold_x, dim3((unsigned)((3L * nzg * N0 + TB / 64 - 1) / (TB / 64))), dim3(TB), 0, h->stream,
+                           (const double2 *)cf, N0, N1, nzg, dex);
+        hipLaunchKernelGGL(k_fold_y, dim3((unsigned)(3 * nzg * ((N1h + 63) / 64))), dim3(TB), 0, h->stream,
+                           (const double2 *)cf, N0, N1, nzg, dey);
         SPCHK(h, hipGetLastError());
     }
     SPCHK(h, hipMemcpyAsync(ex, dex, 3 * (size_t)N0 * nzg * sizeof(double), hipMemcpyDeviceToHost, h->stream));
