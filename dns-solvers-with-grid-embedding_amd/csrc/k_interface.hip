@@ -24,6 +24,7 @@
 
 #include "internal.hpp"
 #include "lattice.hpp"
+#include "stream_common.hpp"
 
 namespace dnsg {
 
@@ -294,237 +295,319 @@ __device__ __forceinline__ void store_pair(__half *p, float a, float b) {
 }
 
 // ---- fused interface fill ----------------------------------------------------------
-// One workgroup = one TX x TY tile of coarse cells of one band.  For each of the
-// 23 plane values in turn it
-//   1. forms the Hermite-in-time value on the tile plus a 2-cell halo, in LDS
-//      (the loads of the next value are issued before this value is processed);
-//   2. takes d/dx, d/dy at the tile's (TX+1) x (TY+1) corners (d/dy also on the
-//      halo columns), in LDS;
-//   3. forms d2/dxdy = d/dx of d/dy at its cell's 4 corners, builds the cell's 16
-//      bicubic coefficients and evaluates them at its GR x GR fine columns;
-//   4. keeps rho and u (the first four values, each a phase of its own with a
-//      fixed destination register set) in registers; for a distribution value
-//      writes f = feq + tau_f/(GR tau_c) f_neq straight from registers, GR
-//      adjacent fine values per store.
+// One workgroup = one TX x TY tile of coarse cells of one band.  The 23 plane values
+// are taken two at a time: rho and u_x, u_y and u_z, then nine pairs of directions and
+// the rest direction alone.  For each two
+//   1. the Hermite-in-time values on the tile plus a 2-cell halo go to LDS (the loads
+//      of the next two are issued before these are processed);
+//   2. d/dx, d/dy at the tile's (TX+1) x (TY+1) corners (and on the halo columns) are
+//      formed in LDS;
+//   3. each thread forms d2/dxdy = d/dx of d/dy at its cell's 4 corners, builds the
+//      cell's 16 bicubic coefficients and evaluates them at its GR x GR fine columns;
+//   4. rho and u stay in registers; distribution values are written as
+//      f = feq + tau_f/(GR tau_c) f_neq straight from registers, GR adjacent fine
+//      values per store.
+// Bound by its own vector work and the wait for the planes about equally.  Re_tau=180,
+// both bands, us a launch, first / last substep: FP64 97 / 73 (3.1 TB/s; with one value
+// at a time and all planes read 108 / 108), FP32 53 / 39 (57 / 57), FP16 50 / 39
+// (54 / 54); the serving queue's step of 16 channels 1096 -> 1040 us.  Two at a time
+// halves the waits and gives the loads of the next two twice the time; both directions'
+// results kept so that opposite ones share the even part of feq take more registers
+// and are slower in FP64 (100 / 75).
+// LAST: the substep at t = 1, where the Hermite weights are 0, 0, 1, 0 and the value is
+// the newest plane's: the two older planes are not read.
 struct IfaceItem {
     const void *ln, *lp, *lpp;  // newest, previous, oldest plane levels [23][Yc][Xc]
     void *band;                 // band post-stream lattice
     int layer;                  // stored interface layer
     int Xc, Yc;
-    int groups;                 // workgroups per tile, each filling a share of the 19 directions
+    int groups;                 // workgroups per tile, each filling a share of the direction units
     double rescale;             // tau_f / (GR tau_c)
 };
 
-template <class S, class P, int GR, int TX, int TY>
+// units of directions: (1, 2), (3, 4) .. (17, 18), then the rest direction
+constexpr int IF_UNITS = 10;
+constexpr int if_dir(int unit, int i) { return unit < IF_UNITS - 1 ? 2 * unit + 1 + i : 0; }
+
+template <class S, class P, int GR, bool LAST, int TX, int TY>
 __global__ __launch_bounds__(TX *TY) void k_iface(Batch<IfaceItem> BT, HermiteW<P> H) {
     if (halted(BT.halt)) return;
+    static_assert(64 % TX == 0 && TX * TY % 64 == 0, "a wave holds whole tile rows");
     constexpr int NT = TX * TY, HX = TX + 5, HY = TY + 5, NP = GR * GR;
     constexpr int NH = (HX * HY + NT - 1) / NT;  // halo points per thread
-    // The value tile has two sets, used by alternate values: the next value is
-    // written there before the first wait, while slower threads still read this
-    // one.  The derivative tiles are written only after that wait, when every
-    // thread has finished reading them, so one set serves.
-    __shared__ P s0[2][HY][HX];       // value, halo 2 on each side (+1 corner)
-    __shared__ P s1[TY + 1][TX + 1];  // d/dx at the corners
-    __shared__ P s2[TY + 1][HX];      // d/dy at the corners and the halo columns
-    const int itm = batch_find(BT.first, BT.n, blockIdx.x);
+    constexpr int NL = LAST ? 1 : 3;             // plane levels read
+    constexpr int ND = (TY + 1) * HX;            // derivative points, the halo columns included
+    // The value tiles have two sets, used by alternate steps: the next values are
+    // written there before the first wait, while slower threads still read these.
+    // The derivative tiles are written only after that wait, when every thread has
+    // finished reading them, so one set serves.  All have rows of HX, so a derivative
+    // point's own value is 2 HX further on in the value tile; the d/dx of the halo
+    // columns are formed from neighbours in the next rows and never read.
+    __shared__ P s0[2][2][HX * HY];  // value, halo 2 on each side (+1 corner)
+    __shared__ P s1[2][ND];          // d/dx
+    __shared__ P s2[2][ND];          // d/dy
+    const int bid = xcd_remap(blockIdx.x, gridDim.x);
+    const int itm = batch_find(BT.first, BT.n, bid);
     const IfaceItem &B = BT.it[itm];
-    const int lbg = blockIdx.x - BT.first[itm];
+    const int lbg = bid - BT.first[itm];
     const int G = B.groups, lb = lbg / G, grp = lbg % G;
-    // this workgroup's directions [q0, q1); rho and u (values 0..3) are formed by every group
-    const int q0 = (Q * grp) / G, q1 = (Q * (grp + 1)) / G, nv = 4 + q1 - q0;
+    // this workgroup's units [q0, q1); rho and u are formed by every group
+    const int q0 = (IF_UNITS * grp) / G, q1 = (IF_UNITS * (grp + 1)) / G, steps = 2 + q1 - q0;
     const int Xc = B.Xc, Yc = B.Yc;
     const P rescale = (P)B.rescale;
-    const P *__restrict__ Ln = static_cast<const P *>(B.ln);
-    const P *__restrict__ Lp = static_cast<const P *>(B.lp);
-    const P *__restrict__ Lpp = static_cast<const P *>(B.lpp);
     const int ntx = (Xc + TX - 1) / TX;
     const int x0 = (lb % ntx) * TX, y0 = (lb / ntx) * TY;
     const int tid = threadIdx.x, cx = tid % TX, cy = tid / TX;
-    const int n = Xc * Yc, Xf = GR * Xc, Yf = GR * Yc;
-    S *band = static_cast<S *>(B.band);
-    // halo points of this thread and their plane offsets (fixed for every value)
-    int hoff[NH];
+    const size_t n = (size_t)Xc * Yc;
+    const int Xf = GR * Xc, Yf = GR * Yc;
+    // halo points of this thread: byte offsets in a plane (fixed for every value)
+    unsigned hoff[NH];
     bool hok[NH];
 #pragma unroll
     for (int k = 0; k < NH; k++) {
         const int p = tid + k * NT;
         hok[k] = p < HX * HY;
         const int gx = ((x0 - 2 + p % HX) % Xc + Xc) % Xc, gy = ((y0 - 2 + p / HX) % Yc + Yc) % Yc;
-        hoff[k] = hok[k] ? gy * Xc + gx : 0;
+        hoff[k] = hok[k] ? (unsigned)(gy * Xc + gx) * (unsigned)sizeof(P) : 0u;
     }
-    P a[NH][3];
+    // plane values of a step: 0, 1 / 2, 3 / 4 + direction, the second < 0 for the rest unit
+    auto values_of = [&](int st, int &va, int &vb) {
+        if (st < 2) { va = 2 * st; vb = va + 1; return; }
+        const int u = q0 + st - 2;
+        va = 4 + if_dir(u, 0);
+        vb = u < IF_UNITS - 1 ? 4 + if_dir(u, 1) : -1;
+    };
+    P a[2][NH][NL];
+    auto fetch = [&](int st) __attribute__((always_inline)) {
+        int v[2];
+        values_of(st, v[0], v[1]);
 #pragma unroll
-    for (int k = 0; k < NH; k++)
-        if (hok[k]) { a[k][0] = Ln[hoff[k]]; a[k][1] = Lp[hoff[k]]; a[k][2] = Lpp[hoff[k]]; }
-    // value phase iv (value 0..3: rho, u; then directions q0..q1-1): steps 1-3 for
-    // that value, its bicubic result at the cell's fine columns into r
-    auto phase = [&](int iv, P *r) __attribute__((always_inline)) {
-        const int sb = iv & 1;
-        // 1. Hermite value on the halo tile (tinterpolate_hrmt.c:28-34)
+        for (int i = 0; i < 2; i++) {
+            if (i == 1 && v[1] < 0) continue;
+            const size_t vo = (size_t)v[i] * n;
+            const char *L0 = reinterpret_cast<const char *>(static_cast<const P *>(B.ln) + vo);
+            const char *L1 = reinterpret_cast<const char *>(static_cast<const P *>(B.lp) + vo);
+            const char *L2 = reinterpret_cast<const char *>(static_cast<const P *>(B.lpp) + vo);
 #pragma unroll
-        for (int k = 0; k < NH; k++) {
-            if (!hok[k]) continue;
-            const int p = tid + k * NT;
-            const P ln = a[k][0], lp = a[k][1], lpp = a[k][2];
-            const P c1 = lp;
-            const P c2 = (ln - lpp) * (P)0.5;
-            const P c3 = ln;
-            const P c4 = (fma_exact((P)-4., lp, (P)3. * ln) + lpp) * (P)0.5;  // 3 ln - 4 lp
-            P hv;
-            if (H.exact) hv = fma_exact(H.h11, c4, fma_exact(H.h01, c3, fma_exact(H.h10, c2, H.h00 * c1)));
-            else hv = H.h00 * c1 + H.h10 * c2 + H.h01 * c3 + H.h11 * c4;
-            s0[sb][p / HX][p % HX] = hv;
+            for (int k = 0; k < NH; k++) {
+                if (!hok[k]) continue;
+                a[i][k][0] = *reinterpret_cast<const P *>(L0 + hoff[k]);
+                if constexpr (!LAST) {
+                    a[i][k][1] = *reinterpret_cast<const P *>(L1 + hoff[k]);
+                    a[i][k][2] = *reinterpret_cast<const P *>(L2 + hoff[k]);
+                }
+            }
         }
-        if (iv + 1 < nv) {  // prefetch the next value
-            const size_t vo = (size_t)(iv + 1 < 4 ? iv + 1 : 4 + q0 + (iv + 1 - 4)) * n;
+    };
+    // 1. and 2. of a step; leaves its values and derivatives in LDS
+    auto stage = [&](int st) __attribute__((always_inline)) {
+        const int sb = st & 1;
 #pragma unroll
-            for (int k = 0; k < NH; k++)
-                if (hok[k]) { a[k][0] = Ln[vo + hoff[k]]; a[k][1] = Lp[vo + hoff[k]]; a[k][2] = Lpp[vo + hoff[k]]; }
+        for (int i = 0; i < 2; i++)
+#pragma unroll
+            for (int k = 0; k < NH; k++) {
+                if (!hok[k]) continue;
+                P hv;
+                if constexpr (LAST) {
+                    hv = a[i][k][0];
+                } else {  // tinterpolate_hrmt.c:28-34
+                    const P ln = a[i][k][0], lp = a[i][k][1], lpp = a[i][k][2];
+                    const P c1 = lp;
+                    const P c2 = (ln - lpp) * (P)0.5;
+                    const P c3 = ln;
+                    const P c4 = (fma_exact((P)-4., lp, (P)3. * ln) + lpp) * (P)0.5;  // 3 ln - 4 lp
+                    if (H.exact)
+                        hv = fma_exact(H.h11, c4, fma_exact(H.h01, c3, fma_exact(H.h10, c2, H.h00 * c1)));
+                    else hv = H.h00 * c1 + H.h10 * c2 + H.h01 * c3 + H.h11 * c4;
+                }
+                s0[sb][i][tid + k * NT] = hv;
+            }
+        if (st + 1 < steps) fetch(st + 1);
+        __syncthreads();
+        // d/dx, d/dy (derivative.c:41-42, 63-64)
+#pragma unroll 1
+        for (int p = tid; p < 2 * ND; p += NT) {
+            const int i = p >= ND ? 1 : 0, r = p - i * ND;
+            const P *c = &s0[sb][i][r + 2 * HX];
+            s2[i][r] = d4(c[-2 * HX], c[-HX], c[HX], c[2 * HX]);
+            s1[i][r] = d4(c[-2], c[-1], c[1], c[2]);
         }
         __syncthreads();
-        // 2. d/dy on corner rows for every halo column; d/dx at the corners (derivative.c:41-42, 63-64)
-        P(*t0)[HX] = s0[sb];
-        for (int p = tid; p < (TY + 1) * HX; p += NT) {
-            const int rr = p / HX, hx = p % HX, hy = rr + 2;
-            s2[rr][hx] = d4(t0[hy - 2][hx], t0[hy - 1][hx], t0[hy + 1][hx], t0[hy + 2][hx]);
-            if (hx >= 2 && hx <= TX + 2)
-                s1[rr][hx - 2] = d4(t0[hy][hx - 2], t0[hy][hx - 1], t0[hy][hx + 1], t0[hy][hx + 2]);
-        }
-        __syncthreads();
-        // 3. bicubic patch of this cell (bcucof_opt.c:47-61) at its fine columns;
-        //    d2/dxdy = d/dx of d/dy (derivative.c:84) at the cell's corners, from
-        //    the d/dy of columns cx .. cx+5 on its two corner rows
+    };
+    // 3. bicubic patch of this cell (bcucof_opt.c:47-61) at its fine columns for value i
+    //    of the step; d2/dxdy = d/dx of d/dy (derivative.c:84) at the cell's corners,
+    //    from the d/dy of columns cx .. cx+5 on its two corner rows
+    const int c0 = cy * HX + cx;
+    auto patch = [&](int st, int i, P *r) __attribute__((always_inline)) {
+        const P *t0 = &s0[st & 1][i][c0 + 2 * HX + 2], *dx = &s1[i][c0 + 2], *dy = &s2[i][c0];
         P xv[16];
         P dyr[2][6];
 #pragma unroll
         for (int j = 0; j < 2; j++)
 #pragma unroll
-            for (int i = 0; i < 6; i++) dyr[j][i] = s2[cy + j][cx + i];
-        xv[0] = t0[cy + 2][cx + 2]; xv[4] = s1[cy][cx];         xv[8] = dyr[0][2];
-        xv[1] = t0[cy + 2][cx + 3]; xv[5] = s1[cy][cx + 1];     xv[9] = dyr[0][3];
-        xv[2] = t0[cy + 3][cx + 3]; xv[6] = s1[cy + 1][cx + 1]; xv[10] = dyr[1][3];
-        xv[3] = t0[cy + 3][cx + 2]; xv[7] = s1[cy + 1][cx];     xv[11] = dyr[1][2];
+            for (int k = 0; k < 6; k++) dyr[j][k] = dy[j * HX + k];
+        xv[0] = t0[0];      xv[4] = dx[0];      xv[8] = dyr[0][2];
+        xv[1] = t0[1];      xv[5] = dx[1];      xv[9] = dyr[0][3];
+        xv[2] = t0[HX + 1]; xv[6] = dx[HX + 1]; xv[10] = dyr[1][3];
+        xv[3] = t0[HX];     xv[7] = dx[HX];     xv[11] = dyr[1][2];
         xv[12] = d4(dyr[0][0], dyr[0][1], dyr[0][3], dyr[0][4]);
         xv[13] = d4(dyr[0][1], dyr[0][2], dyr[0][4], dyr[0][5]);
         xv[14] = d4(dyr[1][1], dyr[1][2], dyr[1][4], dyr[1][5]);
         xv[15] = d4(dyr[1][0], dyr[1][1], dyr[1][3], dyr[1][4]);
         bicubic_patch<GR>(xv, r);
     };
+    // the fine columns of this cell for direction q: the wave's first row and the
+    // direction are uniform, the rest is this lane's offset
+    const bool inside = x0 + cx < Xc && y0 + cy < Yc;
+    const int wave_row = (__builtin_amdgcn_readfirstlane(tid >> 6)) * (64 / TX);
+    S *const wbase = static_cast<S *>(B.band) + lat_at(0, (size_t)B.layer * Yf + (size_t)GR * (y0 + wave_row), 0, Xf);
+    const unsigned lane_off =
+        ((unsigned)((cy - wave_row) * GR * Q) * (unsigned)Xf + (unsigned)(GR * (x0 + cx))) * (unsigned)sizeof(S);
+    auto put = [&](auto qc, S *wb, const P *out) __attribute__((always_inline)) {
+        constexpr int QD = decltype(qc)::value;
+        if (!inside) return;
+#pragma unroll
+        for (int jj = 0; jj < GR; jj++) {
+            S *dst = reinterpret_cast<S *>(reinterpret_cast<char *>(wb + (size_t)(jj * Q + QD) * Xf) + lane_off);
+            if constexpr (GR == 2) {
+                store_pair(dst, out[jj], out[GR + jj]);  // ii = 0, 1
+            } else {  // pairs are slower at gratio 4 (FP64: 102 against 79 us)
+#pragma unroll
+                for (int ii = 0; ii < GR; ii++) store_s(dst + ii, out[ii * GR + jj]);
+            }
+        }
+    };
+    fetch(0);
     // rho and u stay in registers for every direction of this workgroup
     P dens[NP], u0[NP], u1[NP], u2[NP];
-    phase(0, dens);
-    phase(1, u0);
-    phase(2, u1);
-    phase(3, u2);
-    for (int iv = 4; iv < nv; iv++) {
-        P r[NP];
-        phase(iv, r);
-        // 4. f = feq + tau_f/(GR tau_c) f_neq for direction q (uniform over the
-        //    workgroup): one branch per direction, so e_q . u is edot<q> itself
-        const int q = q0 + iv - 4;
-        // feq depends on rho and u only: without this (empty) register constraint
-        // the compiler hoists it out of the loop for all 19 directions at once,
-        // which holds 19 NP values in registers and lowers occupancy
+    stage(0);
+    patch(0, 0, dens);
+    patch(0, 1, u0);
+    stage(1);
+    patch(1, 0, u1);
+    patch(1, 1, u2);
+    for (int st = 2; st < steps; st++) {
+        stage(st);
+        // 4. the unit is uniform over the workgroup: one branch per unit, so e_q . u is
+        //    edot<q> itself
+        const int unit = q0 + st - 2;
+        // feq depends on rho and u only, the stores' addresses on the tile only: without
+        // these (empty) register constraints the compiler forms both for many directions
+        // ahead, and the registers that hold them cost half of the waves (137 against 66
+        // in FP32)
+        S *wb = wbase;
+        auto keep = [&]() __attribute__((always_inline)) {
+            asm volatile("" : "+s"(wb));
 #pragma unroll
-        for (int pp = 0; pp < NP; pp++) asm volatile("" : "+v"(dens[pp]), "+v"(u0[pp]), "+v"(u1[pp]), "+v"(u2[pp]));
-        unroll<0, Q>([&](auto qc) {
+            for (int pp = 0; pp < NP; pp++)
+                asm volatile("" : "+v"(dens[pp]), "+v"(u0[pp]), "+v"(u1[pp]), "+v"(u2[pp]));
+        };
+        auto value = [&](auto qc, int pp, P r) __attribute__((always_inline)) {
             constexpr int QD = decltype(qc)::value;
-            if (q != QD) return;
             const P wq = (P)WQ[QD];
-            P out[NP];
-#pragma unroll
-            for (int pp = 0; pp < NP; pp++) {
-                const P eu = edot<QD>(u0[pp], u1[pp], u2[pp]);
-                // u.u formed again for every direction, the same expression each time,
-                // rather than held through the loop (registers)
-                const P vsq = u0[pp] * u0[pp] + u1[pp] * u1[pp] + u2[pp] * u2[pp];
-                if constexpr (sizeof(S) == 8) {
-                    const P feq = wq * dens[pp] * ((P)1. + (P)3. * eu + (P)4.5 * eu * eu - (P)1.5 * vsq);
-                    out[pp] = feq + rescale * r[pp];  // ctfdtransfer_opt.c:93
-                } else {  // dens holds rho - 1
-                    const P rho = (P)1. + dens[pp];
-                    const P geq = wq * (dens[pp] + rho * ((P)3. * eu + (P)4.5 * eu * eu - (P)1.5 * vsq));
-                    out[pp] = geq + rescale * r[pp];
-                }
+            const P eu = edot<QD>(u0[pp], u1[pp], u2[pp]);
+            // u.u formed again for every direction, the same expression each time,
+            // rather than held through the loop (registers)
+            const P vsq = u0[pp] * u0[pp] + u1[pp] * u1[pp] + u2[pp] * u2[pp];
+            if constexpr (sizeof(S) == 8) {
+                const P feq = wq * dens[pp] * ((P)1. + (P)3. * eu + (P)4.5 * eu * eu - (P)1.5 * vsq);
+                return feq + rescale * r;  // ctfdtransfer_opt.c:93
+            } else {  // dens holds rho - 1
+                const P rho = (P)1. + dens[pp];
+                const P geq = wq * (dens[pp] + rho * ((P)3. * eu + (P)4.5 * eu * eu - (P)1.5 * vsq));
+                return geq + rescale * r;
             }
-            // the fine columns of this cell, straight from registers: a half-wave's
-            // cells cover one contiguous run of each fine row
-            if (x0 + cx < Xc && y0 + cy < Yc) {
+        };
+        auto direction = [&](auto ic) __attribute__((always_inline)) {
+            constexpr int i = decltype(ic)::value;
+            P r[NP];
+            patch(st, i, r);
+            unroll<0, IF_UNITS - i>([&](auto uc) {  // the rest unit has no second direction
+                constexpr int U = decltype(uc)::value;
+                if (unit != U) return;
+                constexpr std::integral_constant<int, if_dir(U, i)> qd;
 #pragma unroll
-                for (int jj = 0; jj < GR; jj++) {
-                    S *dst = band + lat_at(QD, (size_t)B.layer * Yf + GR * (y0 + cy) + jj, GR * (x0 + cx), Xf);
-                    if constexpr (GR == 2) {
-                        store_pair(dst, out[jj], out[GR + jj]);  // ii = 0, 1
-                    } else {
-#pragma unroll
-                        for (int ii = 0; ii < GR; ii++) store_s(dst + ii, out[ii * GR + jj]);
-                    }
-                }
-            }
-        });
+                for (int pp = 0; pp < NP; pp++) r[pp] = value(qd, pp, r[pp]);
+                put(qd, wb, r);
+            });
+        };
+        keep();
+        direction(std::integral_constant<int, 0>{});
+        keep();
+        if (unit < IF_UNITS - 1) direction(std::integral_constant<int, 1>{});
     }
 }
 
-// Coarse tile of one workgroup.  The 19 directions can be shared out over G
+// Coarse tile of one workgroup.  The direction units can be shared out over G
 // workgroups per tile, each forming rho and u itself: that multiplies the work by
-// (4 + 19/G) G / 23 but shortens each workgroup's chain of sequential value phases
-// to 4 + 19/G.  G fills the workgroup slots the GPU holds at once for this kernel
+// (4 + 19/G) G / 23 but shortens each workgroup's chain of sequential steps
+// to 2 + 10/G.  G fills the workgroup slots the GPU holds at once for this kernel
 // (CUs x resident workgroups per CU, from the occupancy query): a launch whose
 // tiles alone fill them (the Re_tau=180 bands: 1024 tiles) takes G = 1, a launch of
-// small channels (the serving queue) shortens its chains, up to G = 19.
+// small channels (the serving queue) shortens its chains, up to G = 10.
 constexpr int IF_TX = 32, IF_TY = 8;
 
-template <class S, class P, int GR>
+template <class S, class P, int GR, bool LAST>
 static int iface_slots() {
     static int slots = 0;  // per kernel; concurrent first calls compute the same value
     if (slots == 0) {
         int dev = 0, cus = 0, per_cu = 0;
         if (hipGetDevice(&dev) == hipSuccess &&
             hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess &&
-            hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_iface<S, P, GR, IF_TX, IF_TY>, IF_TX * IF_TY, 0) ==
-                hipSuccess &&
+            hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_iface<S, P, GR, LAST, IF_TX, IF_TY>,
+                                                         IF_TX * IF_TY, 0) == hipSuccess &&
             cus > 0 && per_cu > 0)
             slots = cus * per_cu;
-        else
+        else {
+            (void)hipGetLastError();  // answered here: not the launch's error
             slots = 1024;
+        }
     }
     return slots;
 }
 
 static int iface_groups(long tiles, int slots) {
     if (tiles >= slots) return 1;
-    return (int)std::min<long>(Q, slots / tiles);
+    return (int)std::min<long>(IF_UNITS, slots / tiles);
 }
 
-template <class S, class P, int GR>
+template <class S, class P, int GR, bool LAST>
 static hipError_t iface_launch(hipStream_t s, IfaceItem *items, int n, HermiteW<P> H, const int *halt) {
     for (int i0 = 0; i0 < n; i0 += BATCH_MAX) {
         const int m = std::min(BATCH_MAX, n - i0);
         long tiles = 0;
         for (int i = i0; i < i0 + m; i++)
             tiles += (long)((items[i].Xc + IF_TX - 1) / IF_TX) * ((items[i].Yc + IF_TY - 1) / IF_TY);
-        const int G = iface_groups(tiles, iface_slots<S, P, GR>());
+        const int G = iface_groups(tiles, iface_slots<S, P, GR, LAST>());
         for (int i = i0; i < i0 + m; i++) items[i].groups = G;
         Batch<IfaceItem> B;
         B.halt = halt;
         const int blocks = fill_batch(B, items + i0, m, [](const IfaceItem &a) {
             return ((a.Xc + IF_TX - 1) / IF_TX) * ((a.Yc + IF_TY - 1) / IF_TY) * a.groups;
         });
-        hipLaunchKernelGGL((k_iface<S, P, GR, IF_TX, IF_TY>), dim3(blocks), dim3(IF_TX * IF_TY), 0, s, B, H);
+        hipLaunchKernelGGL((k_iface<S, P, GR, LAST, IF_TX, IF_TY>), dim3(blocks), dim3(IF_TX * IF_TY), 0, s, B, H);
         const hipError_t e = hipGetLastError();
         if (e != hipSuccess) return e;
     }
     return hipSuccess;
 }
 
+template <class S, class P, int GR>
+static hipError_t iface_gr(hipStream_t s, IfaceItem *items, int n, HermiteW<P> H, const int *halt) {
+    // weights 0, 0, 1, 0: the last substep, and the only one at gratio 1
+    if (H.h00 == (P)0 && H.h10 == (P)0 && H.h01 == (P)1 && H.h11 == (P)0)
+        return iface_launch<S, P, GR, true>(s, items, n, H, halt);
+    if constexpr (GR > 1) return iface_launch<S, P, GR, false>(s, items, n, H, halt);
+    return hipErrorInvalidValue;
+}
+
 template <class S, class P>
 static hipError_t iface_items(hipStream_t s, int GR, IfaceItem *items, int n, HermiteW<P> H, const int *halt) {
     switch (GR) {
-    case 1: return iface_launch<S, P, 1>(s, items, n, H, halt);
-    case 2: return iface_launch<S, P, 2>(s, items, n, H, halt);
-    case 3: return iface_launch<S, P, 3>(s, items, n, H, halt);
-    default: return iface_launch<S, P, 4>(s, items, n, H, halt);
+    case 1: return iface_gr<S, P, 1>(s, items, n, H, halt);
+    case 2: return iface_gr<S, P, 2>(s, items, n, H, halt);
+    case 3: return iface_gr<S, P, 3>(s, items, n, H, halt);
+    default: return iface_gr<S, P, 4>(s, items, n, H, halt);
     }
 }
 
