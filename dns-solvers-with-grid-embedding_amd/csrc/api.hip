@@ -10,8 +10,11 @@
 #include <stdlib.h>
 #include <string.h>
 
+#include <algorithm>
 #include <mutex>
 #include <new>
+#include <system_error>
+#include <thread>
 #include <vector>
 
 #include "internal.hpp"
@@ -125,7 +128,7 @@ int ensure_diag(dnsg_t *h, int n) {
     if (h->d_diag) HIPCHK(h, hipFree(h->d_diag));
     h->d_diag = nullptr;
     h->diag_cap = 0;
-    HIPCHK(h, hipMalloc(&h->d_diag, sizeof(double) * DIAG_WORDS * (size_t)n));
+    HIPCHK(h, dev_malloc(&h->d_diag, sizeof(double) * DIAG_WORDS * (size_t)n));
     h->diag_cap = n;
     return DNSG_OK;
 }
@@ -661,17 +664,175 @@ int get_levels(dnsg_t *h, double *const *lv, void *const *dev, HostLayout L = {}
     return DNSG_OK;
 }
 
+}  // namespace
+
+namespace {
+
+struct ScratchBlock {
+    void *p;
+    size_t bytes;
+    int dev;
+    bool used;
+};
+struct ScratchPool {
+    std::mutex m;
+    ScratchBlock b[64];
+    int n = 0, users = 0;  // b[0, n): handed out or kept, the longest kept first
+    void drop(int i) {
+        (void)hipFree(b[i].p);
+        std::move(b + i + 1, b + n, b + i);
+        n--;
+    }
+    void trim() {
+        for (int i = n - 1; i >= 0; i--)
+            if (!b[i].used) drop(i);
+    }
+};
+// never destroyed: handles may outlive the static objects of this library
+ScratchPool &pool() {
+    static ScratchPool &p = *new ScratchPool;
+    return p;
+}
+
+}  // namespace
+
+void dnsg::scratch_trim() {
+    std::lock_guard<std::mutex> l(pool().m);
+    pool().trim();
+}
+
+void dnsg::scratch_users(int change) {
+    std::lock_guard<std::mutex> l(pool().m);
+    pool().users += change;
+    if (pool().users == 0) pool().trim();
+}
+
+hipError_t dnsg::scratch_get(void **p, size_t bytes) {
+    int dev = 0;
+    hipError_t e = hipGetDevice(&dev);
+    if (e != hipSuccess) return e;
+    ScratchPool &P = pool();
+    {
+        // the smallest kept block that is large enough and no more than twice the size
+        std::lock_guard<std::mutex> l(P.m);
+        ScratchBlock *best = nullptr;
+        for (int i = 0; i < P.n; i++) {
+            ScratchBlock &c = P.b[i];
+            if (!c.used && c.dev == dev && c.bytes >= bytes && c.bytes / 2 <= bytes && (!best || c.bytes < best->bytes)) best = &c;
+        }
+        if (best) {
+            best->used = true;
+            *p = best->p;
+            return hipSuccess;
+        }
+    }
+    e = dev_malloc(p, bytes);
+    if (e != hipSuccess) return e;
+    std::lock_guard<std::mutex> l(P.m);
+    if (P.n == 64)
+        for (int i = 0; i < P.n; i++)
+            if (!P.b[i].used) {
+                P.drop(i);
+                break;
+            }
+    if (P.n < 64) P.b[P.n++] = {*p, bytes, dev, true};  // else it is freed when given back
+    return hipSuccess;
+}
+
+void dnsg::scratch_put(void *p) {
+    if (!p) return;
+    ScratchPool &P = pool();
+    std::lock_guard<std::mutex> l(P.m);
+    int i = 0;
+    while (i < P.n && P.b[i].p != p) i++;
+    if (i == P.n) {
+        (void)hipFree(p);
+        return;
+    }
+    std::rotate(P.b + i, P.b + i + 1, P.b + P.n);
+    ScratchBlock &mine = P.b[P.n - 1];
+    mine.used = false;
+    const int dev = mine.dev;
+    size_t total = 0, kept = 0;
+    if (hipDeviceTotalMem(&total, dev) != hipSuccess) total = 0;
+    for (int j = 0; j < P.n; j++)
+        if (!P.b[j].used && P.b[j].dev == dev) kept += P.b[j].bytes;
+    for (int j = 0; j < P.n && kept > total / 64;) {  // the longest kept go first
+        if (P.b[j].used || P.b[j].dev != dev) {
+            j++;
+            continue;
+        }
+        kept -= P.b[j].bytes;
+        P.drop(j);
+    }
+}
+
+// A plain copy into pageable memory runs at the rate of one host thread that also takes
+// the page faults of a fresh array (4 to 10 GB/s against 57 of the link).  From two
+// pieces on, the data comes through two pinned buffers instead: while the link fills one,
+// a few threads move the other on (20 to 29 GB/s).  The buffers live for the call, about
+// 0.5 ms, so a single piece (1.6 ms) is left to the plain copy; so is an array that the
+// device can write itself (pinned or device memory).
+hipError_t dnsg::copy_out(hipStream_t s, void *dst, const void *src, size_t bytes) {
+    constexpr size_t PIECE = (size_t)16 << 20;
+    hipPointerAttribute_t at;
+    const bool pageable = hipPointerGetAttributes(&at, dst) != hipSuccess || at.type == hipMemoryTypeUnregistered;
+    if (pageable) (void)hipGetLastError();  // an unknown pointer is an answer, not an error
+    char *buf = nullptr;
+    if (!pageable || bytes < 2 * PIECE || hipHostMalloc((void **)&buf, 2 * PIECE, hipHostMallocDefault) != hipSuccess) {
+        if (pageable) (void)hipGetLastError();
+        const hipError_t e = hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, s);
+        const hipError_t w = hipStreamSynchronize(s);
+        return e != hipSuccess ? e : w;
+    }
+    const int nt = (int)std::min(4u, std::max(1u, std::thread::hardware_concurrency()));
+    const size_t pieces = (bytes + PIECE - 1) / PIECE;
+    auto len = [&](size_t p) { return std::min(PIECE, bytes - p * PIECE); };
+    auto fetch = [&](size_t p) {
+        return hipMemcpyAsync(buf + (p & 1) * PIECE, static_cast<const char *>(src) + p * PIECE, len(p),
+                              hipMemcpyDeviceToHost, s);
+    };
+    hipError_t e = fetch(0);
+    for (size_t p = 0; p < pieces && e == hipSuccess; p++) {
+        e = hipStreamSynchronize(s);
+        if (e == hipSuccess && p + 1 < pieces) e = fetch(p + 1);
+        if (e != hipSuccess) break;
+        const size_t n = len(p);
+        auto share = [&](int t) {
+            const size_t a = n * t / nt, b = n * (t + 1) / nt;
+            memcpy(static_cast<char *>(dst) + p * PIECE + a, buf + (p & 1) * PIECE + a, b - a);
+        };
+        std::thread th[4];
+        for (int t = 1; t < nt; t++) {
+            try {
+                th[t] = std::thread(share, t);
+            } catch (const std::system_error &) {  // no thread to be had
+                share(t);
+            }
+        }
+        share(0);
+        for (int t = 1; t < nt; t++)
+            if (th[t].joinable()) th[t].join();
+    }
+    const hipError_t w = hipStreamSynchronize(s);
+    (void)hipHostFree(buf);
+    return e != hipSuccess ? e : w;
+}
+
+namespace {
+
 // AoS [X(+1)][Y(+1)][zaos][19] host array <-> SoA device lattice (stored layers z0..z0+nz-1)
 int put_lattice(dnsg_t *h, const double *aos, Grid &g, int zaos, int z0, HostLayout L = {}) {
     const int gl = L.gl();
     const size_t n = (size_t)(g.nx + gl) * (g.ny + gl) * zaos * 19;
     double *stage = nullptr;
-    HIPCHK(h, hipMalloc(&stage, n * 8));
+    HIPCHK(h, scratch_get(&stage, n * 8));
     hipError_t e = hipMemcpyAsync(stage, aos, n * 8, hipMemcpyHostToDevice, h->stream);
     if (e == hipSuccess)
         e = launch_aos_to_soa(h->stream, stage, g.c(), g.nx, g.ny, zaos, z0, g.nz, h->p.precision, gl);
-    if (e == hipSuccess) e = hipStreamSynchronize(h->stream);
-    (void)hipFree(stage);
+    const hipError_t w = hipStreamSynchronize(h->stream);
+    if (e == hipSuccess) e = w;
+    scratch_put(stage);
     HIPCHK(h, e);
     return DNSG_OK;
 }
@@ -680,13 +841,13 @@ int get_lattice(dnsg_t *h, double *aos, const Grid &g, int zaos, int z0, HostLay
     const int gl = L.gl();
     const size_t n = (size_t)(g.nx + gl) * (g.ny + gl) * zaos * 19;
     double *stage = nullptr;
-    HIPCHK(h, hipMalloc(&stage, n * 8));
+    HIPCHK(h, scratch_get(&stage, n * 8));
     hipError_t e = hipMemsetAsync(stage, 0, n * 8, h->stream);
     if (e == hipSuccess)
         e = launch_soa_to_aos(h->stream, g.c(), stage, g.nx, g.ny, zaos, z0, g.nz, h->p.precision, gl);
-    if (e == hipSuccess) e = hipMemcpyAsync(aos, stage, n * 8, hipMemcpyDeviceToHost, h->stream);
-    if (e == hipSuccess) e = hipStreamSynchronize(h->stream);
-    (void)hipFree(stage);
+    if (e == hipSuccess) e = copy_out(h->stream, aos, stage, n * 8);
+    else (void)hipStreamSynchronize(h->stream);
+    scratch_put(stage);
     HIPCHK(h, e);
     return DNSG_OK;
 }
@@ -832,10 +993,12 @@ int dnsg_destroy(dnsg_t *h) {
     for (void *q : ptrs)
         if (q) (void)hipFree(q);
     if (h->h_pinned) (void)hipHostFree(h->h_pinned);
+    dnsg::spectra_release(h);
     free(h->host_wall_lo);
     free(h->host_wall_up);
     if (h->stream && h->own_stream) (void)hipStreamDestroy(h->stream);
     delete h;
+    dnsg::scratch_users(-1);
     return DNSG_OK;
 }
 
@@ -849,6 +1012,7 @@ int dnsg::create_ctx(const dnsg_params *p, hipStream_t ext, dnsg_t **out) {
     *out = nullptr;
     dnsg_t *h = new (std::nothrow) dnsg_ctx();
     if (!h) return DNSG_ERR_OOM;
+    scratch_users(1);
     h->p = *p;
     int rc = derive(p, &h->d, &h->err);
     if (rc) {
@@ -887,44 +1051,44 @@ int dnsg::create_ctx(const dnsg_params *p, hipStream_t ext, dnsg_t **out) {
     for (auto *g : gs)
         for (int b = 0; b < 2; b++) {
             const size_t bytes = g->qs() * 19 * h->elem;
-            HIPCHK(h, hipMalloc(&g->buf[b], bytes));
+            HIPCHK(h, dev_malloc(&g->buf[b], bytes));
             HIPCHK(h, hipMemsetAsync(g->buf[b], 0, bytes, h->stream));
         }
     const size_t np = (size_t)d.Xc * d.Yc * NVP;
     for (int l = 0; l < 4; l++) {
-        HIPCHK(h, hipMalloc(&h->lev_lo[l], np * 8));
-        HIPCHK(h, hipMalloc(&h->lev_up[l], np * 8));
+        HIPCHK(h, dev_malloc(&h->lev_lo[l], np * 8));
+        HIPCHK(h, dev_malloc(&h->lev_up[l], np * 8));
         HIPCHK(h, hipMemsetAsync(h->lev_lo[l], 0, np * 8, h->stream));
         HIPCHK(h, hipMemsetAsync(h->lev_up[l], 0, np * 8, h->stream));
     }
     const std::vector<int8_t> w = wall_codes(p, &d);
-    HIPCHK(h, hipMalloc(&h->wall_lo, w.size()));
-    HIPCHK(h, hipMalloc(&h->wall_up, w.size()));
+    HIPCHK(h, dev_malloc(&h->wall_lo, w.size()));
+    HIPCHK(h, dev_malloc(&h->wall_up, w.size()));
     HIPCHK(h, hipMemcpy(h->wall_lo, w.data(), w.size(), hipMemcpyHostToDevice));
     HIPCHK(h, hipMemcpy(h->wall_up, w.data(), w.size(), hipMemcpyHostToDevice));
     h->part_cap = partial_doubles(h);
-    HIPCHK(h, hipMalloc(&h->part, h->part_cap * 8));
+    HIPCHK(h, dev_malloc(&h->part, h->part_cap * 8));
     {
         const size_t nred =
             (coarse_parts_max(d) + 2 * band_parts_max(d)) * RED_W;
-        HIPCHK(h, hipMalloc(&h->red, nred * 8));
+        HIPCHK(h, dev_malloc(&h->red, nred * 8));
         HIPCHK(h, hipMemsetAsync(h->red, 0, nred * 8, h->stream));
-        HIPCHK(h, hipMalloc(&h->seg, enc_seg_doubles(h) * 8));
-        HIPCHK(h, hipMalloc(&h->dsum, dsum_doubles(h) * 8));
-        HIPCHK(h, hipMalloc(&h->fsum, 2 * (size_t)ftcd_blocks(h) * 8));
-        HIPCHK(h, hipMalloc(&h->enc_next, 8 * 8));
+        HIPCHK(h, dev_malloc(&h->seg, enc_seg_doubles(h) * 8));
+        HIPCHK(h, dev_malloc(&h->dsum, dsum_doubles(h) * 8));
+        HIPCHK(h, dev_malloc(&h->fsum, 2 * (size_t)ftcd_blocks(h) * 8));
+        HIPCHK(h, dev_malloc(&h->enc_next, 8 * 8));
     }
-    HIPCHK(h, hipMalloc(&h->d_force, 4 * 8));
+    HIPCHK(h, dev_malloc(&h->d_force, 4 * 8));
     HIPCHK(h, hipMemsetAsync(h->d_force, 0, 4 * 8, h->stream));
-    HIPCHK(h, hipMalloc(&h->d_halt, sizeof(int)));
+    HIPCHK(h, dev_malloc(&h->d_halt, sizeof(int)));
     HIPCHK(h, hipMemsetAsync(h->d_halt, 0, sizeof(int), h->stream));
     h->halt_flag = h->d_halt;
     if ((rc = noalloc_scratch(h, nullptr))) return rc;
     h->err.reserve(256);  // error texts of dnsg_step_noalloc fit without a reallocation
     const size_t nred = 4 * ((size_t)d.zdc + 2 * (d.zdf - 1)) + 2 * 9 * (size_t)d.NZ + 64;
-    HIPCHK(h, hipMalloc(&h->d_red, nred * 8));
+    HIPCHK(h, dev_malloc(&h->d_red, nred * 8));
     HIPCHK(h, hipMemsetAsync(h->d_red, 0, nred * 8, h->stream));
-    HIPCHK(h, hipMalloc(&h->d_acc, 14 * (size_t)d.NZ * 8));
+    HIPCHK(h, dev_malloc(&h->d_acc, 14 * (size_t)d.NZ * 8));
     HIPCHK(h, hipMemsetAsync(h->d_acc, 0, 14 * (size_t)d.NZ * 8, h->stream));
     if ((rc = ensure_diag(h, 64))) return rc;
     if ((rc = ensure_pinned(h, 64 + 9 * (size_t)d.NZ))) return rc;
@@ -935,8 +1099,8 @@ int dnsg::create_ctx(const dnsg_params *p, hipStream_t ext, dnsg_t **out) {
         return DNSG_ERR_OOM;
     }
     if (p->fltr) {
-        HIPCHK(h, hipMalloc(&h->fneq, fltr_fneq_doubles(h) * 8));
-        HIPCHK(h, hipMalloc(&h->fwall, fltr_wall_doubles(h) * 8));
+        HIPCHK(h, dev_malloc(&h->fneq, fltr_fneq_doubles(h) * 8));
+        HIPCHK(h, dev_malloc(&h->fwall, fltr_wall_doubles(h) * 8));
         HIPCHK(h, hipMemsetAsync(h->fwall, 0, fltr_wall_doubles(h) * 8, h->stream));
     }
     HIPCHK(h, hipStreamSynchronize(h->stream));
@@ -960,7 +1124,7 @@ static int sync_fwall(dnsg_t *h) {
 // once allocated, fwall is refreshed by every call that sets the state
 int dnsg::ensure_fwall(dnsg_t *h) {
     if (h->fwall) return DNSG_OK;
-    HIPCHK(h, hipMalloc(&h->fwall, fltr_wall_doubles(h) * 8));
+    HIPCHK(h, dev_malloc(&h->fwall, fltr_wall_doubles(h) * 8));
     return sync_fwall(h);
 }
 
@@ -1076,11 +1240,11 @@ int dnsg_init_uniform(dnsg_t *h, const double *uniform, int xdu, int ydu, int zd
     h->flux_fused = false;
     const size_t nu = (size_t)xdu * ydu * (zdu + 2) * 19;
     double *du = nullptr;
-    HIPCHK(h, hipMalloc(&du, nu * 8));
+    HIPCHK(h, scratch_get(&du, nu * 8));
     hipError_t e = hipMemcpy(du, uniform, nu * 8, hipMemcpyHostToDevice);
     if (e == hipSuccess) e = launch_uniform(h->stream, h, du, xdu, ydu, zdu);
     if (e == hipSuccess) e = hipStreamSynchronize(h->stream);
-    (void)hipFree(du);
+    scratch_put(du);
     HIPCHK(h, e);
     // main:986-987 call init() before solid_init(), so the band wall layers start at
     // rest like every other node (init.c:17-52) and the interpolation leaves them so
@@ -1414,13 +1578,12 @@ int dnsg_velocity_snapshot(dnsg_t *h, int grid, double *vel, double *den) {
     const int Z = grid == 0 ? h->d.zdc : h->d.zdf;
     const size_t nn = (size_t)X * Y * Z;
     double *dv = nullptr;
-    HIPCHK(h, hipMalloc(&dv, nn * 4 * 8));
+    HIPCHK(h, scratch_get(&dv, nn * 4 * 8));
     hipError_t e = launch_snapshot(h, grid, dv, dv + 3 * nn);
-    if (e == hipSuccess && vel) e = hipMemcpyAsync(vel, dv, nn * 3 * 8, hipMemcpyDeviceToHost, h->stream);
-    if (e == hipSuccess && den) e = hipMemcpyAsync(den, dv + 3 * nn, nn * 8, hipMemcpyDeviceToHost, h->stream);
-    if (e == hipSuccess) e = hipStreamSynchronize(h->stream);
-    else (void)hipStreamSynchronize(h->stream);
-    (void)hipFree(dv);
+    if (e == hipSuccess && vel) e = copy_out(h->stream, vel, dv, nn * 3 * 8);
+    if (e == hipSuccess && den) e = copy_out(h->stream, den, dv + 3 * nn, nn * 8);
+    (void)hipStreamSynchronize(h->stream);
+    scratch_put(dv);
     HIPCHK(h, e);
     return DNSG_OK;
 }

@@ -548,10 +548,10 @@ extern "C" int dnsg_budget2d(dnsg_t *h, double *turb, double *vort, double *ke, 
         nsum = std::max(nsum, (size_t)F.Z * NACC);
         nv += 4 * (size_t)F.X * F.Y * F.Z;
     }
-    BCHK(h, hipMalloc(&dv, nv * 8));
-    BCHK(h, hipMalloc(&dmean, 4 * (size_t)NZ * 8));
-    BCHK(h, hipMalloc(&dpart, npart * 8));
-    BCHK(h, hipMalloc(&dsum, 3 * nsum * 8));
+    BCHK(h, scratch_get(&dv, nv * 8));
+    BCHK(h, scratch_get(&dmean, 4 * (size_t)NZ * 8));
+    BCHK(h, scratch_get(&dpart, npart * 8));
+    BCHK(h, scratch_get(&dsum, 3 * nsum * 8));
     A.g[0].v = dv;
     for (int g = 1; g < 3; g++) A.g[g].v = A.g[g - 1].v + 4 * (size_t)A.g[g - 1].X * A.g[g - 1].Y * A.g[g - 1].Z;
     lay.resize(3 * nsum);
@@ -598,7 +598,7 @@ extern "C" int dnsg_budget2d(dnsg_t *h, double *turb, double *vort, double *ke, 
     }
     if (ufl) {
         const size_t np = (size_t)A.g[1].X * A.g[1].Y;
-        BCHK(h, hipMalloc(&dpl, 2 * np * 8));
+        BCHK(h, scratch_get(&dpl, 2 * np * 8));
         hipLaunchKernelGGL(k_bud_plane, dim3((unsigned)((np + BT - 1) / BT)), dim3(BT), 0, h->stream, A, 4, dpl, dpl + np);
         BCHK(h, hipGetLastError());
         BCHK(h, hipMemcpyAsync(ufl, dpl, np * 8, hipMemcpyDeviceToHost, h->stream));
@@ -610,11 +610,11 @@ extern "C" int dnsg_budget2d(dnsg_t *h, double *turb, double *vort, double *ke, 
     bud_finish(h->p, mean.data(), dUdz.data(), acc, turb, vort, ke);
 done:
     if (rc) (void)hipStreamSynchronize(h->stream);
-    if (dv) (void)hipFree(dv);
-    if (dmean) (void)hipFree(dmean);
-    if (dpart) (void)hipFree(dpart);
-    if (dsum) (void)hipFree(dsum);
-    if (dpl) (void)hipFree(dpl);
+    scratch_put(dv);
+    scratch_put(dmean);
+    scratch_put(dpart);
+    scratch_put(dsum);
+    scratch_put(dpl);
     return rc;
 }
 

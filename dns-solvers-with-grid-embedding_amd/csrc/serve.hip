@@ -365,7 +365,7 @@ int dnsg_queue_create(const dnsg_queue_opts *o, dnsg_queue_t **out) {
         q->use_graph = !(e && e[0] == '0');
     }
     QCHK(q, hipStreamCreateWithFlags(&q->stream, hipStreamNonBlocking));
-    QCHK(q, hipMalloc(&q->d_u, 2 * sizeof(double) * DNSG_QUEUE_MAX_ACTIVE));
+    QCHK(q, dev_malloc(&q->d_u, 2 * sizeof(double) * DNSG_QUEUE_MAX_ACTIVE));
     QCHK(q, hipHostMalloc((void **)&q->h_u, 2 * sizeof(double) * DNSG_QUEUE_MAX_ACTIVE, hipHostMallocDefault));
     if (o->hbm_budget) {
         q->budget = o->hbm_budget;

@@ -12,6 +12,8 @@
 // per E_x value and a workgroup per 64 E_y values.
 #include <hipfft/hipfft.h>
 
+#include <new>
+
 #include "internal.hpp"
 #include "lattice.hpp"
 
@@ -106,7 +108,43 @@ __global__ __launch_bounds__(TB) void k_fold_y(const double2 *__restrict__ cf, i
     }
 }
 
+// A plan's preparation takes 8 ms of host time, its transforms of the Re_tau=180 grids
+// under 1 ms, so a handle keeps the plans of its coarse grid and of its bands (equal in
+// size) from their first use; the work area, as large as the data, lives for the call.
+struct FftPlan {
+    hipfftHandle plan;
+    size_t work;
+};
+
+FftPlan *fft_plan(void **slot, int N0, int N1, int batch) {
+    if (*slot) return static_cast<FftPlan *>(*slot);
+    FftPlan *f = new (std::nothrow) FftPlan{};
+    if (!f) return nullptr;
+    if (hipfftCreate(&f->plan) != HIPFFT_SUCCESS) {
+        delete f;
+        return nullptr;
+    }
+    int dims[2] = {N0, N1};
+    if (hipfftSetAutoAllocation(f->plan, 0) != HIPFFT_SUCCESS ||
+        hipfftMakePlanMany(f->plan, 2, dims, nullptr, 1, 0, nullptr, 1, 0, HIPFFT_D2Z, batch, &f->work) != HIPFFT_SUCCESS) {
+        (void)hipfftDestroy(f->plan);
+        delete f;
+        return nullptr;
+    }
+    *slot = f;
+    return f;
+}
+
 }  // namespace
+
+void spectra_release(dnsg_ctx *h) {
+    for (void *&p : h->fft) {
+        if (!p) continue;
+        (void)hipfftDestroy(static_cast<FftPlan *>(p)->plan);
+        delete static_cast<FftPlan *>(p);
+        p = nullptr;
+    }
+}
 
 }  // namespace dnsg
 
@@ -137,12 +175,12 @@ extern "C" int dnsg_spectra(dnsg_t *h, int grid, double *ex, double *ey) {
     if (rc) return rc;
     double *vel = nullptr, *dex = nullptr, *dey = nullptr;
     double2 *cf = nullptr;
-    hipfftHandle plan = 0;
-    bool have_plan = false;
-    SPCHK(h, hipMalloc(&vel, 3 * (size_t)nzg * plane * sizeof(double)));
-    SPCHK(h, hipMalloc(&cf, 3 * (size_t)nzg * N0 * N1h * sizeof(double2)));
-    SPCHK(h, hipMalloc(&dex, 3 * (size_t)N0 * nzg * sizeof(double)));
-    SPCHK(h, hipMalloc(&dey, 3 * (size_t)N1h * nzg * sizeof(double)));
+    void *work = nullptr;
+    FftPlan *plan = nullptr;
+    SPCHK(h, scratch_get(&vel, 3 * (size_t)nzg * plane * sizeof(double)));
+    SPCHK(h, scratch_get(&cf, 3 * (size_t)nzg * N0 * N1h * sizeof(double2)));
+    SPCHK(h, scratch_get(&dex, 3 * (size_t)N0 * nzg * sizeof(double)));
+    SPCHK(h, scratch_get(&dey, 3 * (size_t)N1h * nzg * sizeof(double)));
     {
         const int kwall = grid == 0 ? -1 : (grid == 1 ? 0 : nzg - 1);
         const double *wall = grid == 2 ? h->fwall + plane * Q : h->fwall;
@@ -156,15 +194,20 @@ extern "C" int dnsg_spectra(dnsg_t *h, int grid, double *ex, double *ey) {
         SPCHK(h, hipGetLastError());
     }
     {
-        int dims[2] = {N0, N1};
-        if (hipfftPlanMany(&plan, 2, dims, nullptr, 1, 0, nullptr, 1, 0, HIPFFT_D2Z, 3 * nzg) != HIPFFT_SUCCESS) {
-            h->err = "hipfftPlanMany failed";
+        plan = fft_plan(&h->fft[grid == 0 ? 0 : 1], N0, N1, 3 * nzg);
+        if (!plan) {  // its tables found no memory
+            scratch_trim();
+            plan = fft_plan(&h->fft[grid == 0 ? 0 : 1], N0, N1, 3 * nzg);
+        }
+        if (!plan) {
+            h->err = "hipfftMakePlanMany failed";
             rc = DNSG_ERR_HIP;
             goto done;
         }
-        have_plan = true;
-        if (hipfftSetStream(plan, h->stream) != HIPFFT_SUCCESS ||
-            hipfftExecD2Z(plan, vel, reinterpret_cast<hipfftDoubleComplex *>(cf)) != HIPFFT_SUCCESS) {
+        if (plan->work) SPCHK(h, scratch_get(&work, plan->work));
+        if (hipfftSetStream(plan->plan, h->stream) != HIPFFT_SUCCESS ||
+            (work && hipfftSetWorkArea(plan->plan, work) != HIPFFT_SUCCESS) ||
+            hipfftExecD2Z(plan->plan, vel, reinterpret_cast<hipfftDoubleComplex *>(cf)) != HIPFFT_SUCCESS) {
             h->err = "hipfftExecD2Z failed";
             rc = DNSG_ERR_HIP;
             goto done;
@@ -182,10 +225,10 @@ extern "C" int dnsg_spectra(dnsg_t *h, int grid, double *ex, double *ey) {
     SPCHK(h, hipStreamSynchronize(h->stream));
 done:
     if (rc) (void)hipStreamSynchronize(h->stream);
-    if (have_plan) hipfftDestroy(plan);
-    if (vel) (void)hipFree(vel);
-    if (cf) (void)hipFree(cf);
-    if (dex) (void)hipFree(dex);
-    if (dey) (void)hipFree(dey);
+    scratch_put(work);
+    scratch_put(vel);
+    scratch_put(cf);
+    scratch_put(dex);
+    scratch_put(dey);
     return rc;
 }
