@@ -351,8 +351,11 @@ __global__ __launch_bounds__(TX *TY) void k_iface(Batch<IfaceItem> BT, HermiteW<
     const IfaceItem &B = BT.it[itm];
     const int lbg = bid - BT.first[itm];
     const int G = B.groups, lb = lbg / G, grp = lbg % G;
-    // this workgroup's units [q0, q1); rho and u are formed by every group
-    const int q0 = (IF_UNITS * grp) / G, q1 = (IF_UNITS * (grp + 1)) / G, steps = 2 + q1 - q0;
+    // this workgroup's units [q0, q1), or with G = 19 one direction i0 of one unit; rho and
+    // u are formed by every group
+    const bool single = G == Q;
+    const int q0 = single ? grp / 2 : (IF_UNITS * grp) / G, q1 = single ? q0 + 1 : (IF_UNITS * (grp + 1)) / G;
+    const int i0 = single ? grp & 1 : 0, steps = 2 + q1 - q0;
     const int Xc = B.Xc, Yc = B.Yc;
     const P rescale = (P)B.rescale;
     const int ntx = (Xc + TX - 1) / TX;
@@ -370,21 +373,16 @@ __global__ __launch_bounds__(TX *TY) void k_iface(Batch<IfaceItem> BT, HermiteW<
         const int gx = ((x0 - 2 + p % HX) % Xc + Xc) % Xc, gy = ((y0 - 2 + p / HX) % Yc + Yc) % Yc;
         hoff[k] = hok[k] ? (unsigned)(gy * Xc + gx) * (unsigned)sizeof(P) : 0u;
     }
-    // plane values of a step: 0, 1 / 2, 3 / 4 + direction, the second < 0 for the rest unit
-    auto values_of = [&](int st, int &va, int &vb) {
-        if (st < 2) { va = 2 * st; vb = va + 1; return; }
-        const int u = q0 + st - 2;
-        va = 4 + if_dir(u, 0);
-        vb = u < IF_UNITS - 1 ? 4 + if_dir(u, 1) : -1;
-    };
+    // plane value i of a step: 0, 1 / 2, 3 / 4 + direction; the values [lo, hi) it has
+    auto value_of = [&](int st, int i) { return st < 2 ? 2 * st + i : 4 + if_dir(q0 + st - 2, i); };
+    auto lo = [&](int st) { return st < 2 ? 0 : i0; };
+    auto hi = [&](int st) { return st < 2 || (!single && q0 + st - 2 < IF_UNITS - 1) ? 2 : i0 + 1; };
     P a[2][NH][NL];
     auto fetch = [&](int st) __attribute__((always_inline)) {
-        int v[2];
-        values_of(st, v[0], v[1]);
 #pragma unroll
         for (int i = 0; i < 2; i++) {
-            if (i == 1 && v[1] < 0) continue;
-            const size_t vo = (size_t)v[i] * n;
+            if (i < lo(st) || i >= hi(st)) continue;
+            const size_t vo = (size_t)value_of(st, i) * n;
             const char *L0 = reinterpret_cast<const char *>(static_cast<const P *>(B.ln) + vo);
             const char *L1 = reinterpret_cast<const char *>(static_cast<const P *>(B.lp) + vo);
             const char *L2 = reinterpret_cast<const char *>(static_cast<const P *>(B.lpp) + vo);
@@ -403,7 +401,8 @@ __global__ __launch_bounds__(TX *TY) void k_iface(Batch<IfaceItem> BT, HermiteW<
     auto stage = [&](int st) __attribute__((always_inline)) {
         const int sb = st & 1;
 #pragma unroll
-        for (int i = 0; i < 2; i++)
+        for (int i = 0; i < 2; i++) {
+            if (i < lo(st) || i >= hi(st)) continue;
 #pragma unroll
             for (int k = 0; k < NH; k++) {
                 if (!hok[k]) continue;
@@ -422,11 +421,12 @@ __global__ __launch_bounds__(TX *TY) void k_iface(Batch<IfaceItem> BT, HermiteW<
                 }
                 s0[sb][i][tid + k * NT] = hv;
             }
+        }
         if (st + 1 < steps) fetch(st + 1);
         __syncthreads();
         // d/dx, d/dy (derivative.c:41-42, 63-64)
 #pragma unroll 1
-        for (int p = tid; p < 2 * ND; p += NT) {
+        for (int p = tid + lo(st) * ND; p < hi(st) * ND; p += NT) {
             const int i = p >= ND ? 1 : 0, r = p - i * ND;
             const P *c = &s0[sb][i][r + 2 * HX];
             s2[i][r] = d4(c[-2 * HX], c[-HX], c[HX], c[2 * HX]);
@@ -532,9 +532,9 @@ __global__ __launch_bounds__(TX *TY) void k_iface(Batch<IfaceItem> BT, HermiteW<
             });
         };
         keep();
-        direction(std::integral_constant<int, 0>{});
+        if (lo(st) == 0) direction(std::integral_constant<int, 0>{});
         keep();
-        if (unit < IF_UNITS - 1) direction(std::integral_constant<int, 1>{});
+        if (hi(st) == 2) direction(std::integral_constant<int, 1>{});
     }
 }
 
@@ -544,30 +544,35 @@ __global__ __launch_bounds__(TX *TY) void k_iface(Batch<IfaceItem> BT, HermiteW<
 // to 2 + 10/G.  G fills the workgroup slots the GPU holds at once for this kernel
 // (CUs x resident workgroups per CU, from the occupancy query): a launch whose
 // tiles alone fill them (the Re_tau=180 bands: 1024 tiles) takes G = 1, a launch of
-// small channels (the serving queue) shortens its chains, up to G = 10.
+// small channels (the serving queue) shortens its chains, up to G = 10, or
+// G = 19 with one direction each where every workgroup then has a CU of its own (gratio 3,
+// 4 tiles: 11.4 and 10.0 us a launch against 13.2 and 11.6 with G = 10; gratio 2,
+// 16 tiles, whose 304 workgroups share CUs: 12.5 and 11.4 against 11.8 and 10.2).
 constexpr int IF_TX = 32, IF_TY = 8;
 
 template <class S, class P, int GR, bool LAST>
-static int iface_slots() {
-    static int slots = 0;  // per kernel; concurrent first calls compute the same value
+static int iface_slots(int &cus) {
+    static int slots = 0, ncu = 0;  // per kernel; concurrent first calls compute the same values
     if (slots == 0) {
-        int dev = 0, cus = 0, per_cu = 0;
+        int dev = 0, per_cu = 0;
         if (hipGetDevice(&dev) == hipSuccess &&
-            hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess &&
+            hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess &&
             hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_iface<S, P, GR, LAST, IF_TX, IF_TY>,
                                                          IF_TX * IF_TY, 0) == hipSuccess &&
-            cus > 0 && per_cu > 0)
-            slots = cus * per_cu;
+            ncu > 0 && per_cu > 0)
+            slots = ncu * per_cu;
         else {
             (void)hipGetLastError();  // answered here: not the launch's error
             slots = 1024;
         }
     }
+    cus = ncu;
     return slots;
 }
 
-static int iface_groups(long tiles, int slots) {
+static int iface_groups(long tiles, int slots, int cus) {
     if (tiles >= slots) return 1;
+    if (tiles * Q <= cus) return Q;
     return (int)std::min<long>(IF_UNITS, slots / tiles);
 }
 
@@ -578,7 +583,8 @@ static hipError_t iface_launch(hipStream_t s, IfaceItem *items, int n, HermiteW<
         long tiles = 0;
         for (int i = i0; i < i0 + m; i++)
             tiles += (long)((items[i].Xc + IF_TX - 1) / IF_TX) * ((items[i].Yc + IF_TY - 1) / IF_TY);
-        const int G = iface_groups(tiles, iface_slots<S, P, GR, LAST>());
+        int cus = 0;
+        const int slots = iface_slots<S, P, GR, LAST>(cus), G = iface_groups(tiles, slots, cus);
         for (int i = i0; i < i0 + m; i++) items[i].groups = G;
         Batch<IfaceItem> B;
         B.halt = halt;
