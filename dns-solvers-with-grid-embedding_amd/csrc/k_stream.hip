@@ -1,10 +1,9 @@
 // k_stream.hip -- fused BGK collide + push-stream on the coarse grid and the
 // wall bands, the initial-state kernel and the AoS <-> SoA transposes.
 //
-// One workgroup owns a chunk of CS_THREADS nodes of one (y, z) row: its reads
-// are 19 contiguous vectors of the row block, its writes the same vectors of
-// the 9 neighbouring rows shifted by e_x.  A lattice narrower than CS_THREADS
-// packs CS_THREADS / nx whole rows into each workgroup instead.
+// A workgroup owns CS_THREADS nodes of a row (two chunks of them in the paired form, a run
+// of consecutive nodes of the layer in the flat form): its reads are 19 contiguous vectors
+// of the row block, its writes the same vectors of the 9 neighbouring rows shifted by e_x.
 //
 // Boundary rules at the stored z ends (xfcomputations.c:215-442):
 //   BOUND_DROP  populations leaving the lattice are not written (the bounded
