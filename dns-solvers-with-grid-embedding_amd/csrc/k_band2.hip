@@ -237,8 +237,8 @@ __device__ __forceinline__ void band2_tile(const LatArgs &L, int tile, typename 
             if (core) {
                 constexpr int up = SIDE ? 1 : -1;  // stored-layer step toward the wall
                 const double w0 = dest_w(L, m), w1 = t < nz - 1 ? dest_w(L, m + up) : 0., w2 = t >= 1 ? dest_w(L, m - up) : 0.;
-                sdm += w0 * sx[0] + w1 * sx[1] + w2 * sx[2];
-                sdd += w0 * sd[0] + w1 * sd[1] + w2 * sd[2];
+                sdm += weighted(w0, sx[0]) + weighted(w1, sx[1]) + weighted(w2, sx[2]);
+                sdd += weighted(w0, sd[0]) + weighted(w1, sd[1]) + weighted(w2, sd[2]);
             }
         }
     };

@@ -46,8 +46,8 @@ struct DestSums {
     }
     __device__ __forceinline__ void into(RowSums &rs, const LatArgs &L, int z) const {
         const double wl = dest_w(L, z - 1), wc = dest_w(L, z), wh = dest_w(L, z + 1);
-        rs.dd += wl * dl + wc * dc + wh * dh;
-        rs.dm += wl * xl + wc * xc + wh * xh;
+        rs.dd += weighted(wl, dl) + weighted(wc, dc) + weighted(wh, dh);
+        rs.dm += weighted(wl, xl) + weighted(wc, xc) + weighted(wh, xh);
     }
 };
 

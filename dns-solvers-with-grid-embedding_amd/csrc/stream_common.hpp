@@ -124,5 +124,8 @@ struct RowSums {
 __device__ __forceinline__ double dest_w(const LatArgs &L, int zt) {
     return (zt < L.klo || zt > L.khi) ? 0. : (zt == L.khalf ? 0.5 * L.kscale : L.kscale);
 }
+// a layer's part of those sums; nothing from a layer of weight 0, also where its sum is
+// not finite (0 x NaN would reach the force)
+__device__ __forceinline__ double weighted(double w, double sum) { return w != 0. ? w * sum : 0.; }
 
 }  // namespace dnsg
