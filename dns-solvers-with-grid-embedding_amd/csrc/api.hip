@@ -238,6 +238,7 @@ void rotate_levels(dnsg_t *h) {  // xcomputations.c:548-556
     h->lev_lo[3] = h->lev_lo[2]; h->lev_lo[2] = h->lev_lo[1]; h->lev_lo[1] = h->lev_lo[0]; h->lev_lo[0] = t;
     t = h->lev_up[3];
     h->lev_up[3] = h->lev_up[2]; h->lev_up[2] = h->lev_up[1]; h->lev_up[1] = h->lev_up[0]; h->lev_up[0] = t;
+    if (h->given_levels > 0) h->given_levels--;
 }
 
 }  // namespace dnsg
@@ -469,6 +470,7 @@ struct StepTop {
     int cur[3];
     void *lo[4], *up[4];
     bool flux_fused;
+    int given_levels;
 };
 
 StepTop step_top(const dnsg_t *h) {
@@ -476,6 +478,7 @@ StepTop step_top(const dnsg_t *h) {
     t.cur[0] = h->coarse.cur; t.cur[1] = h->lower.cur; t.cur[2] = h->upper.cur;
     for (int l = 0; l < 4; l++) { t.lo[l] = h->lev_lo[l]; t.up[l] = h->lev_up[l]; }
     t.flux_fused = h->flux_fused;
+    t.given_levels = h->given_levels;
     return t;
 }
 
@@ -491,6 +494,7 @@ StepTop top_after(const dnsg_t *h, StepTop t, long s) {
         void *a = t.lo[3]; t.lo[3] = t.lo[2]; t.lo[2] = t.lo[1]; t.lo[1] = t.lo[0]; t.lo[0] = a;
         a = t.up[3]; t.up[3] = t.up[2]; t.up[2] = t.up[1]; t.up[1] = t.up[0]; t.up[0] = a;
         t.flux_fused = h->p.force_mode == DNSG_FORCE_FLUX;
+        if (t.given_levels > 0) t.given_levels--;
     }
     return t;
 }
@@ -499,6 +503,7 @@ void restore_top(dnsg_t *h, const StepTop &t) {
     h->coarse.cur = t.cur[0]; h->lower.cur = t.cur[1]; h->upper.cur = t.cur[2];
     for (int l = 0; l < 4; l++) { h->lev_lo[l] = t.lo[l]; h->lev_up[l] = t.up[l]; }
     h->flux_fused = t.flux_fused;
+    h->given_levels = t.given_levels;
 }
 
 // clears the halt flag with a kernel rather than a memset node, so a caller that
@@ -619,6 +624,7 @@ int put_levels(dnsg_t *h, const double *const *lv, void *const *dev, HostLayout 
     const int Xc = h->d.Xc, Yc = h->d.Yc;
     const size_t np = (size_t)Xc * Yc * NVP;
     const bool f32 = h->p.precision != DNSG_PREC_FP64;
+    h->given_levels = 3;
     std::vector<double> t(np);
     std::vector<float> tf(f32 ? np : 0);
     for (int l = 0; l < 3; l++) {
@@ -1140,6 +1146,7 @@ static int set_force(dnsg_t *h, double g) {
 int dnsg_init_state(dnsg_t *h) {
     if (!h || !h->stream) return DNSG_ERR_ARG;
     h->flux_fused = false;
+    h->given_levels = 0;
     HIPCHK(h, launch_init_lattice(h->stream, h, 0, h->coarse.c()));
     HIPCHK(h, launch_init_lattice(h->stream, h, 1, h->lower.c()));
     HIPCHK(h, launch_init_lattice(h->stream, h, 2, h->upper.c()));

@@ -160,6 +160,7 @@ struct dnsg_ctx {
     // the step's wall-stress check has passed
     void *lev_lo[4] = {nullptr, nullptr, nullptr, nullptr};
     void *lev_up[4] = {nullptr, nullptr, nullptr, nullptr};
+    int given_levels = 0;  // of the three levels a fill reads, how many the caller uploaded
     // the steps use the two-substep band kernel (gratio 2); band_tiled: the bands'
     // fused-reduction partials of the last launch that wrote them are that kernel's
     bool band2 = false;

@@ -315,7 +315,9 @@ __device__ __forceinline__ void store_pair(__half *p, float a, float b) {
 // results kept so that opposite ones share the even part of feq take more registers
 // and are slower in FP64 (100 / 75).
 // LAST: the substep at t = 1, where the Hermite weights are 0, 0, 1, 0 and the value is
-// the newest plane's: the two older planes are not read.
+// the newest plane's: the two older planes are not read.  0 x NaN is NaN, so planes that
+// the caller uploaded are read all the same (dnsg_ctx::given_levels); the solver's own
+// ones were the newest once, and what was not finite in them is in the state already.
 struct IfaceItem {
     const void *ln, *lp, *lpp;  // newest, previous, oldest plane levels [23][Yc][Xc]
     void *band;                 // band post-stream lattice
@@ -599,21 +601,20 @@ static hipError_t iface_launch(hipStream_t s, IfaceItem *items, int n, HermiteW<
 }
 
 template <class S, class P, int GR>
-static hipError_t iface_gr(hipStream_t s, IfaceItem *items, int n, HermiteW<P> H, const int *halt) {
+static hipError_t iface_gr(hipStream_t s, IfaceItem *items, int n, HermiteW<P> H, bool given, const int *halt) {
     // weights 0, 0, 1, 0: the last substep, and the only one at gratio 1
-    if (H.h00 == (P)0 && H.h10 == (P)0 && H.h01 == (P)1 && H.h11 == (P)0)
+    if (!given && H.h00 == (P)0 && H.h10 == (P)0 && H.h01 == (P)1 && H.h11 == (P)0)
         return iface_launch<S, P, GR, true>(s, items, n, H, halt);
-    if constexpr (GR > 1) return iface_launch<S, P, GR, false>(s, items, n, H, halt);
-    return hipErrorInvalidValue;
+    return iface_launch<S, P, GR, false>(s, items, n, H, halt);
 }
 
 template <class S, class P>
-static hipError_t iface_items(hipStream_t s, int GR, IfaceItem *items, int n, HermiteW<P> H, const int *halt) {
+static hipError_t iface_items(hipStream_t s, int GR, IfaceItem *items, int n, HermiteW<P> H, bool given, const int *halt) {
     switch (GR) {
-    case 1: return iface_gr<S, P, 1>(s, items, n, H, halt);
-    case 2: return iface_gr<S, P, 2>(s, items, n, H, halt);
-    case 3: return iface_gr<S, P, 3>(s, items, n, H, halt);
-    default: return iface_gr<S, P, 4>(s, items, n, H, halt);
+    case 1: return iface_gr<S, P, 1>(s, items, n, H, given, halt);
+    case 2: return iface_gr<S, P, 2>(s, items, n, H, given, halt);
+    case 3: return iface_gr<S, P, 3>(s, items, n, H, given, halt);
+    default: return iface_gr<S, P, 4>(s, items, n, H, given, halt);
     }
 }
 
@@ -647,13 +648,17 @@ hipError_t launch_interface_many(hipStream_t s, dnsg_ctx *const *hs, int n, int 
     IfaceItem one[2];
     std::vector<IfaceItem> many(n > 1 ? 2 * (size_t)n : 0);
     IfaceItem *v = n > 1 ? many.data() : one;
-    for (int i = 0; i < n; i++) iface_pair(hs[i], &v[2 * (size_t)i]);
+    bool given = false;
+    for (int i = 0; i < n; i++) {
+        iface_pair(hs[i], &v[2 * (size_t)i]);
+        given = given || hs[i]->given_levels > 0;
+    }
     // one handle: its own halt flag; a batch of several (the serving queue): none
     const int *halt = n == 1 ? hs[0]->halt() : nullptr;
-    if (prec == DNSG_PREC_FP64) return iface_items<double, double>(s, GR, v, 2 * n, H, halt);
+    if (prec == DNSG_PREC_FP64) return iface_items<double, double>(s, GR, v, 2 * n, H, given, halt);
     HermiteW<float> Hf = {(float)H.h00, (float)H.h10, (float)H.h01, (float)H.h11, H.exact};
-    if (prec == DNSG_PREC_FP32) return iface_items<float, float>(s, GR, v, 2 * n, Hf, halt);
-    return iface_items<__half, float>(s, GR, v, 2 * n, Hf, halt);
+    if (prec == DNSG_PREC_FP32) return iface_items<float, float>(s, GR, v, 2 * n, Hf, given, halt);
+    return iface_items<__half, float>(s, GR, v, 2 * n, Hf, given, halt);
 }
 
 hipError_t launch_interface(hipStream_t s, dnsg_ctx *h, int iter) { return launch_interface_many(s, &h, 1, iter); }
