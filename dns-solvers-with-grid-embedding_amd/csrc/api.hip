@@ -10,11 +10,8 @@
 #include <stdlib.h>
 #include <string.h>
 
-#include <algorithm>
 #include <mutex>
 #include <new>
-#include <system_error>
-#include <thread>
 #include <vector>
 
 #include "internal.hpp"
@@ -670,163 +667,6 @@ int get_levels(dnsg_t *h, double *const *lv, void *const *dev, HostLayout L = {}
     return DNSG_OK;
 }
 
-}  // namespace
-
-namespace {
-
-struct ScratchBlock {
-    void *p;
-    size_t bytes;
-    int dev;
-    bool used;
-};
-struct ScratchPool {
-    std::mutex m;
-    ScratchBlock b[64];
-    int n = 0, users = 0;  // b[0, n): handed out or kept, the longest kept first
-    void drop(int i) {
-        (void)hipFree(b[i].p);
-        std::move(b + i + 1, b + n, b + i);
-        n--;
-    }
-    void trim() {
-        for (int i = n - 1; i >= 0; i--)
-            if (!b[i].used) drop(i);
-    }
-};
-// never destroyed: handles may outlive the static objects of this library
-ScratchPool &pool() {
-    static ScratchPool &p = *new ScratchPool;
-    return p;
-}
-
-}  // namespace
-
-void dnsg::scratch_trim() {
-    std::lock_guard<std::mutex> l(pool().m);
-    pool().trim();
-}
-
-void dnsg::scratch_users(int change) {
-    std::lock_guard<std::mutex> l(pool().m);
-    pool().users += change;
-    if (pool().users == 0) pool().trim();
-}
-
-hipError_t dnsg::scratch_get(void **p, size_t bytes) {
-    int dev = 0;
-    hipError_t e = hipGetDevice(&dev);
-    if (e != hipSuccess) return e;
-    ScratchPool &P = pool();
-    {
-        // the smallest kept block that is large enough and no more than twice the size
-        std::lock_guard<std::mutex> l(P.m);
-        ScratchBlock *best = nullptr;
-        for (int i = 0; i < P.n; i++) {
-            ScratchBlock &c = P.b[i];
-            if (!c.used && c.dev == dev && c.bytes >= bytes && c.bytes / 2 <= bytes && (!best || c.bytes < best->bytes)) best = &c;
-        }
-        if (best) {
-            best->used = true;
-            *p = best->p;
-            return hipSuccess;
-        }
-    }
-    e = dev_malloc(p, bytes);
-    if (e != hipSuccess) return e;
-    std::lock_guard<std::mutex> l(P.m);
-    if (P.n == 64)
-        for (int i = 0; i < P.n; i++)
-            if (!P.b[i].used) {
-                P.drop(i);
-                break;
-            }
-    if (P.n < 64) P.b[P.n++] = {*p, bytes, dev, true};  // else it is freed when given back
-    return hipSuccess;
-}
-
-void dnsg::scratch_put(void *p) {
-    if (!p) return;
-    ScratchPool &P = pool();
-    std::lock_guard<std::mutex> l(P.m);
-    int i = 0;
-    while (i < P.n && P.b[i].p != p) i++;
-    if (i == P.n) {
-        (void)hipFree(p);
-        return;
-    }
-    std::rotate(P.b + i, P.b + i + 1, P.b + P.n);
-    ScratchBlock &mine = P.b[P.n - 1];
-    mine.used = false;
-    const int dev = mine.dev;
-    size_t total = 0, kept = 0;
-    if (hipDeviceTotalMem(&total, dev) != hipSuccess) total = 0;
-    for (int j = 0; j < P.n; j++)
-        if (!P.b[j].used && P.b[j].dev == dev) kept += P.b[j].bytes;
-    for (int j = 0; j < P.n && kept > total / 64;) {  // the longest kept go first
-        if (P.b[j].used || P.b[j].dev != dev) {
-            j++;
-            continue;
-        }
-        kept -= P.b[j].bytes;
-        P.drop(j);
-    }
-}
-
-// A plain copy into pageable memory runs at the rate of one host thread that also takes
-// the page faults of a fresh array (4 to 10 GB/s against 57 of the link).  From two
-// pieces on, the data comes through two pinned buffers instead: while the link fills one,
-// a few threads move the other on (20 to 29 GB/s).  The buffers live for the call, about
-// 0.5 ms, so a single piece (1.6 ms) is left to the plain copy; so is an array that the
-// device can write itself (pinned or device memory).
-hipError_t dnsg::copy_out(hipStream_t s, void *dst, const void *src, size_t bytes) {
-    constexpr size_t PIECE = (size_t)16 << 20;
-    hipPointerAttribute_t at;
-    const bool pageable = hipPointerGetAttributes(&at, dst) != hipSuccess || at.type == hipMemoryTypeUnregistered;
-    if (pageable) (void)hipGetLastError();  // an unknown pointer is an answer, not an error
-    char *buf = nullptr;
-    if (!pageable || bytes < 2 * PIECE || hipHostMalloc((void **)&buf, 2 * PIECE, hipHostMallocDefault) != hipSuccess) {
-        if (pageable) (void)hipGetLastError();
-        const hipError_t e = hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, s);
-        const hipError_t w = hipStreamSynchronize(s);
-        return e != hipSuccess ? e : w;
-    }
-    const int nt = (int)std::min(4u, std::max(1u, std::thread::hardware_concurrency()));
-    const size_t pieces = (bytes + PIECE - 1) / PIECE;
-    auto len = [&](size_t p) { return std::min(PIECE, bytes - p * PIECE); };
-    auto fetch = [&](size_t p) {
-        return hipMemcpyAsync(buf + (p & 1) * PIECE, static_cast<const char *>(src) + p * PIECE, len(p),
-                              hipMemcpyDeviceToHost, s);
-    };
-    hipError_t e = fetch(0);
-    for (size_t p = 0; p < pieces && e == hipSuccess; p++) {
-        e = hipStreamSynchronize(s);
-        if (e == hipSuccess && p + 1 < pieces) e = fetch(p + 1);
-        if (e != hipSuccess) break;
-        const size_t n = len(p);
-        auto share = [&](int t) {
-            const size_t a = n * t / nt, b = n * (t + 1) / nt;
-            memcpy(static_cast<char *>(dst) + p * PIECE + a, buf + (p & 1) * PIECE + a, b - a);
-        };
-        std::thread th[4];
-        for (int t = 1; t < nt; t++) {
-            try {
-                th[t] = std::thread(share, t);
-            } catch (const std::system_error &) {  // no thread to be had
-                share(t);
-            }
-        }
-        share(0);
-        for (int t = 1; t < nt; t++)
-            if (th[t].joinable()) th[t].join();
-    }
-    const hipError_t w = hipStreamSynchronize(s);
-    (void)hipHostFree(buf);
-    return e != hipSuccess ? e : w;
-}
-
-namespace {
-
 // AoS [X(+1)][Y(+1)][zaos][19] host array <-> SoA device lattice (stored layers z0..z0+nz-1)
 int put_lattice(dnsg_t *h, const double *aos, Grid &g, int zaos, int z0, HostLayout L = {}) {
     const int gl = L.gl();
@@ -836,9 +676,8 @@ int put_lattice(dnsg_t *h, const double *aos, Grid &g, int zaos, int z0, HostLay
     hipError_t e = hipMemcpyAsync(stage, aos, n * 8, hipMemcpyHostToDevice, h->stream);
     if (e == hipSuccess)
         e = launch_aos_to_soa(h->stream, stage, g.c(), g.nx, g.ny, zaos, z0, g.nz, h->p.precision, gl);
-    const hipError_t w = hipStreamSynchronize(h->stream);
+    const hipError_t w = scratch_put(h->stream, {stage});
     if (e == hipSuccess) e = w;
-    scratch_put(stage);
     HIPCHK(h, e);
     return DNSG_OK;
 }
@@ -852,8 +691,7 @@ int get_lattice(dnsg_t *h, double *aos, const Grid &g, int zaos, int z0, HostLay
     if (e == hipSuccess)
         e = launch_soa_to_aos(h->stream, g.c(), stage, g.nx, g.ny, zaos, z0, g.nz, h->p.precision, gl);
     if (e == hipSuccess) e = copy_out(h->stream, aos, stage, n * 8);
-    else (void)hipStreamSynchronize(h->stream);
-    scratch_put(stage);
+    (void)scratch_put(h->stream, {stage});
     HIPCHK(h, e);
     return DNSG_OK;
 }
@@ -1250,8 +1088,8 @@ int dnsg_init_uniform(dnsg_t *h, const double *uniform, int xdu, int ydu, int zd
     HIPCHK(h, scratch_get(&du, nu * 8));
     hipError_t e = hipMemcpy(du, uniform, nu * 8, hipMemcpyHostToDevice);
     if (e == hipSuccess) e = launch_uniform(h->stream, h, du, xdu, ydu, zdu);
-    if (e == hipSuccess) e = hipStreamSynchronize(h->stream);
-    scratch_put(du);
+    const hipError_t w = scratch_put(h->stream, {du});
+    if (e == hipSuccess) e = w;
     HIPCHK(h, e);
     // main:986-987 call init() before solid_init(), so the band wall layers start at
     // rest like every other node (init.c:17-52) and the interpolation leaves them so
@@ -1589,8 +1427,7 @@ int dnsg_velocity_snapshot(dnsg_t *h, int grid, double *vel, double *den) {
     hipError_t e = launch_snapshot(h, grid, dv, dv + 3 * nn);
     if (e == hipSuccess && vel) e = copy_out(h->stream, vel, dv, nn * 3 * 8);
     if (e == hipSuccess && den) e = copy_out(h->stream, den, dv + 3 * nn, nn * 8);
-    (void)hipStreamSynchronize(h->stream);
-    scratch_put(dv);
+    (void)scratch_put(h->stream, {dv});
     HIPCHK(h, e);
     return DNSG_OK;
 }

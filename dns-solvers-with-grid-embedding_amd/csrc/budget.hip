@@ -609,12 +609,7 @@ extern "C" int dnsg_budget2d(dnsg_t *h, double *turb, double *vort, double *ke, 
     bud_dudz(mean.data(), zdf, zdc, GR, dUdz.data());
     bud_finish(h->p, mean.data(), dUdz.data(), acc, turb, vort, ke);
 done:
-    if (rc) (void)hipStreamSynchronize(h->stream);
-    scratch_put(dv);
-    scratch_put(dmean);
-    scratch_put(dpart);
-    scratch_put(dsum);
-    scratch_put(dpl);
+    (void)scratch_put(h->stream, {dv, dmean, dpart, dsum, dpl});
     return rc;
 }
 

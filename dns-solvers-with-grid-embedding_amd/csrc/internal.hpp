@@ -22,6 +22,7 @@
 #include <vector>
 
 #include "../../include/dnsg.h"
+#include "scratch.hpp"
 
 namespace dnsg {
 
@@ -285,34 +286,6 @@ hipError_t launch_snapshot(dnsg_ctx *h, int g, double *vel, double *den);
 // device copies of the band wall layers (fwall), allocated and filled from the
 // host copies on first use; every call that sets the state refreshes them
 int ensure_fwall(dnsg_t *h);
-// Working memory of the calls that write results out (budget, spectra, snapshots,
-// checkpoints).  The driver clears a freed block before it hands it out again, so an
-// allocation of the size just freed waits for that: 1 GB a call costs up to 30 ms where
-// the kernels take 3.  Blocks given back are therefore kept for the next such call of
-// any handle: at most 1/64 of the device's memory and 64 blocks, all freed with the last
-// handle, and freed and tried again where an allocation finds no memory (dev_malloc).
-// Safe with any number of threads; a block is given back only after its stream has
-// finished with it.
-hipError_t scratch_get(void **p, size_t bytes);
-void scratch_put(void *p);
-void scratch_trim();
-void scratch_users(int change);  // handles alive
-template <class T>
-inline hipError_t scratch_get(T **p, size_t bytes) {
-    return scratch_get(reinterpret_cast<void **>(p), bytes);
-}
-template <class T>
-inline hipError_t dev_malloc(T **p, size_t bytes) {
-    hipError_t e = hipMalloc(reinterpret_cast<void **>(p), bytes);
-    if (e == hipErrorOutOfMemory) {
-        (void)hipGetLastError();
-        scratch_trim();
-        e = hipMalloc(reinterpret_cast<void **>(p), bytes);
-    }
-    return e;
-}
-// device memory to the caller's array, in stream order; complete on return
-hipError_t copy_out(hipStream_t s, void *dst, const void *src, size_t bytes);
 void spectra_release(dnsg_ctx *h);  // the spectra plans of a handle
 // doubles of the filtered injection's f_neq scratch and of the wall-layer copies
 size_t fltr_fneq_doubles(const dnsg_ctx *h);

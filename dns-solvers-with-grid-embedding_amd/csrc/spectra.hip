@@ -224,11 +224,6 @@ extern "C" int dnsg_spectra(dnsg_t *h, int grid, double *ex, double *ey) {
     SPCHK(h, hipMemcpyAsync(ey, dey, 3 * (size_t)N1h * nzg * sizeof(double), hipMemcpyDeviceToHost, h->stream));
     SPCHK(h, hipStreamSynchronize(h->stream));
 done:
-    if (rc) (void)hipStreamSynchronize(h->stream);
-    scratch_put(work);
-    scratch_put(vel);
-    scratch_put(cf);
-    scratch_put(dex);
-    scratch_put(dey);
+    (void)scratch_put(h->stream, {work, vel, cf, dex, dey});
     return rc;
 }
