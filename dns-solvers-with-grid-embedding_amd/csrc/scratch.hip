@@ -3,6 +3,7 @@
 #include "scratch.hpp"
 
 #include <algorithm>
+#include <condition_variable>
 #include <cstring>
 #include <mutex>
 #include <system_error>
@@ -18,18 +19,29 @@ struct ScratchBlock {
     int dev;
     bool used;
 };
+constexpr int BLOCKS = 64;
+// blocks taken out of the pool under its lock, freed after it is released (declared before
+// the lock): hipFree waits for the device, and other handles must not wait with it
+struct Victims {
+    void *p[BLOCKS];
+    int n = 0;
+    ~Victims();
+};
 struct ScratchPool {
     std::mutex m;
-    ScratchBlock b[64];
+    std::condition_variable freed;
+    ScratchBlock b[BLOCKS];
     int n = 0, users = 0;  // b[0, n): handed out or kept, the longest kept first
-    void drop(int i) {
-        (void)hipFree(b[i].p);
+    int leaving = 0;       // victims not freed yet
+    void drop(int i, Victims &v) {
+        v.p[v.n++] = b[i].p;
+        leaving++;
         std::move(b + i + 1, b + n, b + i);
         n--;
     }
-    void trim() {
+    void trim(Victims &v) {
         for (int i = n - 1; i >= 0; i--)
-            if (!b[i].used) drop(i);
+            if (!b[i].used) drop(i, v);
     }
 };
 // never destroyed: handles may outlive the static objects of this library
@@ -37,18 +49,33 @@ ScratchPool &pool() {
     static ScratchPool &p = *new ScratchPool;
     return p;
 }
+Victims::~Victims() {
+    if (n == 0) return;
+    for (int i = 0; i < n; i++) (void)hipFree(p[i]);
+    std::lock_guard<std::mutex> l(pool().m);
+    pool().leaving -= n;
+    pool().freed.notify_all();
+}
 
 }  // namespace
 
+// what other threads are freeing is waited for: their blocks are as good as kept ones to a
+// caller that found no memory
 void dnsg::scratch_trim() {
-    std::lock_guard<std::mutex> l(pool().m);
-    pool().trim();
+    {
+        Victims v;
+        std::lock_guard<std::mutex> l(pool().m);
+        pool().trim(v);
+    }
+    std::unique_lock<std::mutex> l(pool().m);
+    pool().freed.wait(l, [] { return pool().leaving == 0; });
 }
 
 void dnsg::scratch_users(int change) {
+    Victims v;
     std::lock_guard<std::mutex> l(pool().m);
     pool().users += change;
-    if (pool().users == 0) pool().trim();
+    if (pool().users == 0) pool().trim(v);
 }
 
 hipError_t dnsg::scratch_get(void **p, size_t bytes) {
@@ -72,14 +99,15 @@ hipError_t dnsg::scratch_get(void **p, size_t bytes) {
     }
     e = dev_malloc(p, bytes);
     if (e != hipSuccess) return e;
+    Victims v;
     std::lock_guard<std::mutex> l(P.m);
-    if (P.n == 64)
+    if (P.n == BLOCKS)
         for (int i = 0; i < P.n; i++)
             if (!P.b[i].used) {
-                P.drop(i);
+                P.drop(i, v);
                 break;
             }
-    if (P.n < 64) P.b[P.n++] = {*p, bytes, dev, true};  // else it is freed when given back
+    if (P.n < BLOCKS) P.b[P.n++] = {*p, bytes, dev, true};  // else it is freed when given back
     return hipSuccess;
 }
 
@@ -87,11 +115,13 @@ namespace {
 
 void put_back(void *p) {
     ScratchPool &P = pool();
+    Victims v;
     std::lock_guard<std::mutex> l(P.m);
     int i = 0;
     while (i < P.n && P.b[i].p != p) i++;
     if (i == P.n) {
-        (void)hipFree(p);
+        v.p[v.n++] = p;
+        P.leaving++;
         return;
     }
     std::rotate(P.b + i, P.b + i + 1, P.b + P.n);
@@ -100,6 +130,10 @@ void put_back(void *p) {
     const int dev = mine.dev;
     size_t total = 0, kept = 0;
     if (hipDeviceTotalMem(&total, dev) != hipSuccess) total = 0;
+    if (mine.bytes > total / 64) {  // never kept: the others stay
+        P.drop(P.n - 1, v);
+        return;
+    }
     for (int j = 0; j < P.n; j++)
         if (!P.b[j].used && P.b[j].dev == dev) kept += P.b[j].bytes;
     for (int j = 0; j < P.n && kept > total / 64;) {  // the longest kept go first
@@ -108,7 +142,7 @@ void put_back(void *p) {
             continue;
         }
         kept -= P.b[j].bytes;
-        P.drop(j);
+        P.drop(j, v);
     }
 }
 

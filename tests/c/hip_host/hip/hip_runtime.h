@@ -27,7 +27,7 @@ struct FakeDevice {
     std::recursive_mutex m;
     size_t total = (size_t)1 << 30, in_use = 0;
     std::map<void *, size_t> blocks;
-    void (*on_free)(void *) = nullptr;  // called by hipFree
+    void (*on_free)() = nullptr;  // called by hipFree
     void (*on_sync)() = nullptr;        // called by hipStreamSynchronize
     size_t copies = 0, host_buffers = 0;
 };
@@ -48,7 +48,7 @@ inline hipError_t hipMalloc(void **p, size_t bytes) {
     return hipSuccess;
 }
 inline hipError_t hipFree(void *p) {
-    if (fake().on_free) fake().on_free(p);
+    if (fake().on_free) fake().on_free();
     std::lock_guard<std::recursive_mutex> l(fake().m);
     const auto it = fake().blocks.find(p);
     if (it == fake().blocks.end()) return hipErrorInvalidValue;
