@@ -6,7 +6,7 @@
 #include <condition_variable>
 #include <cstring>
 #include <mutex>
-#include <system_error>
+#include <new>
 #include <thread>
 
 using namespace dnsg;
@@ -46,7 +46,8 @@ struct ScratchPool {
 };
 // never destroyed: handles may outlive the static objects of this library
 ScratchPool &pool() {
-    static ScratchPool &p = *new ScratchPool;
+    alignas(ScratchPool) static unsigned char room[sizeof(ScratchPool)];
+    static ScratchPool &p = *new (room) ScratchPool;
     return p;
 }
 Victims::~Victims() {
@@ -194,7 +195,7 @@ hipError_t dnsg::copy_out(hipStream_t s, void *dst, const void *src, size_t byte
         for (int t = 1; t < nt; t++) {
             try {
                 th[t] = std::thread(share, t);
-            } catch (const std::system_error &) {  // no thread to be had
+            } catch (...) {  // no thread, or no memory for one, to be had
                 share(t);
             }
         }

@@ -6,7 +6,9 @@
 #include <cstdio>
 #include <functional>
 #include <future>
+#include <new>
 #include <string>
+#include <vector>
 
 #define CHECK(x)                                                     \
     do {                                                             \
@@ -15,6 +17,16 @@
             exit(1);                                                 \
         }                                                            \
     } while (0)
+
+// no host memory for a new thread, from the first wait for a piece on
+static std::atomic<bool> no_memory{false};
+void *operator new(size_t n) {
+    void *p = no_memory ? nullptr : malloc(n ? n : 1);
+    if (!p) throw std::bad_alloc();
+    return p;
+}
+void operator delete(void *p) noexcept { free(p); }
+void operator delete(void *p, size_t) noexcept { free(p); }
 
 static void *get(size_t bytes) {
     void *p = nullptr;
@@ -105,6 +117,17 @@ static void allocation_waits_for_frees() {
     t.join();
 }
 
+// the calling thread moves what no other thread can be had for
+static void copy_without_threads() {
+    const size_t n = (size_t)37 << 20;
+    std::vector<unsigned char> src(n), dst(n);
+    for (size_t i = 0; i < n; i++) src[i] = (unsigned char)(i * 2654435761u >> 16);
+    fake().on_sync = [] { no_memory = true; };
+    const hipError_t e = copy_out(&idle, dst.data(), src.data(), n);
+    no_memory = false;
+    CHECK(e == hipSuccess && fake().host_buffers == 1 && dst == src);
+}
+
 int main(int argc, char **argv) {
     const std::map<std::string, std::function<void()>> tests = {
         {"waits_for_the_stream", waits_for_the_stream},
@@ -112,9 +135,12 @@ int main(int argc, char **argv) {
         {"oldest_go_first", oldest_go_first},
         {"frees_hold_no_lock", frees_hold_no_lock},
         {"allocation_waits_for_frees", allocation_waits_for_frees},
+        {"copy_without_threads", copy_without_threads},
     };
     CHECK(argc == 2 && tests.count(argv[1]));
+    no_memory = true;  // the first handle asks for none
     scratch_users(1);
+    no_memory = false;
     tests.at(argv[1])();
     return 0;
 }
