@@ -79,6 +79,20 @@ void dnsg::scratch_users(int change) {
     if (pool().users == 0) pool().trim(v);
 }
 
+hipError_t dnsg::scratch_available(size_t *bytes) {
+    int dev = 0;
+    size_t total = 0;
+    ScratchPool &P = pool();
+    std::unique_lock<std::mutex> l(P.m);  // held over the query: no block changes sides meanwhile
+    P.freed.wait(l, [&] { return P.leaving == 0; });
+    hipError_t e = hipGetDevice(&dev);
+    if (e == hipSuccess) e = hipMemGetInfo(bytes, &total);
+    if (e != hipSuccess) return e;
+    for (int i = 0; i < P.n; i++)
+        if (!P.b[i].used && P.b[i].dev == dev) *bytes += P.b[i].bytes;
+    return hipSuccess;
+}
+
 hipError_t dnsg::scratch_get(void **p, size_t bytes) {
     int dev = 0;
     hipError_t e = hipGetDevice(&dev);

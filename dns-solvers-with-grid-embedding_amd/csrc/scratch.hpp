@@ -21,6 +21,9 @@ hipError_t scratch_get(void **p, size_t bytes);
 hipError_t scratch_put(hipStream_t s, std::initializer_list<void *> ps);
 void scratch_trim();
 void scratch_users(int change);  // handles alive
+// free memory of the current device, kept blocks included: dev_malloc finds them where
+// nothing else is left, so whether and when they are freed does not change it
+hipError_t scratch_available(size_t *bytes);
 template <class T>
 inline hipError_t scratch_get(T **p, size_t bytes) {
     return scratch_get(reinterpret_cast<void **>(p), bytes);

@@ -143,11 +143,11 @@ int admit(dnsg_queue *q) {
         // the device bytes the solve actually takes (the runtime rounds and pools
         // allocations), measured around its creation; accounted as the larger of that
         // and the estimate the admission used
-        size_t fr0 = 0, fr1 = 0, tot = 0;
-        const bool measured = hipMemGetInfo(&fr0, &tot) == hipSuccess;
+        size_t fr0 = 0, fr1 = 0;
+        const bool measured = scratch_available(&fr0) == hipSuccess;
         int rc = create_ctx(&s->p, q->stream, &s->h);
         if (!rc) rc = dnsg_init_state(s->h);
-        if (!rc && measured && hipMemGetInfo(&fr1, &tot) == hipSuccess && fr0 > fr1)
+        if (!rc && measured && scratch_available(&fr1) == hipSuccess && fr0 > fr1)
             s->bytes = std::max(s->bytes, fr0 - fr1);
         if (rc) {
             q->err = std::string("admitting solve: ") + (s->h ? dnsg_last_error(s->h) : "");
@@ -370,8 +370,8 @@ int dnsg_queue_create(const dnsg_queue_opts *o, dnsg_queue_t **out) {
     if (o->hbm_budget) {
         q->budget = o->hbm_budget;
     } else {
-        size_t fr = 0, tot = 0;
-        QCHK(q, hipMemGetInfo(&fr, &tot));
+        size_t fr = 0;
+        QCHK(q, scratch_available(&fr));
         const size_t reserve = (size_t)4 << 30;
         q->budget = fr > reserve ? fr - reserve : 0;
     }

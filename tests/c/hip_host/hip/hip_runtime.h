@@ -39,6 +39,10 @@ inline FakeDevice &fake() {
 inline hipError_t hipGetDevice(int *d) { return *d = 0, hipSuccess; }
 inline hipError_t hipGetLastError() { return hipSuccess; }
 inline hipError_t hipDeviceTotalMem(size_t *b, int) { return *b = fake().total, hipSuccess; }
+inline hipError_t hipMemGetInfo(size_t *free, size_t *total) {
+    std::lock_guard<std::recursive_mutex> l(fake().m);
+    return *total = fake().total, *free = fake().total - fake().in_use, hipSuccess;
+}
 inline hipError_t hipMalloc(void **p, size_t bytes) {
     std::lock_guard<std::recursive_mutex> l(fake().m);
     if (fake().in_use + bytes > fake().total) return hipErrorOutOfMemory;

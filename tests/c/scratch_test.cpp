@@ -128,6 +128,27 @@ static void copy_without_threads() {
     CHECK(e == hipSuccess && fake().host_buffers == 1 && dst == src);
 }
 
+// memory counts as available whether it is kept or free
+static size_t available() {
+    size_t n = 0;
+    CHECK(scratch_available(&n) == hipSuccess);
+    return n;
+}
+static void kept_memory_is_available() {
+    const size_t all = fake().total;
+    void *a = get(10 * MB);
+    CHECK(available() == all - 10 * MB);
+    put(a);
+    CHECK(fake().in_use == 10 * MB && available() == all);
+    CHECK(get(8 * MB) == a && available() == all - 10 * MB);
+    put(a);
+    // what an allocation takes, also where it empties the pool
+    void *p = nullptr;
+    CHECK(dev_malloc(&p, all - 4 * MB) == hipSuccess);
+    CHECK(available() == 4 * MB);
+    CHECK(hipFree(p) == hipSuccess && available() == all);
+}
+
 int main(int argc, char **argv) {
     const std::map<std::string, std::function<void()>> tests = {
         {"waits_for_the_stream", waits_for_the_stream},
@@ -136,6 +157,7 @@ int main(int argc, char **argv) {
         {"frees_hold_no_lock", frees_hold_no_lock},
         {"allocation_waits_for_frees", allocation_waits_for_frees},
         {"copy_without_threads", copy_without_threads},
+        {"kept_memory_is_available", kept_memory_is_available},
     };
     CHECK(argc == 2 && tests.count(argv[1]));
     no_memory = true;  // the first handle asks for none
