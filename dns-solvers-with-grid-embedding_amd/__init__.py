@@ -107,6 +107,7 @@ SIGNATURES = {
     "dnsg_run_timed_sections": [_P, ctypes.c_int, ctypes.POINTER(Diag), _DP, _DP, ctypes.c_int],
     "dnsg_kernel_times": [_P, ctypes.c_int, _DP],
     "dnsg_band_launch_substeps": [_P, ctypes.POINTER(ctypes.c_int)],
+    "dnsg_release_memory": [],
     "dnsg_hbm_probe": [ctypes.c_size_t, ctypes.c_int, ctypes.c_int, _DP],
     "dnsg_encalc2": [_P, ctypes.c_long, ctypes.POINTER(Diag)],
     "dnsg_wshearstr": [_P, ctypes.c_long, ctypes.POINTER(Diag)],
@@ -467,6 +468,14 @@ class Queue:
 
 def solve_bytes(params):
     return load().dnsg_solve_bytes(ctypes.byref(params))
+
+
+def release_memory():
+    """give back the device memory kept between output calls (for another allocator in
+    the process); the next such call allocates again"""
+    rc = load().dnsg_release_memory()
+    if rc:
+        raise DnsgError(rc, "release_memory")
 
 
 def hbm_probe(nbytes=2 << 30, kind=0, reps=5):

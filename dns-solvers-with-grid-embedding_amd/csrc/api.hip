@@ -846,6 +846,11 @@ int dnsg_destroy(dnsg_t *h) {
     return DNSG_OK;
 }
 
+int dnsg_release_memory(void) {
+    dnsg::scratch_trim();
+    return DNSG_OK;
+}
+
 int dnsg_create(const dnsg_params *p, dnsg_t **out) { return dnsg::create_ctx(p, nullptr, out); }
 
 }  // extern "C"

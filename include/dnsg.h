@@ -277,6 +277,13 @@ int dnsg_kernel_times(dnsg_t *h, int n, double *ms);
  * default FP32 / FP16 rows of a multiple of 512 nodes take two nodes per thread). */
 int dnsg_band_launch_substeps(const dnsg_t *h, int *substeps);
 
+/* Gives back the device memory that the calls writing results out (budget, spectra,
+ * snapshots, checkpoints) keep for the next such call of any handle (at most 1/64 of the
+ * device's memory; no counterpart in the reference, which allocates per call).  For a
+ * program with another allocator on the same device; safe at any time, with any number of
+ * threads: what a call in progress uses stays. */
+int dnsg_release_memory(void);
+
 /* Instrumentation (no counterpart in the reference): achievable HBM bandwidth of
  * a plain kernel over a buffer of `bytes` -- kind 0 copy (read + write),
  * 1 read-only, 2 write-only, 3 the collide-stream's data movement without its
