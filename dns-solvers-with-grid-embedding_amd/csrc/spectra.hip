@@ -171,7 +171,7 @@ extern "C" int dnsg_spectra(dnsg_t *h, int grid, double *ex, double *ey) {
     const int nzg = grid == 0 ? h->d.zdc : h->d.zdf;  // planes in the velocity file
     const int k0 = grid == 1 ? 1 : 0;                 // lower band: the wall is plane 0
     const size_t plane = (size_t)N0 * N1;
-    int rc = ensure_fwall(h);
+    int rc = grid == 0 ? DNSG_OK : ensure_fwall(h);  // the coarse grid has no wall layer
     if (rc) return rc;
     double *vel = nullptr, *dex = nullptr, *dey = nullptr;
     double2 *cf = nullptr;
@@ -183,7 +183,7 @@ extern "C" int dnsg_spectra(dnsg_t *h, int grid, double *ex, double *ey) {
     SPCHK(h, scratch_get(&dey, 3 * (size_t)N1h * nzg * sizeof(double)));
     {
         const int kwall = grid == 0 ? -1 : (grid == 1 ? 0 : nzg - 1);
-        const double *wall = grid == 2 ? h->fwall + plane * Q : h->fwall;
+        const double *wall = grid == 2 ? h->fwall + plane * Q : h->fwall;  // not read where kwall < 0
         const dim3 grd((unsigned)(((N0 + TS - 1) / TS) * ((N1 + TS - 1) / TS) * nzg)), blk(TB);
         if (h->p.precision == DNSG_PREC_FP64)
             hipLaunchKernelGGL(k_vel_planes<double>, grd, blk, 0, h->stream, (const double *)g.c(), wall, N0, N1, k0, kwall, nzg, vel);

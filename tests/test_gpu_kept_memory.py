@@ -34,3 +34,21 @@ def test_release():
     for u, v in zip(a, s.budget2d()[:3]):
         assert np.array_equal(u, v)
     s.close()
+
+
+def test_coarse_spectra_keep_no_wall_layers():
+    """the coarse grid has no wall layer: its spectra leave the handle without the device
+    copies of the bands' (2 x 512 x 256 x 19 doubles), which a band's spectra read"""
+    wall = 2 * 512 * 256 * 19 * 8
+    first = channel(256, 128, 12)  # what the first use of a plan's kernels keeps
+    first.spectra(0), first.spectra(1)
+    s = channel(256, 128, 12)
+    dnsg.release_memory()
+    before = free()
+    s.spectra(0)
+    dnsg.release_memory()
+    assert before - free() < wall // 2
+    s.spectra(1)
+    dnsg.release_memory()
+    assert before - free() >= wall
+    s.close(), first.close()
