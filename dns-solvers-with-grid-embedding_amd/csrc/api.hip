@@ -195,7 +195,7 @@ LatArgs coarse_args(dnsg_t *h) {
     L.red = nullptr;
     L.force = h->d_force;
     L.dsum = nullptr;
-    L.form = cs_form(L.nx, L.ny, (int)h->elem, h->cs_pair);
+    L.form = coarse_form(h);
     set_dest_weights(h, 0, &L);
     return L;
 }
@@ -220,7 +220,7 @@ void band_args(dnsg_t *h, LatArgs *L) {
         L[b].red = nullptr;
         L[b].force = h->d_force;
         L[b].dsum = nullptr;
-        L[b].form = cs_form(g.nx, g.ny, (int)h->elem, h->cs_pair);
+        L[b].form = band_form(h);
         set_dest_weights(h, 1 + b, &L[b]);
     }
 }
@@ -879,9 +879,12 @@ int dnsg::create_ctx(const dnsg_params *p, hipStream_t ext, dnsg_t **out) {
     h->elem = p->precision == DNSG_PREC_FP64 ? 8 : (p->precision == DNSG_PREC_FP32 ? 4 : 2);
     {
         // FP32 / FP16 rows of a multiple of 2 CS_THREADS nodes: the paired collide-stream
-        // form (k_stream.hip), unless DNSG_CS_PAIRED=0 (the scatter form; same state)
-        const char *cp = getenv("DNSG_CS_PAIRED");
+        // form (k_stream.hip), unless DNSG_CS_PAIRED=0 (the flat form; same state).
+        // DNSG_CS_WIDE=1, 2, 3: the form of layers of 2 GiB and more on the coarse grid, the
+        // bands, both, so that it can be run at any size (same state)
+        const char *cp = getenv("DNSG_CS_PAIRED"), *cw = getenv("DNSG_CS_WIDE");
         h->cs_pair = !(cp && cp[0] == '0');
+        h->cs_wide = cw && cw[0] >= '0' && cw[0] <= '3' ? cw[0] - '0' : 0;
         // gratio 2: both band substeps in one pass (k_band2.hip), by default in FP64 and FP32
         // where the lattice is large enough (band2_pays); FP16 storage keeps one launch per
         // substep (Re_tau=180 step 0.92 against 0.94 ms).  DNSG_BAND2=1 / DNSG_BAND2=0 in the
@@ -889,7 +892,7 @@ int dnsg::create_ctx(const dnsg_params *p, hipStream_t ext, dnsg_t **out) {
         // reductions' partials differ)
         const char *e = getenv("DNSG_BAND2");
         const int elem = (int)h->elem;
-        h->band2 = h->d.GR == 2 && buf_fits(h->d.Xf, h->d.Yf, elem) &&
+        h->band2 = h->d.GR == 2 && buf_fits(h->d.Xf, h->d.Yf, elem) && !(h->cs_wide & 2) &&
                    ((e && e[0]) ? e[0] == '1' : elem != 2 && band2_pays(h->d.Xf, h->d.Yf, h->d.zdf - 1, elem));
     }
     const dnsg_dims &d = h->d;

@@ -167,6 +167,7 @@ struct dnsg_ctx {
     bool band2 = false;
     bool band_tiled = false;
     bool cs_pair = true;  // FP32 / FP16: CS_PAIRED where the rows allow it
+    int cs_wide = 0;      // CS_WIDE also where the layers are small: bit 0 the coarse grid, bit 1 the bands
     int8_t *wall_lo = nullptr, *wall_up = nullptr;     // [Yf][Xf]
 
     // reductions
@@ -220,15 +221,20 @@ struct dnsg_ctx {
 
 namespace dnsg {
 
+// the collide-stream form of a handle's coarse grid and of its bands
+inline int coarse_form(const dnsg_ctx *h) {
+    return (h->cs_wide & 1) ? CS_WIDE : cs_form(h->coarse.nx, h->coarse.ny, (int)h->elem, h->cs_pair);
+}
+inline int band_form(const dnsg_ctx *h) {
+    return (h->cs_wide & 2) ? CS_WIDE : cs_form(h->lower.nx, h->lower.ny, (int)h->elem, h->cs_pair);
+}
 // fused-reduction partials of a coarse layer, and of a band: of a layer, or of the whole
 // band where band_tiled
-inline int coarse_parts(const dnsg_ctx *h) {
-    return cs_parts(cs_form(h->coarse.nx, h->coarse.ny, (int)h->elem, h->cs_pair), h->coarse.nx, h->coarse.ny);
-}
+inline int coarse_parts(const dnsg_ctx *h) { return cs_parts(coarse_form(h), h->coarse.nx, h->coarse.ny); }
 inline int band_parts(const dnsg_ctx *h) {
     const Grid &g = h->lower;
     if (h->band_tiled) return g.ny * ((g.nx + b2_cols((int)h->elem) - 1) / b2_cols((int)h->elem));
-    return cs_parts(cs_form(g.nx, g.ny, (int)h->elem, h->cs_pair), g.nx, g.ny);
+    return cs_parts(band_form(h), g.nx, g.ny);
 }
 // the partials of RED_W values the buffers are sized for: any layout of the coarse grid,
 // and of one band

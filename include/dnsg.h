@@ -274,7 +274,9 @@ int dnsg_kernel_times(dnsg_t *h, int n, double *ms);
  * to the order of the reductions' sums under the flux controller): DNSG_BAND2=1 / 0
  * forces the one-pass band kernel on / off at gratio 2 (layers of 2 GiB or more never
  * take it); DNSG_CS_PAIRED=0 keeps every collide-stream launch in its one-node form (by
- * default FP32 / FP16 rows of a multiple of 512 nodes take two nodes per thread). */
+ * default FP32 / FP16 rows of a multiple of 512 nodes take two nodes per thread);
+ * DNSG_CS_WIDE=1 / 2 / 3 takes the coarse grid / the bands / both through the form that
+ * layers of 2 GiB or more always take (the bands then one launch per substep). */
 int dnsg_band_launch_substeps(const dnsg_t *h, int *substeps);
 
 /* Gives back the device memory that the calls writing results out (budget, spectra,
