@@ -149,6 +149,25 @@ static void kept_memory_is_available() {
     CHECK(hipFree(p) == hipSuccess && available() == all);
 }
 
+// which way a copy goes, and that it is whole: one plain copy below two pieces of 16 MiB;
+// from there on through one pinned buffer, a copy a piece, the last of any length
+static void copies_of_every_length() {
+    const size_t piece = 16 * MB;
+    const struct {
+        size_t bytes, pieces;  // pieces 0: the plain copy
+    } cases[] = {{1, 0}, {piece, 0}, {2 * piece - 1, 0}, {2 * piece, 2}, {2 * piece + 1, 3}, {2 * piece + 3, 3},
+                 {3 * piece - 1, 3}, {3 * piece, 3}, {3 * piece + 7, 4}};
+    for (const auto &c : cases) {
+        std::vector<unsigned char> src(c.bytes), dst(c.bytes + 64, 0xa5);
+        for (size_t i = 0; i < c.bytes; i++) src[i] = (unsigned char)(i * 2654435761u >> 16);
+        fake().copies = fake().host_buffers = 0;
+        CHECK(copy_out(&idle, dst.data(), src.data(), c.bytes) == hipSuccess);
+        CHECK(fake().host_buffers == (c.pieces ? 1 : 0) && fake().copies == (c.pieces ? c.pieces : 1));
+        CHECK(memcmp(dst.data(), src.data(), c.bytes) == 0);
+        for (size_t i = 0; i < 64; i++) CHECK(dst[c.bytes + i] == 0xa5);
+    }
+}
+
 int main(int argc, char **argv) {
     const std::map<std::string, std::function<void()>> tests = {
         {"waits_for_the_stream", waits_for_the_stream},
@@ -157,6 +176,7 @@ int main(int argc, char **argv) {
         {"frees_hold_no_lock", frees_hold_no_lock},
         {"allocation_waits_for_frees", allocation_waits_for_frees},
         {"copy_without_threads", copy_without_threads},
+        {"copies_of_every_length", copies_of_every_length},
         {"kept_memory_is_available", kept_memory_is_available},
     };
     CHECK(argc == 2 && tests.count(argv[1]));

@@ -19,7 +19,7 @@ def program(tmp_path_factory):
 
 @pytest.mark.parametrize("name", ["waits_for_the_stream", "large_block_leaves_the_others", "oldest_go_first",
                                   "frees_hold_no_lock", "allocation_waits_for_frees", "copy_without_threads",
-                                  "kept_memory_is_available"])
+                                  "kept_memory_is_available", "copies_of_every_length"])
 def test_scratch(program, name):
     r = subprocess.run([program, name], capture_output=True, text=True, timeout=60)
     assert r.returncode == 0, r.stdout + r.stderr
