@@ -552,24 +552,24 @@ __global__ __launch_bounds__(TX *TY) void k_iface(Batch<IfaceItem> BT, HermiteW<
 // 16 tiles, whose 304 workgroups share CUs: 12.5 and 11.4 against 11.8 and 10.2).
 constexpr int IF_TX = 32, IF_TY = 8;
 
+// workgroups of the kernel that the GPU holds at once, and its CUs
+struct IfaceSlots {
+    int slots, cus;
+};
 template <class S, class P, int GR, bool LAST>
-static int iface_slots(int &cus) {
-    static int slots = 0, ncu = 0;  // per kernel; concurrent first calls compute the same values
-    if (slots == 0) {
-        int dev = 0, per_cu = 0;
+static const IfaceSlots &iface_slots() {
+    static const IfaceSlots n = [] {  // once per kernel, both values together for every thread
+        int dev = 0, cus = 0, per_cu = 0;
         if (hipGetDevice(&dev) == hipSuccess &&
-            hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess &&
+            hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess &&
             hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_iface<S, P, GR, LAST, IF_TX, IF_TY>,
                                                          IF_TX * IF_TY, 0) == hipSuccess &&
-            ncu > 0 && per_cu > 0)
-            slots = ncu * per_cu;
-        else {
-            (void)hipGetLastError();  // answered here: not the launch's error
-            slots = 1024;
-        }
-    }
-    cus = ncu;
-    return slots;
+            cus > 0 && per_cu > 0)
+            return IfaceSlots{cus * per_cu, cus};
+        (void)hipGetLastError();  // answered here: not the launch's error
+        return IfaceSlots{1024, cus};
+    }();
+    return n;
 }
 
 static int iface_groups(long tiles, int slots, int cus) {
@@ -585,8 +585,8 @@ static hipError_t iface_launch(hipStream_t s, IfaceItem *items, int n, HermiteW<
         long tiles = 0;
         for (int i = i0; i < i0 + m; i++)
             tiles += (long)((items[i].Xc + IF_TX - 1) / IF_TX) * ((items[i].Yc + IF_TY - 1) / IF_TY);
-        int cus = 0;
-        const int slots = iface_slots<S, P, GR, LAST>(cus), G = iface_groups(tiles, slots, cus);
+        const IfaceSlots &gpu = iface_slots<S, P, GR, LAST>();
+        const int G = iface_groups(tiles, gpu.slots, gpu.cus);
         for (int i = i0; i < i0 + m; i++) items[i].groups = G;
         Batch<IfaceItem> B;
         B.halt = halt;
