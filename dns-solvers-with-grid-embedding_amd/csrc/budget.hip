@@ -26,6 +26,7 @@
 #include <type_traits>
 #include <vector>
 
+#include "budget_split.hpp"
 #include "internal.hpp"
 #include "lattice.hpp"
 
@@ -40,7 +41,6 @@ enum {
     A_PU, A_PV, A_PW, A_WX, A_WY, A_WZ, A_PAIUU, A_PAIVV, A_PAIWW, A_PAIUW,
     A_USUW, A_VSVW, A_WSWW, A_WSUW, A_USWW, A_EPUU, A_EPVV, A_EPWW, A_EPUW, NACC
 };
-constexpr int BT = 256;  // threads per workgroup
 
 // one grid of the snapshot: planes [4][Z][Y][X] of u, v, w, rho
 struct BudGrid {
@@ -49,6 +49,7 @@ struct BudGrid {
     int k0, k1;         // layers taking part in the statistics
     int m0, m1;         // layers whose mean is taken (and subtracted)
     int base;           // profile index of layer 0
+    int rows;           // rows a thread takes (bud_rows)
 };
 
 struct BudArgs {
@@ -117,34 +118,27 @@ __device__ __forceinline__ void wg_sum(double *v, double *out) {
     }
 }
 
-// A workgroup takes BT consecutive columns x of BR rows of one layer: its partials are
-// summed over BR nodes per thread before the workgroup reduction (44 values: reduced at
-// every node, the reduction cost more than the terms).
-constexpr int BR = 8;
-__host__ __device__ inline int bud_xc(int X) { return (X + BT - 1) / BT; }
-__host__ __device__ inline int bud_chunks(int X, int Y) { return bud_xc(X) * ((Y + BR - 1) / BR); }
-
 // 1. planes of one grid, and per-(layer, chunk) sums of u, v, w, rho/3
 template <class S>
 __global__ __launch_bounds__(BT) void k_bud_fill(const S *__restrict__ lat, const double *__restrict__ wall, BudGrid G,
                                                  int zlo, int kwall, double *__restrict__ part) {
-    const int nch = bud_chunks(G.X, G.Y), nxc = bud_xc(G.X);
-    const int k = (int)blockIdx.x / nch, ch = (int)blockIdx.x % nch;
-    const int x = (ch % nxc) * BT + threadIdx.x, y0 = ch / nxc * BR;
+    const int nch = bud_chunks(G.X, G.Y, G.rows);
+    const int k = (int)blockIdx.x / nch;
+    int x, y0;
+    bud_column(G.X, G.rows, (int)blockIdx.x % nch, threadIdx.x, x, y0);
     double v[4] = {0., 0., 0., 0.};
-    if (x < G.X)
-        for (int y = y0; y < min(y0 + BR, G.Y); y++) {
-            const Vel r = file_vel(lat, wall, G.X, G.Y, zlo, kwall, x, y, k);
-            const size_t plane = (size_t)G.Z * G.Y * G.X, e = ((size_t)k * G.Y + y) * G.X + x;
-            G.v[e] = r.u;
-            G.v[plane + e] = r.v;
-            G.v[2 * plane + e] = r.w;
-            G.v[3 * plane + e] = r.rho;
-            v[0] += r.u;
-            v[1] += r.v;
-            v[2] += r.w;
-            v[3] += (1. / 3.) * r.rho;
-        }
+    for (int y = y0; y < min(y0 + G.rows, G.Y); y++) {
+        const Vel r = file_vel(lat, wall, G.X, G.Y, zlo, kwall, x, y, k);
+        const size_t plane = (size_t)G.Z * G.Y * G.X, e = ((size_t)k * G.Y + y) * G.X + x;
+        G.v[e] = r.u;
+        G.v[plane + e] = r.v;
+        G.v[2 * plane + e] = r.w;
+        G.v[3 * plane + e] = r.rho;
+        v[0] += r.u;
+        v[1] += r.v;
+        v[2] += r.w;
+        v[3] += (1. / 3.) * r.rho;
+    }
     wg_sum<4>(v, part + (size_t)blockIdx.x * 4);
 }
 
@@ -214,58 +208,58 @@ __device__ __forceinline__ double bud_ddz(const BudArgs &A, int g, int i, int j,
 //    per (layer, chunk) -> part[(k - k0) * chunks + chunk][NACC]
 __global__ __launch_bounds__(BT) void k_bud_nodes(BudArgs A, int g, double *__restrict__ part) {
     const BudGrid &G = A.g[g];
-    const int X = G.X, Y = G.Y, nch = bud_chunks(X, Y), nxc = bud_xc(X);
-    const int k = G.k0 + (int)blockIdx.x / nch, ch = (int)blockIdx.x % nch;
-    const int i = (ch % nxc) * BT + threadIdx.x, y0 = ch / nxc * BR;
+    const int X = G.X, Y = G.Y, nch = bud_chunks(X, Y, G.rows);
+    const int k = G.k0 + (int)blockIdx.x / nch;
+    int i, y0;
+    bud_column(X, G.rows, (int)blockIdx.x % nch, threadIdx.x, i, y0);
     double a[NACC];
 #pragma unroll
     for (int c = 0; c < NACC; c++) a[c] = 0.;
     const int im = i == 0 ? X - 1 : i - 1, imm = im == 0 ? X - 1 : im - 1;
     const int ip = i == X - 1 ? 0 : i + 1, ipp = ip == X - 1 ? 0 : ip + 1;
     const size_t plane = (size_t)Y * X;
-    if (i < X)
-        for (int j = y0; j < min(y0 + BR, Y); j++) {
-            const int jp = j == 0 ? Y - 1 : j - 1, jpp = jp == 0 ? Y - 1 : jp - 1;
-            const int jn = j == Y - 1 ? 0 : j + 1, jnn = jn == Y - 1 ? 0 : jn + 1;
-            double w0[3], d[3][3];
+    for (int j = y0; j < min(y0 + G.rows, Y); j++) {
+        const int jp = j == 0 ? Y - 1 : j - 1, jpp = jp == 0 ? Y - 1 : jp - 1;
+        const int jn = j == Y - 1 ? 0 : j + 1, jnn = jn == Y - 1 ? 0 : jn + 1;
+        double w0[3], d[3][3];
 #pragma unroll
-            for (int c = 0; c < 3; c++) {
-                const double *p = G.v + ((size_t)c * G.Z + k) * plane;
-                const double m = (k >= G.m0 && k < G.m1) ? A.mean[c * A.NZ + G.base + k] : 0.;
-                auto at = [&](int ii, int jj) { return p[(size_t)jj * X + ii] - m; };
-                const double gx = (2. / 3.) * (at(ip, j) - at(im, j)) - (1. / 12.) * (at(ipp, j) - at(imm, j));
-                const double gy = (2. / 3.) * (at(i, jn) - at(i, jp)) - (1. / 12.) * (at(i, jnn) - at(i, jpp));
-                w0[c] = at(i, j);
-                d[c][0] = g == 0 ? A.coef * gx : gx;
-                d[c][1] = g == 0 ? A.coef * gy : gy;
-                d[c][2] = bud_ddz(A, g, i, j, k, c);
-            }
-            const double u = w0[0], vv = w0[1], w = w0[2];
-            const double dfl = (1. / 3.) * G.v[((size_t)3 * G.Z + k) * plane + (size_t)j * X + i] - A.mean[3 * A.NZ + G.base + k];
-            const double dudx = d[0][0], dudy = d[0][1], dudz = d[0][2];
-            const double dvdx = d[1][0], dvdy = d[1][1], dvdz = d[1][2];
-            const double dwdx = d[2][0], dwdy = d[2][1], dwdz = d[2][2];
-            const double ox = (dwdy - dvdz), oy = (dudz - dwdx), oz = (dvdx - dudy);
-            a[A_UU] += u * u; a[A_UV] += u * vv; a[A_UW] += u * w; a[A_VV] += vv * vv; a[A_VW] += vv * w; a[A_WW] += w * w;
-            a[A_SKU] += u * u * u; a[A_SKV] += vv * vv * vv; a[A_SKW] += w * w * w; a[A_SKP] += dfl * dfl * dfl;
-            a[A_SKUW] += u * u * u * w * w * w; a[A_SKUV] += u * u * u * vv * vv * vv; a[A_SKVW] += vv * vv * vv * w * w * w;
-            a[A_KUU] += u * u * u * u; a[A_KUV] += vv * vv * vv * vv; a[A_KUW] += w * w * w * w;
-            a[A_KUP] += dfl * dfl * dfl * dfl;
-            a[A_KUUW] += u * u * u * u * w * w * w * w; a[A_KUVW] += vv * vv * vv * vv * w * w * w * w;
-            a[A_KUUV] += u * u * u * u * vv * vv * vv * vv;
-            a[A_DD] += dfl * dfl;
-            a[A_UUW] += u * u * w; a[A_VVW] += vv * vv * w; a[A_WWW] += w * w * w; a[A_UWW] += u * w * w;
-            a[A_PU] += u * dfl; a[A_PV] += vv * dfl; a[A_PW] += w * dfl;
-            a[A_WX] += ox * ox; a[A_WY] += oy * oy; a[A_WZ] += oz * oz;
-            a[A_PAIUU] += dfl * dudx; a[A_PAIVV] += dfl * dvdy; a[A_PAIWW] += dfl * dwdz; a[A_PAIUW] += dfl * (dudz + dwdx);
-            a[A_USUW] += 0.5 * u * (dudz + dwdx); a[A_VSVW] += 0.5 * vv * (dvdz + dwdy);
-            a[A_WSWW] += 0.5 * w * (dwdz + dwdz); a[A_WSUW] += 0.5 * w * (dudz + dwdx); a[A_USWW] += 0.5 * u * (dwdz + dwdz);
-            a[A_EPUU] += dudx * (dudx + dudx) + dudy * (dudy + dvdx) + dudz * (dudz + dwdx);
-            a[A_EPVV] += dvdx * (dvdx + dudy) + dvdy * (dvdy + dvdy) + dvdz * (dvdz + dwdy);
-            a[A_EPWW] += dwdx * (dwdx + dudz) + dwdy * (dwdy + dvdz) + dwdz * (dwdz + dwdz);
-            a[A_EPUW] += dudx * (dwdx + dudz) + dudy * (dwdy + dvdz) + dudz * (dwdz + dwdz) + dwdx * (dudx + dudx) +
-                         dwdy * (dudy + dvdx) + dwdz * (dudz + dwdx);
+        for (int c = 0; c < 3; c++) {
+            const double *p = G.v + ((size_t)c * G.Z + k) * plane;
+            const double m = (k >= G.m0 && k < G.m1) ? A.mean[c * A.NZ + G.base + k] : 0.;
+            auto at = [&](int ii, int jj) { return p[(size_t)jj * X + ii] - m; };
+            const double gx = (2. / 3.) * (at(ip, j) - at(im, j)) - (1. / 12.) * (at(ipp, j) - at(imm, j));
+            const double gy = (2. / 3.) * (at(i, jn) - at(i, jp)) - (1. / 12.) * (at(i, jnn) - at(i, jpp));
+            w0[c] = at(i, j);
+            d[c][0] = g == 0 ? A.coef * gx : gx;
+            d[c][1] = g == 0 ? A.coef * gy : gy;
+            d[c][2] = bud_ddz(A, g, i, j, k, c);
         }
+        const double u = w0[0], vv = w0[1], w = w0[2];
+        const double dfl = (1. / 3.) * G.v[((size_t)3 * G.Z + k) * plane + (size_t)j * X + i] - A.mean[3 * A.NZ + G.base + k];
+        const double dudx = d[0][0], dudy = d[0][1], dudz = d[0][2];
+        const double dvdx = d[1][0], dvdy = d[1][1], dvdz = d[1][2];
+        const double dwdx = d[2][0], dwdy = d[2][1], dwdz = d[2][2];
+        const double ox = (dwdy - dvdz), oy = (dudz - dwdx), oz = (dvdx - dudy);
+        a[A_UU] += u * u; a[A_UV] += u * vv; a[A_UW] += u * w; a[A_VV] += vv * vv; a[A_VW] += vv * w; a[A_WW] += w * w;
+        a[A_SKU] += u * u * u; a[A_SKV] += vv * vv * vv; a[A_SKW] += w * w * w; a[A_SKP] += dfl * dfl * dfl;
+        a[A_SKUW] += u * u * u * w * w * w; a[A_SKUV] += u * u * u * vv * vv * vv; a[A_SKVW] += vv * vv * vv * w * w * w;
+        a[A_KUU] += u * u * u * u; a[A_KUV] += vv * vv * vv * vv; a[A_KUW] += w * w * w * w;
+        a[A_KUP] += dfl * dfl * dfl * dfl;
+        a[A_KUUW] += u * u * u * u * w * w * w * w; a[A_KUVW] += vv * vv * vv * vv * w * w * w * w;
+        a[A_KUUV] += u * u * u * u * vv * vv * vv * vv;
+        a[A_DD] += dfl * dfl;
+        a[A_UUW] += u * u * w; a[A_VVW] += vv * vv * w; a[A_WWW] += w * w * w; a[A_UWW] += u * w * w;
+        a[A_PU] += u * dfl; a[A_PV] += vv * dfl; a[A_PW] += w * dfl;
+        a[A_WX] += ox * ox; a[A_WY] += oy * oy; a[A_WZ] += oz * oz;
+        a[A_PAIUU] += dfl * dudx; a[A_PAIVV] += dfl * dvdy; a[A_PAIWW] += dfl * dwdz; a[A_PAIUW] += dfl * (dudz + dwdx);
+        a[A_USUW] += 0.5 * u * (dudz + dwdx); a[A_VSVW] += 0.5 * vv * (dvdz + dwdy);
+        a[A_WSWW] += 0.5 * w * (dwdz + dwdz); a[A_WSUW] += 0.5 * w * (dudz + dwdx); a[A_USWW] += 0.5 * u * (dwdz + dwdz);
+        a[A_EPUU] += dudx * (dudx + dudx) + dudy * (dudy + dvdx) + dudz * (dudz + dwdx);
+        a[A_EPVV] += dvdx * (dvdx + dudy) + dvdy * (dvdy + dvdy) + dvdz * (dvdz + dwdy);
+        a[A_EPWW] += dwdx * (dwdx + dudz) + dwdy * (dwdy + dvdz) + dwdz * (dwdz + dwdz);
+        a[A_EPUW] += dudx * (dwdx + dudz) + dudy * (dwdy + dvdz) + dudz * (dwdz + dwdz) + dwdx * (dudx + dudx) +
+                     dwdy * (dudy + dvdx) + dwdz * (dudz + dwdx);
+    }
     wg_sum<NACC>(a, part + (size_t)blockIdx.x * NACC);
 }
 
@@ -507,6 +501,8 @@ hipError_t launch_snapshot(dnsg_ctx *h, int g, double *vel, double *den) {
 
 using namespace dnsg;
 
+constexpr size_t BUD_SMALL = (size_t)1 << 20;
+
 #define BCHK(h, expr)                                                                       \
     do {                                                                                    \
         hipError_t e_ = (expr);                                                             \
@@ -538,63 +534,81 @@ extern "C" int dnsg_budget2d(dnsg_t *h, double *turb, double *vort, double *ke, 
     const int k0[3] = {2, 1, 0}, k1[3] = {zdc - 2, zdf, zdf - 1};    // node passes
     const int m0[3] = {2, 0, 0}, m1[3] = {zdc - 2, zdf, zdf};        // means and subtraction
     const int base[3] = {zdf - 2, 0, zdf + zdc - 4};
-    size_t npart = 0, nsum = 0, nv = 0;
+    int cus = 0;
+    if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, h->device) != hipSuccess) cus = 0;
+    size_t npart = 0, nv[3], off[3][2], n4 = 0, nacc = 0;  // off: of a grid's sums, layer means and node terms
     std::vector<double> mean(4 * (size_t)NZ, 0.), acc((size_t)NACC * NZ, 0.), dUdz(NZ, 0.), lay;
-    double *dmean = nullptr, *dpart = nullptr, *dsum = nullptr, *dpl = nullptr, *dv = nullptr;
+    double *dmean = nullptr, *dpart = nullptr, *dsum = nullptr, *dpl = nullptr, *dv[3] = {nullptr, nullptr, nullptr};
     for (int g = 0; g < 3; g++) {
         const FileGrid F = file_grid(h, g);
-        A.g[g] = BudGrid{nullptr, F.X, F.Y, F.Z, k0[g], k1[g], m0[g], m1[g], base[g]};
-        npart = std::max(npart, (size_t)bud_chunks(F.X, F.Y) * F.Z * NACC);
-        nsum = std::max(nsum, (size_t)F.Z * NACC);
-        nv += 4 * (size_t)F.X * F.Y * F.Z;
+        const int rows = bud_rows(F.X, F.Y, k1[g] - k0[g], cus);
+        A.g[g] = BudGrid{nullptr, F.X, F.Y, F.Z, k0[g], k1[g], m0[g], m1[g], base[g], rows};
+        npart = std::max(npart, (size_t)bud_chunks(F.X, F.Y, rows) * F.Z * NACC);
+        off[g][0] = n4;
+        off[g][1] = nacc;
+        n4 += (size_t)F.Z * 4;
+        nacc += (size_t)(k1[g] - k0[g]) * NACC;
+        nv[g] = 4 * (size_t)F.X * F.Y * F.Z;
     }
-    BCHK(h, scratch_get(&dv, nv * 8));
+    // one block for the planes of all grids, or one a grid where each is below 1 MiB: the
+    // runtime cuts those from a larger one, while a block of its own takes 0.3 ms or more
+    // (the first budget of a 32 x 24 x 16 handle 560 us with one block, 280 with three)
+    if (nv[0] * 8 < BUD_SMALL && nv[1] * 8 < BUD_SMALL) {
+        for (int g = 0; g < 3; g++) {
+            BCHK(h, scratch_get(&dv[g], nv[g] * 8));
+            A.g[g].v = dv[g];
+        }
+    } else {
+        BCHK(h, scratch_get(&dv[0], (nv[0] + nv[1] + nv[2]) * 8));
+        for (int g = 0; g < 3; g++) A.g[g].v = g == 0 ? dv[0] : A.g[g - 1].v + nv[g - 1];
+    }
     BCHK(h, scratch_get(&dmean, 4 * (size_t)NZ * 8));
     BCHK(h, scratch_get(&dpart, npart * 8));
-    BCHK(h, scratch_get(&dsum, 3 * nsum * 8));
-    A.g[0].v = dv;
-    for (int g = 1; g < 3; g++) A.g[g].v = A.g[g - 1].v + 4 * (size_t)A.g[g - 1].X * A.g[g - 1].Y * A.g[g - 1].Z;
-    lay.resize(3 * nsum);
+    // the sums lie end to end: copies of up to 16 KiB to the host are made by a kernel, larger
+    // ones by the DMA engines, which also clear freed memory and may be busy with that (a
+    // small budget took 260 us for 12 ms after another handle's 300 MB were freed, now 155)
+    BCHK(h, scratch_get(&dsum, std::max(n4, nacc) * 8));
+    lay.resize(std::max(n4, nacc));
     // 1. snapshot planes and layer means
     for (int g = 0; g < 3; g++) {
         const FileGrid F = file_grid(h, g);
         const BudGrid &G = A.g[g];
-        const int nch = bud_chunks(G.X, G.Y);
+        const int nch = bud_chunks(G.X, G.Y, G.rows);
         by_storage(h, F.lat->c(), [&](auto *lat) {
             using S = std::remove_const_t<std::remove_pointer_t<decltype(lat)>>;
             hipLaunchKernelGGL(k_bud_fill<S>, dim3((unsigned)(G.Z * nch)), dim3(BT), 0, h->stream, lat, F.wall, G, F.zlo,
                                F.kwall, dpart);
         });
         hipLaunchKernelGGL(k_bud_segsum, dim3((unsigned)((G.Z * 4 + 3) / 4)), dim3(BT), 0, h->stream,
-                           (const double *)dpart, G.Z, nch, 4, dsum + g * nsum);
+                           (const double *)dpart, G.Z, nch, 4, dsum + off[g][0]);
         BCHK(h, hipGetLastError());
     }
-    BCHK(h, hipMemcpyAsync(lay.data(), dsum, lay.size() * 8, hipMemcpyDeviceToHost, h->stream));
+    BCHK(h, hipMemcpyAsync(lay.data(), dsum, n4 * 8, hipMemcpyDeviceToHost, h->stream));
     BCHK(h, hipStreamSynchronize(h->stream));
     for (int g = 0; g < 3; g++) {
         const BudGrid &G = A.g[g];
         for (int k = G.m0; k < G.m1; k++)
             for (int c = 0; c < 4; c++)
-                mean[(size_t)c * NZ + G.base + k] = lay[g * nsum + (size_t)k * 4 + c] / (double)(G.X * G.Y);
+                mean[(size_t)c * NZ + G.base + k] = lay[off[g][0] + (size_t)k * 4 + c] / (double)(G.X * G.Y);
     }
     BCHK(h, hipMemcpyAsync(dmean, mean.data(), mean.size() * 8, hipMemcpyHostToDevice, h->stream));
     // 2. per-node terms over the layers of the node passes
     A.mean = dmean;
     for (int g = 0; g < 3; g++) {
         const BudGrid &G = A.g[g];
-        const int nch = bud_chunks(G.X, G.Y), nk = G.k1 - G.k0;
+        const int nch = bud_chunks(G.X, G.Y, G.rows), nk = G.k1 - G.k0;
         hipLaunchKernelGGL(k_bud_nodes, dim3((unsigned)(nk * nch)), dim3(BT), 0, h->stream, A, g, dpart);
         hipLaunchKernelGGL(k_bud_segsum, dim3((unsigned)((nk * NACC + 3) / 4)), dim3(BT), 0, h->stream,
-                           (const double *)dpart, nk, nch, (int)NACC, dsum + g * nsum);
+                           (const double *)dpart, nk, nch, (int)NACC, dsum + off[g][1]);
         BCHK(h, hipGetLastError());
     }
-    BCHK(h, hipMemcpyAsync(lay.data(), dsum, lay.size() * 8, hipMemcpyDeviceToHost, h->stream));
+    BCHK(h, hipMemcpyAsync(lay.data(), dsum, nacc * 8, hipMemcpyDeviceToHost, h->stream));
     BCHK(h, hipStreamSynchronize(h->stream));
     for (int g = 0; g < 3; g++) {
         const BudGrid &G = A.g[g];
         for (int k = G.k0; k < G.k1; k++)
             for (int c = 0; c < NACC; c++)
-                acc[(size_t)c * NZ + G.base + k] = lay[g * nsum + (size_t)(k - G.k0) * NACC + c];
+                acc[(size_t)c * NZ + G.base + k] = lay[off[g][1] + (size_t)(k - G.k0) * NACC + c];
     }
     if (ufl) {
         const size_t np = (size_t)A.g[1].X * A.g[1].Y;
@@ -609,7 +623,7 @@ extern "C" int dnsg_budget2d(dnsg_t *h, double *turb, double *vort, double *ke, 
     bud_dudz(mean.data(), zdf, zdc, GR, dUdz.data());
     bud_finish(h->p, mean.data(), dUdz.data(), acc, turb, vort, ke);
 done:
-    (void)scratch_put(h->stream, {dv, dmean, dpart, dsum, dpl});
+    (void)scratch_put(h->stream, {dv[0], dv[1], dv[2], dmean, dpart, dsum, dpl});
     return rc;
 }
 

@@ -1,5 +1,6 @@
-// The few HIP runtime calls of csrc/scratch.hip on host memory, so that its bookkeeping
-// can be tested without a GPU.  A test sets the device's size and reads what was done.
+// The few HIP runtime calls of csrc/scratch.hip on host memory, so that its bookkeeping (and
+// plain host code of other headers) can be tested without a GPU.  A test sets the device's
+// size and reads what was done.
 #pragma once
 #include <pthread.h>
 #include <stddef.h>
@@ -10,6 +11,8 @@
 #include <map>
 #include <mutex>
 
+#define __host__
+#define __device__
 typedef int hipError_t;
 enum { hipSuccess = 0, hipErrorInvalidValue = 1, hipErrorOutOfMemory = 2 };
 struct ihipStream_t {
