@@ -358,7 +358,7 @@ int do_step_band2(dnsg_t *h, double *rec, SecTimer *T) {
         B[1].dsum = dsum_band(h, 1);
     }
     if (T) T->begin(h->stream, SEC_BAND);
-    HIPCHK(h, launch_band2(h->stream, B, h->p.precision, h->halt()));
+    HIPCHK(h, launch_band2(h->stream, B, h->p.precision, h->band2, h->halt()));
     if (T) T->end(h->stream, SEC_BAND);
     if (T) T->begin(h->stream, SEC_REDUCE);
     if (!flux) HIPCHK(h, launch_reductions_fused(h->stream, h, rec));
@@ -886,14 +886,18 @@ int dnsg::create_ctx(const dnsg_params *p, hipStream_t ext, dnsg_t **out) {
         h->cs_pair = !(cp && cp[0] == '0');
         h->cs_wide = cw && cw[0] >= '0' && cw[0] <= '3' ? cw[0] - '0' : 0;
         // gratio 2: both band substeps in one pass (k_band2.hip), by default in FP64 and FP32
-        // where the lattice is large enough (band2_pays); FP16 storage keeps one launch per
-        // substep (Re_tau=180 step 0.92 against 0.94 ms).  DNSG_BAND2=1 / DNSG_BAND2=0 in the
-        // environment selects it / the one-launch-per-substep path (the same state; the
-        // reductions' partials differ)
+        // where that is the faster path (band2_pick); FP16 storage keeps one launch per
+        // substep (Re_tau=180 step 0.92 against 0.94 ms).  DNSG_BAND2=0, 1, 2 in the
+        // environment: one launch per substep, the pass with large tiles, with small ones (the
+        // same state; the reductions' partials differ)
         const char *e = getenv("DNSG_BAND2");
         const int elem = (int)h->elem;
-        h->band2 = h->d.GR == 2 && buf_fits(h->d.Xf, h->d.Yf, elem) && !(h->cs_wide & 2) &&
-                   ((e && e[0]) ? e[0] == '1' : elem != 2 && band2_pays(h->d.Xf, h->d.Yf, h->d.zdf - 1, elem));
+        int cus = 0;
+        if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, h->device) != hipSuccess) cus = 0;
+        if (h->d.GR == 2 && buf_fits(h->d.Xf, h->d.Yf, elem) && !(h->cs_wide & 2)) {
+            if (e && e[0]) h->band2 = e[0] == '1' ? B2_LARGE : (e[0] == '2' ? (elem == 2 ? B2_LARGE : B2_SMALL) : B2_OFF);
+            else if (elem != 2 && cus > 0) h->band2 = band2_pick(h->d.Xf, h->d.Yf, h->d.zdf - 1, elem, cus);
+        }
     }
     const dnsg_dims &d = h->d;
     h->coarse.nx = d.Xc; h->coarse.ny = d.Yc; h->coarse.nz = d.zdc;

@@ -22,6 +22,7 @@
 #include <vector>
 
 #include "../../include/dnsg.h"
+#include "band2_pick.hpp"
 #include "scratch.hpp"
 
 namespace dnsg {
@@ -120,21 +121,14 @@ struct Grid {
     void swap() { cur ^= 1; }
 };
 
-// Tile of the two-substep band kernel (k_band2.hip): rows of a workgroup (ring
-// included), nodes per lane and output columns for elements of `elem` bytes.  When a
-// step runs it (dnsg_ctx::band_tiled), the bands' fused-reduction partials are per
-// (row, b2_cols columns) instead of per layer and workgroup, with the layer weights
-// applied: LatArgs::dsum the pair above, LatArgs::red the B2_RED values
+// When a step runs the two-substep band kernel (dnsg_ctx::band_tiled), the bands'
+// fused-reduction partials are per (row, b2_cols columns) instead of per layer and
+// workgroup, with the layer weights applied: LatArgs::dsum the pair above, LatArgs::red the
+// B2_RED values
 //   [0], [1] sum of rho, rho u_x weighted by encalc2's layer weights
 //   [2]      sum of rho over the layer whose density wshearstr takes
 //   [3..5]   sum of u_x over the three layers next to the wall, nearest first
 constexpr int B2_RED = 6;
-#ifndef DNSG_B2_ROWS
-#define DNSG_B2_ROWS 12
-#endif
-constexpr int B2_ROWS = DNSG_B2_ROWS;
-constexpr int b2_npl(int elem) { return elem == 8 ? 1 : 2; }
-constexpr int b2_cols(int elem) { return 62 * b2_npl(elem); }
 
 // number of doubles in one diag record written by the reduction finalisers
 constexpr int DIAG_WORDS = 9;
@@ -162,9 +156,10 @@ struct dnsg_ctx {
     void *lev_lo[4] = {nullptr, nullptr, nullptr, nullptr};
     void *lev_up[4] = {nullptr, nullptr, nullptr, nullptr};
     int given_levels = 0;  // of the three levels a fill reads, how many the caller uploaded
-    // the steps use the two-substep band kernel (gratio 2); band_tiled: the bands'
-    // fused-reduction partials of the last launch that wrote them are that kernel's
-    bool band2 = false;
+    // whether, and with which tiles (Band2), the steps use the two-substep band kernel
+    // (gratio 2); band_tiled: the bands' fused-reduction partials of the last launch that
+    // wrote them are that kernel's
+    int band2 = dnsg::B2_OFF;
     bool band_tiled = false;
     bool cs_pair = true;  // FP32 / FP16: CS_PAIRED where the rows allow it
     int cs_wide = 0;      // CS_WIDE also where the layers are small: bit 0 the coarse grid, bit 1 the bands
@@ -233,14 +228,15 @@ inline int band_form(const dnsg_ctx *h) {
 inline int coarse_parts(const dnsg_ctx *h) { return cs_parts(coarse_form(h), h->coarse.nx, h->coarse.ny); }
 inline int band_parts(const dnsg_ctx *h) {
     const Grid &g = h->lower;
-    if (h->band_tiled) return g.ny * ((g.nx + b2_cols((int)h->elem) - 1) / b2_cols((int)h->elem));
+    if (h->band_tiled) return g.ny * ((g.nx + b2_cols(h->band2, (int)h->elem) - 1) / b2_cols(h->band2, (int)h->elem));
     return cs_parts(band_form(h), g.nx, g.ny);
 }
 // the partials of RED_W values the buffers are sized for: any layout of the coarse grid,
 // and of one band
 inline size_t coarse_parts_max(const dnsg_dims &d) { return (size_t)d.Yc * d.zdc * cs_chunks(d.Xc); }
 inline size_t band_parts_max(const dnsg_dims &d) {
-    const size_t b2 = (size_t)d.Yf * ((d.Xf + b2_cols(8) - 1) / b2_cols(8)) * (B2_RED / RED_W);
+    constexpr int cols = b2_cols(B2_SMALL, 8);  // the narrowest tiles
+    const size_t b2 = (size_t)d.Yf * ((d.Xf + cols - 1) / cols) * (B2_RED / RED_W);
     const size_t cs = (size_t)d.Yf * (d.zdf - 1) * cs_chunks(d.Xf);
     return b2 > cs ? b2 : cs;
 }
@@ -261,10 +257,7 @@ hipError_t launch_collide_stream(hipStream_t s, const LatArgs *lats, int nlat, i
 // the lower band, bands[1] the upper band, as band_args builds them; the first fill
 // must already be in their nxt lattices' interface layers; red / dsum in its own
 // partial layout (B2_RED)
-hipError_t launch_band2(hipStream_t s, const LatArgs *bands, int prec, const int *halt = nullptr);
-int band2_tiles(int nx, int ny, int elem);
-// the one-pass path is the faster one for a handle's two bands of nx x ny x nz nodes
-bool band2_pays(int nx, int ny, int nz, int elem);
+hipError_t launch_band2(hipStream_t s, const LatArgs *bands, int prec, int tile, const int *halt = nullptr);
 hipError_t launch_init_lattice(hipStream_t s, dnsg_ctx *h, int grid, void *dst);
 // gl = 1: the host array carries one ghost x-plane and y-row (the reference's in-memory
 // layout); downloads write them as periodic images

@@ -12,7 +12,9 @@
 //   * a workgroup has NR waves, one per row of the tile and its ring; a lane holds NPL
 //     adjacent nodes of its row.  The first substep is collided on all 64 NPL columns
 //     and NR rows, the second on all but the outermost lane and row on each side (the
-//     ring), so a tile is 62 NPL columns by NR - 2 rows, all layers;
+//     ring), so a tile is 62 NPL columns by NR - 2 rows, all layers.  Large tiles have 12
+//     waves and two nodes per lane (FP64 one), small ones 8 waves and one node, which
+//     halves a layer's chain and leaves fewer CUs idle on small lattices (band2_pick.hpp);
 //   * the workgroup marches through the layers from the interface towards the wall.
 //     At layer t it collides the first substep's input and puts the 18 streamed
 //     values of each node into LDS; after a barrier every node of the tile takes the
@@ -48,13 +50,10 @@ namespace dnsg {
 
 namespace {
 
-constexpr int NR = B2_ROWS;  // rows of a workgroup, ring included: one wave each
-constexpr int TY = NR - 2;   // output rows of a tile
-constexpr int B2_THREADS = 64 * NR;
-template <class S>
-constexpr int npl() { return b2_npl(sizeof(S)); }  // nodes per lane
-template <class S>
-constexpr bool early() { return sizeof(S) == 8; }  // when the next layer is loaded (band2_tile)
+template <class S, int TILE>
+constexpr int npl() { return b2_npl(TILE, sizeof(S)); }  // nodes per lane
+template <class S, int TILE>
+constexpr bool early() { return npl<S, TILE>() == 1; }  // when the next layer is loaded (band2_tile)
 
 // March coordinate t: 0 at the interface layer, nz-1 next to the wall.  A direction
 // moves t by ez for the upper band (interface = stored layer 0) and by -ez for the
@@ -81,10 +80,14 @@ __device__ __forceinline__ void load_n(Rsrc R, unsigned v, unsigned s, const dou
 template <class S>
 __device__ __forceinline__ void load_n(Rsrc R, unsigned v, unsigned s, const S *p, float (&o)[2]) { buf_load_pair(R, v, s, p, o[0], o[1]); }
 
-template <class S, int SIDE, bool DS>
+template <class S>
+__device__ __forceinline__ void load_n(Rsrc R, unsigned v, unsigned s, const S *p, float (&o)[1]) { o[0] = buf_load(R, v, s, p); }
+
+template <class S, int TILE, int SIDE, bool DS>
 __device__ __forceinline__ void band2_tile(const LatArgs &L, int tile, typename ComputeOf<S>::T *lds, int8_t *wcl) {
     using T = typename ComputeOf<S>::T;
-    constexpr int NPL = npl<S>(), CW = 64 * NPL, OX = 62 * NPL;
+    constexpr int NR = b2_rows(TILE), TY = NR - 2;  // rows of the workgroup, one wave each, and of the tile
+    constexpr int NPL = npl<S, TILE>(), CW = 64 * NPL, OX = 62 * NPL;
     auto each_n = [](auto &&f) __attribute__((always_inline)) { unroll<0, NPL>(f); };
     const int nx = L.nx, ny = L.ny, nz = L.nz;
     const int tilesx = (nx + OX - 1) / OX;
@@ -252,13 +255,13 @@ __device__ __forceinline__ void band2_tile(const LatArgs &L, int tile, typename 
     for (int t = 0; t < nz; t++) {
         T *const me0 = me + (t & 1) * ALONG * PL;               // along-layer copy of layer t
         const T *const me1 = me + ((t & 1) ^ 1) * ALONG * PL;   // ... of layer t-1
-        // The next layer's loads: issued here, before this layer's collision, in FP64, so
-        // they have the whole iteration to arrive (Re_tau=180 launch 1.250 -> 1.203 ms);
-        // in FP32 and FP16, whose two nodes per lane would spill (0.749 -> 0.812 ms), after
-        // it, into the registers it frees.
+        // The next layer's loads: issued here, before this layer's collision, with one node
+        // per lane, so they have the whole iteration to arrive (FP64 Re_tau=180 launch 1.250
+        // -> 1.203 ms, FP32 small tiles on 512 x 256 x 8 bands 99 -> 86 us); with two, which
+        // would spill (FP32 0.749 -> 0.812 ms), after it, into the registers it frees.
         T f[NPL][Q];
-        T(&F)[NPL][Q] = early<S>() ? f : fin;
-        if constexpr (early<S>()) {
+        T(&F)[NPL][Q] = early<S, TILE>() ? f : fin;
+        if constexpr (early<S, TILE>()) {
             unroll<0, Q>([&](auto qc) {
                 constexpr int q = decltype(qc)::value;
                 each_n([&](auto nc) { f[decltype(nc)::value][q] = fin[decltype(nc)::value][q]; });
@@ -310,7 +313,7 @@ __device__ __forceinline__ void band2_tile(const LatArgs &L, int tile, typename 
         T f0[NPL];
         each_n([&](auto nc) { f0[decltype(nc)::value] = F[decltype(nc)::value][0]; });
         __syncthreads();
-        if constexpr (!early<S>()) {
+        if constexpr (!early<S, TILE>()) {
             if (rowok && t + 1 < nz) load_layer(layer_rsrc(cur, t + 1), fin);
         }
         __builtin_amdgcn_sched_barrier(0);
@@ -411,10 +414,14 @@ __device__ __forceinline__ void band2_tile(const LatArgs &L, int tile, typename 
     }
 }
 
-template <class S, bool DS>
-__global__ __launch_bounds__(B2_THREADS) void k_band2(Batch<LatArgs> P) {
+// waves per SIMD that the registers must allow: FP32 in small tiles four, two workgroups a CU
+template <class S, int TILE>
+constexpr int min_waves() { return TILE == B2_SMALL && sizeof(S) == 4 ? 4 : 1; }
+
+template <class S, int TILE, bool DS>
+__global__ __launch_bounds__(64 * b2_rows(TILE), (min_waves<S, TILE>())) void k_band2(Batch<LatArgs> P) {
     using T = typename ComputeOf<S>::T;
-    constexpr int CW = 64 * npl<S>(), PAD = 2;  // PAD: ring lanes read one value beside the array and ignore it
+    constexpr int NR = b2_rows(TILE), CW = 64 * npl<S, TILE>(), PAD = 2;  // PAD: ring lanes read one value beside the array and ignore it
     __shared__ T lds[NPLANES * NR * CW + 2 * PAD];
     __shared__ int8_t wcl[NR * CW + 2 * PAD];  // the tile's wall codes, ring included
     if (halted(P.halt)) return;
@@ -422,36 +429,22 @@ __global__ __launch_bounds__(B2_THREADS) void k_band2(Batch<LatArgs> P) {
     const int it = batch_find(P.first, P.n, bg);
     const LatArgs &L = P.it[it];
     const int tile = bg - P.first[it];
-    if (L.lo_kind == BOUND_WALL) band2_tile<S, 0, DS>(L, tile, lds + PAD, wcl + PAD);
-    else band2_tile<S, 1, DS>(L, tile, lds + PAD, wcl + PAD);
+    if (L.lo_kind == BOUND_WALL) band2_tile<S, TILE, 0, DS>(L, tile, lds + PAD, wcl + PAD);
+    else band2_tile<S, TILE, 1, DS>(L, tile, lds + PAD, wcl + PAD);
 }
 
 }  // namespace
 
-int band2_tiles(int nx, int ny, int elem) {
-    const int ox = b2_cols(elem);
-    return ((nx + ox - 1) / ox) * ((ny + TY - 1) / TY);
+template <class S, int TILE>
+static void band2_launch(hipStream_t s, const Batch<LatArgs> &P, bool ds) {
+    const dim3 g(P.first[BATCH_MAX]), b(64 * b2_rows(TILE));
+    if (ds) hipLaunchKernelGGL((k_band2<S, TILE, true>), g, b, 0, s, P);
+    else hipLaunchKernelGGL((k_band2<S, TILE, false>), g, b, 0, s, P);
 }
 
-// Which path a gratio-2 handle takes.  A tile holds a CU to itself and marches nz + 1
-// layers, each a chain of two collisions, two barriers and their memory accesses that
-// takes 6.5-8 us with few tiles and 9-10 us with the chip full, so the pass takes whole
-// rounds of tiles over the CUs; the two launches it replaces move twice the bytes at
-// 5.5 TB/s.  Measured, pass against two launches (band time a step): FP64 512 x 256 x 8
-// bands (468 tiles, 2 rounds) 165 / 237 us, 128 x 64 x 8 (42 tiles) 58 / 47 us, 256 x
-// 256 x 8 (260 tiles, a second round for 4 of them) 124 / 112 us; FP32 420 x 252 x 11
-// (208 tiles) 128 / 154 us, 512 x 256 x 16 (260 tiles) 264 / 251 us.
-bool band2_pays(int nx, int ny, int nz, int elem) {
-    int dev = 0, cus = 0;
-    if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus < 1)
-        return false;
-    const int rounds = (2 * band2_tiles(nx, ny, elem) + cus - 1) / cus;
-    const double pass = rounds * (nz + 1) * 9e-6, two = 2. * 2. * nx * (double)ny * nz * 2 * Q * elem / 5.5e12;
-    return pass <= two;
-}
-
-hipError_t launch_band2(hipStream_t s, const LatArgs *bands, int prec, const int *halt) {
+hipError_t launch_band2(hipStream_t s, const LatArgs *bands, int prec, int tile, const int *halt) {
     const int elem = prec == DNSG_PREC_FP64 ? 8 : (prec == DNSG_PREC_FP32 ? 4 : 2);
+    if (tile != B2_LARGE && (tile != B2_SMALL || elem == 2)) return hipErrorInvalidValue;
     Batch<LatArgs> P;
     P.halt = halt;
     P.n = 2;
@@ -459,20 +452,18 @@ hipError_t launch_band2(hipStream_t s, const LatArgs *bands, int prec, const int
     for (int i = 0; i < BATCH_MAX; i++) {
         P.it[i] = bands[i < 2 ? i : 0];
         P.first[i] = blocks;
-        if (i < 2) blocks += band2_tiles(bands[i].nx, bands[i].ny, elem);
+        if (i < 2) blocks += band2_tiles(bands[i].nx, bands[i].ny, elem, tile);
     }
     P.first[BATCH_MAX] = blocks;
-    const bool ds = bands[0].dsum != nullptr || bands[1].dsum != nullptr;
-    const dim3 g(blocks), b(B2_THREADS);
+    const bool ds = bands[0].dsum != nullptr || bands[1].dsum != nullptr, small = tile == B2_SMALL;
     if (prec == DNSG_PREC_FP64) {
-        if (ds) hipLaunchKernelGGL((k_band2<double, true>), g, b, 0, s, P);
-        else hipLaunchKernelGGL((k_band2<double, false>), g, b, 0, s, P);
+        if (small) band2_launch<double, B2_SMALL>(s, P, ds);
+        else band2_launch<double, B2_LARGE>(s, P, ds);
     } else if (prec == DNSG_PREC_FP32) {
-        if (ds) hipLaunchKernelGGL((k_band2<float, true>), g, b, 0, s, P);
-        else hipLaunchKernelGGL((k_band2<float, false>), g, b, 0, s, P);
+        if (small) band2_launch<float, B2_SMALL>(s, P, ds);
+        else band2_launch<float, B2_LARGE>(s, P, ds);
     } else {
-        if (ds) hipLaunchKernelGGL((k_band2<__half, true>), g, b, 0, s, P);
-        else hipLaunchKernelGGL((k_band2<__half, false>), g, b, 0, s, P);
+        band2_launch<__half, B2_LARGE>(s, P, ds);
     }
     return hipGetLastError();
 }
