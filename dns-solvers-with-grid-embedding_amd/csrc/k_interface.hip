@@ -22,6 +22,7 @@
 #include <cmath>
 #include <vector>
 
+#include "iface_split.hpp"
 #include "internal.hpp"
 #include "lattice.hpp"
 #include "stream_common.hpp"
@@ -328,7 +329,6 @@ struct IfaceItem {
 };
 
 // units of directions: (1, 2), (3, 4) .. (17, 18), then the rest direction
-constexpr int IF_UNITS = 10;
 constexpr int if_dir(int unit, int i) { return unit < IF_UNITS - 1 ? 2 * unit + 1 + i : 0; }
 
 template <class S, class P, int GR, bool LAST, int TX, int TY>
@@ -543,13 +543,7 @@ __global__ __launch_bounds__(TX *TY) void k_iface(Batch<IfaceItem> BT, HermiteW<
 // Coarse tile of one workgroup.  The direction units can be shared out over G
 // workgroups per tile, each forming rho and u itself: that multiplies the work by
 // (4 + 19/G) G / 23 but shortens each workgroup's chain of sequential steps
-// to 2 + 10/G.  G fills the workgroup slots the GPU holds at once for this kernel
-// (CUs x resident workgroups per CU, from the occupancy query): a launch whose
-// tiles alone fill them (the Re_tau=180 bands: 1024 tiles) takes G = 1, a launch of
-// small channels (the serving queue) shortens its chains, up to G = 10, or
-// G = 19 with one direction each where every workgroup then has a CU of its own (gratio 3,
-// 4 tiles: 11.4 and 10.0 us a launch against 13.2 and 11.6 with G = 10; gratio 2,
-// 16 tiles, whose 304 workgroups share CUs: 12.5 and 11.4 against 11.8 and 10.2).
+// to 2 + 10/G (iface_split.hpp).
 constexpr int IF_TX = 32, IF_TY = 8;
 
 // workgroups of the kernel that the GPU holds at once, and its CUs
@@ -572,12 +566,6 @@ static const IfaceSlots &iface_slots() {
     return n;
 }
 
-static int iface_groups(long tiles, int slots, int cus) {
-    if (tiles >= slots) return 1;
-    if (tiles * Q <= cus) return Q;
-    return (int)std::min<long>(IF_UNITS, slots / tiles);
-}
-
 template <class S, class P, int GR, bool LAST>
 static hipError_t iface_launch(hipStream_t s, IfaceItem *items, int n, HermiteW<P> H, const int *halt) {
     for (int i0 = 0; i0 < n; i0 += BATCH_MAX) {
@@ -586,7 +574,7 @@ static hipError_t iface_launch(hipStream_t s, IfaceItem *items, int n, HermiteW<
         for (int i = i0; i < i0 + m; i++)
             tiles += (long)((items[i].Xc + IF_TX - 1) / IF_TX) * ((items[i].Yc + IF_TY - 1) / IF_TY);
         const IfaceSlots &gpu = iface_slots<S, P, GR, LAST>();
-        const int G = iface_groups(tiles, gpu.slots, gpu.cus);
+        const int G = iface_groups(tiles, gpu.slots, gpu.cus, sizeof(P) == 4 && GR >= 3);
         for (int i = i0; i < i0 + m; i++) items[i].groups = G;
         Batch<IfaceItem> B;
         B.halt = halt;
