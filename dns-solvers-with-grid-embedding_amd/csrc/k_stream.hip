@@ -19,11 +19,6 @@
 
 namespace dnsg {
 
-// FP64 rows of whole chunks take the aligned-store form, with non-temporal stores; FP32 and
-// FP16 rows that cannot pair are faster in the scatter form (Re_tau=180 lattices).
-template <class S>
-constexpr bool cs_aligned() { return sizeof(S) == 8; }
-
 // Sums of a node's stores by the layer step k = -1, 0, 1 of their destination; the layer
 // weights are applied once at the end (LatArgs::dsum).  Every direction is added at its
 // own step, stored or not: the layers that take no store (beyond an end, or rewritten by

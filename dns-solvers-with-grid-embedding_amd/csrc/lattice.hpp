@@ -208,12 +208,5 @@ __device__ __forceinline__ double read_back(T v) {
     else if constexpr (sizeof(S) == 4) return (double)(float)v + WQ[q];
     else return (double)__half2float(__float2half((float)v)) + WQ[q];
 }
-// streaming stores that bypass the caches' normal allocation (written once, read next step)
-__device__ __forceinline__ void store_nt(float *p, float v) { __builtin_nontemporal_store(v, p); }
-__device__ __forceinline__ void store_nt(double *p, double v) { __builtin_nontemporal_store(v, p); }
-__device__ __forceinline__ void store_nt(__half *p, float v) {
-    const __half h = __float2half(v);
-    __builtin_nontemporal_store(*reinterpret_cast<const unsigned short *>(&h), reinterpret_cast<unsigned short *>(p));
-}
 
 }  // namespace dnsg

@@ -53,3 +53,28 @@ def test_flux_control_over_several_tiles(x, y, prec, tile, monkeypatch):
     for f in ("momentum", "density", "flowrate"):
         assert relmax(ra[f], rb[f]) <= tol, f
     assert np.max(np.abs(ra["force"] - rb["force"])) <= tol * 0.05
+
+
+@pytest.mark.parametrize("prec", ["fp64", "fp32"])
+@pytest.mark.parametrize("force", ["const", "flux"])
+def test_nan_stops_every_path_at_the_same_step(force, prec, monkeypatch):
+    """a NaN planted in the middle of the coarse grid: each path returns the NaN status at the
+    same step of one call and holds NaN at the same places of that step's top"""
+    out = []
+    for band2 in "012":
+        monkeypatch.setenv("DNSG_BAND2", band2)
+        s = dnsg.Solver(dnsg.make_params(xdv=40, ydv=9, zdv=12, gratio=2, zds=5, tau_c=0.53, ub=0.05, force_mode=force,
+                                         g_const=2e-5, CFL=1.0, precision=prec, init_kind="laminar_noise", seed=5,
+                                         u_max=0.05, noise=0.1))
+        s.init_state()
+        st = s.download()
+        st["coarse"][20, 3, 6, 0] = np.nan
+        s.upload(st["coarse"], st["lower"], st["upper"], st["lin"], st["uin"], st["force"])
+        d = (dnsg.Diag * 60)()
+        assert s.lib.dnsg_step(s.h, 60, d) == -3
+        out.append((s.lib.dnsg_last_error(s.h).decode(), {k: np.isnan(v) for k, v in s.download().items() if k != "force"}))
+        s.close()
+    for msg, nan in out[1:]:
+        assert msg == out[0][0]
+        for k in KEYS:
+            assert np.array_equal(nan[k], out[0][1][k]), k
