@@ -880,23 +880,26 @@ int dnsg::create_ctx(const dnsg_params *p, hipStream_t ext, dnsg_t **out) {
     {
         // FP32 / FP16 rows of a multiple of 2 CS_THREADS nodes: the paired collide-stream
         // form (k_stream.hip), unless DNSG_CS_PAIRED=0 (the flat form; same state).
-        // DNSG_CS_WIDE=1, 2, 3: the form of layers of 2 GiB and more on the coarse grid, the
-        // bands, both, so that it can be run at any size (same state)
+        // DNSG_CS_WIDE=1, 2, 3: the form that rows of no whole chunks take in layers of 2 GiB
+        // and more on the coarse grid, the bands, both, so that it can be run at any size
+        // (same state)
         const char *cp = getenv("DNSG_CS_PAIRED"), *cw = getenv("DNSG_CS_WIDE");
         h->cs_pair = !(cp && cp[0] == '0');
         h->cs_wide = cw && cw[0] >= '0' && cw[0] <= '3' ? cw[0] - '0' : 0;
         // gratio 2: both band substeps in one pass (k_band2.hip), by default in FP64 and FP32
         // where that is the faster path (band2_pick); FP16 storage keeps one launch per
-        // substep (Re_tau=180 step 0.92 against 0.94 ms).  DNSG_BAND2=0, 1, 2 in the
-        // environment: one launch per substep, the pass with large tiles, with small ones (the
-        // same state; the reductions' partials differ)
+        // substep (Re_tau=180 step 0.92 against 0.94 ms).  DNSG_BAND2=0, 1, 2, 3 in the
+        // environment: one launch per substep, the pass with large tiles, with small ones, with
+        // large ones in the form for layers of 2 GiB and more (the same state; the
+        // reductions' partials differ)
         const char *e = getenv("DNSG_BAND2");
         const int elem = (int)h->elem;
         int cus = 0;
         if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, h->device) != hipSuccess) cus = 0;
-        if (h->d.GR == 2 && buf_fits(h->d.Xf, h->d.Yf, elem) && !(h->cs_wide & 2)) {
-            if (e && e[0]) h->band2 = e[0] == '1' ? B2_LARGE : (e[0] == '2' ? (elem == 2 ? B2_LARGE : B2_SMALL) : B2_OFF);
-            else if (elem != 2 && cus > 0) h->band2 = band2_pick(h->d.Xf, h->d.Yf, h->d.zdf - 1, elem, cus);
+        if (h->d.GR == 2 && !(h->cs_wide & 2)) {
+            if (e && e[0] >= '1' && e[0] <= '3') h->band2 = e[0] == '2' && elem == 2 ? B2_LARGE : e[0] - '0';
+            else if (!(e && e[0]) && elem != 2 && cus > 0) h->band2 = band2_pick(h->d.Xf, h->d.Yf, h->d.zdf - 1, elem, cus);
+            if (h->band2 && !buf_fits(h->d.Xf, h->d.Yf, elem)) h->band2 = B2_HUGE;
         }
     }
     const dnsg_dims &d = h->d;

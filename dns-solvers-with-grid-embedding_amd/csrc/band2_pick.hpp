@@ -7,7 +7,12 @@ namespace dnsg {
 
 // rows of a workgroup (ring included) and nodes per lane, hence output columns, for
 // elements of `elem` bytes
-enum Band2 { B2_OFF, B2_LARGE, B2_SMALL };  // two launches; tiles of 10 rows; of 6 rows
+enum Band2 {
+    B2_OFF,    // two launches
+    B2_LARGE,  // tiles of 10 rows
+    B2_SMALL,  // tiles of 6 rows
+    B2_HUGE    // tiles of 10 rows, for layers of 2 GiB and more
+};
 constexpr int b2_rows(int tile) { return tile == B2_SMALL ? 8 : 12; }
 constexpr int b2_npl(int tile, int elem) { return tile == B2_SMALL || elem == 8 ? 1 : 2; }
 constexpr int b2_cols(int tile, int elem) { return 62 * b2_npl(tile, elem); }

@@ -84,7 +84,8 @@ constexpr int RED_W = 3;
 // threads per collide-stream workgroup and chunks of them per lattice row
 constexpr int CS_THREADS = 256;
 __host__ __device__ __forceinline__ int cs_chunks(int nx) { return (nx + CS_THREADS - 1) / CS_THREADS; }
-// a layer can be addressed with 31-bit byte offsets (the buffer-resource forms)
+// a layer can be addressed with 31-bit byte offsets (the flat form; the others' resources
+// are single rows)
 __host__ __device__ __forceinline__ bool buf_fits(int nx, int ny, int elem) {
     return (size_t)nx * ny * 19 * elem < ((size_t)1 << 31);
 }
@@ -94,13 +95,13 @@ __host__ __device__ __forceinline__ bool buf_fits(int nx, int ny, int elem) {
 //               Measured on the Re_tau=180 lattices against one node per thread: FP32
 //               coarse launch 0.956 -> 0.852 ms, FP16 0.599 -> 0.586 ms
 //   CS_FLAT     any other rows: consecutive nodes of a layer, whatever rows they fall in
-//   CS_WIDE     layers of 2 GiB and more: one row chunk per workgroup, 64-bit addresses
+//   CS_WIDE     such rows in layers of 2 GiB and more: one row chunk per workgroup, 64-bit
+//               addresses
 enum CsForm { CS_ALIGNED, CS_PAIRED, CS_FLAT, CS_WIDE };
 inline int cs_form(int nx, int ny, int elem, bool pair) {
-    if (!buf_fits(nx, ny, elem)) return CS_WIDE;
     if (elem == 8 && nx % CS_THREADS == 0) return CS_ALIGNED;
     if (elem != 8 && pair && nx % (2 * CS_THREADS) == 0) return CS_PAIRED;
-    return CS_FLAT;
+    return buf_fits(nx, ny, elem) ? CS_FLAT : CS_WIDE;
 }
 // partials of the fused sums per layer, and workgroups of a launch per layer
 __host__ __device__ __forceinline__ int cs_parts(int form, int nx, int ny) {

@@ -15,6 +15,8 @@
 //     ring), so a tile is 62 NPL columns by NR - 2 rows, all layers.  Large tiles have 12
 //     waves and two nodes per lane (FP64 one), small ones 8 waves and one node, which
 //     halves a layer's chain and leaves fewer CUs idle on small lattices (band2_pick.hpp);
+//     huge ones are large tiles whose buffer resources are rows, for layers of 2 GiB and more
+//     (a resource for each row costs the FP64 launch 9 more spilled registers and 3%);
 //   * the workgroup marches through the layers from the interface towards the wall.
 //     At layer t it collides the first substep's input and puts the 18 streamed
 //     values of each node into LDS; after a barrier every node of the tile takes the
@@ -118,8 +120,11 @@ __device__ __forceinline__ void band2_tile(const LatArgs &L, int tile, typename 
     // a pair of targets across the periodic edge is stored one value at a time
     const bool edge = NPL == 2 && (x0 == 0 || x0 + w == nx);
     const bool ep = core && x + NPL == nx, em = core && x == 0;
-    const unsigned layer_bytes = (unsigned)ny * Q * nx * ES;
-    auto soff = [&](int yy, int q) { return (unsigned)(yy * Q + q) * nx * ES; };  // row and direction within a layer
+    // a resource is a layer, or a row where layers are too large for one
+    constexpr bool ROWS = TILE == B2_HUGE;
+    const unsigned layer_bytes = ROWS ? (unsigned)Q * nx * ES : (unsigned)ny * Q * nx * ES;
+    // scalar offset of direction q of row yy within it
+    auto soff = [&](int yy, int q) { return ROWS ? (unsigned)q * nx * ES : (unsigned)(yy * Q + q) * nx * ES; };
     // LDS: plane q-1 of [NR][CW]; this lane's place in it
     T *const me = lds + r * CW + NPL * lane;
     constexpr int PL = NR * CW;
@@ -136,8 +141,12 @@ __device__ __forceinline__ void band2_tile(const LatArgs &L, int tile, typename 
         for (int k = 0; k < 5; k++) wo[n][k] = wn[n][k] = T(0);
     });
 
-    auto layer_rsrc = [&](const S *lat, int t) {
-        return buf_rsrc(lat + (size_t)(SIDE ? t : nz - 1 - t) * ny * Q * nx, layer_bytes);
+    auto row_rsrc = [&](const S *lat, int t, int yy) {
+        return buf_rsrc(lat + ((size_t)(SIDE ? t : nz - 1 - t) * ny + yy) * Q * nx, layer_bytes);
+    };
+    auto layer_rsrc = [&](const S *lat, int t) {  // ... of layer t, or of its row y
+        if constexpr (ROWS) return row_rsrc(lat, t, y);
+        else return buf_rsrc(lat + (size_t)(SIDE ? t : nz - 1 - t) * ny * Q * nx, layer_bytes);
     };
     auto load_q = [&](Rsrc R, int q, T (&v)[NPL]) __attribute__((always_inline)) { load_n(R, vx, soff(y, q), cur, v); };
     auto load_layer = [&](Rsrc R, T (&f)[NPL][Q]) __attribute__((always_inline)) {
@@ -165,6 +174,8 @@ __device__ __forceinline__ void band2_tile(const LatArgs &L, int tile, typename 
         auto put = [&](Rsrc R, auto qc) {  // R: the target layer
             constexpr int q = decltype(qc)::value;
             const unsigned so = soff(EY[q] > 0 ? yp : (EY[q] < 0 ? ym : y), q);
+            if constexpr (ROWS && EY[q] != 0)
+                R = row_rsrc(nxt, cls<SIDE>(q) == 1 ? t + 1 : (cls<SIDE>(q) == 2 ? t - 1 : t), EY[q] > 0 ? yp : ym);
             const unsigned vo = EX[q] > 0 ? vsp : (EX[q] < 0 ? vsm : vs0);
             if constexpr (NPL == 1) {
                 buf_store<0>(R, vo, so, nxt, g[0][q]);
@@ -442,9 +453,17 @@ static void band2_launch(hipStream_t s, const Batch<LatArgs> &P, bool ds) {
     else hipLaunchKernelGGL((k_band2<S, TILE, false>), g, b, 0, s, P);
 }
 
+template <class S>
+static void band2_launch(hipStream_t s, const Batch<LatArgs> &P, bool ds, int tile) {
+    if (tile == B2_HUGE) band2_launch<S, B2_HUGE>(s, P, ds);
+    else if (sizeof(S) == 2 || tile == B2_LARGE) band2_launch<S, B2_LARGE>(s, P, ds);
+    else if constexpr (sizeof(S) != 2) band2_launch<S, B2_SMALL>(s, P, ds);
+}
+
 hipError_t launch_band2(hipStream_t s, const LatArgs *bands, int prec, int tile, const int *halt) {
     const int elem = prec == DNSG_PREC_FP64 ? 8 : (prec == DNSG_PREC_FP32 ? 4 : 2);
-    if (tile != B2_LARGE && (tile != B2_SMALL || elem == 2)) return hipErrorInvalidValue;
+    if (tile == B2_OFF || (tile == B2_SMALL && elem == 2) || (tile != B2_HUGE && !buf_fits(bands[0].nx, bands[0].ny, elem)))
+        return hipErrorInvalidValue;
     Batch<LatArgs> P;
     P.halt = halt;
     P.n = 2;
@@ -455,16 +474,10 @@ hipError_t launch_band2(hipStream_t s, const LatArgs *bands, int prec, int tile,
         if (i < 2) blocks += band2_tiles(bands[i].nx, bands[i].ny, elem, tile);
     }
     P.first[BATCH_MAX] = blocks;
-    const bool ds = bands[0].dsum != nullptr || bands[1].dsum != nullptr, small = tile == B2_SMALL;
-    if (prec == DNSG_PREC_FP64) {
-        if (small) band2_launch<double, B2_SMALL>(s, P, ds);
-        else band2_launch<double, B2_LARGE>(s, P, ds);
-    } else if (prec == DNSG_PREC_FP32) {
-        if (small) band2_launch<float, B2_SMALL>(s, P, ds);
-        else band2_launch<float, B2_LARGE>(s, P, ds);
-    } else {
-        band2_launch<__half, B2_LARGE>(s, P, ds);
-    }
+    const bool ds = bands[0].dsum != nullptr || bands[1].dsum != nullptr;
+    if (prec == DNSG_PREC_FP64) band2_launch<double>(s, P, ds, tile);
+    else if (prec == DNSG_PREC_FP32) band2_launch<float>(s, P, ds, tile);
+    else band2_launch<__half>(s, P, ds, tile);
     return hipGetLastError();
 }
 

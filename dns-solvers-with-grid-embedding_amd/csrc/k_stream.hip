@@ -105,29 +105,45 @@ __device__ __forceinline__ void cs_scatter(const LatArgs &L, const S *__restrict
 // positions of the target row: whole cache lines, written once.  Each thread
 // stores, at its own x, the value arriving there from x - e_x; the set of writes
 // is exactly the scatter form's.
-// The three layers a row's values go to, as buffer resources, and the scalar offsets of
-// their rows y - 1, y, y + 1 and of a direction's line: formed once per workgroup, so a
-// store costs one scalar add.
+// The nine rows (y + e_y, z + e_z) that a row's values go to, each a buffer resource of its
+// own, so that layers of any size can be addressed: what is kept is the addresses of the
+// three layers and the row offsets, uniform over the workgroup.
 template <class S>
 struct RowTargets {
-    Rsrc lo, mid, hi;
-    unsigned ym, yc, yp, line;
+    const char *lo, *mid, *hi;
+    size_t ym, yc, yp;
+    unsigned line, row;
     __device__ __forceinline__ RowTargets(const LatArgs &L, const S *nxt, int y, int z) {
         line = __builtin_amdgcn_readfirstlane(L.nx * (int)sizeof(S));
         y = __builtin_amdgcn_readfirstlane(y);
-        const unsigned row = Q * line, bytes = row * (unsigned)L.ny;
+        row = Q * line;
+        const size_t bytes = (size_t)row * L.ny;
+        mid = reinterpret_cast<const char *>(nxt) + z * bytes;
+        lo = mid - bytes;  // beyond an end: takes no stores
+        hi = mid + bytes;
+        ym = (size_t)row * (y == 0 ? L.ny - 1 : y - 1);
+        yc = (size_t)row * y;
+        yp = (size_t)row * (y == L.ny - 1 ? 0 : y + 1);
+    }
+    template <int ey, int ez>
+    __device__ __forceinline__ Rsrc at() const {
+        return buf_rsrc((ez < 0 ? lo : (ez > 0 ? hi : mid)) + (ey < 0 ? ym : (ey > 0 ? yp : yc)), row);
+    }
+};
+
+// The three layers a layer's values go to, as buffer resources (layers below 2 GiB)
+template <class S>
+struct LayerTargets {
+    Rsrc lo, mid, hi;
+    __device__ __forceinline__ LayerTargets(const LatArgs &L, const S *nxt, int z) {
+        const unsigned bytes = Q * (unsigned)L.nx * sizeof(S) * (unsigned)L.ny;
         const char *m = reinterpret_cast<const char *>(nxt) + (size_t)z * bytes;
         lo = buf_rsrc(z > 0 ? m - bytes : m, bytes);  // the layer beyond an end takes no stores
         mid = buf_rsrc(m, bytes);
         hi = buf_rsrc(z < L.nz - 1 ? m + bytes : m, bytes);
-        ym = row * (unsigned)(y == 0 ? L.ny - 1 : y - 1);
-        yc = row * (unsigned)y;
-        yp = row * (unsigned)(y == L.ny - 1 ? 0 : y + 1);
     }
     template <int ez>
     __device__ __forceinline__ Rsrc layer() const { return ez < 0 ? lo : (ez > 0 ? hi : mid); }
-    template <int ey>
-    __device__ __forceinline__ unsigned off(int q) const { return (ey < 0 ? ym : (ey > 0 ? yp : yc)) + q * line; }
 };
 
 // Flat form: the workgroup takes CS_THREADS consecutive nodes of layer z, from node n0 on,
@@ -144,7 +160,7 @@ __device__ __forceinline__ void cs_flat(const LatArgs &L, const S *__restrict__ 
     const int y = (int)(id / (unsigned)nx), x = (int)id - y * nx;
     constexpr unsigned ES = sizeof(S);
     const unsigned line = __builtin_amdgcn_readfirstlane(nx * (int)ES), row = Q * line;
-    const RowTargets<S> in(L, lat, 0, z), to(L, nxt, 0, z);
+    const LayerTargets<S> in(L, lat, z), to(L, nxt, z);
     T f[Q];
     unroll<0, Q>([&](auto qc) {
         constexpr int q = decltype(qc)::value;
@@ -281,7 +297,7 @@ __device__ __forceinline__ void cs_aligned_chunk(const LatArgs &L, const S *__re
         }
         const int zt = z + EZ[q];
         if ((zt == 0 && L.skip_lo) || (zt == nz - 1 && L.skip_hi)) return;
-        buf_store<NT>(to.template layer<EZ[q]>(), vx, to.template off<EY[q]>(q), nxt, v);
+        buf_store<NT>(to.template at<EY[q], EZ[q]>(), vx, q * lb, nxt, v);
     });
     if constexpr (DS) dst.into(rs, L, z);
 }
@@ -402,7 +418,7 @@ __device__ __forceinline__ void cs_paired_chunk(const LatArgs &L, const S *__res
         }
         const int zt = z + EZ[q];
         if ((zt == 0 && L.skip_lo) || (zt == nz - 1 && L.skip_hi)) return;
-        buf_store_pair<2>(to.template layer<EZ[q]>(), vx, to.template off<EY[q]>(q), nxt, va, vb);
+        buf_store_pair<2>(to.template at<EY[q], EZ[q]>(), vx, q * lb, nxt, va, vb);
     });
     if constexpr (DS) dst.into(rs, L, z);
 }

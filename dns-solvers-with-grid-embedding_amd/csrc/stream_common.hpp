@@ -24,8 +24,8 @@ __device__ __forceinline__ PreSums<float> collide_any(float *f, float G, float o
 // direction offset are scalars, so a lane holds one 32-bit offset for all 19 directions
 // (as 64-bit addresses, 19 loads or stores in flight take 38 VGPRs), and a lane that
 // must not store takes the offset DROP, which lies past every resource and is dropped
-// by the resource's bounds check, so that stores need no branches.  Layers must be
-// below 2 GiB (buf_fits).
+// by the resource's bounds check, so that stores need no branches.  A resource, a row or
+// a layer, must be below 2 GiB.
 constexpr unsigned DROP = 0x80000000u;
 typedef __amdgpu_buffer_rsrc_t Rsrc;
 typedef unsigned u2v __attribute__((ext_vector_type(2)));

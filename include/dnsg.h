@@ -271,13 +271,13 @@ int dnsg_kernel_times(dnsg_t *h, int n, double *ms);
  * (the default at gratio 2 in FP64 and FP32 where the lattice is large enough for it to
  * be the faster path), else 1.  Read from the environment at dnsg_create (no counterpart
  * in the reference; every choice gives the same state under constant force, and the same
- * to the order of the reductions' sums under the flux controller): DNSG_BAND2=1 / 2 / 0
- * takes the one-pass band kernel with large tiles / with small ones (FP16: large) / not at
- * all at gratio 2 (layers of 2 GiB or more never take it); DNSG_CS_PAIRED=0 keeps every
- * collide-stream launch in its one-node form (by default FP32 / FP16 rows of a multiple of
- * 512 nodes take two nodes per thread); DNSG_CS_WIDE=1 / 2 / 3 takes the coarse grid / the
- * bands / both through the form that layers of 2 GiB or more always take (the bands then
- * one launch per substep). */
+ * to the order of the reductions' sums under the flux controller): DNSG_BAND2=1 / 2 / 3 / 0
+ * takes the one-pass band kernel with large tiles / with small ones (FP16: large) / with
+ * large ones in the form for layers of 2 GiB and more / not at all at gratio 2;
+ * DNSG_CS_PAIRED=0 keeps every collide-stream launch in its one-node form (by default FP32
+ * / FP16 rows of a multiple of 512 nodes take two nodes per thread); DNSG_CS_WIDE=1 / 2 / 3
+ * takes the coarse grid / the bands / both through the form for layers of 2 GiB and more
+ * whose rows are no whole chunks (the bands then one launch per substep). */
 int dnsg_band_launch_substeps(const dnsg_t *h, int *substeps);
 
 /* Gives back the device memory that the calls writing results out (budget, spectra,
