@@ -84,8 +84,8 @@ constexpr int RED_W = 3;
 // threads per collide-stream workgroup and chunks of them per lattice row
 constexpr int CS_THREADS = 256;
 __host__ __device__ __forceinline__ int cs_chunks(int nx) { return (nx + CS_THREADS - 1) / CS_THREADS; }
-// a layer can be addressed with 31-bit byte offsets (the flat form; the others' resources
-// are single rows)
+// a layer can be addressed with 31-bit byte offsets (the flat form and, below 2 GiB, FP16
+// pairs; the others' resources are single rows)
 __host__ __device__ __forceinline__ bool buf_fits(int nx, int ny, int elem) {
     return (size_t)nx * ny * 19 * elem < ((size_t)1 << 31);
 }

@@ -129,6 +129,8 @@ struct RowTargets {
     __device__ __forceinline__ Rsrc at() const {
         return buf_rsrc((ez < 0 ? lo : (ez > 0 ? hi : mid)) + (ey < 0 ? ym : (ey > 0 ? yp : yc)), row);
     }
+    template <int ey>
+    __device__ __forceinline__ unsigned off(unsigned q_line) const { return q_line; }
 };
 
 // The three layers a layer's values go to, as buffer resources (layers below 2 GiB)
@@ -144,6 +146,26 @@ struct LayerTargets {
     }
     template <int ez>
     __device__ __forceinline__ Rsrc layer() const { return ez < 0 ? lo : (ez > 0 ? hi : mid); }
+};
+
+// The nine rows as offsets into the three layers' resources (layers below 2 GiB): 46 scalar
+// instructions fewer a wave than a resource for each row.  It shows where instructions bound
+// the launch, in FP16: a Re_tau=180 step 880 us against 886 (flux control 966 against 975).
+// FP64 and FP32 take the rows in all sizes (no difference).
+template <class S>
+struct LayerRowTargets : LayerTargets<S> {
+    unsigned ym, yc, yp;
+    __device__ __forceinline__ LayerRowTargets(const LatArgs &L, const S *nxt, int y, int z) : LayerTargets<S>(L, nxt, z) {
+        y = __builtin_amdgcn_readfirstlane(y);
+        const unsigned row = Q * __builtin_amdgcn_readfirstlane(L.nx * (int)sizeof(S));
+        ym = row * (unsigned)(y == 0 ? L.ny - 1 : y - 1);
+        yc = row * (unsigned)y;
+        yp = row * (unsigned)(y == L.ny - 1 ? 0 : y + 1);
+    }
+    template <int ey, int ez>
+    __device__ __forceinline__ Rsrc at() const { return this->template layer<ez>(); }
+    template <int ey>
+    __device__ __forceinline__ unsigned off(unsigned q_line) const { return (ey < 0 ? ym : (ey > 0 ? yp : yc)) + q_line; }
 };
 
 // Flat form: the workgroup takes CS_THREADS consecutive nodes of layer z, from node n0 on,
@@ -297,7 +319,7 @@ __device__ __forceinline__ void cs_aligned_chunk(const LatArgs &L, const S *__re
         }
         const int zt = z + EZ[q];
         if ((zt == 0 && L.skip_lo) || (zt == nz - 1 && L.skip_hi)) return;
-        buf_store<NT>(to.template at<EY[q], EZ[q]>(), vx, q * lb, nxt, v);
+        buf_store<NT>(to.template at<EY[q], EZ[q]>(), vx, to.template off<EY[q]>(q * lb), nxt, v);
     });
     if constexpr (DS) dst.into(rs, L, z);
 }
@@ -314,7 +336,7 @@ __device__ __forceinline__ void cs_aligned_chunk(const LatArgs &L, const S *__re
 // Paired stores are non-temporal, like the aligned form's.  Measured on the
 // Re_tau=180 lattices: FP32 coarse 0.952 -> 0.938 ms and band 0.479 -> 0.472 ms; FP16
 // within 1%.
-template <class S, bool DS, class T>
+template <class S, bool DS, template <class> class Targets, class T>
 __device__ __forceinline__ void cs_paired_chunk(const LatArgs &L, const S *__restrict__ cur, S *__restrict__ nxt,
                                                 int row, int x0, T G, T om, bool red, RowSums &rs) {
     constexpr int NW = CS_THREADS / 64, NP = 2 * CS_THREADS;
@@ -364,7 +386,7 @@ __device__ __forceinline__ void cs_paired_chunk(const LatArgs &L, const S *__res
     });
     __syncthreads();
     DestSums dst;
-    const RowTargets<S> to(L, nxt, y, z);
+    const Targets<S> to(L, nxt, y, z);
     unroll<0, Q>([&](auto qc) {
         constexpr int q = decltype(qc)::value;
         // the values arriving at x and x + 1, and the sources they leave from
@@ -418,7 +440,7 @@ __device__ __forceinline__ void cs_paired_chunk(const LatArgs &L, const S *__res
         }
         const int zt = z + EZ[q];
         if ((zt == 0 && L.skip_lo) || (zt == nz - 1 && L.skip_hi)) return;
-        buf_store_pair<2>(to.template at<EY[q], EZ[q]>(), vx, q * lb, nxt, va, vb);
+        buf_store_pair<2>(to.template at<EY[q], EZ[q]>(), vx, to.template off<EY[q]>(q * lb), nxt, va, vb);
     });
     if constexpr (DS) dst.into(rs, L, z);
 }
@@ -459,8 +481,8 @@ __device__ __forceinline__ void write_block_sums(const LatArgs &L, const RowSums
     }
 }
 
-template <class S, bool DS>
-__global__ __launch_bounds__(CS_THREADS) void k_collide_stream(Batch<LatArgs> P) {
+template <class S, bool DS, template <class> class PairedTargets>
+__device__ __forceinline__ void collide_stream(const Batch<LatArgs> &P) {
     using T = typename ComputeOf<S>::T;
     if (halted(P.halt)) return;
     const int bg = xcd_remap(blockIdx.x, gridDim.x);
@@ -489,11 +511,23 @@ __global__ __launch_bounds__(CS_THREADS) void k_collide_stream(Batch<LatArgs> P)
         // CS_PAIRED, two chunks of one row per workgroup, two nodes per thread; the
         // workgroup's halves are the two chunks' partials
         const int cpr = cs_chunks(nx), ppr = cpr / 2, row = b / ppr, pc = b % ppr;
-        cs_paired_chunk<S, DS, T>(L, base + (size_t)row * Q * nx, nxt, row, pc * 2 * CS_THREADS, G, om, red, rs);
+        cs_paired_chunk<S, DS, PairedTargets>(L, base + (size_t)row * Q * nx, nxt, row, pc * 2 * CS_THREADS, G, om, red,
+                                              rs);
         e = (size_t)row * cpr + 2 * pc;
         parts = 2;
     }
     if (red || (DS && L.dsum)) write_block_sums<DS>(L, rs, e, parts);  // uniform per workgroup
+}
+
+template <class S, bool DS>
+__global__ __launch_bounds__(CS_THREADS) void k_collide_stream(Batch<LatArgs> P) {
+    if constexpr (sizeof(S) == 2) collide_stream<S, DS, LayerRowTargets>(P);
+    else collide_stream<S, DS, RowTargets>(P);
+}
+// FP16 where a paired lattice has layers of 2 GiB and more
+template <bool DS>
+__global__ __launch_bounds__(CS_THREADS) void k_collide_half_rows(Batch<LatArgs> P) {
+    collide_stream<__half, DS, RowTargets>(P);
 }
 
 // CS_WIDE: one (row, chunk) of one lattice per workgroup in the scatter form
@@ -521,7 +555,7 @@ hipError_t launch_collide_stream(hipStream_t s, const LatArgs *lats, int nlat, i
         Batch<LatArgs> P;
         P.halt = halt;
         P.n = 0;
-        bool ds = false;
+        bool ds = false, rows = false;
         int blocks = 0;
         for (; i < nlat && P.n < BATCH_MAX; i++) {
             const LatArgs &L = lats[i];
@@ -534,6 +568,7 @@ hipError_t launch_collide_stream(hipStream_t s, const LatArgs *lats, int nlat, i
                 continue;
             }
             ds = ds || L.dsum != nullptr;
+            rows = rows || (L.form == CS_PAIRED && !buf_fits(L.nx, L.ny, sizeof(__half)));
             P.it[P.n] = L;
             P.first[P.n++] = blocks;
             blocks += L.nz * cs_blocks(L.form, L.nx, L.ny);
@@ -547,6 +582,9 @@ hipError_t launch_collide_stream(hipStream_t s, const LatArgs *lats, int nlat, i
         } else if (prec == DNSG_PREC_FP32) {
             if (ds) hipLaunchKernelGGL((k_collide_stream<float, true>), g, b, 0, s, P);
             else hipLaunchKernelGGL((k_collide_stream<float, false>), g, b, 0, s, P);
+        } else if (rows) {
+            if (ds) hipLaunchKernelGGL(k_collide_half_rows<true>, g, b, 0, s, P);
+            else hipLaunchKernelGGL(k_collide_half_rows<false>, g, b, 0, s, P);
         } else {
             if (ds) hipLaunchKernelGGL((k_collide_stream<__half, true>), g, b, 0, s, P);
             else hipLaunchKernelGGL((k_collide_stream<__half, false>), g, b, 0, s, P);

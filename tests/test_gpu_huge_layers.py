@@ -1,8 +1,8 @@
 """Lattice layers of 2 GiB and more.  The two-substep band kernel's form for them at small
 sizes (DNSG_BAND2=3) against one launch per substep, as for its other tiles: bit for bit
 under a constant force, within the tier's rounding under the flux controller.  And the real
-ones, bands of 4096 x 3456 nodes: each path the same statistics, bit for bit (they are sums
-of the state in one fixed order); rows of no whole chunks by a start without noise, whose
+ones, bands of 4096 x 3456 nodes (FP16 8192 x 6912): each path the same statistics, bit for
+bit (they are sums of the state in one fixed order); rows of no whole chunks by a start without noise, whose
 layers must stay uniform and equal those of a small channel."""
 import numpy as np
 import pytest
@@ -45,8 +45,8 @@ def test_flux_control(prec, monkeypatch):
     assert np.max(np.abs(ra["force"] - rb["force"])) <= tol * 0.05
 
 
-def large(x, y, gr, zds, noise, **kw):
-    s = dnsg.Solver(dnsg.make_params(xdv=x, ydv=y, zdv=7, gratio=gr, zds=zds, tau_c=0.53, ub=0.05, force_mode="const",
+def large(x, y, gr, zds, noise, force="const", **kw):
+    s = dnsg.Solver(dnsg.make_params(xdv=x, ydv=y, zdv=7, gratio=gr, zds=zds, tau_c=0.53, ub=0.05, force_mode=force,
                                      g_const=2e-5, CFL=1.0, init_kind="laminar_noise", seed=5, u_max=0.05, noise=noise, **kw))
     s.init_state()
     rec = s.step(2)
@@ -68,6 +68,24 @@ def test_bands_of_2_gib(monkeypatch):
     assert np.isfinite(a).all() and np.array_equal(a, b)
     for f in ("momentum", "density", "str_up", "str_down"):
         assert np.allclose(ra[f], rb[f], rtol=1e-9, atol=0), f
+
+
+@pytest.mark.parametrize("force", ["const", "flux"])
+def test_pairs_in_fp16_bands_of_2_gib(force, monkeypatch):
+    """FP16 bands of 8192 x 6912 (2.15 GB a layer): two nodes a thread, and one"""
+    got = []
+    for pair in "10":
+        monkeypatch.setenv("DNSG_CS_PAIRED", pair)
+        st, sub, rec = large(4096, 3456, 2, 4, 0.1, precision="fp16", force=force)
+        assert sub == 1
+        got.append((st, rec))
+        print("FP16 bands of 2 GiB: done", force, pair, flush=True)
+    (a, ra), (b, rb) = got
+    assert np.isfinite(a).all()
+    if force == "const":
+        assert np.array_equal(a, b)
+    else:
+        assert relmax(a, b) <= 1e-2 and np.max(np.abs(ra["force"] - rb["force"])) <= 1e-2 * 0.05
 
 
 def test_rows_of_no_whole_chunks():
