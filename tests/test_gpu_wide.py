@@ -1,5 +1,5 @@
-"""The collide-stream form of layers of 2 GiB and more (one chunk of a row per workgroup,
-64-bit addresses), which DNSG_CS_WIDE selects at any size: for the coarse grid, the bands or
+"""The collide-stream form that rows of no whole chunks take in layers of 2 GiB and more (one
+chunk of a row per workgroup, 64-bit addresses), which DNSG_CS_WIDE selects at any size: for the coarse grid, the bands or
 both, so that it also shares a step with the other forms.
 
 FP64 against the oracle: bit for bit under a constant force, 1e-12 of the largest value
